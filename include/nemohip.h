@@ -80,13 +80,11 @@ nh_status nh_context_create(const nh_model *model, int device,
 void nh_context_destroy(nh_context *ctx);
 int64_t nh_context_dim(const nh_context *ctx); /* N = n_atoms * nb */
 
-/* Kernel variants (chosen by measured throughput; the same products to
- * rounding: the compiler contracts the block's multiply-adds differently
- * in the two).  NH_SET_HV_STAGED: 1 stages the neighbours'
- * vector entries in LDS (stored-block layout: per workgroup; SK layout: the
- * four lanes of an atom load each neighbour's entries together), 0 reads
- * them from the caches by every lane, -1 (default) picks by layout (SK:
- * staged, stored blocks: direct). */
+/* Kernel variants (the same products to rounding).  NH_SET_HV_STAGED, of
+ * the stored-block layout: 1 stages the neighbours' vector entries in LDS,
+ * 0 reads them from the caches by every lane, -1 (default) direct.  SK and
+ * matrix-free products always stage; there 0 only makes FP32 Lanczos runs
+ * keep FP64 vectors (as NH_SET_LZ_VECTORS = 0 does). */
 enum { NH_SET_HV_STAGED = 1 };
 /* NH_SET_RING_STEPS: Lanczos steps between eigenvector accumulations in the
  * eigenvector pass (ring length; 8, 16, 32, 64 or 128), or 0 (default): 128,
@@ -94,28 +92,20 @@ enum { NH_SET_HV_STAGED = 1 };
  * The eigenvectors agree to rounding whatever the length. */
 enum { NH_SET_RING_STEPS = 2 };
 /* NH_SET_BLOCK_HV: products of several vectors (block H·V): -1 (default)
- * the matrix-core kernel for the row-owner block layout and 0 for the SK
+ * the matrix-core kernel for the row-owner block layout and 1 for the SK
  * and matrix-free layouts (the fastest measured there), 0 one column per
- * grid row, 1 all columns in one launch with the bond records read once
- * (SK and matrix-free), 2 the matrix-core kernel (FP32 SK or block
- * layouts, 8 columns). */
+ * grid row, 1 all columns in one launch with H read once (SK and
+ * matrix-free), 2 the matrix-core kernel (FP32 SK or block layouts, 8
+ * columns). */
 enum { NH_SET_BLOCK_HV = 3 };
-/* NH_SET_SK_ROLES: workgroups of the SK and matrix-free products: 1 holds
- * cation-role and anion-role atoms of the same cells together (both rows of
- * a bond read its record in one workgroup), 0 one role per workgroup (the
- * two roles of the same cells back to back on one XCD), -1 the default
- * (1 with FP64 products, 0 with FP32: the faster of the two measured).
- * The products are identical either way. */
+/* NH_SET_SK_ROLES, NH_SET_SK_LANES: workgroup mappings of earlier SK and
+ * matrix-free products; accepted and without effect (one mapping is the
+ * fastest in every case measured). */
 enum { NH_SET_SK_ROLES = 4 };
-/* NH_SET_SK_LANES: lanes per atom of the SK and matrix-free Lanczos
- * products of 20-band models: 4 (a lane per bond, both spin blocks) or 8
- * (a lane per bond and spin block: half the registers per lane); -1 the
- * default (8 for matrix-free FP32 products, 4 otherwise: the faster of the
- * two measured). */
 enum { NH_SET_SK_LANES = 5 };
 /* NH_SET_LZ_VECTORS: storage of the Lanczos vectors r_k of a Lanczos run
- * with FP32 SK or matrix-free products: 0 FP64 (with an FP32 copy for the
- * products' gathers), 1 FP32: the step runs in Paige's order, u_k = H q_k
+ * with FP32 SK or matrix-free products: 0 FP64 (the product and the update
+ * in two launches), 1 FP32: the step runs in Paige's order, u_k = H q_k
  * - beta_k q_{k-1} computed in FP64 and rounded once to FP32, r_{k+1} =
  * u_k - (alpha_k / beta_k) r_k as two FP32 fmas with the coefficient split
  * into two FP32 parts, and the product of step k
@@ -124,7 +114,11 @@ enum { NH_SET_SK_LANES = 5 };
  * FP64); -1 the default (1 where the products use the
  * LDS gather: measured faster, with the same number of steps).  Either
  * way the eigenvector pass retraces the eigenvalue pass; other layouts
- * and FP64 products always keep FP64 vectors. */
+ * and FP64 products always keep FP64 vectors.  FP64 SK and matrix-free
+ * products run the one-launch step too, with FP64 u and r; there
+ * beta_{k+1}^2 = |u_k|^2 - 2 alpha_k^2 + alpha_k^2 |q_k|^2, and a run in
+ * which it falls below 1e-4 |u_k|^2 (a start in an almost invariant
+ * subspace) is repeated with |r_{k+1}|^2 summed directly. */
 enum { NH_SET_LZ_VECTORS = 6 };
 nh_status nh_context_set(nh_context *ctx, int what, int value);
 

@@ -146,7 +146,9 @@ static void destroy(nh_context *c) {
   }
   (void)hipSetDevice(c->device);
   void *ptrs[] = {c->parmat, c->strnmat, c->species, c->is_cation, c->nbr,
-                  c->bond_q, c->disp, c->phi, c->cations, c->anions, c->bond_of,
+                  c->bond_q, c->disp, c->phi, c->cations, c->bond_of, c->blk_own,
+                  c->blk_local, c->blk_halo, c->blk_bonds, c->mf_geo, c->mf_q,
+                  c->mf_pair, c->mf_ends,
                   c->rev_slot, c->onsite, c->blocks64, c->blocks32,
                   c->onsite32, c->sk64, c->sk32, c->corr, c->red, c->xbuf,
                   c->ybuf};
@@ -159,15 +161,24 @@ static void destroy(nh_context *c) {
   delete c;
 }
 
-// Orders an atom list by 32x32x32-cell bricks (bricks in z, y, x order,
-// cells and atoms in their original order inside a brick).  The SK kernels give
-// consecutive workgroups consecutive list entries and each XCD a contiguous
-// part of the list, so a brick's atoms and most of their neighbours are in
-// flight together and the neighbours' vector entries are reused from the
-// XCD's L2 instead of being fetched again when the next plane of cells is
-// processed.  Ideal positions (units a/4) come from the ideal bond vectors
-// by a walk over the bond graph.
-static void brick_order(const nh_model *m, std::vector<int32_t> &list) {
+// Blocks of atoms for the SK and matrix-free products (nh_hv_sk.h): the atoms
+// are ordered by bricks of 16 cells and inside them by cubes of 2 x 2 x 2
+// cells (ideal positions, from the ideal bond vectors by a walk over the bond
+// graph), and cut into blocks within the kernels' capacities.  A cube starts a
+// new block unless it fits into the open one whole, so the blocks of a
+// crystal coincide with its cubes (64 atoms, at most 57 halo atoms and 170
+// bonds) and only thin rests of cubes at the surface are put together.
+// Bond numbers are 4 (number of the cation in `cations`) + slot, the cations
+// in block order.
+struct BlockTables {
+  std::vector<int32_t> cations, bond_of;  // bond_of [A][4], -1 for none
+  std::vector<int32_t> own, halo, bonds;  // [blocks][64], [64], [192]; -1 pads
+  std::vector<uint8_t> local;  // [blocks][64][2][4]: place of x, of the record
+  int n = 0;
+};
+
+static void cube_order(const nh_model *m, std::vector<int32_t> &order,
+                       std::vector<int64_t> &cube) {
   const int A = m->n_atoms;
   std::vector<int32_t> pos((size_t)A * 3, 0);
   std::vector<char> seen(A, 0);
@@ -192,19 +203,126 @@ static void brick_order(const nh_model *m, std::vector<int32_t> &list) {
   int32_t lo[3] = {INT32_MAX, INT32_MAX, INT32_MAX};
   for (int i = 0; i < A; ++i)
     for (int d = 0; d < 3; ++d) lo[d] = std::min(lo[d], pos[(size_t)i * 3 + d]);
-  // 32 cells of 4 units (a/4).  Measured on the 786,520-atom dot (FP32 /
-  // FP64 fused Lanczos H*v): 4-cell bricks 0.241 / -, 8-cell 0.239 / 0.338,
-  // 16-cell 0.234 / 0.337, 32-cell 0.229-0.232 / 0.337-0.338, 64-cell
-  // 0.234 / 0.339 ms; octants at the medians (one per XCD) with 8-cell
-  // bricks inside 0.245 / 0.343
-  constexpr int kBrick = 128;
-  auto key = [&](int32_t i) {
-    int64_t b[3];
-    for (int d = 0; d < 3; ++d) b[d] = (pos[(size_t)i * 3 + d] - lo[d]) / kBrick;
-    return (b[2] << 42) | (b[1] << 21) | b[0];
+  // units a/4: 8 a cube, 64 a brick (8 cubes): 17 + 3 bits a direction
+  std::vector<std::pair<int64_t, int32_t>> key(A);
+  for (int i = 0; i < A; ++i) {
+    int64_t b = 0, c = 0;
+    for (int d = 2; d >= 0; --d) b = b << 17 | (((pos[(size_t)i * 3 + d] - lo[d]) >> 6) & 0x1ffff);
+    for (int d = 0; d < 3; ++d) c = c << 3 | (((pos[(size_t)i * 3 + d] - lo[d]) >> 3) & 7);
+    key[i] = {b << 9 | c, i};
+  }
+  std::sort(key.begin(), key.end());
+  order.resize(A);
+  cube.resize(A);
+  for (int i = 0; i < A; ++i) {
+    order[i] = key[i].second;
+    cube[i] = key[i].first;
+  }
+}
+
+static void build_blocks(const nh_model *m, const std::vector<int32_t> &rev, BlockTables &T) {
+  constexpr int kOwn = 64, kHalf = 32, kHalo = 64, kBonds = 176, kBondPad = 192;
+  const int A = m->n_atoms;
+  std::vector<int32_t> order;
+  std::vector<int64_t> cube;
+  cube_order(m, order, cube);
+  for (int i : order)
+    if (m->is_cation[i]) T.cations.push_back(i);
+  T.bond_of.assign((size_t)A * 4, -1);
+  for (size_t ci = 0; ci < T.cations.size(); ++ci) {
+    const int i = T.cations[ci];
+    for (int n = 0; n < 4; ++n) {
+      const int j = m->nbr[i * 4 + n];
+      if (j < 0) continue;
+      T.bond_of[(size_t)i * 4 + n] = (int32_t)(ci * 4 + n);
+      T.bond_of[(size_t)j * 4 + rev[(size_t)i * 4 + n]] = (int32_t)(ci * 4 + n);
+    }
+  }
+  // of the open block: an atom's place (own, or kOwn + halo), a bond's place
+  std::vector<int32_t> place(A, -1), bplace(T.cations.size() * 4, -1);
+  std::vector<int32_t> halo, bonds;   // members in order of arrival; a halo
+  int32_t own[kOwn];                  // atom that became an own one leaves a -1
+  int nc = 0, na = 0, nh = 0;
+  std::fill(own, own + kOwn, -1);
+  auto close = [&]() {
+    if (nc + na == 0) return;
+    int k = 0;
+    for (int32_t a : halo)
+      if (a >= 0) {
+        place[a] = kOwn + k++;
+        T.halo.push_back(a);
+      }
+    T.halo.resize((size_t)(T.n + 1) * kHalo, -1);
+    T.bonds.insert(T.bonds.end(), bonds.begin(), bonds.end());
+    T.bonds.resize((size_t)(T.n + 1) * kBondPad, -1);
+    T.own.insert(T.own.end(), own, own + kOwn);
+    const size_t l0 = T.local.size();
+    T.local.resize(l0 + kOwn * 8, 255);
+    for (int s = 0; s < kOwn; ++s) {
+      if (own[s] < 0) continue;
+      for (int n = 0; n < 4; ++n) {
+        const int j = m->nbr[(size_t)own[s] * 4 + n];
+        if (j < 0) continue;
+        T.local[l0 + s * 8 + n] = (uint8_t)place[j];
+        T.local[l0 + s * 8 + 4 + n] = (uint8_t)bplace[T.bond_of[(size_t)own[s] * 4 + n]];
+      }
+    }
+    for (int s = 0; s < kOwn; ++s)
+      if (own[s] >= 0) place[own[s]] = -1;
+    for (int32_t a : halo)
+      if (a >= 0) place[a] = -1;
+    for (int32_t q : bonds) bplace[q] = -1;
+    std::fill(own, own + kOwn, -1);
+    halo.clear();
+    bonds.clear();
+    nc = na = nh = 0;
+    ++T.n;
   };
-  std::stable_sort(list.begin(), list.end(),
-                   [&](int32_t a, int32_t b) { return key(a) < key(b); });
+  for (size_t k = 0; k < order.size(); ++k) {
+    if (k == 0 || cube[k] != cube[k - 1]) {
+      int gc = 0, ga = 0;
+      for (size_t e = k; e < order.size() && cube[e] == cube[k]; ++e)
+        ++(m->is_cation[order[e]] ? gc : ga);
+      if (nc + gc > kHalf || na + ga > kHalf) close();
+    }
+    const int i = order[k];
+    const bool cat = m->is_cation[i] != 0;
+    int dh = 0, db = 0;
+    auto count = [&]() {
+      dh = place[i] >= kOwn ? -1 : 0;
+      db = 0;
+      for (int n = 0; n < 4; ++n) {
+        const int j = m->nbr[(size_t)i * 4 + n];
+        if (j < 0) continue;
+        if (place[j] < 0) ++dh;
+        if (bplace[T.bond_of[(size_t)i * 4 + n]] < 0) ++db;
+      }
+    };
+    count();
+    if ((cat ? nc : na) == kHalf || nh + dh > kHalo || (int)bonds.size() + db > kBonds) {
+      close();
+      count();
+    }
+    if (place[i] >= kOwn) halo[place[i] - kOwn] = -1;
+    const int s = cat ? nc++ : kHalf + na++;
+    own[s] = i;
+    place[i] = s;
+    for (int n = 0; n < 4; ++n) {
+      const int j = m->nbr[(size_t)i * 4 + n];
+      if (j < 0) continue;
+      if (place[j] < 0) {
+        place[j] = kOwn + (int32_t)halo.size();
+        halo.push_back(j);
+      }
+      const int q = T.bond_of[(size_t)i * 4 + n];
+      if (bplace[q] < 0) {
+        bplace[q] = (int32_t)bonds.size();
+        bonds.push_back(q);
+      }
+    }
+    nh += dh;
+  }
+  close();
 }
 
 static nh_status create(const nh_model *m, int device, nh_context **out) {
@@ -216,8 +334,8 @@ static nh_status create(const nh_model *m, int device, nh_context **out) {
            NH_ERR_ARG, "missing model array");
   const int A = m->n_atoms, S = m->n_species;
   NH_CHECK((int64_t)A * m->nb < ((int64_t)1 << 40), NH_ERR_ARG, "too large");
-  std::vector<int32_t> cations, anions, bond_of((size_t)A * 4, -1),
-      rev((size_t)A * 4, -1);
+  std::vector<int32_t> rev((size_t)A * 4, -1);
+  int n_cations = 0;
   for (int i = 0; i < A; ++i) {
     NH_CHECK(m->species[i] >= 0 && m->species[i] < S, NH_ERR_ARG,
              "species[%d] out of range", i);
@@ -239,20 +357,10 @@ static nh_status create(const nh_model *m, int device, nh_context **out) {
     }
     NH_CHECK(present > 0, NH_ERR_ARG, "atom %d has no neighbours", i);
   }
-  for (int i = 0; i < A; ++i)
-    (m->is_cation[i] ? cations : anions).push_back(i);
-  brick_order(m, cations);
-  brick_order(m, anions);
-  for (size_t ci = 0; ci < cations.size(); ++ci) {
-    const int i = cations[ci];
-    for (int n = 0; n < 4; ++n) {
-      const int j = m->nbr[i * 4 + n];
-      if (j < 0) continue;
-      bond_of[i * 4 + n] = (int32_t)(ci * 4 + n);
-      bond_of[j * 4 + rev[i * 4 + n]] = (int32_t)(ci * 4 + n);
-    }
-  }
-  NH_CHECK(!cations.empty(), NH_ERR_ARG, "no cation-role atoms");
+  for (int i = 0; i < A; ++i) n_cations += m->is_cation[i] != 0;
+  NH_CHECK(n_cations > 0, NH_ERR_ARG, "no cation-role atoms");
+  BlockTables blocks;
+  build_blocks(m, rev, blocks);
 
   NH_HIP(hipSetDevice(device));
   NH_TRY(init_noalloc_scratch(device));
@@ -261,8 +369,8 @@ static nh_status create(const nh_model *m, int device, nh_context **out) {
   c->nb = m->nb;
   c->n_atoms = A;
   c->n_species = S;
-  c->n_cations = (int)cations.size();
-  c->n_anions = (int)anions.size();
+  c->n_cations = n_cations;
+  c->n_blocks = blocks.n;
   c->n = (int64_t)A * m->nb;
   for (int k = 0; k < 3; ++k) c->lattice[k] = m->lattice[k];
   c->passivate = m->passivate;
@@ -278,9 +386,12 @@ static nh_status create(const nh_model *m, int device, nh_context **out) {
   UP(bond_q, m->bond_q, (size_t)A * 12);
   UP(disp, m->disp, (size_t)A * 3);
   if (m->phi) UP(phi, m->phi, A);
-  UP(cations, cations.data(), cations.size());
-  if (!anions.empty()) UP(anions, anions.data(), anions.size());
-  UP(bond_of, bond_of.data(), (size_t)A * 4);
+  UP(cations, blocks.cations.data(), blocks.cations.size());
+  UP(bond_of, blocks.bond_of.data(), (size_t)A * 4);
+  UP(blk_own, blocks.own.data(), blocks.own.size());
+  UP(blk_local, reinterpret_cast<const uint2 *>(blocks.local.data()), blocks.local.size() / 8);
+  UP(blk_halo, blocks.halo.data(), blocks.halo.size());
+  UP(blk_bonds, blocks.bonds.data(), blocks.bonds.size());
   UP(rev_slot, rev.data(), (size_t)A * 4);
 #undef UP
   if (st == NH_OK) {
@@ -326,7 +437,6 @@ nh_status nh_context_set(nh_context *ctx, int what, int value) {
     case NH_SET_SK_LANES:
       NH_CHECK(value == -1 || value == 4 || value == 8, NH_ERR_ARG,
                "NH_SET_SK_LANES: value %d not -1, 4 or 8", value);
-      ctx->sk_lanes = value;
       return NH_OK;
     case NH_SET_LZ_VECTORS:
       NH_CHECK(value >= -1 && value <= 1, NH_ERR_ARG,
@@ -336,7 +446,6 @@ nh_status nh_context_set(nh_context *ctx, int what, int value) {
     case NH_SET_SK_ROLES:
       NH_CHECK(value >= -1 && value <= 1, NH_ERR_ARG,
                "NH_SET_SK_ROLES: value %d not in -1..1", value);
-      ctx->sk_roles = value;
       return NH_OK;
     case NH_SET_BLOCK_HV:
       NH_CHECK(value >= -1 && value <= 2, NH_ERR_ARG,

@@ -13,7 +13,7 @@
 // h3d_diag, mb_ham_spds_micro.c:1453-1505;
 // h3d_diag_dangling_bond_shift_zincblende, mb_ham_spds_micro.c:1910-2152).
 #include "nh_internal.h"
-#include "nh_sk.h"
+#include "nh_hv_sk.h"
 
 namespace nh {
 namespace {
@@ -73,11 +73,10 @@ __global__ void k_bond(int n_cations, int S, const int32_t *__restrict__ cations
   }
   if (sk) {
     double *rec = sk + (size_t)t * kSkStride;
-    rec[0] = g.l;
-    rec[1] = g.m;
-    rec[2] = g.n;
+    double k[kSkStride];
+    sk_record(g.l, g.m, g.n, v, k);
 #pragma unroll
-    for (int k = 0; k < 21; ++k) rec[3 + k] = v[k];
+    for (int i = 0; i < kSkStride; ++i) rec[i] = k[i];
   }
   // Boykin terms ((V0^2 - V^2) c_strain / (E_a + E_c)) * c_pair
   // (mb_ham_spds_VoffdEdiag_constructors.h; the pVpE_* macros are not
@@ -222,6 +221,18 @@ __global__ void k_mf_geo(int A, const int32_t *__restrict__ species,
   }
 }
 
+// The two atoms of every bond of the products' blocks: 4 cation atom + slot,
+// anion atom (-1 pads).
+__global__ void k_mf_ends(int n, const int32_t *__restrict__ bonds,
+                          const int32_t *__restrict__ cations,
+                          const int32_t *__restrict__ nbr, int2 *__restrict__ ends) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const int b = bonds[k];
+  const int e = b >= 0 ? cations[b >> 2] * 4 + (b & 3) : -1;
+  ends[k] = make_int2(e, e >= 0 ? nbr[e] : -1);
+}
+
 // Per (cation, anion) species pair: integrals 10..30, strain exponents
 // 0..14, lattice constant (the parameters k_bond reads).
 __global__ void k_mf_pair(int S, const double *__restrict__ parmat,
@@ -264,6 +275,8 @@ static void free_ham(nh_context *c) {
   (void)hipFree(c->mf_geo);
   (void)hipFree(c->mf_q);
   (void)hipFree(c->mf_pair);
+  (void)hipFree(c->mf_ends);
+  c->mf_ends = nullptr;
   c->mf_geo = nullptr;
   c->mf_q = nullptr;
   c->mf_pair = nullptr;
@@ -308,6 +321,10 @@ nh_status assemble(nh_context *c, int layout, int precision) {
     hipLaunchKernelGGL(k_mf_geo, dim3(grid_for(A, 128)), dim3(128), 0, c->stream,
                        A, c->species, c->is_cation, c->bond_q, c->disp,
                        c->mf_geo, c->mf_q);
+    const int ne = c->n_blocks * kSkBondPad;
+    NH_TRY(device_malloc(c, (void **)&c->mf_ends, (size_t)ne * sizeof(int2)));
+    hipLaunchKernelGGL(k_mf_ends, dim3(grid_for(ne, 256)), dim3(256), 0, c->stream, ne,
+                       c->blk_bonds, c->cations, c->nbr, c->mf_ends);
     hipLaunchKernelGGL(k_mf_pair, dim3(1), dim3(64 * ((S * S + 63) / 64)), 0,
                        c->stream, S, c->parmat, c->strnmat, c->mf_pair);
     NH_HIP(hipGetLastError());

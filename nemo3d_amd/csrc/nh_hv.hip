@@ -7,148 +7,65 @@ namespace nh {
 namespace {
 
 // SK-compressed and matrix-free layouts (see nh_hv_sk.h; SRC = SkSrc or
-// MfSrc); workgroup -> atoms by sk_lane_of.
-template <int NSP, typename R, bool QUAD, typename SRC>
-__global__ __launch_bounds__(kSkThreads) void k_hv_sk(
-    int nc, const int32_t *__restrict__ cations, int na,
-    const int32_t *__restrict__ anions, SkGrid grid,
-    const double *__restrict__ onsite, const SRC src,
-    const int32_t *__restrict__ nbr, double shift,
-    const double2 *__restrict__ x, double2 *__restrict__ y, int64_t ld) {
-  constexpr int NB = NSP * 10;
-  const SkLane ln = sk_lane_of(grid, blockIdx.x, threadIdx.x);
+// MfSrc): each workgroup takes block after block.  COLS: `per` columns of a
+// block one after another (its records, tables and onsite terms read once for
+// them; Hmatmult_spds_col_stored, Hmult_stored.c:2359-2474, re-reads H for
+// every column), the next column's entries requested while the current one is
+// computed; a group of columns per grid row.
+template <bool COLS, int NSP, typename R, typename SRC>
+__global__ __launch_bounds__(kSkThreads, 2) void k_hv_sk(
+    SkTable tab, const double *__restrict__ onsite, const SRC src, double shift,
+    const double2 *__restrict__ X, double2 *__restrict__ Y, int64_t ld, int ncol, int per) {
+  __shared__ SkLds<NSP, R, double2> L;
+  using S = SkX<NSP, double2>;
+  const SkThread t;
+  SkWalk w(tab);
+  if (w.b >= w.end) return;
+  const int c0 = COLS ? blockIdx.y * per : blockIdx.y, nc = COLS ? min(per, ncol - c0) : 1;
+  const double2 *x0 = X + (int64_t)c0 * ld;
+  double2 *y0 = Y + (int64_t)c0 * ld;
   // the role is uniform across the wavefront; read as a scalar, the role
   // branches below are scalar branches (one per wave)
-  const bool cat = __builtin_amdgcn_readfirstlane((int)ln.cat) != 0;
-  const int li = ln.li;
-  const int slot = threadIdx.x & 3;
-  const bool active = li < (cat ? nc : na);
-  const int atom = active ? (cat ? cations[li] : anions[li]) : 0;
-  const double2 *xc = x + (int64_t)blockIdx.y * ld;
-  double2 *yc = y + (int64_t)blockIdx.y * ld;
-  constexpr int NO = (NB + 3) / 4;
-  double own_re[NO], own_im[NO];
-  SkQuadStage<NSP, double2> *L = nullptr;
-  if constexpr (QUAD) {
-    __shared__ SkQuadStage<NSP, double2> stage;
-    L = &stage;
-  }
-  if (cat)
-    sk_bonds<NSP, R, true, double2, QUAD>(atom, slot, active, src, nbr, xc,
-                                          own_re, own_im, L);
-  else
-    sk_bonds<NSP, R, false, double2, QUAD>(atom, slot, active, src, nbr, xc,
-                                           own_re, own_im, L);
-  if constexpr (QUAD) {
-    auto &S = *reinterpret_cast<SkOwnStage<NSP> *>(L->buf);
-    const int la = threadIdx.x / 4;
-    // own entries and onsite record loaded before the barrier (the loads
-    // overlap it), staged in the freed LDS after it
-    SkOwnRegs<NSP> own;
-    if (active)
-      sk_load_own<NSP>(slot, xc + (int64_t)atom * NB,
-                       onsite + (size_t)atom * kOnsiteStride, own);
-    __syncthreads();  // every lane has read its staged neighbour entries
-    if (active) sk_store_own<NSP>(la, slot, own, S);
-    __syncthreads();
-    if (!active) return;
-#pragma unroll
-    for (int i = 0; i < NO; ++i) {
-      const int r = 4 * i + slot;
-      if (r >= NB) break;
-      double re = own_re[i], im = own_im[i];
-      onsite_row<NSP>(reinterpret_cast<const double *>(S.os[la]), S.x[la],
-                      r / 10, r % 10, shift, re, im);
-      yc[(int64_t)atom * NB + r] = make_double2(re, im);
-    }
-    return;
-  }
-  if (!active) return;
-  const double *os = onsite + (size_t)atom * kOnsiteStride;
-  const double2 *xa = xc + (int64_t)atom * NB;
-  // all four lanes of the quad active on every step (row r = 4 i + slot)
-#pragma unroll
-  for (int i = 0; i < NO; ++i) {
-    const int r = 4 * i + slot;
-    if (r >= NB) break;
-    double re = own_re[i], im = own_im[i];
-    onsite_row<NSP>(os, xa, r / 10, r % 10, shift, re, im);
-    yc[(int64_t)atom * NB + r] = make_double2(re, im);
-  }
-}
-
-// Block H·V in the SK-compressed and matrix-free layouts: the columns of
-// the block one after another inside each workgroup, the bond records,
-// neighbour indices and onsite records read once for all of them
-// (Hmatmult_spds_col_stored, Hmult_stored.c:2359-2474, re-reads H for every
-// column).  Mapping and the per-column steps as k_hv_sk with the quad LDS
-// gather.
-template <int NSP, typename R, bool CATION, typename SRC>
-__device__ __forceinline__ void sk_columns(int atom, int slot, bool active,
-                                           const SRC &src,
-                                           const int32_t *__restrict__ nbr,
-                                           const double *__restrict__ onsite,
-                                           double shift, const double2 *__restrict__ X,
-                                           double2 *__restrict__ Y, int64_t ld,
-                                           int ncol, SkQuadStage<NSP, double2> &L) {
-  constexpr int NB = NSP * 10;
-  constexpr int NO = (NB + 3) / 4;
-  const int j = active ? nbr[atom * 4 + slot] : -1;
-  R rv[24];
-  if (j >= 0) src.template fetch<CATION>(atom, slot, j, rv);
-  SkOwnRegs<NSP> own;
-  auto &S = *reinterpret_cast<SkOwnStage<NSP> *>(L.buf);
-  const int la = threadIdx.x / 4;
-  for (int col = 0; col < ncol; ++col) {
-    const double2 *xc = X + (int64_t)col * ld;
-    double2 *yc = Y + (int64_t)col * ld;
-    double own_re[NO], own_im[NO];
-    sk_bonds_rec<NSP, R, CATION, double2>(j, slot, rv, xc, own_re, own_im, L);
-    if (active)
-      sk_load_own<NSP>(slot, xc + (int64_t)atom * NB,
-                       onsite + (size_t)atom * kOnsiteStride, own);
-    __syncthreads();  // every lane has read its staged neighbour entries
-    if (active) sk_store_own<NSP>(la, slot, own, S);
-    __syncthreads();
-    if (active) {
-#pragma unroll
-      for (int i = 0; i < NO; ++i) {
-        const int r = 4 * i + slot;
-        if (r >= NB) break;
-        double re = own_re[i], im = own_im[i];
-        onsite_row<NSP>(reinterpret_cast<const double *>(S.os[la]), S.x[la],
-                        r / 10, r % 10, shift, re, im);
-        yc[(int64_t)atom * NB + r] = make_double2(re, im);
+  const bool cat = __builtin_amdgcn_readfirstlane(t.Q) < kSkOwn / 2;
+  uint4 *own = L.x + t.Q * S::kStride, *halo = L.x + (kSkOwn + t.Q) * S::kStride;
+  SkIndex<SRC> ix;
+  ix.read(tab, src, w.b, t.Q);
+  while (w.b < w.end) {
+    typename SRC::Data rec;
+    uint4 xo[S::kLoads], xh[S::kLoads], os[3];
+    const int atom = ix.own, hatom = ix.halo;
+    sk_load_x<NSP>(atom, t.c, x0, xo);
+    sk_load_x<NSP>(hatom, t.c, x0, xh);
+    src.load(ix.rec, rec);
+    sk_load_onsite(atom, t.c, onsite, os);
+    const uint2 local = ix.local;
+    const bool surface = sk_surface(atom, local);
+    w.b += w.step;
+    if (w.b < w.end) ix.read(tab, src, w.b, t.Q);
+    src.stage(rec, L.rec);
+    for (int col = 0; col < nc; ++col) {
+      sk_stage_x<NSP, double2>(own, t.c, xo);
+      sk_stage_x<NSP, double2>(halo, t.c, xh);
+      __syncthreads();
+      if (COLS && col + 1 < nc) {
+        sk_load_x<NSP>(atom, t.c, x0 + (int64_t)(col + 1) * ld, xo);
+        sk_load_x<NSP>(hatom, t.c, x0 + (int64_t)(col + 1) * ld, xh);
       }
+      double acc[10];
+      if (cat) sk_bonds<NSP, R, true, double2>(t, local, L, acc);
+      else sk_bonds<NSP, R, false, double2>(t, local, L, acc);
+      sk_finish<NSP, R, double2>(t, L, os, shift, surface, acc);
+      if (NSP == 2 || t.h == 0) sk_entries(own, t.comp, NSP == 2 ? 10 * t.h : 0, acc);
+      wave_sync();
+      if (atom >= 0) {
+        uint4 *y = reinterpret_cast<uint4 *>(y0 + (int64_t)col * ld) + (int64_t)atom * S::kChunks;
+#pragma unroll
+        for (int i = 0; i < S::kLoads; ++i)
+          if (4 * i + t.c < S::kChunks) y[4 * i + t.c] = own[4 * i + t.c];
+      }
+      wave_sync();
     }
-    __syncthreads();  // the epilogue has read the staging before it is reused
   }
-}
-
-template <int NSP, typename R, typename SRC>
-__global__ __launch_bounds__(kSkThreads) void k_hV_sk(
-    int nc, const int32_t *__restrict__ cations, int na,
-    const int32_t *__restrict__ anions, SkGrid grid,
-    const double *__restrict__ onsite, const SRC src,
-    const int32_t *__restrict__ nbr, double shift,
-    const double2 *__restrict__ X, double2 *__restrict__ Y, int64_t ld, int ncol) {
-  // one role per workgroup (grid.mixed == 0): the role branch below holds
-  // the column loop's barriers
-  const SkLane ln = sk_lane_of(grid, blockIdx.x, threadIdx.x);
-  // the role is uniform across the wavefront; read as a scalar, the role
-  // branches below are scalar branches (one per wave)
-  const bool cat = __builtin_amdgcn_readfirstlane((int)ln.cat) != 0;
-  const int li = ln.li;
-  const int slot = threadIdx.x & 3;
-  const bool active = li < (cat ? nc : na);
-  const int atom = active ? (cat ? cations[li] : anions[li]) : 0;
-  __shared__ SkQuadStage<NSP, double2> stage;
-  if (cat)
-    sk_columns<NSP, R, true>(atom, slot, active, src, nbr, onsite, shift, X, Y,
-                             ld, ncol, stage);
-  else
-    sk_columns<NSP, R, false>(atom, slot, active, src, nbr, onsite, shift, X, Y,
-                              ld, ncol, stage);
 }
 
 template <int NSP, typename TB, typename TA, bool STAGED>
@@ -190,60 +107,35 @@ nh_status launch_hv(nh_context *c, double shift, const nh_cplx *x, nh_cplx *y,
            "H·v: Hamiltonian not built in a supported layout");
   NH_CHECK(ncol >= 1 && ncol <= 65535 && ld >= c->n, NH_ERR_ARG,
            "H·V: bad ncol %d / ld %lld", ncol, (long long)ld);
-  // block products: the matrix-core kernel (FP32, 8 columns), all the
-  // columns in one SK / matrix-free launch with the bond records read once,
-  // or one column per grid row.  Default (-1): the matrix-core kernel for
-  // the row-owner block layout; one column per grid row for the SK and
-  // matrix-free layouts, measured fastest on a 786,520-atom dot (8 columns:
-  // 2.46 ms FP64 / 2.12 ms FP32 against 4.38 / 2.53 ms in one launch and
-  // 4.02 ms on the matrix cores)
+  // block products: the matrix-core kernel (FP32, 8 columns) by default for
+  // the row-owner block layout only; in the SK and matrix-free layouts all the
+  // columns in one launch with H read once, measured fastest for 2 columns and
+  // more (395,136 atoms, 8 columns, FP64: 0.65 ms SK and matrix-free against
+  // 0.83 / 1.06 ms with a column per grid row; 4 columns 0.34 / 0.35 ms)
   const int mode = c->block_hv;
   if ((mode == 2 || (mode == -1 && c->layout == NH_LAYOUT_BLOCKS)) &&
       hV_mfma_supported(c, ncol))
     return launch_hV_mfma(c, shift, x, y, ld);
-  if (sk_like(c) && ncol > 1 && mode == 1) {
-    int blocks = 0;
-    const SkGrid sg = sk_grid(c->n_cations, c->n_anions, false, &blocks);
-    const double2 *xd = reinterpret_cast<const double2 *>(x);
-    double2 *yd = reinterpret_cast<double2 *>(y);
-#define HVK(NSP, R, SRC)                                                      \
-  hipLaunchKernelGGL((k_hV_sk<NSP, R, decltype(SRC)>), dim3(blocks),          \
-                     dim3(kSkThreads), 0, c->stream, c->n_cations,            \
-                     c->cations, c->n_anions, c->anions, sg, c->onsite, SRC,  \
-                     c->nbr, shift, xd, yd, ld, ncol)
-#define HVP(R, SRC)                                                          \
-  do {                                                                       \
-    if (c->nb == 20) HVK(2, R, SRC);                                         \
-    else HVK(1, R, SRC);                                                     \
-  } while (0)
-    if (c->layout == NH_LAYOUT_MATRIX_FREE) {
-      if (c->precision == NH_PREC_FP64) HVP(double, mf_src<double>(c));
-      else HVP(float, mf_src<float>(c));
-    } else if (c->precision == NH_PREC_FP64) {
-      HVP(double, (SkSrc<double>{c->sk64, c->bond_of}));
-    } else {
-      HVP(float, (SkSrc<float>{c->sk32, c->bond_of}));
-    }
-#undef HVP
-#undef HVK
-    NH_HIP(hipGetLastError());
-    return NH_OK;
-  }
   if (sk_like(c)) {
-    int blocks = 0;
-    const SkGrid sg = sk_grid(c->n_cations, c->n_anions, sk_mixed_roles(c), &blocks);
-    const dim3 g(blocks, ncol);
+    const SkTable tab = sk_table_of(c);
     const double2 *xd = reinterpret_cast<const double2 *>(x);
     double2 *yd = reinterpret_cast<double2 *>(y);
-#define SKL1(NSP, R, SRC, QUAD)                                               \
-  hipLaunchKernelGGL((k_hv_sk<NSP, R, QUAD, decltype(SRC)>), g,               \
-                     dim3(kSkThreads), 0, c->stream, c->n_cations,            \
-                     c->cations, c->n_anions, c->anions, sg, c->onsite, SRC,  \
-                     c->nbr, shift, xd, yd, ld)
-#define SKL(NSP, R, SRC)                                                     \
-  do {                                                                       \
-    if (use_staged(c)) SKL1(NSP, R, SRC, true);                               \
-    else SKL1(NSP, R, SRC, false);                                           \
+    const bool cols = ncol > 1 && mode != 0;
+    // one block per workgroup; the matrix-free product of one vector is
+    // faster with as many workgroups as run at a time, their next tables read
+    // ahead (786,520 atoms, FP64: 0.273 against 0.292 ms; SK 0.243 / 0.232)
+    const bool walk = c->layout == NH_LAYOUT_MATRIX_FREE && !cols;
+    const dim3 g(walk ? sk_grid(c, 2) : sk_grid(c, 1 << 20), cols ? 1 : ncol);
+#define SKL(NSP, R, SRC)                                                       \
+  do {                                                                         \
+    if (cols)                                                                  \
+      hipLaunchKernelGGL((k_hv_sk<true, NSP, R, decltype(SRC)>), g,            \
+                         dim3(kSkThreads), 0, c->stream, tab, c->onsite, SRC,  \
+                         shift, xd, yd, ld, ncol, ncol);                       \
+    else                                                                       \
+      hipLaunchKernelGGL((k_hv_sk<false, NSP, R, decltype(SRC)>), g,           \
+                         dim3(kSkThreads), 0, c->stream, tab, c->onsite, SRC,  \
+                         shift, xd, yd, ld, ncol, 1);                          \
   } while (0)
 #define SKP(R, SRC)                                                          \
   do {                                                                       \
@@ -254,13 +146,12 @@ nh_status launch_hv(nh_context *c, double shift, const nh_cplx *x, nh_cplx *y,
       if (c->precision == NH_PREC_FP64) SKP(double, mf_src<double>(c));
       else SKP(float, mf_src<float>(c));
     } else if (c->precision == NH_PREC_FP64) {
-      SKP(double, (SkSrc<double>{c->sk64, c->bond_of}));
+      SKP(double, (SkSrc<double>{c->sk64, c->blk_bonds}));
     } else {
-      SKP(float, (SkSrc<float>{c->sk32, c->bond_of}));
+      SKP(float, (SkSrc<float>{c->sk32, c->blk_bonds}));
     }
 #undef SKP
 #undef SKL
-#undef SKL1
     NH_HIP(hipGetLastError());
     return NH_OK;
   }

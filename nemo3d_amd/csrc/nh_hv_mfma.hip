@@ -14,6 +14,7 @@
 // one bond each).  The epilogue adds the onsite part (diagonal - shift,
 // surface s-p couplings, spin-orbit) in FP64 and writes Y.
 #include "nh_hv_sk.h"
+#include "nh_sk_row.h"
 
 namespace nh {
 namespace {
@@ -39,10 +40,11 @@ struct MfmaShape {
 template <typename R>
 __device__ __forceinline__ void sk_block_to_lds(const R *__restrict__ rec,
                                                 bool cation, float *dst) {
-  R v[21];
+  R k[24], v[21];
 #pragma unroll
-  for (int k = 0; k < 21; ++k) v[k] = rec[3 + k];
-  const R l = rec[0], m = rec[1], n = rec[2];
+  for (int i = 0; i < 24; ++i) k[i] = rec[i];
+  sk_integrals(k, v);
+  const R l = k[K_L], m = k[K_M], n = k[K_N];
   R row[10];
 #define NH_ROW(A)                                                   \
   sk_row<A, R>(l, m, n, v, row);                                    \

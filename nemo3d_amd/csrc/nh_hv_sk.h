@@ -1,74 +1,77 @@
-// H·v in the SK-compressed and matrix-free layouts: per bond only the
-// direction cosines and the 21 strain-scaled two-centre integrals are
-// needed (24 values), stored once per bond (cation-owned) or recomputed
-// from the atoms' displacements (MfSrc); the 10x10 block is rebuilt row by
-// row in registers on every product.  The onsite record (diagonal with
-// Boykin corrections, surface couplings, spin-orbit) is stored per atom as
-// in the block layout.
+// H·v in the SK-compressed and matrix-free layouts: per bond only a record
+// of 24 numbers (direction and combinations of the strain-scaled two-centre
+// integrals, nh_sk_apply.h) is needed, stored once per bond (cation-owned) or
+// recomputed from the atoms' displacements (MfSrc); the 10x10 block is never
+// formed.  The onsite record (diagonal with Boykin corrections, surface
+// couplings, spin-orbit) is stored per atom as in the block layout.
 //
-// Mapping: 4 lanes per atom, lane n owns neighbour slot n.  A workgroup
-// holds only cation-role or only anion-role atoms (lists `cations` /
-// `anions`), so whether the lane applies T (anion row) or its transpose
-// (cation row) is uniform across the wavefront.  Each lane forms its bond's
-// 20 (10) complex products with R-precision arithmetic inside the block,
-// adds them to FP64 accumulators, a 4-lane butterfly sums the four bonds,
-// and lane n then finishes and writes rows r = n, n+4, ... with the onsite
-// terms.
+// Mapping: a workgroup of 256 threads takes a block of up to 32 cations and
+// 32 anions from a cube of cells (2 x 2 x 2 cells in the bulk).  It stages
+// the vector entries of its own atoms and of their other neighbours (the
+// halo: 46 atoms on average) and the records of their bonds (154) in LDS,
+// each once, a quad of lanes (64 bytes a load) per item, all loads in flight
+// together; then a quad per atom computes, its lanes owning the four real
+// component vectors of a 20-band atom (re and im of both spins): each lane
+// applies the atom's four bonds to its component from LDS and adds them up in
+// its own FP64 accumulators, so no sums cross lanes.  (10-band atoms have two
+// components: the quad's halves take two bonds each and are added.)
+// What bounds it: the traffic between L2 and the CUs.  Gathering each atom's
+// four neighbours and both rows' records separately moved 2.55 GB through L2
+// per FP64 product of a 786,520-atom dot (atom entries five times, records
+// twice) and kept the texture addresser busy 76% of 255 us whatever the order
+// of the atoms; the block moves the entries 1.7 times and the records 1.2
+// times: 786,520 atoms FP64 0.312 -> 0.244 ms (SK), 8 columns of 395,136
+// atoms 1.25 -> 0.67 ms (matrix-free); what is left is FP64 VALU (93 FMAs a
+// bond, component and row) and LDS reads about evenly, behind 0.94 GB of HBM.
+// The role (cation or anion) is uniform in a wavefront, so whether T or its
+// transpose is applied is a scalar branch.
 #pragma once
 
+#include <type_traits>
+
 #include "nh_internal.h"
-#include "nh_sk_row.h"
+#include "nh_sk_apply.h"
 
 namespace nh {
 
-constexpr int kSkThreads = 256;
-constexpr int kSkAtomsPerBlock = kSkThreads / 4;
+// ---- blocks of atoms ---------------------------------------------------------
 
-// Workgroup -> atoms.  Consecutive workgroups go to different XCDs (round
-// robin over 8): workgroup b runs on XCD b % 8, and XCD x takes the blocks
-// [x * ppx, (x + 1) * ppx) of the atom lists, so each XCD works on a
-// compact region (the lists are ordered by bricks of cells) and reuses the
-// neighbours' vector entries from its L2.  Cation block k and anion block k
-// cover the same cells.  Two mappings:
-//  * one role per workgroup (mixed = 0): 64 atoms, cation and anion blocks
-//    alternating on each XCD, so the two roles of the same cells run back
-//    to back; grid 16 * ppx, ppx = ceil(max(blocks of 64) / 8);
-//  * both roles (mixed = 1): waves 0-1 hold 32 cations and waves 2-3 the 32
-//    anions of the same list position, so both rows of a bond read its
-//    record within one workgroup; grid 8 * ppx, ppx = ceil(max(blocks of
-//    32) / 8).
-// Either way the role is uniform across a wavefront, so whether a lane
-// applies T (anion row) or its transpose (cation row) is too.
-struct SkGrid {
-  int ppx;
-  int mixed;
+// Blocks (built at context creation): capacity 32 cations and 32 anions of
+// its own, 64 more neighbours (the halo), 176 bonds; -1 pads the tables.
+constexpr int kSkOwn = 64, kSkHalo = 64, kSkBonds = 176, kSkBondPad = 192;
+constexpr int kSkThreads = 256;
+
+struct SkTable {
+  const int32_t *own;   // [blocks][64] atoms (0-31 cations, 32-63 anions)
+  const int32_t *halo;  // [blocks][64] atoms
+  const uint2 *local;   // [blocks][64] a byte per slot: x: neighbour's place
+                        // (own slot or 64 + halo place), y: bond's place; 255
+  int n;                // blocks
+  int per;              // blocks of an XCD, ceil(n / 8)
 };
-struct SkLane {
-  bool cat;
-  int li;  // index into the cation or anion list
-};
-// LANES: lanes per atom (4: lane = bond; 8: lane = bond and spin, SkSplit)
-template <int LANES = 4>
-__device__ __forceinline__ SkLane sk_lane_of(SkGrid g, int b, int t) {
-  constexpr int kAtoms = kSkThreads / LANES;
-  const int x = b & 7, s = b >> 3;
-  if (g.mixed) {
-    constexpr int kHalf = kSkThreads / 2;
-    return {t < kHalf, (x * g.ppx + s) * (kAtoms / 2) + (t & (kHalf - 1)) / LANES};
+inline SkTable sk_table_of(const nh_context *c) {
+  return SkTable{c->blk_own, c->blk_halo, c->blk_local,
+                 c->n_blocks, (c->n_blocks + 7) / 8};
+}
+// Workgroups: as many as run at a time (`groups` a CU, 32 CUs an XCD), each
+// taking block after block.  Consecutive workgroups go to different XCDs
+// (round robin over 8): workgroup g runs on XCD g % 8 and takes the blocks
+// (g % 8) per + g / 8, + grid / 8, ... < (g % 8 + 1) per, so each XCD works
+// on a compact region of the crystal whose vector entries and records are
+// shared in its L2.
+inline int sk_grid(const nh_context *c, int groups) {
+  const int per = (c->n_blocks + 7) / 8;
+  return 8 * (per / 32 < groups ? per : 32 * groups);
+}
+struct SkWalk {
+  int b, step, end;
+  __device__ __forceinline__ explicit SkWalk(const SkTable &t) {
+    const int x = blockIdx.x & 7;
+    b = x * t.per + (int)(blockIdx.x >> 3);
+    step = (int)(gridDim.x >> 3);
+    end = min(t.n, (x + 1) * t.per);
   }
-  return {(s & 1) == 0, (x * g.ppx + (s >> 1)) * kAtoms + t / LANES};
-}
-// the grid of a launch and its mapping
-inline SkGrid sk_grid(int n_cations, int n_anions, bool mixed, int *blocks,
-                      int lanes = 4) {
-  const int atoms = kSkThreads / lanes;
-  const int per = mixed ? atoms / 2 : atoms;
-  const int nbc = (n_cations + per - 1) / per;
-  const int nba = (n_anions + per - 1) / per;
-  const int ppx = ((nbc > nba ? nbc : nba) + 7) / 8;
-  *blocks = (mixed ? 8 : 16) * ppx;
-  return SkGrid{ppx, mixed ? 1 : 0};
-}
+};
 
 // Complex entries of the FP64 vector, or of an FP32 one widened on load
 __device__ __forceinline__ double2 widen2(double2 v) { return v; }
@@ -123,86 +126,157 @@ __device__ __forceinline__ void onsite_row(const double *__restrict__ os,
   }
 }
 
-// Block product of one bond, rows applied by orientation: anion rows
-// acc[s][a] += sum_c T[a][c] x[s][c]; cation rows acc[s][c] += sum_a
-// T[a][c] x[s][a].
-template <int NSP, typename R, bool CATION>
-struct BondApply {
-  template <int A>
-  __device__ __forceinline__ static void run(R l, R m, R n, const R *v,
-                                             const R (&xr)[NSP][10],
-                                             const R (&xi)[NSP][10],
-                                             R (&br)[NSP][10],
-                                             R (&bi)[NSP][10]) {
-    if constexpr (A < 10) {
-      R row[10];
-      sk_row<A, R>(l, m, n, v, row);
-#pragma unroll
-      for (int s = 0; s < NSP; ++s) {
-        if constexpr (!CATION) {
-          R sr = R(0), si = R(0);
-#pragma unroll
-          for (int c = 0; c < 10; ++c) {
-            sr += row[c] * xr[s][c];
-            si += row[c] * xi[s][c];
-          }
-          br[s][A] += sr;
-          bi[s][A] += si;
-        } else {
-#pragma unroll
-          for (int c = 0; c < 10; ++c) {
-            br[s][c] += row[c] * xr[s][A];
-            bi[s][c] += row[c] * xi[s][A];
-          }
-        }
-      }
-      run<A + 1>(l, m, n, v, xr, xi, br, bi);
-    }
-  }
+// LDS accesses of one wavefront execute in order; this keeps the compiler
+// from moving them across (lanes read what other lanes of the wavefront
+// wrote).  No instruction is emitted.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Staged items, in 16-byte chunks; odd strides spread the items of a
+// wavefront's atoms over the LDS banks.
+template <int NSP, typename XT>
+struct SkX {  // the entries of an atom
+  static constexpr int kChunks = NSP * 10 * (int)sizeof(XT) / 16;  // 20/10, 10/5
+  static constexpr int kLoads = (kChunks + 3) / 4;                 // per lane of a quad
+  // a place also holds an onsite record (9) or ten FP64 entries
+  static constexpr int kStride = (kChunks < 10 ? 10 : kChunks) | 1;
+};
+template <typename R>
+struct SkRec {  // a bond record (24 numbers)
+  static constexpr int kChunks = 24 * (int)sizeof(R) / 16;  // 12 / 6
+  static constexpr int kLoads = (kChunks + 3) / 4;
+  static constexpr int kStride = kChunks + 1;
+};
+constexpr int kOsChunks = kOnsiteStride / 2;
+
+template <int NSP, typename R, typename XT>
+struct SkLds {
+  uint4 x[(kSkOwn + kSkHalo) * SkX<NSP, XT>::kStride];
+  uint4 rec[kSkBonds * SkRec<R>::kStride];
 };
 
-// The 24 record values of a bond as 16-byte loads (12 for FP64, 6 for
-// FP32): the records are 16-byte aligned (24 values per bond).  Across a
-// wavefront every lane reads its own record, so the number of load
-// instructions, each touching 64 cache lines, is what the texture
-// addresser pays for.
-__device__ __forceinline__ void sk_load_record(const double *rec, double (&v)[24]) {
-  const double2 *p = reinterpret_cast<const double2 *>(rec);
-#pragma unroll
-  for (int q = 0; q < 12; ++q) {
-    const double2 t = p[q];
-    v[2 * q] = t.x;
-    v[2 * q + 1] = t.y;
+// Exchange of a double between lanes through DPP moves
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)b, CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), CTRL, 0xF, 0xF, true);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
+                                          (unsigned)lo));
+}
+constexpr int kQuadXor1 = 0xB1;  // quad_perm [1, 0, 3, 2]
+constexpr int kQuadXor2 = 0x4E;  // quad_perm [2, 3, 0, 1]
+constexpr int kQuadXor3 = 0x1B;  // quad_perm [3, 2, 1, 0]
+
+// ---- FP32 / deferred Lanczos vectors ---------------------------------------
+
+// Lanczos vectors in Paige's order: r_k = u_{k-1} - a r_{k-1}, a =
+// alpha_{k-1} / beta_{k-1} (so that a r_{k-1} = alpha_{k-1} q_{k-1}),
+// formed by the product as it reads u_{k-1} and r_{k-1}.
+// FP32 vectors: a is split into two FP32 parts (a = hi + lo to 2^-48
+// relative): two fmas, rounding entry by entry.  The coefficient must not be
+// rounded to FP32 alone: its error is the same for every entry, i.e. an
+// error along q_{k-1} in every step, which cost a 786,520-atom dot 10,251
+// steps instead of 7,901 (and a level, from another start); with the split
+// it takes the same 7,826 steps as one FP64 fma per entry.
+// FP64 vectors: one fma.  Every kernel that forms r_k (the products that
+// read u_{k-1} and r_{k-1}, the eigenvector pass that writes r_k) evaluates
+// these expressions on the same operands, so they agree bit for bit.
+template <typename XT>
+struct LzCoef;
+template <>
+struct LzCoef<float2> {
+  float hi, lo;
+};
+template <>
+struct LzCoef<double2> {
+  double a;
+};
+template <typename XT>
+__device__ __forceinline__ LzCoef<XT> lz_defer_coef(double al, double inv) {
+  const double a = al * inv;
+  if constexpr (sizeof(XT) == 8) {
+    const float hi = (float)a;
+    return LzCoef<XT>{hi, (float)(a - (double)hi)};
+  } else {
+    return LzCoef<XT>{a};
   }
 }
-__device__ __forceinline__ void sk_load_record(const float *rec, float (&v)[24]) {
-  const float4 *p = reinterpret_cast<const float4 *>(rec);
-#pragma unroll
-  for (int q = 0; q < 6; ++q) {
-    const float4 t = p[q];
-    v[4 * q] = t.x;
-    v[4 * q + 1] = t.y;
-    v[4 * q + 2] = t.z;
-    v[4 * q + 3] = t.w;
+__device__ __forceinline__ float lz_defer1(float u, float rp, LzCoef<float2> a) {
+  // the cancellation u - hi rp happens inside the first fma (one rounding
+  // of the exact difference), then the small correction: about one ulp of
+  // r in all (the other order adds half an ulp of u, which can be larger)
+  return __builtin_fmaf(-a.lo, rp, __builtin_fmaf(-a.hi, rp, u));
+}
+__device__ __forceinline__ double lz_defer1(double u, double rp, LzCoef<double2> a) {
+  return __builtin_fma(-a.a, rp, u);
+}
+// a 16-byte chunk of r_k: two FP32 entries or one FP64 entry
+template <typename XT>
+__device__ __forceinline__ uint4 lz_defer_chunk(uint4 u, uint4 rp, LzCoef<XT> a) {
+  uint4 o;
+  if constexpr (sizeof(XT) == 8) {
+    o.x = __float_as_uint(lz_defer1(__uint_as_float(u.x), __uint_as_float(rp.x), a));
+    o.y = __float_as_uint(lz_defer1(__uint_as_float(u.y), __uint_as_float(rp.y), a));
+    o.z = __float_as_uint(lz_defer1(__uint_as_float(u.z), __uint_as_float(rp.z), a));
+    o.w = __float_as_uint(lz_defer1(__uint_as_float(u.w), __uint_as_float(rp.w), a));
+  } else {
+    const double2 du = *reinterpret_cast<const double2 *>(&u);
+    const double2 dr = *reinterpret_cast<const double2 *>(&rp);
+    double2 r;
+    r.x = lz_defer1(du.x, dr.x, a);
+    r.y = lz_defer1(du.y, dr.y, a);
+    o = *reinterpret_cast<const uint4 *>(&r);
   }
+  return o;
 }
 
-// Where a lane's bond record comes from.
+// ---- bond records ------------------------------------------------------------
+
+// A source of bond records: index() reads which records a block needs,
+// load() requests what they are made of, stage() writes them to LDS.
 //
-// SkSrc: the stored SK layout, 24 values per bond (each bond once), found
-// through bond_of.
+// SkSrc: the stored SK layout, 24 numbers per bond (each bond once); the
+// block's records are loaded by quads, one record a quad and round.
 template <typename R>
 struct SkSrc {
   const R *__restrict__ sk;
-  const int32_t *__restrict__ bond_of;
-  // FP64: the record is requested before the neighbour gather, whose
-  // barrier its loads then overlap (measured: plain solve -4%); FP32: after
-  // it (requested early, the 24 values spill at 128 VGPRs: +3% per product)
-  static constexpr bool kEarly = sizeof(R) == 8;
-  template <bool CATION>
-  __device__ __forceinline__ void fetch(int atom, int slot, int /*j*/,
-                                        R (&rv)[24]) const {
-    sk_load_record(sk + (size_t)bond_of[atom * 4 + slot] * kSkStride, rv);
+  const int32_t *__restrict__ bonds;
+
+  static constexpr int kRounds = kSkBondPad / 64;
+  struct Index {
+    int b[kRounds];
+  };
+  struct Data {
+    uint4 r[kRounds][SkRec<R>::kLoads];
+  };
+  __device__ __forceinline__ void index(int blk, Index &i) const {
+#pragma unroll
+    for (int k = 0; k < kRounds; ++k)
+      i.b[k] = bonds[blk * kSkBondPad + 64 * k + (int)(threadIdx.x >> 2)];
+  }
+  __device__ __forceinline__ void load(const Index &i, Data &d) const {
+    const int c = threadIdx.x & 3;
+#pragma unroll
+    for (int k = 0; k < kRounds; ++k)
+#pragma unroll
+      for (int q = 0; q < SkRec<R>::kLoads; ++q) {
+        d.r[k][q] = make_uint4(0, 0, 0, 0);
+        if (i.b[k] >= 0 && 4 * q + c < SkRec<R>::kChunks)
+          d.r[k][q] = reinterpret_cast<const uint4 *>(sk + (size_t)i.b[k] * kSkStride)[4 * q + c];
+      }
+  }
+  __device__ __forceinline__ void stage(const Data &d, uint4 *rec) const {
+    const int Q = threadIdx.x >> 2, c = threadIdx.x & 3;
+#pragma unroll
+    for (int k = 0; k < kRounds; ++k)
+#pragma unroll
+      for (int q = 0; q < SkRec<R>::kLoads; ++q)
+        if (64 * k + Q < kSkBonds && 4 * q + c < SkRec<R>::kChunks)
+          rec[(64 * k + Q) * SkRec<R>::kStride + 4 * q + c] = d.r[k][q];
   }
 };
 
@@ -212,19 +286,20 @@ struct SkSrc {
 // and species and the slot's ideal bond vector, as the assembly computes it
 // (strain_corr_prep, mb_ham_spds_micro.c:2848-2978): direction cosines of
 // the strained bond and the 21 integrals scaled by (d0/d)^eta, with
-// (d0/d)^eta = exp(eta log(d0/d)) (one log and 15 exp per bond).  The bond
-// vector is formed in the cation's frame from either end, so both rows of
-// a bond get bit-identical records and H stays exactly Hermitian.  With
-// R = float the integrals are scaled in FP32 (geometry and the log in FP64).
+// (d0/d)^eta = exp(eta log(d0/d)) (one log and 15 exp per bond and block, a
+// lane per bond).  Both rows of a bond get
+// bit-identical records (the bond vector is formed in the cation's frame), so
+// H stays exactly Hermitian.  With R = float the integrals are scaled in
+// FP32 (geometry and the log in FP64).
 template <typename R>
 struct MfSrc {
+  const int2 *__restrict__ ends;    // [blocks][192] 4 cation atom + slot, anion
   const double4 *__restrict__ geo;  // [A] displacement x, y, z (nm), species
   const int32_t *__restrict__ q;    // [A][4] packed int8 ideal bond vector,
                                     // cation frame
   const double *__restrict__ pair;  // [S][S][kMfPair]
   int S;
   double lx, ly, lz;
-  static constexpr bool kEarly = true;
 
   __device__ __forceinline__ static void scale(const double *__restrict__ P,
                                                double lb, R *__restrict__ v) {
@@ -238,12 +313,9 @@ struct MfSrc {
     for (int k = 0; k < 21; ++k) v[k] = R(P[k]) * f[eta_index(k)];
   }
 
-  template <bool CATION>
-  __device__ __forceinline__ void fetch(int atom, int slot, int j,
-                                        R (&rv)[24]) const {
-    const double4 gi = geo[atom], gj = geo[j];
-    const int qp = q[atom * 4 + slot];
-    const double4 gc = CATION ? gi : gj, ga = CATION ? gj : gi;
+  // the record of a bond from its two atoms and its ideal vector
+  __device__ __forceinline__ void make(const double4 &gc, const double4 &ga, int qp,
+                                       R (&rec)[24]) const {
     const double qx = (double)(int8_t)(qp & 0xff);
     const double qy = (double)(int8_t)((qp >> 8) & 0xff);
     const double qz = (double)(int8_t)((qp >> 16) & 0xff);
@@ -253,400 +325,235 @@ struct MfSrc {
     const double ny = -(ly * (0.25 * qy) + ga.y - gc.y);
     const double nz = -(lz * (0.25 * qz) + ga.z - gc.z);
     const double den = sqrt(nx * nx + ny * ny + nz * nz);
-    rv[0] = R(nx / den);
-    rv[1] = R(ny / den);
-    rv[2] = R(nz / den);
+    R v[21];
     const int p = (int)gc.w * S + (int)ga.w;
     // the common case, one species pair across the wavefront, reads the
     // pair constants through the scalar cache
     const int pu = __builtin_amdgcn_readfirstlane(p);
     if (__all(p == pu)) {
       const double *P = pair + pu * kMfPair;
-      scale(P, log((0.25 * kSqrt3Ref * P[kMfA0]) / den), rv + 3);
+      scale(P, log((0.25 * kSqrt3Ref * P[kMfA0]) / den), v);
     } else {
       const double *P = pair + p * kMfPair;
-      scale(P, log((0.25 * kSqrt3Ref * P[kMfA0]) / den), rv + 3);
+      scale(P, log((0.25 * kSqrt3Ref * P[kMfA0]) / den), v);
+    }
+    sk_record(R(nx / den), R(ny / den), R(nz / den), v, rec);
+  }
+
+
+  struct Index {
+    int2 e;
+  };
+  struct Data {
+    double4 gc, ga;
+    int q;
+  };
+  __device__ __forceinline__ void index(int blk, Index &i) const {
+    i.e = make_int2(-1, -1);
+    if (threadIdx.x < kSkBonds) i.e = ends[blk * kSkBondPad + (int)threadIdx.x];
+  }
+  __device__ __forceinline__ void load(const Index &i, Data &d) const {
+    d.q = -1;
+    if (i.e.x >= 0) {
+      d.gc = geo[i.e.x >> 2];
+      d.ga = geo[i.e.y];
+      d.q = q[i.e.x] & 0xffffff;
+    }
+  }
+  __device__ __forceinline__ void stage(const Data &d, uint4 *rec) const {
+    if (d.q >= 0) {
+      R k[24];
+      make(d.gc, d.ga, d.q, k);
+      const uint4 *r = reinterpret_cast<const uint4 *>(k);
+#pragma unroll
+      for (int i = 0; i < SkRec<R>::kChunks; ++i)
+        rec[threadIdx.x * SkRec<R>::kStride + i] = r[i];
     }
   }
 };
 
 template <typename R>
 inline MfSrc<R> mf_src(const nh_context *c) {
-  return MfSrc<R>{c->mf_geo, c->mf_q, c->mf_pair, c->n_species,
+  return MfSrc<R>{c->mf_ends, c->mf_geo, c->mf_q, c->mf_pair, c->n_species,
                   c->lattice[0], c->lattice[1], c->lattice[2]};
 }
 
-// The neighbour's NB complex entries, from the FP64 vector (one double2
-// per entry) or from its FP32 copy (one float4 per two entries; the entries
-// of an atom start on a 16-byte boundary, NB * 8 bytes per atom).
-template <int NSP, typename R>
-__device__ __forceinline__ void sk_load_x(const double2 *__restrict__ x,
-                                          int64_t j, R (&xr)[NSP][10],
-                                          R (&xi)[NSP][10]) {
-  const double2 *xj = x + j * (NSP * 10);
-#pragma unroll
-  for (int s = 0; s < NSP; ++s)
-#pragma unroll
-    for (int c = 0; c < 10; ++c) {
-      const double2 t = xj[s * 10 + c];
-      xr[s][c] = R(t.x);
-      xi[s][c] = R(t.y);
-    }
-}
-template <int NSP, typename R>
-__device__ __forceinline__ void sk_load_x(const float2 *__restrict__ x,
-                                          int64_t j, R (&xr)[NSP][10],
-                                          R (&xi)[NSP][10]) {
-  const float4 *xj = reinterpret_cast<const float4 *>(x + j * (NSP * 10));
-#pragma unroll
-  for (int s = 0; s < NSP; ++s)
-#pragma unroll
-    for (int c = 0; c < 10; c += 2) {
-      const float4 t = xj[(s * 10 + c) / 2];
-      xr[s][c] = R(t.x);
-      xi[s][c] = R(t.y);
-      xr[s][c + 1] = R(t.z);
-      xi[s][c + 1] = R(t.w);
-    }
+// ---- one block ------------------------------------------------------------------
+
+// What a thread is: quad Q of lanes, its atom's slot in the block; lane c of
+// the quad: chunks c, c + 4, ... when the quad moves an item, component re /
+// im (comp) of spin h (20 bands) or of bond half h (10 bands) when it computes.
+struct SkThread {
+  int Q, c, comp, h;
+  __device__ __forceinline__ SkThread() {
+    Q = threadIdx.x >> 2;
+    c = threadIdx.x & 3;
+    comp = c & 1;
+    h = c >> 1;
+  }
+};
+
+// The thread's part of a block's tables: the two atoms whose entries its quad
+// stages (its own and one of the halo), the neighbours' and records' places,
+// the records.
+template <typename SRC>
+struct SkIndex {
+  int own, halo;
+  uint2 local;
+  typename SRC::Index rec;
+  __device__ __forceinline__ void read(const SkTable &tab, const SRC &src, int blk, int Q) {
+    own = tab.own[blk * kSkOwn + Q];
+    halo = tab.halo[blk * kSkHalo + Q];
+    local = tab.local[blk * kSkOwn + Q];
+    src.index(blk, rec);
+  }
+};
+
+// whether some own atom of the wavefront lacks a neighbour (a byte of all ones)
+__device__ __forceinline__ bool sk_surface(int own, uint2 local) {
+  const unsigned z = ~local.x;
+  return __any(own >= 0 && ((z - 0x01010101u) & ~z & 0x80808080u) != 0);
 }
 
-// Quad-cooperative gather of the neighbours' entries through LDS: the four
-// lanes of an atom load the entries of each of its four neighbours in turn,
-// lane `slot` taking the 16-byte chunks slot, slot + 4, ..., so one load
-// instruction touches one 64-byte piece per quad (16 cache lines per
-// wavefront instead of 64 when every lane reads its own neighbour); every
-// lane then reads its own neighbour's entries back from LDS.  Entries are
-// those of XT (double2: the FP64 vector; float2: its FP32 copy).
+// The entries of an atom, chunks c, c + 4, ... by lane c
 template <int NSP, typename XT>
-struct SkQuadStage {
-  static constexpr int kChunks = NSP * 10 * (int)sizeof(XT) / 16;  // 20/10/5
-  // Lane t keeps its item in chunks [t kChunks, (t + 1) kChunks), no
-  // padding.  A multiple of 4 chunks: chunk index XOR-swizzled by
-  // (t >> 2) & 3 (16 lanes then cover all 64 banks); 2 mod 4: chunk index
-  // rotated by one for lanes with bit 2 ^ bit 3 set, so the reads of 8 or
-  // 16 consecutive lanes hit distinct banks (the quad writes stay 2-way);
-  // odd: already conflict-free.
-  static constexpr bool kSwizzle = kChunks % 4 == 0;
-  static constexpr bool kRotate = kChunks % 4 == 2;
-  static constexpr int kStride = kChunks;
-  __device__ static int pos(int t, int c) {
-    if constexpr (kSwizzle) return t * kStride + (c ^ ((t >> 2) & 3));
-    if constexpr (kRotate) {
-      const int r = c + (((t >> 2) ^ (t >> 3)) & 1);
-      return t * kStride + (r >= kChunks ? r - kChunks : r);
-    }
-    return t * kStride + c;
-  }
-  uint4 buf[kSkThreads * kStride];
-};
-
-// FP32 Lanczos vectors: r_k = u_{k-1} - a r_{k-1}, a = alpha_{k-1} /
-// beta_{k-1} (so that a r_{k-1} = alpha_{k-1} q_{k-1}), in FP32 with a
-// split into two FP32 parts (a = hi + lo to 2^-48 relative): two fmas,
-// rounding entry by entry.  The coefficient must not be rounded to FP32
-// alone: its error is the same for every entry, i.e. an error along
-// q_{k-1} in every step, which cost a 786,520-atom dot 10,251 steps
-// instead of 7,901 (and a level, from another start); with the split it
-// takes the same 7,826 steps as one FP64 fma per entry, 6% faster in the
-// product.  Every kernel that forms r_k (the products that read u_{k-1}
-// and r_{k-1}, the eigenvector pass that writes r_k) evaluates these
-// expressions on the same operands, so they agree bit for bit.
-struct LzCoef {
-  float hi, lo;
-};
-__device__ __forceinline__ LzCoef lz_defer_coef(double al, double inv) {
-  const double a = al * inv;
-  const float hi = (float)a;
-  return LzCoef{hi, (float)(a - (double)hi)};
-}
-__device__ __forceinline__ float lz_defer1(float u, float rp, LzCoef a) {
-  // the cancellation u - hi rp happens inside the first fma (one rounding
-  // of the exact difference), then the small correction: about one ulp of
-  // r in all (the other order adds half an ulp of u, which can be larger)
-  return __builtin_fmaf(-a.lo, rp, __builtin_fmaf(-a.hi, rp, u));
-}
-// where the products read r_k from: x holds u_{k-1}, rp r_{k-1}
-struct LzDeferSrc {
-  const float2 *rp;
-  LzCoef a;  // lz_defer_coef(alpha_{k-1}, 1 / beta_{k-1})
-};
-__device__ __forceinline__ uint4 lz_defer_chunk(uint4 u, uint4 rp, const LzDeferSrc &d) {
-  uint4 o;
-  o.x = __float_as_uint(lz_defer1(__uint_as_float(u.x), __uint_as_float(rp.x), d.a));
-  o.y = __float_as_uint(lz_defer1(__uint_as_float(u.y), __uint_as_float(rp.y), d.a));
-  o.z = __float_as_uint(lz_defer1(__uint_as_float(u.z), __uint_as_float(rp.z), d.a));
-  o.w = __float_as_uint(lz_defer1(__uint_as_float(u.w), __uint_as_float(rp.w), d.a));
-  return o;
-}
-
-// The NSP * 10 entries of an item start at entry `off` of the neighbour's
-// `stride` entries (stride = NSP * 10, off = 0: the whole atom; stride =
-// 20, off = 10 s: spin block s of a 20-band atom).  DEFER (XT = float2):
-// the staged entries are r_k formed from x = u_{k-1} and d.rp = r_{k-1}.
-template <int NSP, typename R, typename XT, bool DEFER = false>
-__device__ __forceinline__ void sk_quad_gather(int j, int slot,
-                                               const XT *__restrict__ x,
-                                               SkQuadStage<NSP, XT> &L,
-                                               R (&xr)[NSP][10],
-                                               R (&xi)[NSP][10],
-                                               int stride = NSP * 10, int off = 0,
-                                               LzDeferSrc d = {nullptr, {0.0f, 0.0f}}) {
-  static_assert(!DEFER || sizeof(XT) == 8, "deferred r_k needs FP32 vectors");
-  using S = SkQuadStage<NSP, XT>;
-  constexpr int NB = NSP * 10;
-  constexpr int C = S::kChunks;
-  const int t = threadIdx.x, q0 = t & ~3;
+__device__ __forceinline__ void sk_load_x(int atom, int c, const XT *__restrict__ x,
+                                          uint4 (&X)[SkX<NSP, XT>::kLoads]) {
+  const uint4 *p = reinterpret_cast<const uint4 *>(x) + (int64_t)atom * SkX<NSP, XT>::kChunks;
 #pragma unroll
-  for (int n = 0; n < 4; ++n) {
-    const int jn = __shfl(j, (t & 63 & ~3) | n, 64);
-    if (jn >= 0) {
-      const uint4 *src = reinterpret_cast<const uint4 *>(x + (int64_t)jn * stride + off);
-      if constexpr (DEFER) {
-        const uint4 *srp =
-            reinterpret_cast<const uint4 *>(d.rp + (int64_t)jn * stride + off);
-#pragma unroll
-        for (int c0 = 0; c0 < C; c0 += 4) {
-          const int c = c0 + slot;
-          if (c < C) L.buf[S::pos(q0 + n, c)] = lz_defer_chunk(src[c], srp[c], d);
-        }
-      } else {
-#pragma unroll
-        for (int c0 = 0; c0 < C; c0 += 4) {
-          const int c = c0 + slot;
-          if (c < C) L.buf[S::pos(q0 + n, c)] = src[c];
-        }
-      }
-    }
-  }
-  __syncthreads();
-  if (j >= 0) {
-    if constexpr (sizeof(XT) == 16) {
-#pragma unroll
-      for (int e = 0; e < NB; ++e) {
-        const double2 v = *reinterpret_cast<const double2 *>(&L.buf[S::pos(t, e)]);
-        xr[e / 10][e % 10] = R(v.x);
-        xi[e / 10][e % 10] = R(v.y);
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < NB; e += 2) {
-        const float4 v = *reinterpret_cast<const float4 *>(&L.buf[S::pos(t, e / 2)]);
-        xr[e / 10][e % 10] = R(v.x);
-        xi[e / 10][e % 10] = R(v.y);
-        xr[(e + 1) / 10][(e + 1) % 10] = R(v.z);
-        xi[(e + 1) / 10][(e + 1) % 10] = R(v.w);
-      }
-    }
+  for (int i = 0; i < SkX<NSP, XT>::kLoads; ++i) {
+    X[i] = make_uint4(0, 0, 0, 0);
+    if (atom >= 0 && 4 * i + c < SkX<NSP, XT>::kChunks) X[i] = p[4 * i + c];
   }
 }
-
-// Epilogue staging (after the quad gather, in the same LDS): every atom's
-// own entries and onsite record, loaded by its quad with lane `slot` taking
-// rows slot, slot + 4, ... (64 contiguous bytes per quad and load), so that
-// the onsite couplings read their partner entries from LDS instead of
-// issuing scattered loads per row.
-template <int NSP, int ATOMS = kSkAtomsPerBlock>
-struct SkOwnStage {
-  double2 x[ATOMS][NSP * 10];
-  double2 os[ATOMS][kOnsiteStride / 2];
-};
-
-// Own entries and onsite record loaded into registers (before the barrier
-// that frees the staging LDS, so the loads overlap it) ...
-// (LANES lanes per atom; lane `lane` takes entries lane, lane + LANES, ...)
-template <int NSP, int LANES = 4>
-struct SkOwnRegs {
-  static constexpr int kOs = (kOnsiteStride / 2 + LANES - 1) / LANES;  // onsite chunks per lane
-  double2 x[(NSP * 10 + LANES - 1) / LANES];
-  double2 os[kOs];
-};
-// (xa: the FP64 vector, or the FP32 one whose entries are widened on load)
-template <int NSP, int LANES = 4, typename XO = double2>
-__device__ __forceinline__ void sk_load_own(int lane, const XO *__restrict__ xa,
-                                            const double *__restrict__ os,
-                                            SkOwnRegs<NSP, LANES> &g) {
-  constexpr int NB = NSP * 10;
+template <int NSP, typename XT>
+__device__ __forceinline__ void sk_stage_x(uint4 *place, int c,
+                                           const uint4 (&X)[SkX<NSP, XT>::kLoads]) {
 #pragma unroll
-  for (int i = 0; i < (NB + LANES - 1) / LANES; ++i) {
-    const int r = LANES * i + lane;
-    g.x[i] = r < NB ? widen2(xa[r]) : make_double2(0.0, 0.0);
-  }
-  const double2 *o2 = reinterpret_cast<const double2 *>(os);  // 144-byte records
-#pragma unroll
-  for (int i = 0; i < SkOwnRegs<NSP, LANES>::kOs; ++i) {
-    const int c = LANES * i + lane;
-    g.os[i] = c < kOnsiteStride / 2 ? o2[c] : make_double2(0.0, 0.0);
-  }
+  for (int i = 0; i < SkX<NSP, XT>::kLoads; ++i)
+    if (4 * i + c < SkX<NSP, XT>::kChunks) place[4 * i + c] = X[i];
 }
-// ... and stored to the epilogue staging after it
-template <int NSP, int LANES = 4, int ATOMS = kSkAtomsPerBlock>
-__device__ __forceinline__ void sk_store_own(int la, int lane,
-                                             const SkOwnRegs<NSP, LANES> &g,
-                                             SkOwnStage<NSP, ATOMS> &S) {
-  constexpr int NB = NSP * 10;
+// r_k from the chunks of u_{k-1} and r_{k-1}
+template <typename XT, int K>
+__device__ __forceinline__ void sk_defer(uint4 (&X)[K], const uint4 (&P)[K], LzCoef<XT> a) {
 #pragma unroll
-  for (int i = 0; i < (NB + LANES - 1) / LANES; ++i)
-    if (LANES * i + lane < NB) S.x[la][LANES * i + lane] = g.x[i];
-#pragma unroll
-  for (int i = 0; i < SkOwnRegs<NSP, LANES>::kOs; ++i)
-    if (LANES * i + lane < kOnsiteStride / 2) S.os[la][LANES * i + lane] = g.os[i];
+  for (int i = 0; i < K; ++i) X[i] = lz_defer_chunk<XT>(X[i], P[i], a);
 }
 
-// Exchange of a double with lane ^ 1 / lane ^ 2 inside the quad through
-// DPP quad permutations (VALU moves; a __shfl_xor is an LDS permute).
-template <int CTRL>
-__device__ __forceinline__ double quad_perm_f64(double v) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)b, CTRL, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), CTRL, 0xF, 0xF, true);
-  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
-                                          (unsigned)lo));
-}
-constexpr int kQuadXor1 = 0xB1;  // quad_perm [1, 0, 3, 2]
-constexpr int kQuadXor2 = 0x4E;  // quad_perm [2, 3, 0, 1]
-
-// The 4 bonds of `atom` (lane = slot), summed over the quad in FP64 (fixed
-// order); lane `slot` keeps rows r = 4 i + slot in own_re[i] / own_im[i].
-// SRC: where the bond records come from (SkSrc, MfSrc).
-// XT: double2 (the FP64 vector) or float2 (its FP32 copy, R = float).
-// QUAD: gather through LDS (sk_quad_gather; every thread of the workgroup
-// must call, there is a barrier) in the caller's LDS area L, or directly
-// from the caches.  Callers branch on the role with a wave-uniform
-// (scalar) condition, so every wave runs exactly one instantiation and
-// reaches the same number of barriers whichever role it holds.
-template <int NSP, typename R, bool CATION, typename XT, bool QUAD, bool DEFER = false,
-          typename SRC>
-__device__ __forceinline__ void sk_bonds(int atom, int slot, bool active,
-                                         const SRC &src,
-                                         const int32_t *__restrict__ nbr,
-                                         const XT *__restrict__ xc,
-                                         double (&own_re)[(NSP * 10 + 3) / 4],
-                                         double (&own_im)[(NSP * 10 + 3) / 4],
-                                         SkQuadStage<NSP, XT> *L = nullptr,
-                                         LzDeferSrc d = {nullptr, {0.0f, 0.0f}}) {
-  static_assert(!DEFER || QUAD, "deferred r_k needs the LDS gather");
-  R br[NSP][10], bi[NSP][10];
+// The thread's component of the item at `place`, from entry `first` on
+template <typename R, typename XT>
+__device__ __forceinline__ void sk_read_x(const uint4 *place, int comp, int first, R (&x)[10]) {
+  using E = typename std::conditional<sizeof(XT) == 16, double, float>::type;
+  const E *p = reinterpret_cast<const E *>(place) + 2 * first + comp;
 #pragma unroll
-  for (int s = 0; s < NSP; ++s)
-#pragma unroll
-    for (int c = 0; c < 10; ++c) br[s][c] = bi[s][c] = R(0);
-  const int j = active ? nbr[atom * 4 + slot] : -1;
-  R xr[NSP][10], xi[NSP][10];
-  if constexpr (QUAD) {
-    R rv[24];
-    if (SRC::kEarly && j >= 0) src.template fetch<CATION>(atom, slot, j, rv);
-    sk_quad_gather<NSP, R, XT, DEFER>(j, slot, xc, *L, xr, xi, NSP * 10, 0, d);
-    if (!SRC::kEarly && j >= 0) src.template fetch<CATION>(atom, slot, j, rv);
-    if (j >= 0)
-      BondApply<NSP, R, CATION>::template run<0>(rv[0], rv[1], rv[2], rv + 3,
-                                                  xr, xi, br, bi);
-  } else if (j >= 0) {
-    R rv[24];
-    src.template fetch<CATION>(atom, slot, j, rv);
-    sk_load_x<NSP, R>(xc, j, xr, xi);
-    BondApply<NSP, R, CATION>::template run<0>(rv[0], rv[1], rv[2], rv + 3, xr,
-                                                xi, br, bi);
-  }
-  // sum over the quad (lanes 4k..4k+3); the owner lane keeps the row
-#pragma unroll
-  for (int s = 0; s < NSP; ++s)
-#pragma unroll
-    for (int c = 0; c < 10; ++c) {
-      const int r = s * 10 + c;
-      double re = double(br[s][c]), im = double(bi[s][c]);
-      re += quad_perm_f64<kQuadXor1>(re);
-      im += quad_perm_f64<kQuadXor1>(im);
-      re += quad_perm_f64<kQuadXor2>(re);
-      im += quad_perm_f64<kQuadXor2>(im);
-      if ((r & 3) == slot) {
-        own_re[r >> 2] = re;
-        own_im[r >> 2] = im;
-      }
-    }
+  for (int o = 0; o < 10; ++o) x[o] = R(p[2 * o]);
 }
 
-// SkSplit: 8 lanes per atom of a 20-band model, lane = (spin s, bond n):
-// lanes 4 s .. 4 s + 3 of an atom hold the four bonds for spin block s, so
-// each lane applies its bond's 10 x 10 block to one spin block only (half
-// the vector registers of sk_bonds), the record is read by both spin lanes
-// of a bond, and the four-lane sums stay within the spin group.  Lane
-// `slot` of spin group s keeps rows s * 10 + 4 i + slot (i < 3) in
-// own_re[i] / own_im[i].  QUAD only (LDS gather of the spin block).
-struct SkSplit {
-  static constexpr int kLanes = 8;
-  static constexpr int kAtoms = kSkThreads / kLanes;
-  static constexpr int kOwn = 3;  // rows per lane
-};
-
-template <typename R, bool CATION, typename XT, bool DEFER = false, typename SRC>
-__device__ __forceinline__ void sk_bonds_split(int atom, int slot, int spin,
-                                               bool active, const SRC &src,
-                                               const int32_t *__restrict__ nbr,
-                                               const XT *__restrict__ xc,
-                                               double (&own_re)[SkSplit::kOwn],
-                                               double (&own_im)[SkSplit::kOwn],
-                                               SkQuadStage<1, XT> &L,
-                                               LzDeferSrc d = {nullptr, {0.0f, 0.0f}}) {
-  R br[1][10], bi[1][10];
-#pragma unroll
-  for (int c = 0; c < 10; ++c) br[0][c] = bi[0][c] = R(0);
-  const int j = active ? nbr[atom * 4 + slot] : -1;
-  R xr[1][10], xi[1][10];
-  R rv[24];
-  if (SRC::kEarly && j >= 0) src.template fetch<CATION>(atom, slot, j, rv);
-  sk_quad_gather<1, R, XT, DEFER>(j, slot, xc, L, xr, xi, 20, 10 * spin, d);
-  if (!SRC::kEarly && j >= 0) src.template fetch<CATION>(atom, slot, j, rv);
-  if (j >= 0)
-    BondApply<1, R, CATION>::template run<0>(rv[0], rv[1], rv[2], rv + 3, xr,
-                                              xi, br, bi);
-#pragma unroll
-  for (int c = 0; c < 10; ++c) {
-    double re = double(br[0][c]), im = double(bi[0][c]);
-    re += quad_perm_f64<kQuadXor1>(re);
-    im += quad_perm_f64<kQuadXor1>(im);
-    re += quad_perm_f64<kQuadXor2>(re);
-    im += quad_perm_f64<kQuadXor2>(im);
-    if ((c & 3) == slot) {
-      own_re[c >> 2] = re;
-      own_im[c >> 2] = im;
-    }
-  }
-}
-
-// The same with the bond record already in registers (rv; j < 0: no bond)
-// and the quad LDS gather of XT entries: the block products of several
-// vectors reuse one record.
+// acc = the thread's component of sum_n T_n x_n from the staged block; R
+// inside a bond, FP64 over the bonds.  20 bands: the lane applies the atom's
+// four bonds; 10 bands: the two lanes of a component two each.
 template <int NSP, typename R, bool CATION, typename XT>
-__device__ __forceinline__ void sk_bonds_rec(int j, int slot, const R (&rv)[24],
-                                             const XT *__restrict__ xc,
-                                             double (&own_re)[(NSP * 10 + 3) / 4],
-                                             double (&own_im)[(NSP * 10 + 3) / 4],
-                                             SkQuadStage<NSP, XT> &L) {
-  R br[NSP][10], bi[NSP][10];
+__device__ __forceinline__ void sk_bonds(const SkThread &t, uint2 local,
+                                         const SkLds<NSP, R, XT> &L, double (&acc)[10]) {
 #pragma unroll
-  for (int s = 0; s < NSP; ++s)
+  for (int o = 0; o < 10; ++o) acc[o] = 0.0;
 #pragma unroll
-    for (int c = 0; c < 10; ++c) br[s][c] = bi[s][c] = R(0);
-  R xr[NSP][10], xi[NSP][10];
-  sk_quad_gather<NSP, R, XT>(j, slot, xc, L, xr, xi);
-  if (j >= 0)
-    BondApply<NSP, R, CATION>::template run<0>(rv[0], rv[1], rv[2], rv + 3, xr,
-                                                xi, br, bi);
+  for (int n = 0; n < 2 * NSP; ++n) {
+    const int sh = NSP == 2 ? 8 * n : 8 * n + 16 * t.h;
+    const int lx = (local.x >> sh) & 0xff, lb = (local.y >> sh) & 0xff;
+    if (lx != 0xff) {
+      R k[24], x[10];
 #pragma unroll
-  for (int s = 0; s < NSP; ++s)
+      for (int i = 0; i < SkRec<R>::kChunks; ++i)
+        *reinterpret_cast<uint4 *>(&k[i * (16 / (int)sizeof(R))]) =
+            L.rec[lb * SkRec<R>::kStride + i];
+      sk_read_x<R, XT>(L.x + lx * SkX<NSP, XT>::kStride, t.comp, NSP == 2 ? 10 * t.h : 0, x);
+      if constexpr (sizeof(R) == 8) {
+        sk_apply<CATION, double>(k, x, acc);
+      } else {
+        float y[10];
 #pragma unroll
-    for (int c = 0; c < 10; ++c) {
-      const int r = s * 10 + c;
-      double re = double(br[s][c]), im = double(bi[s][c]);
-      re += quad_perm_f64<kQuadXor1>(re);
-      im += quad_perm_f64<kQuadXor1>(im);
-      re += quad_perm_f64<kQuadXor2>(re);
-      im += quad_perm_f64<kQuadXor2>(im);
-      if ((r & 3) == slot) {
-        own_re[r >> 2] = re;
-        own_im[r >> 2] = im;
+        for (int o = 0; o < 10; ++o) y[o] = 0.0f;
+        sk_apply<CATION, float>(k, x, y);
+#pragma unroll
+        for (int o = 0; o < 10; ++o) acc[o] += (double)y[o];
       }
     }
+  }
+  if constexpr (NSP == 1) {
+#pragma unroll
+    for (int o = 0; o < 10; ++o) acc[o] += dpp_f64<kQuadXor2>(acc[o]);
+  }
+}
+
+// y += the onsite terms of the thread's component x: diagonal - shift, surface
+// s-p couplings (surface: some atom of the wavefront has them), spin-orbit.
+template <int NSP>
+__device__ __forceinline__ void sk_onsite(const SkThread &t, const double (&x)[10],
+                                          const uint4 *place, double shift, bool surface,
+                                          double (&y)[10]) {
+  const double *os = reinterpret_cast<const double *>(place);
+#pragma unroll
+  for (int o = 0; o < 10; ++o) y[o] = __builtin_fma(os[o] - shift, x[o], y[o]);
+  if (surface) {
+    // couplings (1,2) (1,3) (1,4) (2,3) (2,4) (3,4)
+    const double s0 = os[10], s1 = os[11], s2 = os[12], s3 = os[13], s4 = os[14], s5 = os[15];
+    y[1] = __builtin_fma(s2, x[4], __builtin_fma(s1, x[3], __builtin_fma(s0, x[2], y[1])));
+    y[2] = __builtin_fma(s4, x[4], __builtin_fma(s3, x[3], __builtin_fma(s0, x[1], y[2])));
+    y[3] = __builtin_fma(s5, x[4], __builtin_fma(s3, x[2], __builtin_fma(s1, x[1], y[3])));
+    y[4] = __builtin_fma(s5, x[3], __builtin_fma(s4, x[2], __builtin_fma(s2, x[1], y[4])));
+  }
+  if constexpr (NSP == 2) {
+    // lambda L.S on the p orbitals; lanes 0..3: up re, up im, down re, down im
+    const double lam = os[16];
+    const double a1 = t.comp != t.h ? -lam : lam;  // + - - +
+    const double a2 = t.h ? -lam : lam;            // + + - -
+    const double a3 = t.comp ? -lam : lam;         // + - + -
+    const double x2_1 = dpp_f64<kQuadXor1>(x[2]), x3_1 = dpp_f64<kQuadXor1>(x[3]);
+    const double x4_2 = dpp_f64<kQuadXor2>(x[4]), x2_2 = dpp_f64<kQuadXor2>(x[2]);
+    const double x4_3 = dpp_f64<kQuadXor3>(x[4]), x3_3 = dpp_f64<kQuadXor3>(x[3]);
+    y[2] = __builtin_fma(a2, x4_2, __builtin_fma(a1, x3_1, y[2]));
+    y[3] = __builtin_fma(a3, x4_3, __builtin_fma(-a1, x2_1, y[3]));
+    y[4] = __builtin_fma(-a3, x3_3, __builtin_fma(-a2, x2_2, y[4]));
+  }
+}
+
+// The rest of a product once its bonds are summed: acc += the onsite terms
+// (own entries from LDS, onsite record os in the quad's chunks).  The barrier:
+// every wavefront has read the staged block; from then on each quad works on
+// its own two places only, of which the halo one is free for reuse.
+template <int NSP, typename R, typename XT>
+__device__ __forceinline__ void sk_finish(const SkThread &t, SkLds<NSP, R, XT> &L,
+                                          const uint4 (&os)[3], double shift, bool surface,
+                                          double (&acc)[10]) {
+  const uint4 *own = L.x + t.Q * SkX<NSP, XT>::kStride;
+  uint4 *halo = L.x + (kSkOwn + t.Q) * SkX<NSP, XT>::kStride;
+  double xo[10];
+  sk_read_x<double, XT>(own, t.comp, NSP == 2 ? 10 * t.h : 0, xo);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    if (4 * i + t.c < kOsChunks) halo[4 * i + t.c] = os[i];
+  wave_sync();
+  sk_onsite<NSP>(t, xo, halo, shift, surface, acc);
+  wave_sync();
+}
+// components -> entries (FP64) at `place`, from entry `first` on
+__device__ __forceinline__ void sk_entries(uint4 *place, int comp, int first,
+                                           const double (&y)[10]) {
+  double *p = reinterpret_cast<double *>(place + first) + comp;
+#pragma unroll
+  for (int o = 0; o < 10; ++o) p[2 * o] = y[o];
+}
+// the quad's chunks of the atom's onsite record
+__device__ __forceinline__ void sk_load_onsite(int atom, int c, const double *__restrict__ onsite,
+                                               uint4 (&os)[3]) {
+  const uint4 *p = reinterpret_cast<const uint4 *>(onsite) + (int64_t)atom * kOsChunks;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    os[i] = make_uint4(0, 0, 0, 0);
+    if (atom >= 0 && 4 * i + c < kOsChunks) os[i] = p[4 * i + c];
+  }
 }
 
 }  // namespace nh

@@ -60,7 +60,6 @@ struct nh_context {
   int n_atoms = 0;
   int n_species = 0;
   int n_cations = 0;
-  int n_anions = 0;
   int64_t n = 0;     // n_atoms * nb
   double lattice[3] = {0, 0, 0};
   int passivate = 0;
@@ -77,9 +76,12 @@ struct nh_context {
   double *disp = nullptr;       // [A][3]
   double *phi = nullptr;        // [A] or null
   int32_t *cations = nullptr;   // [Nc] atom index of each cation
-  int32_t *anions = nullptr;    // [Na] atom index of each anion
   int32_t *bond_of = nullptr;   // [A][4] cation-owned bond id (ci*4+slot)
   int32_t *rev_slot = nullptr;  // [A][4] slot of this atom in the nbr's list
+  // blocks of atoms of the SK / matrix-free products (SkTable, nh_hv_sk.h)
+  int n_blocks = 0;
+  int32_t *blk_own = nullptr, *blk_halo = nullptr, *blk_bonds = nullptr;
+  uint2 *blk_local = nullptr;
 
   // kernel variants (nh_context_set)
   // stored-block H·v: neighbour x staged in LDS (measured on the 786,520-
@@ -88,8 +90,6 @@ struct nh_context {
   int hv_staged = -1;  // NH_SET_HV_STAGED (-1: by layout, see use_staged)
   int ring_steps = 0;  // NH_SET_RING_STEPS (0: by free memory)
   int block_hv = -1;   // NH_SET_BLOCK_HV (-1: by measurement)
-  int sk_roles = -1;   // NH_SET_SK_ROLES (-1: default, sk_mixed_roles)
-  int sk_lanes = -1;   // NH_SET_SK_LANES (-1: default, sk_split_lanes)
   int lz_vectors = -1; // NH_SET_LZ_VECTORS (-1: default, lz_fp32_vectors)
 
   // assembled Hamiltonian
@@ -107,6 +107,7 @@ struct nh_context {
   int32_t *mf_q = nullptr;      // [A][4] ideal bond vector of the slot seen
                                 // from its cation, units a/4, 3 x int8
   double *mf_pair = nullptr;    // [S][S][kMfPair] (cation, anion) constants
+  int2 *mf_ends = nullptr;      // [blocks][192] atoms of the blocks' bonds
 
   // work buffers
   double *red = nullptr;        // reduction partials
@@ -137,27 +138,6 @@ inline bool sk_like(const nh_context *c) {
 }
 inline bool use_staged(const nh_context *c) {
   return c->hv_staged < 0 ? sk_like(c) : c->hv_staged != 0;
-}
-// SK / matrix-free products: both roles in one workgroup (waves 0-1 the
-// cations, waves 2-3 the anions at the same list position, so both rows of
-// a bond read its record within one workgroup) or one role per workgroup.
-// Default: both roles with FP64 products, one role with FP32 (measured on
-// a 786,520-atom dot, fused Lanczos kernel: FP64 0.329 against 0.338 ms,
-// FP32 0.230 against 0.229 ms)
-inline bool sk_mixed_roles(const nh_context *c) {
-  return c->sk_roles < 0 ? c->precision == NH_PREC_FP64 : c->sk_roles != 0;
-}
-// SK / matrix-free products of 20-band models with the LDS gather: 8 lanes
-// per atom (one per bond and spin block) instead of 4 (one per bond).
-// Default: 8 for matrix-free FP32 products only (measured on a 786,520-atom
-// dot, fused Lanczos kernel: matrix-free FP32 0.301 against 0.345 ms; SK
-// FP32 0.283 against 0.230, SK FP64 0.467 against 0.330, matrix-free FP64
-// 0.487 against 0.334 ms)
-inline bool sk_split_lanes(const nh_context *c) {
-  if (c->nb != 20 || !use_staged(c)) return false;
-  if (c->sk_lanes < 0)
-    return c->layout == NH_LAYOUT_MATRIX_FREE && c->precision == NH_PREC_FP32;
-  return c->sk_lanes == 8;
 }
 // Lanczos vectors stored in FP32 (FP32 SK or matrix-free products with the
 // LDS gather only).  Default on (measured on a 786,520-atom dot, FP32 SK

@@ -6,10 +6,11 @@
 //   k_lz_hv     q = r / beta_{k-1} (written into a ring slot), y = H q, and
 //               per-workgroup partials of alpha = Re<q, y>;
 //   k_lz_update r = y - alpha q - beta_{k-1} q_prev with partials of |r|^2.
-// With FP32 products and FP32 Lanczos vectors (SK and matrix-free layouts)
-// it is one kernel and one reduction: the product forms r_k from u_{k-1}
-// and r_{k-1} as it reads them, computes u_k = H q_k - beta_k q_{k-1} and
-// the partials of alpha_k, |u_k|^2 and |q_k|^2 (k_lz_hv_sk, Paige's order).
+// In the SK and matrix-free layouts it is one kernel (k_lz_sk, Paige's order;
+// FP32 products keep FP32 vectors): the product sums the previous step's
+// partials to alpha_{k-1} and beta_k, forms r_k from u_{k-1} and r_{k-1} as it
+// reads them, computes u_k = H q_k - beta_k q_{k-1} and the partials of
+// alpha_k, |u_k|^2 and |q_k|^2.
 // The reference's REDUCE_OPT variant of the iteration (lanczos.c:441-456)
 // defers the vector update into the next iteration in the same spirit, to
 // merge its two reductions into one.
@@ -21,9 +22,9 @@
 // recurrence (eigenvectorsLanczos, lanczos.c:1364-1689): the Lanczos
 // vectors land in a ring (K = 128 steps, fewer when memory is short) and
 // every K iterations one kernel adds Ring * Z to the eigenvector block.
-// The second pass reuses alpha and beta, so with the SK layout its H*v
-// kernel also applies the three-term step (no separate update kernel, no
-// reductions), and the ring holds the r vectors themselves.
+// The second pass reuses alpha and beta, so with the SK and matrix-free layouts
+// its H*v kernel writes r_{k+1} straight into the ring (no reductions), and the
+// ring holds the r vectors themselves.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -99,25 +100,6 @@ __global__ __launch_bounds__(kThreads) void k_lz_hv(
   }
 }
 
-// SK-layout variant of k_lz_hv (mapping of nh_hv_sk.h: 4 lanes per atom,
-// cation and anion workgroups).
-// Workgroup sum for the fused SK kernel: with the LDS gather the staging
-// area is reused (the kernel's LDS stays at 80 KB for two groups per CU).
-template <bool QUAD>
-struct LzBlockSum {
-  template <typename S>
-  __device__ __forceinline__ static void run(double &a, double &b, S *) {
-    block_sum2(a, b);
-  }
-};
-template <>
-struct LzBlockSum<true> {
-  template <typename S>
-  __device__ __forceinline__ static void run(double &a, double &b, S *L) {
-    block_sum2_lds(a, b, reinterpret_cast<double *>(L->buf));
-  }
-};
-
 // One element of the three-term step y - alpha q - beta_prev q_prev with
 // q_prev = r_prev * (1 / beta_prev2); rp null on the first step.  The
 // operations are spelled out (explicit fma, y kept opaque) so that the
@@ -149,406 +131,249 @@ __device__ __forceinline__ double2 lz_three_term(double2 y, double2 q,
                          rp ? widen2(*rp) : make_double2(0.0, 0.0), al, be, invp);
 }
 
-// FP32 Lanczos vectors (Paige's order of the step): u_k = H q_k - beta_k
-// q_{k-1} computed in FP64 and rounded to FP32, alpha_k = <q_k, u_k>,
-// r_{k+1} = u_k - alpha_k q_k (lz_defer1).  y is kept opaque so that every
-// kernel rounds u_k from the same two operations.
-__device__ __forceinline__ float2 lz_u32(double2 y, double2 rp, double be, double invp) {
-  asm volatile("" : "+v"(y.x), "+v"(y.y));
-  return make_float2((float)__builtin_fma(-be, rp.x * invp, y.x),
-                     (float)__builtin_fma(-be, rp.y * invp, y.y));
+// Paige's order of the step: u_k = H q_k - beta_k q_{k-1} (FP64 arithmetic,
+// rounded once to FP32 vectors), alpha_k = <q_k, u_k>, r_{k+1} = u_k -
+// alpha_k q_k (lz_defer1).
+__device__ __forceinline__ double lz_u(double y, double rp, double be, double invp) {
+  return __builtin_fma(-be, rp * invp, y);
 }
-// per-workgroup partials of the FP32-vector eigenvalue pass: alpha_k,
-// |u_k|^2, |q_k|^2 (beta_{k+1}^2 = |u|^2 - 2 alpha^2 + alpha^2 |q|^2)
+// partials of an eigenvalue-pass step: alpha_k, |u_k|^2, |q_k|^2
+// (beta_{k+1}^2 = |u|^2 - 2 alpha^2 + alpha^2 |q|^2)
 struct LzPart3 {
   double a = 0.0, u = 0.0, q = 0.0;
-  __device__ __forceinline__ void add(double2 qv, float2 uv) {
-    const double ux = uv.x, uy = uv.y;
-    a += qv.x * ux + qv.y * uy;
-    u += ux * ux + uy * uy;
-    q += qv.x * qv.x + qv.y * qv.y;
-  }
-  template <bool QUAD, typename S>
-  __device__ __forceinline__ void store(double *part, S *L) {
-    LzBlockSum<QUAD>::run(a, u, L);
-    double z = 0.0;
-    LzBlockSum<QUAD>::run(q, z, L);
-    if (threadIdx.x == 0) {
-      part[3 * blockIdx.x] = a;
-      part[3 * blockIdx.x + 1] = u;
-      part[3 * blockIdx.x + 2] = q;
-    }
+  __device__ __forceinline__ void add(double qv, double uv) {
+    a = __builtin_fma(qv, uv, a);
+    u = __builtin_fma(uv, uv, u);
+    q = __builtin_fma(qv, qv, q);
   }
 };
-
-// Epilogue staging of the FP32-vector kernels: the atom's own entries of
-// r_k and r_{k-1} (FP32) and its onsite record
-template <int NSP, int ATOMS = kSkAtomsPerBlock>
-struct SkOwnStage32 {
-  float2 x[ATOMS][NSP * 10];
-  float2 rp[ATOMS][NSP * 10];
-  double2 os[ATOMS][kOnsiteStride / 2];
-};
-
-// XO: storage of the Lanczos vectors r.  double2: FP64 r (own entries,
-// r_prev) with an FP32 copy for the gathers of FP32 products.  float2
-// (FP32 products, LDS gather): the vectors are FP32 and the step runs in
-// Paige's order (lz_u32, lz_defer1).  Eigenvalue pass: Rv = u_{k-1}, Rp =
-// r_{k-1}; r_k is formed on the fly (gather and own entries) and written
-// to Rout, u_k to Y32, the partials of LzPart3 to part (no update
-// kernel).  Eigenvector pass (FUSE): Rv = Rv32 = r_k, Rp = r_{k-1}, the
-// rounded r_{k+1} to Y32.  The step's arithmetic stays FP64.
-template <int NSP, typename R, bool QUAD, bool FUSE, typename SRC, typename XO = double2>
-__global__ __launch_bounds__(kSkThreads, sizeof(R) == 4 ? 4 : 2) void k_lz_hv_sk(
-    int nc, const int32_t *__restrict__ cations, int na,
-    const int32_t *__restrict__ anions, SkGrid grid,
-    const double *__restrict__ onsite, const SRC src,
-    const int32_t *__restrict__ nbr, const XO *__restrict__ Rv, const float2 *__restrict__ Rv32,
-    double2 *__restrict__ Q, double2 *__restrict__ Y,
-    const double *__restrict__ beta_prev, double *__restrict__ part,
-    const double *__restrict__ alpha, const XO *__restrict__ Rp,
-    const double *__restrict__ beta_prev2, float2 *__restrict__ Y32,
-    float2 *__restrict__ Rout, const double *__restrict__ alpha_prev) {
-  constexpr int NB = NSP * 10;
-  constexpr bool V32 = std::is_same<XO, float2>::value;
-  constexpr bool DEFER = V32 && !FUSE;
-  static_assert(!V32 || (sizeof(R) == 4 && QUAD),
-                "FP32 Lanczos vectors need FP32 products and the LDS gather");
-  constexpr int NO = (NB + 3) / 4;
-  const SkLane ln = sk_lane_of(grid, blockIdx.x, threadIdx.x);
-  // the role is uniform across the wavefront; read as a scalar, the role
-  // branches below are scalar branches (one per wave)
-  const bool cat = __builtin_amdgcn_readfirstlane((int)ln.cat) != 0;
-  const int li = ln.li;
-  const int slot = threadIdx.x & 3;
-  const bool active = li < (cat ? nc : na);
-  const int atom = active ? (cat ? cations[li] : anions[li]) : 0;
-  const double inv = beta_prev ? 1.0 / beta_prev[0] : 1.0;
-  // FUSE (eigenvector pass): alpha is known, so the three-term step of
-  // k_lz_update is applied here and Y receives r_{k+1}
-  const double al = FUSE ? alpha[0] : 0.0;
-  const double be = beta_prev ? beta_prev[0] : 0.0;
-  const double invp = beta_prev2 ? 1.0 / beta_prev2[0] : 1.0;
-  double own_re[NO], own_im[NO];
-  // FP32 products gather from the FP32 copy of r (the same rounding as
-  // converting the FP64 entries on load)
-  using XT = typename std::conditional<sizeof(R) == 4, float2, double2>::type;
-  const XT *xg;
-  if constexpr (sizeof(R) == 4) xg = Rv32;
-  else xg = Rv;
-  // DEFER: r_k = lz_defer1(u_{k-1}, r_{k-1}, alpha_{k-1} / beta_{k-1});
-  // FUSE: r_{k+1} = lz_defer1(u_k, r_k, alpha_k / beta_k)
-  const double alp = DEFER && alpha_prev ? alpha_prev[0] : 0.0;
-  const LzCoef ap = lz_defer_coef(alp, invp), af = lz_defer_coef(al, inv);
-  LzDeferSrc dsrc{nullptr, ap};
-  if constexpr (DEFER) dsrc.rp = Rp;
-  SkQuadStage<NSP, XT> *L = nullptr;
-  if constexpr (QUAD) {
-    __shared__ SkQuadStage<NSP, XT> stage;
-    L = &stage;
+// sums of three values over a workgroup of kRedThreads in a fixed order, in
+// every thread; scratch: 3 * kRedThreads / 64 doubles
+__device__ __forceinline__ void lz_block_sum3(double (&s)[3], double *scratch) {
+  constexpr int kWaves = kRedThreads / 64;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s[c] += __shfl_xor(s[c], off, 64);
+    if ((threadIdx.x & 63) == 0) scratch[c * kWaves + (threadIdx.x >> 6)] = s[c];
   }
-  if (cat)
-    sk_bonds<NSP, R, true, XT, QUAD, DEFER>(atom, slot, active, src, nbr, xg, own_re,
-                                            own_im, L, dsrc);
-  else
-    sk_bonds<NSP, R, false, XT, QUAD, DEFER>(atom, slot, active, src, nbr, xg, own_re,
-                                             own_im, L, dsrc);
-  double local = 0.0;
-  LzPart3 p3;
-  if constexpr (V32) {
-    // FP32 vectors: the atom's own entries of r_k (DEFER: of u_{k-1}) and
-    // r_{k-1} are requested in 16-byte pieces of two entries (lane `slot`
-    // takes pieces slot, slot + 4, ...), with the onsite record, before the
-    // epilogue's barriers, and staged in FP32 in the freed LDS; each lane
-    // then finishes its rows 4 i + slot from there
-    static_assert(sizeof(SkOwnStage32<NSP>) <= sizeof(SkQuadStage<NSP, XT>),
-                  "epilogue staging must fit the gather staging");
-    auto &S = *reinterpret_cast<SkOwnStage32<NSP> *>(L->buf);
-    const int la = threadIdx.x / 4;
-    constexpr int NC = NB / 2, NCL = (NC + 3) / 4;
-    constexpr int KOS = SkOwnRegs<NSP>::kOs;
-    float4 cx[NCL], cp[NCL];
-    double2 co[KOS];
+  __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NCL; ++i) cx[i] = cp[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int c = 0; c < 3; ++c) {
+    s[c] = scratch[c * kWaves];
 #pragma unroll
-    for (int i = 0; i < KOS; ++i) co[i] = make_double2(0.0, 0.0);
-    if (active) {
-      const float4 *xs = reinterpret_cast<const float4 *>(Rv + (int64_t)atom * NB);
-      const float4 *ps = reinterpret_cast<const float4 *>(Rp + (int64_t)atom * NB);
-#pragma unroll
-      for (int i = 0; i < NCL; ++i) {
-        const int c = 4 * i + slot;
-        if (c < NC) {
-          cx[i] = xs[c];
-          cp[i] = ps[c];
-        }
-      }
-      const double2 *o2 = reinterpret_cast<const double2 *>(onsite + (size_t)atom * kOnsiteStride);
-#pragma unroll
-      for (int i = 0; i < KOS; ++i) {
-        const int c = 4 * i + slot;
-        if (c < kOnsiteStride / 2) co[i] = o2[c];
-      }
-      if constexpr (DEFER) {
-        // r_k from u_{k-1} and r_{k-1}, written out for the next step
-#pragma unroll
-        for (int i = 0; i < NCL; ++i) {
-          const int c = 4 * i + slot;
-          if (c < NC) {
-            cx[i] = make_float4(lz_defer1(cx[i].x, cp[i].x, ap), lz_defer1(cx[i].y, cp[i].y, ap),
-                                lz_defer1(cx[i].z, cp[i].z, ap), lz_defer1(cx[i].w, cp[i].w, ap));
-            if (Rout) reinterpret_cast<float4 *>(Rout + (int64_t)atom * NB)[c] = cx[i];
-          }
-        }
-      }
-    }
-    __syncthreads();  // every lane has read its staged neighbour entries
-    if (active) {
-#pragma unroll
-      for (int i = 0; i < NCL; ++i) {
-        const int c = 4 * i + slot;
-        if (c < NC) {
-          S.x[la][2 * c] = make_float2(cx[i].x, cx[i].y);
-          S.x[la][2 * c + 1] = make_float2(cx[i].z, cx[i].w);
-          S.rp[la][2 * c] = make_float2(cp[i].x, cp[i].y);
-          S.rp[la][2 * c + 1] = make_float2(cp[i].z, cp[i].w);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < KOS; ++i) {
-        const int c = 4 * i + slot;
-        if (c < kOnsiteStride / 2) S.os[la][c] = co[i];
-      }
-    }
-    __syncthreads();
-    if (active) {
-#pragma unroll
-      for (int i = 0; i < NO; ++i) {
-        const int r = 4 * i + slot;
-        if (r >= NB) break;
-        double re = own_re[i], im = own_im[i];
-        onsite_row<NSP>(reinterpret_cast<const double *>(S.os[la]), S.x[la],
-                        r / 10, r % 10, 0.0, re, im);
-        const float2 xf = S.x[la][r];
-        const double2 q = make_double2((double)xf.x * inv, (double)xf.y * inv);
-        const int64_t e = (int64_t)atom * NB + r;
-        const double2 y = make_double2(re * inv, im * inv);
-        const float2 u = lz_u32(y, widen2(S.rp[la][r]), be, invp);
-        if constexpr (FUSE) {
-          Y32[e] = make_float2(lz_defer1(u.x, xf.x, af), lz_defer1(u.y, xf.y, af));
-        } else {
-          Y32[e] = u;
-          p3.add(q, u);
-        }
-      }
-    }
-  } else if constexpr (QUAD) {
-    static_assert(sizeof(SkOwnStage<NSP>) <= sizeof(SkQuadStage<NSP, XT>),
-                  "epilogue staging must fit the gather staging");
-    auto &S = *reinterpret_cast<SkOwnStage<NSP> *>(L->buf);
-    const int la = threadIdx.x / 4;
-    // own entries, onsite record and (FUSE) r_prev of the lane's rows are
-    // loaded before the epilogue's barriers, so the loads overlap them; the
-    // first two are staged in the freed LDS after the first barrier
-    SkOwnRegs<NSP> own;
-    if (active)
-      sk_load_own<NSP>(slot, Rv + (int64_t)atom * NB,
-                       onsite + (size_t)atom * kOnsiteStride, own);
-    double2 rpv[NO];
-#pragma unroll
-    for (int i = 0; i < NO; ++i) rpv[i] = make_double2(0.0, 0.0);
-    if constexpr (FUSE) {
-      if (active && Rp) {
-#pragma unroll
-        for (int i = 0; i < NO; ++i)
-          if (4 * i + slot < NB) rpv[i] = widen2(Rp[(int64_t)atom * NB + 4 * i + slot]);
-      }
-    }
-    __syncthreads();  // every lane has read its staged neighbour entries
-    if (active) sk_store_own<NSP>(la, slot, own, S);
-    __syncthreads();
-    if (active) {
-#pragma unroll
-      for (int i = 0; i < NO; ++i) {
-        const int r = 4 * i + slot;
-        if (r >= NB) break;
-        double re = own_re[i], im = own_im[i];
-        onsite_row<NSP>(reinterpret_cast<const double *>(S.os[la]), S.x[la],
-                        r / 10, r % 10, 0.0, re, im);
-        const double2 q = make_double2(own.x[i].x * inv, own.x[i].y * inv);
-        const int64_t e = (int64_t)atom * NB + r;
-        double2 y = make_double2(re * inv, im * inv);
-        if constexpr (FUSE) {
-          y = lz_three_term_v(y, q, Rp != nullptr, rpv[i], al, be, invp);
-          if (Y32) Y32[e] = make_float2((float)y.x, (float)y.y);
-        }
-        if (Q) Q[e] = q;
-        Y[e] = y;
-        local += q.x * y.x + q.y * y.y;
-      }
-    }
-  } else if (active) {
-    const double *os = onsite + (size_t)atom * kOnsiteStride;
-    const XO *xa = Rv + (int64_t)atom * NB;
-#pragma unroll
-    for (int i = 0; i < NO; ++i) {
-      const int r = 4 * i + slot;
-      if (r >= NB) break;
-      double re = own_re[i], im = own_im[i];
-      onsite_row<NSP>(os, xa, r / 10, r % 10, 0.0, re, im);
-      const double2 xr = widen2(xa[r]);
-      const double2 q = make_double2(xr.x * inv, xr.y * inv);
-      const int64_t e = (int64_t)atom * NB + r;
-      double2 y = make_double2(re * inv, im * inv);
-      if constexpr (FUSE) {
-        y = lz_three_term(y, q, Rp ? Rp + e : nullptr, al, be, invp);
-        if (Y32) Y32[e] = make_float2((float)y.x, (float)y.y);
-      }
-      if (Q) Q[e] = q;
-      Y[e] = y;
-      local += q.x * y.x + q.y * y.y;
-    }
+    for (int w = 1; w < kWaves; ++w) s[c] += scratch[c * kWaves + w];
   }
-  if (part) {
-    if constexpr (DEFER) {
-      p3.store<QUAD>(part, L);
-    } else {
-      double z = 0.0;
-      LzBlockSum<QUAD>::run(local, z, L);  // QUAD: reuses the staging LDS
-      if (threadIdx.x == 0) part[blockIdx.x] = local;
-    }
+}
+// alpha_k and beta_{k+1} from the partials of nparts workgroups (fixed order:
+// every workgroup that evaluates it gets the same bits)
+__device__ __forceinline__ void lz_scalars3(int nparts, const double *__restrict__ part,
+                                            double *scratch, double &alpha, double &beta) {
+  double s[3] = {0.0, 0.0, 0.0};
+  for (int k = threadIdx.x; k < nparts; k += kRedThreads)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) s[c] += part[3 * k + c];
+  lz_block_sum3(s, scratch);
+  alpha = s[0];
+  beta = sqrt(fmax(s[1] - 2.0 * s[0] * s[0] + s[0] * s[0] * s[2], 0.0));
+}
+__global__ __launch_bounds__(kRedThreads) void k_lz_scalars3(
+    int nparts, const double *__restrict__ part, double *__restrict__ alpha,
+    double *__restrict__ beta) {
+  __shared__ double scratch[3 * kRedThreads / 64];
+  double a, b;
+  lz_scalars3(nparts, part, scratch, a, b);
+  if (threadIdx.x == 0) {
+    alpha[0] = a;
+    beta[0] = b;
   }
 }
 
-// k_lz_hv_sk with 8 lanes per atom of a 20-band model (SkSplit: lane =
-// spin block and bond), LDS gather; the same epilogue with lane (spin s,
-// slot) finishing rows s * 10 + 4 i + slot.  Fewer vector registers per
-// lane than k_lz_hv_sk (one spin block of the neighbour and of the
-// accumulators), so more waves fit on a SIMD.
-template <typename R, bool FUSE, typename SRC, typename XO = double2>
-__global__ __launch_bounds__(kSkThreads, sizeof(R) == 4 ? 5 : 3) void k_lz_hv_sk_split(
-    int nc, const int32_t *__restrict__ cations, int na,
-    const int32_t *__restrict__ anions, SkGrid grid,
-    const double *__restrict__ onsite, const SRC src,
-    const int32_t *__restrict__ nbr, const XO *__restrict__ Rv, const float2 *__restrict__ Rv32,
-    double2 *__restrict__ Q, double2 *__restrict__ Y,
-    const double *__restrict__ beta_prev, double *__restrict__ part,
-    const double *__restrict__ alpha, const XO *__restrict__ Rp,
-    const double *__restrict__ beta_prev2, float2 *__restrict__ Y32,
-    float2 *__restrict__ Rout, const double *__restrict__ alpha_prev) {
-  constexpr int NSP = 2, NB = 20;
-  constexpr bool V32 = std::is_same<XO, float2>::value;
-  constexpr bool DEFER = V32 && !FUSE;
-  static_assert(!V32 || sizeof(R) == 4, "FP32 Lanczos vectors need FP32 products");
-  constexpr int kLanes = SkSplit::kLanes, kAtoms = SkSplit::kAtoms;
-  const SkLane ln = sk_lane_of<kLanes>(grid, blockIdx.x, threadIdx.x);
-  // the role is uniform across the wavefront (scalar role branches)
-  const bool cat = __builtin_amdgcn_readfirstlane((int)ln.cat) != 0;
-  const int li = ln.li;
-  const int lane = threadIdx.x & (kLanes - 1), slot = lane & 3, spin = lane >> 2;
-  const bool active = li < (cat ? nc : na);
-  const int atom = active ? (cat ? cations[li] : anions[li]) : 0;
-  const double inv = beta_prev ? 1.0 / beta_prev[0] : 1.0;
-  const double al = FUSE ? alpha[0] : 0.0;
-  const double be = beta_prev ? beta_prev[0] : 0.0;
-  const double invp = beta_prev2 ? 1.0 / beta_prev2[0] : 1.0;
-  double own_re[SkSplit::kOwn], own_im[SkSplit::kOwn];
-  using XT = typename std::conditional<sizeof(R) == 4, float2, double2>::type;
-  const XT *xg;
-  if constexpr (sizeof(R) == 4) xg = Rv32;
-  else xg = Rv;
-  const double alp = DEFER && alpha_prev ? alpha_prev[0] : 0.0;
-  const LzCoef ap = lz_defer_coef(alp, invp), af = lz_defer_coef(al, inv);
-  LzDeferSrc dsrc{nullptr, ap};
-  if constexpr (DEFER) dsrc.rp = Rp;
-  __shared__ SkQuadStage<1, XT> stage;
-  if (cat)
-    sk_bonds_split<R, true, XT, DEFER>(atom, slot, spin, active, src, nbr, xg, own_re,
-                                       own_im, stage, dsrc);
-  else
-    sk_bonds_split<R, false, XT, DEFER>(atom, slot, spin, active, src, nbr, xg, own_re,
-                                        own_im, stage, dsrc);
-  static_assert(sizeof(SkOwnStage<NSP, kAtoms>) <= sizeof(SkQuadStage<1, XT>),
-                "epilogue staging must fit the gather staging");
-  auto &S = *reinterpret_cast<SkOwnStage<NSP, kAtoms> *>(stage.buf);
-  const int la = threadIdx.x / kLanes;
-  SkOwnRegs<NSP, kLanes> own;
-  if (active)
-    sk_load_own<NSP, kLanes>(lane, Rv + (int64_t)atom * NB,
-                             onsite + (size_t)atom * kOnsiteStride, own);
-  double2 rpv[SkSplit::kOwn];
-#pragma unroll
-  for (int i = 0; i < SkSplit::kOwn; ++i) rpv[i] = make_double2(0.0, 0.0);
-  if constexpr (FUSE || DEFER) {
-    if (active && Rp) {
-#pragma unroll
-      for (int i = 0; i < SkSplit::kOwn; ++i)
-        if (4 * i + slot < 10)
-          rpv[i] = widen2(Rp[(int64_t)atom * NB + spin * 10 + 4 * i + slot]);
-    }
-  }
-  if constexpr (DEFER) {
-    // own entries of r_k (entries 8 i + lane, as loaded) from u_{k-1} and
-    // r_{k-1}; written out for the next step
-    if (active) {
-#pragma unroll
-      for (int i = 0; i < (NB + kLanes - 1) / kLanes; ++i) {
-        const int r = kLanes * i + lane;
-        if (r >= NB) break;
-        const float2 rq = Rp[(int64_t)atom * NB + r];
-        const float2 rk = make_float2(lz_defer1((float)own.x[i].x, rq.x, ap),
-                                      lz_defer1((float)own.x[i].y, rq.y, ap));
-        own.x[i] = widen2(rk);
-        if (Rout) Rout[(int64_t)atom * NB + r] = rk;
+// The SK / matrix-free product of a Lanczos step (block mapping of
+// nh_hv_sk.h), V: storage of the vectors.
+//  Deferred (Paige's order; FP64 vectors with FP64 products, FP32 vectors
+//  with FP32 products):
+//   kLzValues  eigenvalue pass, the whole step in one launch: the previous
+//     launch's partials give alpha_{k-1}, beta_k (each workgroup sums them,
+//     workgroup 0 stores them); r_k = u_{k-1} - .. r_{k-1} is formed from x =
+//     u_{k-1} and rp = r_{k-1} as the block is staged, u_k goes to out, r_k to
+//     rout, the partials to part;
+//   kLzVectors eigenvector pass: x = r_k, rp = r_{k-1}, r_{k+1} to out.
+//  Classic (FP64 vectors; products of either precision):
+//   kLzProduct eigenvalue pass, before k_lz_update: y = H q_k to out, partials
+//     of alpha_k;
+//   kLzFused   eigenvector pass: with the three-term step, r_{k+1} to out.
+// In both pairs the second pass evaluates the first one's expressions on the
+// same operands and so retraces it bit for bit (sk_apply and the step spell
+// their multiply-adds out).
+// Why deferred: an FP64 step moves H and four vectors (u, r read, u, r
+// written) instead of H and six in two launches with two reductions between
+// them: 786,520 atoms, SK 0.528 -> 0.366 ms a step, 4,336,640 atoms,
+// matrix-free 3.07 -> 2.07 ms, 3,888 atoms 21 -> 10 us.
+enum { kLzProduct = 0, kLzFused = 1, kLzValues = 2, kLzVectors = 3 };
+template <typename V>
+struct LzArgs {
+  const V *x, *rp;
+  V *out, *rout;
+  const double *alpha, *beta_prev, *beta_prev2;  // beta null: 1 (start vector)
+  const double *part_prev;  // kLzValues: partials of the previous step
+  int nparts;
+  double *alpha_out, *beta_out;  // .. whose alpha and beta go here
+  double *part;
+};
+template <int MODE, int NSP, typename R, typename V, typename SRC>
+__global__ __launch_bounds__(kSkThreads, sizeof(V) == 8 ? 3 : 2) void k_lz_sk(
+    SkTable tab, const double *__restrict__ onsite, const SRC src, const LzArgs<V> g) {
+  constexpr bool VALUES = MODE == kLzValues, DEFER = MODE >= kLzValues;
+  static_assert(DEFER || sizeof(V) == 16, "the classic step keeps FP64 vectors");
+  static_assert(sizeof(R) == sizeof(V) / 2 || !DEFER, "deferred vectors have the products' type");
+  static_assert(kSkThreads == kRedThreads, "block sums");
+  using S = SkX<NSP, V>;
+  __shared__ SkLds<NSP, R, V> L;
+  const SkThread t;
+  SkWalk w(tab);
+  const bool cat = __builtin_amdgcn_readfirstlane(t.Q) < kSkOwn / 2;
+  uint4 *own = L.x + t.Q * S::kStride, *halo = L.x + (kSkOwn + t.Q) * S::kStride;
+  double *scratch = reinterpret_cast<double *>(L.rec);
+  double be = g.beta_prev ? g.beta_prev[0] : 0.0;
+  double inv = g.beta_prev ? 1.0 / be : 1.0;
+  const double invp = g.beta_prev2 ? 1.0 / g.beta_prev2[0] : 1.0;
+  const double al = MODE == kLzFused || MODE == kLzVectors ? g.alpha[0] : 0.0;
+  SkIndex<SRC> ix;
+  if (w.b < w.end) ix.read(tab, src, w.b, t.Q);
+  LzCoef<V> ap{};
+  if constexpr (VALUES) {
+    double alp = 0.0;
+    if (g.part_prev) {
+      lz_scalars3(g.nparts, g.part_prev, scratch, alp, be);
+      inv = 1.0 / be;
+      if (blockIdx.x == 0 && threadIdx.x == 0) {
+        g.alpha_out[0] = alp;
+        g.beta_out[0] = be;
       }
+      __syncthreads();  // the scratch is the records' place
     }
+    ap = lz_defer_coef<V>(alp, invp);
   }
-  __syncthreads();  // every lane has read its staged neighbour entries
-  if (active) sk_store_own<NSP, kLanes, kAtoms>(la, lane, own, S);
-  __syncthreads();
-  double local = 0.0;
+  const LzCoef<V> af = lz_defer_coef<V>(al, inv);
   LzPart3 p3;
-  if (active) {
+  double local = 0.0;
+  while (w.b < w.end) {
+    const int atom = ix.own;
+    typename SRC::Data rec;
+    uint4 xo[S::kLoads], xh[S::kLoads], os[3];
+    sk_load_x<NSP>(atom, t.c, g.x, xo);
+    sk_load_x<NSP>(ix.halo, t.c, g.x, xh);
+    if constexpr (VALUES) {
+      uint4 po[S::kLoads], ph[S::kLoads];
+      sk_load_x<NSP>(atom, t.c, g.rp, po);
+      sk_load_x<NSP>(ix.halo, t.c, g.rp, ph);
+      src.load(ix.rec, rec);
+      sk_load_onsite(atom, t.c, onsite, os);
+      sk_defer<V>(xo, po, ap);
+      sk_defer<V>(xh, ph, ap);
+      if (g.rout && atom >= 0) {
+        uint4 *o = reinterpret_cast<uint4 *>(g.rout) + (int64_t)atom * S::kChunks;
 #pragma unroll
-    for (int i = 0; i < SkSplit::kOwn; ++i) {
-      const int c = 4 * i + slot;
-      if (c >= 10) break;
-      const int r = spin * 10 + c;
-      double re = own_re[i], im = own_im[i];
-      onsite_row<NSP>(reinterpret_cast<const double *>(S.os[la]), S.x[la], spin, c,
-                      0.0, re, im);
-      const double2 xo = S.x[la][r];
-      const double2 q = make_double2(xo.x * inv, xo.y * inv);
-      const int64_t e = (int64_t)atom * NB + r;
-      double2 y = make_double2(re * inv, im * inv);
-      if constexpr (V32) {
-        const float2 u = lz_u32(y, rpv[i], be, invp);
-        if constexpr (FUSE) {
-          Y32[e] = make_float2(lz_defer1(u.x, (float)xo.x, af),
-                               lz_defer1(u.y, (float)xo.y, af));
-        } else {
-          Y32[e] = u;
-          p3.add(q, u);
-        }
-      } else {
-        if constexpr (FUSE) {
-          y = lz_three_term_v(y, q, Rp != nullptr, rpv[i], al, be, invp);
-          if (Y32) Y32[e] = make_float2((float)y.x, (float)y.y);
-        }
-        if (Q) Q[e] = q;
-        Y[e] = y;
-        local += q.x * y.x + q.y * y.y;
+        for (int i = 0; i < S::kLoads; ++i)
+          if (4 * i + t.c < S::kChunks) o[4 * i + t.c] = xo[i];
       }
+    } else {
+      src.load(ix.rec, rec);
+      sk_load_onsite(atom, t.c, onsite, os);
+    }
+    const uint2 lc = ix.local;
+    const bool surface = sk_surface(atom, lc);
+    w.b += w.step;
+    if (w.b < w.end) ix.read(tab, src, w.b, t.Q);
+    src.stage(rec, L.rec);
+    sk_stage_x<NSP, V>(own, t.c, xo);
+    sk_stage_x<NSP, V>(halo, t.c, xh);
+    __syncthreads();
+    double acc[10];
+    if (cat) sk_bonds<NSP, R, true, V>(t, lc, L, acc);
+    else sk_bonds<NSP, R, false, V>(t, lc, L, acc);
+    // own r_{k-1}, requested before the barrier of sk_finish
+    constexpr int kSpins = sizeof(V) == 8 ? NSP : 1;      // FP32: a spin at a time
+    constexpr int kPer = S::kChunks / kSpins, kPl = (kPer + 3) / 4;
+    uint4 rp[kSpins][kPl];
+#pragma unroll
+    for (int s = 0; s < kSpins; ++s)
+#pragma unroll
+      for (int i = 0; i < kPl; ++i) {
+        rp[s][i] = make_uint4(0, 0, 0, 0);
+        if (MODE != kLzProduct && g.rp && atom >= 0 && 4 * i + t.c < kPer)
+          rp[s][i] = reinterpret_cast<const uint4 *>(g.rp)[(int64_t)atom * S::kChunks + s * kPer +
+                                                           4 * i + t.c];
+      }
+    sk_finish<NSP, R, V>(t, L, os, 0.0, surface, acc);
+    uint4 *out = reinterpret_cast<uint4 *>(g.out) + (int64_t)atom * S::kChunks;
+#pragma unroll
+    for (int s = 0; s < kSpins; ++s) {
+      // entries of y = H r_k in the halo place: all of them, or those of spin s
+      if (kSpins == 1 ? NSP == 2 || t.h == 0 : t.h == s)
+        sk_entries(halo, t.comp, kSpins == 1 && NSP == 2 ? 10 * t.h : 0, acc);
+      wave_sync();
+      if (atom >= 0) {
+#pragma unroll
+        for (int i = 0; i < kPl; ++i) {
+          const int q = 4 * i + t.c;
+          if (q >= kPer) break;
+          const uint4 rk4 = own[s * kPer + q];
+          uint4 o4;
+          if constexpr (sizeof(V) == 16) {
+            const double2 y = *reinterpret_cast<const double2 *>(&halo[q]);
+            const double2 rk = *reinterpret_cast<const double2 *>(&rk4);
+            const double2 rm = *reinterpret_cast<const double2 *>(&rp[s][i]);
+            const double2 qk = make_double2(rk.x * inv, rk.y * inv);
+            double2 o = make_double2(y.x * inv, y.y * inv);
+            if constexpr (MODE == kLzFused) {
+              o = lz_three_term_v(o, qk, g.rp != nullptr, rm, al, be, invp);
+            } else if constexpr (DEFER) {
+              o = make_double2(lz_u(o.x, rm.x, be, invp), lz_u(o.y, rm.y, be, invp));
+              if constexpr (MODE == kLzVectors) {
+                o = make_double2(lz_defer1(o.x, rk.x, af), lz_defer1(o.y, rk.y, af));
+              } else {
+                p3.add(qk.x, o.x);
+                p3.add(qk.y, o.y);
+              }
+            } else {
+              local += qk.x * o.x + qk.y * o.y;
+            }
+            o4 = *reinterpret_cast<const uint4 *>(&o);
+          } else {
+            const float *rk = reinterpret_cast<const float *>(&rk4);
+            const float *rm = reinterpret_cast<const float *>(&rp[s][i]);
+            const double *y = reinterpret_cast<const double *>(&halo[2 * q]);
+            float *o = reinterpret_cast<float *>(&o4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float u = (float)lz_u(y[e] * inv, (double)rm[e], be, invp);
+              if constexpr (MODE == kLzVectors) {
+                o[e] = lz_defer1(u, rk[e], af);
+              } else {
+                o[e] = u;
+                p3.add((double)rk[e] * inv, (double)u);
+              }
+            }
+          }
+          out[s * kPer + q] = o4;
+        }
+      }
+      wave_sync();
     }
   }
-  if (part) {
-    if constexpr (DEFER) {
-      p3.store<true>(part, &stage);
-    } else {
-      double z = 0.0;
-      LzBlockSum<true>::run(local, z, &stage);
-      if (threadIdx.x == 0) part[blockIdx.x] = local;
+  if constexpr (VALUES || MODE == kLzProduct) {
+    double s[3] = {VALUES ? p3.a : local, p3.u, p3.q};
+    __syncthreads();  // the last block's records have been read
+    lz_block_sum3(s, scratch);
+    if (threadIdx.x == 0) {
+      if constexpr (VALUES) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) g.part[3 * blockIdx.x + c] = s[c];
+      } else {
+        g.part[blockIdx.x] = s[0];
+      }
     }
   }
 }
@@ -558,12 +383,11 @@ __global__ __launch_bounds__(kSkThreads, sizeof(R) == 4 ? 5 : 3) void k_lz_hv_sk
 // as the fused H·v kernel's q, so the trajectory does not depend on whether
 // q was stored), partial sums of |y|^2.  Rp may be null (first step), and
 // beta_prev / beta_prev2 null mean 1 (the start vector is normalised).
-// Y32 (optional): FP32 copy of the new r for the next FP32 product.
 __global__ __launch_bounds__(kRedThreads) void k_lz_update(
     int64_t n, double2 *__restrict__ Y, const double2 *__restrict__ Rk,
     const double2 *__restrict__ Rp, const double *__restrict__ alpha,
     const double *__restrict__ beta_prev, const double *__restrict__ beta_prev2,
-    double *__restrict__ part, float2 *__restrict__ Y32) {
+    double *__restrict__ part) {
   const double al = alpha[0];
   const double be = beta_prev ? beta_prev[0] : 0.0;
   const double inv = beta_prev ? 1.0 / beta_prev[0] : 1.0;
@@ -575,7 +399,6 @@ __global__ __launch_bounds__(kRedThreads) void k_lz_update(
     const double2 q = make_double2(r.x * inv, r.y * inv);
     const double2 y = lz_three_term(Y[k], q, Rp ? Rp + k : nullptr, al, be, invp);
     Y[k] = y;
-    if (Y32) Y32[k] = make_float2((float)y.x, (float)y.y);
     s += y.x * y.x + y.y * y.y;
   }
   if (part) {
@@ -600,51 +423,6 @@ __global__ __launch_bounds__(kRedThreads) void k_lz_scalar(
   double a = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])), b = 0.0;
   block_sum2(a, b);
   if (threadIdx.x == 0) out[0] = take_sqrt ? sqrt(a) : a;
-}
-
-// FP32 Lanczos vectors: alpha_k and beta_{k+1} from the LzPart3 partials
-// of nparts workgroups (fixed summation order):
-// beta_{k+1}^2 = |u_k - alpha_k q_k|^2 = |u|^2 - 2 alpha^2 + alpha^2 |q|^2
-__global__ __launch_bounds__(kRedThreads) void k_lz_scalars3(
-    int nparts, const double *__restrict__ part, double *__restrict__ alpha,
-    double *__restrict__ beta) {
-  // four independent partial sums per component and thread (the loads of
-  // a trip in flight together; constant indices keep them in registers),
-  // combined in a fixed order
-  double p[4][3] = {};
-  int k = threadIdx.x;
-  for (; k + 3 * kRedThreads < nparts; k += 4 * kRedThreads) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) p[u][c] += part[3 * (k + u * kRedThreads) + c];
-  }
-#pragma unroll
-  for (int u = 0; u < 3; ++u)
-    if (k + u * kRedThreads < nparts)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) p[u][c] += part[3 * (k + u * kRedThreads) + c];
-  double s[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) s[c] = (p[0][c] + p[1][c]) + (p[2][c] + p[3][c]);
-  __shared__ double w[3][kRedThreads / 64];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s[c] += __shfl_down(s[c], off, 64);
-    if ((threadIdx.x & 63) == 0) w[c][threadIdx.x >> 6] = s[c];
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int k = 0; k < kRedThreads / 64; ++k) t[c] += w[c][k];
-    const double a = t[0];
-    alpha[0] = a;
-    beta[0] = sqrt(fmax(t[1] - 2.0 * a * a + a * a * t[2], 0.0));
-  }
 }
 
 // V[e] += sum_k Z[e][k] Ring[k] for e < ne, k < K <= kRingMax (ring of
@@ -861,7 +639,8 @@ struct Converged {
 
 class LanczosRun {
  public:
-  LanczosRun(nh_context *c) : c_(c) {}
+  // classic: no deferred step
+  LanczosRun(nh_context *c, bool classic) : c_(c), classic_(classic) {}
   ~LanczosRun() {
     release_events();
     for (void *p : allocs_) pool_release(c_, p);
@@ -869,6 +648,8 @@ class LanczosRun {
     if (fetch_ev_) (void)hipEventDestroy(fetch_ev_);
   }
   nh_status run(const nh_lanczos_opts *o, nh_eig_result *res);
+  // run() ended because the deferred step's beta has lost digits
+  bool small_beta() const { return small_beta_; }
 
  private:
   // from the context's workspace pool, handed back when the run ends
@@ -884,30 +665,33 @@ class LanczosRun {
   bool window_done(int w, int req, int rule) const;
 
   nh_context *c_;
+  bool classic_;
   std::vector<void *> allocs_;
   int64_t n_ = 0;
   double2 *R_ = nullptr, *Y_ = nullptr, *Rm1_ = nullptr, *ring_ = nullptr;
-  // FP32 copies of r for the FP32 SK products (null otherwise)
-  float2 *R32_ = nullptr, *Y32_ = nullptr;
-  // FP32 Lanczos vectors (lz_fp32_vectors): the eigenvalue pass keeps
-  // r_{k-1} in R32_ and u_{k-1} in U32_ and writes r_k, u_k to Y32_, UN32_
-  // (step k = one launch plus k_lz_scalars3); R_ and Rm1_ are not allocated
-  bool v32_ = false;
-  float2 *U32_ = nullptr, *UN32_ = nullptr;
+  // SK and matrix-free layouts: the deferred step (k_lz_sk), with vectors of
+  // the products' type (vbytes_ an entry).  The eigenvalue pass keeps r_{k-1},
+  // u_{k-1} in r_[0], u_[0] and writes r_k, u_k to r_[1], u_[1]; part_ holds
+  // the partials of two steps in turn, grid_ of each.
+  bool defer_ = false, small_beta_ = false;
+  size_t vbytes_ = sizeof(double2);
+  char *r_[2] = {nullptr, nullptr}, *u_[2] = {nullptr, nullptr};
+  int grid_ = 0, last_ = -1;  // the last step of the eigenvalue pass queued
   // ring length of the eigenvector pass (<= kRingMax)
   int ring_k_ = kRingMax;
-  // eigenvector pass with FP32 products: 2 K FP32 copies of r, slot
-  // k % (2 K) holding r_k; the gather of step k reads slot k and writes
-  // r_{k+1} to slot k + 1, and the accumulation reads them as its ring
-  // (1 / beta_{k-1} folded into the coefficients)
-  float2 *ring32_ = nullptr;
-  // eigenvector pass with FP64 SK products: the r vectors themselves live in
-  // a ring of 2 K FP64 slots (slot k % (2 K) holds r_k: read as own entries
+  // SK and matrix-free layouts: the eigenvector pass keeps the r vectors
+  // themselves in 2 K slots, slot k % (2 K) holding r_k: read as own entries
   // and gathered at step k, r_(k-1) from slot k - 1, r_(k+1) written to slot
-  // k + 1), so no q is stored; the accumulation reads them like the FP32 ring
-  double2 *ringr_ = nullptr;
+  // k + 1; the accumulation reads them as its ring (1 / beta_{k-1} folded into
+  // the coefficients), so no q is stored
+  char *ringr_ = nullptr;
+  char *slot(int k) const { return ringr_ + (size_t)((k + 2 * ring_k_) % (2 * ring_k_)) * n_ * vbytes_; }
+  template <int NSP, typename R, typename V, typename SRC>
+  void launch_sk(int k, bool red, const SRC &src);
+  template <int NSP>
+  void launch_sk(int k, bool red);
   nh_status build_start(const nh_lanczos_opts *o);
-  nh_status upload_start(float2 *f32);
+  nh_status upload_start(void *r, size_t bytes);
   double2 *R0_ = nullptr;  // the normalised start vector (device)
   double *alpha_ = nullptr, *beta_ = nullptr, *part_ = nullptr;
   int nparts_ = 0;
@@ -1027,198 +811,161 @@ nh_status LanczosRun::build_start(const nh_lanczos_opts *o) {
   return NH_OK;
 }
 
-// r <- r0 (and its FP32 copy f32 when the products are FP32; only the
-// latter with FP32 Lanczos vectors)
-nh_status LanczosRun::upload_start(float2 *f32) {
-  if (!v32_)
-    NH_HIP(hipMemcpyAsync(R_, R0_, n_ * sizeof(double2), hipMemcpyDeviceToDevice,
+// r <- r0 as FP64 or FP32 entries
+nh_status LanczosRun::upload_start(void *r, size_t bytes) {
+  if (bytes == sizeof(double2)) {
+    NH_HIP(hipMemcpyAsync(r, R0_, n_ * sizeof(double2), hipMemcpyDeviceToDevice,
                           c_->stream));
-  if (f32) {
+  } else {
     hipLaunchKernelGGL(k_to_f32, dim3(reduce_blocks(n_)), dim3(256), 0,
-                       c_->stream, n_, R0_, f32);
+                       c_->stream, n_, R0_, reinterpret_cast<float2 *>(r));
     NH_HIP(hipGetLastError());
   }
   return NH_OK;
 }
 
-nh_status LanczosRun::iterate(int k, bool red) {
+// One product of the SK / matrix-free layouts in the run's mode.
+// Eigenvalue pass, step 0 of the deferred step: u_{-1} = r_{-1} = r_0 with
+// alpha_{-1} = beta_0 = 0, which leaves r_0 as it is; nothing is written back
+// for it.  Eigenvector pass: r_{-1} is slot 0 itself (the eigenvalue pass's
+// operands), none in the classic step.
+template <int NSP, typename R, typename V, typename SRC>
+void LanczosRun::launch_sk(int k, bool red, const SRC &src) {
   nh_context *c = c_;
-  int sk_blocks = 0;
-  const bool split = sk_like(c) && sk_split_lanes(c);
-  const SkGrid sg = sk_grid(c->n_cations, c->n_anions, sk_mixed_roles(c), &sk_blocks,
-                            split ? SkSplit::kLanes : 4);
-  const int gridA = sk_like(c)
-                        ? sk_blocks
-                        : (c->n_atoms + kAtomsPerBlock - 1) / kAtomsPerBlock;
-  // q_k is stored (ring slot) only in the eigenvector pass, which
-  // accumulates from it; the update forms q_k, q_{k-1} from r_k, r_{k-1}
-  double2 *Q = red || ring32_ || ringr_ ? nullptr : ring_ + (int64_t)(k % ring_k_) * n_;
-  // FP64 vectors of the step: r_k, r_(k-1), r_(k+1)
-  double2 *Rk = R_, *Rkm1 = Rm1_, *Yk = Y_;
-  if (!red && ringr_) {
-    Rk = ringr_ + (int64_t)(k % (2 * ring_k_)) * n_;
-    Rkm1 = ringr_ + (int64_t)((k + 2 * ring_k_ - 1) % (2 * ring_k_)) * n_;
-    Yk = ringr_ + (int64_t)((k + 1) % (2 * ring_k_)) * n_;
+  LzArgs<V> g{};
+  g.alpha = alpha_ + k;
+  g.beta_prev = k > 0 ? beta_ + (k - 1) : nullptr;
+  g.beta_prev2 = k > 1 ? beta_ + (k - 2) : nullptr;
+  g.part = part_ + (size_t)(k & 1) * 3 * nparts_;
+  auto vec = [](char *p) { return reinterpret_cast<V *>(p); };
+  if (red && defer_) {
+    g.x = vec(k == 0 ? r_[0] : u_[0]);
+    g.rp = vec(r_[0]);
+    g.out = vec(u_[1]);
+    g.rout = k == 0 ? nullptr : vec(r_[1]);
+    g.beta_prev = nullptr;  // summed by this launch
+    if (k > 0) {
+      g.part_prev = part_ + (size_t)((k - 1) & 1) * 3 * nparts_;
+      g.nparts = grid_;
+      g.alpha_out = alpha_ + (k - 1);
+      g.beta_out = beta_ + (k - 1);
+    }
+  } else if (red) {
+    g.x = reinterpret_cast<V *>(R_);
+    g.out = reinterpret_cast<V *>(Y_);
+    g.part = part_;
+  } else {
+    g.x = vec(slot(k));
+    g.rp = k > 0 ? vec(slot(k - 1)) : defer_ ? g.x : nullptr;
+    g.out = vec(slot(k + 1));
   }
-  // FP32 copies: gathered (r_k) and written (r_{k+1})
-  const float2 *g32 = R32_;
-  float2 *y32 = Y32_;
-  if (!red && ring32_) {
-    g32 = ring32_ + (int64_t)(k % (2 * ring_k_)) * n_;
-    y32 = ring32_ + (int64_t)((k + 1) % (2 * ring_k_)) * n_;
-  }
-  const double *bprev = k > 0 ? beta_ + (k - 1) : nullptr;
-  const double *bprev2 = k > 1 ? beta_ + (k - 2) : nullptr;
-  double *part = red ? part_ : nullptr;
-  const bool timed = (k % kTimeEvery) == 0;
-  // the eigenvector pass knows alpha_k: the SK kernel applies the update
-  const bool fuse = !red && sk_like(c);
-  // FP32 Lanczos vectors.  Eigenvalue pass: the product reads u_{k-1}
-  // (own entries and gathers) and r_{k-1}, forms r_k, writes r_k and u_k
-  // (step 0: u_{-1} = r_{-1} = r_0 with alpha_{-1} = beta_0 = 0, which
-  // leaves r_0 as it is; nothing is written back for it).  Eigenvector
-  // pass: own entries and gathers from ring slot k, r_{k-1} from slot k - 1
-  // (slot 0 itself at step 0, the eigenvalue pass's operands), r_{k+1} to
-  // slot k + 1; no FP64 vector at all.
-  const float2 *rp32 = nullptr;
-  float2 *rout = nullptr;
-  const double *aprev = nullptr;
-  if (v32_) {
-    if (red) {
-      g32 = k == 0 ? R32_ : U32_;
-      rp32 = R32_;
-      rout = k == 0 ? nullptr : Y32_;
-      y32 = UN32_;
-      aprev = k > 0 ? alpha_ + (k - 1) : nullptr;
-      Yk = nullptr;
-      part = part_;
-    } else {
-      rp32 = ring32_ + (int64_t)((k + 2 * ring_k_ - (k > 0 ? 1 : 0)) % (2 * ring_k_)) * n_;
-      Yk = nullptr;
+  const SkTable tab = sk_table_of(c);
+#define LZ_SK(MODE)                                                            \
+  hipLaunchKernelGGL((k_lz_sk<MODE, NSP, R, V, SRC>), dim3(grid_),             \
+                     dim3(kSkThreads), 0, c->stream, tab, c->onsite, src, g)
+  if constexpr (sizeof(V) == 2 * sizeof(R)) {
+    if (defer_) {
+      if (red) LZ_SK(kLzValues);
+      else LZ_SK(kLzVectors);
+      return;
     }
   }
-  const double2 *rp64 = k > 0 ? Rkm1 : nullptr;
+  if constexpr (sizeof(V) == 16) {
+    if (red) LZ_SK(kLzProduct);
+    else LZ_SK(kLzFused);
+  }
+#undef LZ_SK
+}
+
+template <int NSP>
+void LanczosRun::launch_sk(int k, bool red) {
+  nh_context *c = c_;
+  const bool f64 = c->precision == NH_PREC_FP64, v64 = vbytes_ == sizeof(double2);
+#define LZ_SRC(S64, S32)                                                       \
+  do {                                                                         \
+    if (f64) launch_sk<NSP, double, double2>(k, red, S64);                     \
+    else if (v64) launch_sk<NSP, float, double2>(k, red, S32);                 \
+    else launch_sk<NSP, float, float2>(k, red, S32);                           \
+  } while (0)
+  if (c->layout == NH_LAYOUT_MATRIX_FREE)
+    LZ_SRC(mf_src<double>(c), mf_src<float>(c));
+  else
+    LZ_SRC((SkSrc<double>{c->sk64, c->blk_bonds}), (SkSrc<float>{c->sk32, c->blk_bonds}));
+#undef LZ_SRC
+}
+
+nh_status LanczosRun::iterate(int k, bool red) {
+  nh_context *c = c_;
+  const bool sk = sk_like(c);
+  const double *bprev = k > 0 ? beta_ + (k - 1) : nullptr;
+  const double *bprev2 = k > 1 ? beta_ + (k - 2) : nullptr;
+  const bool timed = (k % kTimeEvery) == 0;
   Timed evp{nullptr, nullptr, red};
   if (timed) {
     NH_HIP(hipEventCreate(&evp.start));
     NH_HIP(hipEventCreate(&evp.stop));
     NH_HIP(hipEventRecord(evp.start, c->stream));
   }
+  if (sk) {
+    if (c->nb == 20) launch_sk<2>(k, red);
+    else launch_sk<1>(k, red);
+  } else {
+    // q_k is stored (ring slot) only in the eigenvector pass, which
+    // accumulates from it; the update forms q_k, q_{k-1} from r_k, r_{k-1}
+    double2 *Q = red ? nullptr : ring_ + (int64_t)(k % ring_k_) * n_;
+    double *part = red ? part_ : nullptr;
 #define LZ_HV(NSP, TB, BLK)                                                    \
   do {                                                                         \
-    if (use_staged(c))                                                          \
-      hipLaunchKernelGGL((k_lz_hv<NSP, TB, TB, true>), dim3(gridA),            \
+    if (use_staged(c))                                                         \
+      hipLaunchKernelGGL((k_lz_hv<NSP, TB, TB, true>), dim3(grid_),            \
                          dim3(kThreads), 0, c->stream, c->n_atoms, c->onsite,  \
                          BLK, c->nbr, R_, Q, Y_, bprev, part);                 \
     else                                                                       \
-      hipLaunchKernelGGL((k_lz_hv<NSP, TB, TB, false>), dim3(gridA),           \
+      hipLaunchKernelGGL((k_lz_hv<NSP, TB, TB, false>), dim3(grid_),           \
                          dim3(kThreads), 0, c->stream, c->n_atoms, c->onsite,  \
                          BLK, c->nbr, R_, Q, Y_, bprev, part);                 \
   } while (0)
-// XO, RV, RP: storage type of r, own entries r_k, r_{k-1}
-#define LZ_SK2(NSP, R, SRC, QUAD, FUSE, XO, RV, RP)                             \
-  hipLaunchKernelGGL((k_lz_hv_sk<NSP, R, QUAD, FUSE, decltype(SRC), XO>),       \
-                     dim3(gridA), dim3(kSkThreads), 0, c->stream, c->n_cations, \
-                     c->cations, c->n_anions, c->anions, sg, c->onsite, SRC,    \
-                     c->nbr, RV, g32, Q, Yk, bprev, part, alpha_ + k, RP,       \
-                     bprev2, y32, rout, aprev)
-#define LZ_SK1(NSP, R, SRC, QUAD, XO, RV, RP)                                   \
-  do {                                                                          \
-    if (fuse) LZ_SK2(NSP, R, SRC, QUAD, true, XO, RV, RP);                      \
-    else LZ_SK2(NSP, R, SRC, QUAD, false, XO, RV, RP);                          \
-  } while (0)
-#define LZ_SPL2(R, SRC, FUSE, XO, RV, RP)                                        \
-  hipLaunchKernelGGL((k_lz_hv_sk_split<R, FUSE, decltype(SRC), XO>),            \
-                     dim3(gridA), dim3(kSkThreads), 0, c->stream, c->n_cations, \
-                     c->cations, c->n_anions, c->anions, sg, c->onsite, SRC,    \
-                     c->nbr, RV, g32, Q, Yk, bprev, part, alpha_ + k, RP,       \
-                     bprev2, y32, rout, aprev)
-#define LZ_SK0(NSP, R, SRC, XO, RV, RP)                                         \
-  do {                                                                          \
-    if (NSP == 2 && split) {                                                    \
-      if (fuse) LZ_SPL2(R, SRC, true, XO, RV, RP);                              \
-      else LZ_SPL2(R, SRC, false, XO, RV, RP);                                  \
-    } else if (use_staged(c)) LZ_SK1(NSP, R, SRC, true, XO, RV, RP);            \
-    else LZ_SK1(NSP, R, SRC, false, XO, RV, RP);                                \
-  } while (0)
-#define LZ_SK(R, SRC, XO, RV, RP)                                               \
-  do {                                                                          \
-    if (c->nb == 20) LZ_SK0(2, R, SRC, XO, RV, RP);                             \
-    else LZ_SK0(1, R, SRC, XO, RV, RP);                                         \
-  } while (0)
-// FP32 vectors (LDS gather only)
-#define LZ_SKV0(NSP, SRC)                                                       \
-  do {                                                                          \
-    if (NSP == 2 && split) {                                                    \
-      if (fuse) LZ_SPL2(float, SRC, true, float2, g32, rp32);                   \
-      else LZ_SPL2(float, SRC, false, float2, g32, rp32);                       \
-    } else LZ_SK1(NSP, float, SRC, true, float2, g32, rp32);                    \
-  } while (0)
-#define LZ_SKV(SRC)                                                             \
-  do {                                                                          \
-    if (c->nb == 20) LZ_SKV0(2, SRC);                                           \
-    else LZ_SKV0(1, SRC);                                                       \
-  } while (0)
-  if (c->layout == NH_LAYOUT_MATRIX_FREE) {
-    if (c->precision == NH_PREC_FP64) LZ_SK(double, mf_src<double>(c), double2, Rk, rp64);
-    else if (v32_) LZ_SKV(mf_src<float>(c));
-    else LZ_SK(float, mf_src<float>(c), double2, Rk, rp64);
-  } else if (c->layout == NH_LAYOUT_SK) {
-    if (c->precision == NH_PREC_FP64)
-      LZ_SK(double, (SkSrc<double>{c->sk64, c->bond_of}), double2, Rk, rp64);
-    else if (v32_) LZ_SKV((SkSrc<float>{c->sk32, c->bond_of}));
-    else LZ_SK(float, (SkSrc<float>{c->sk32, c->bond_of}), double2, Rk, rp64);
-  } else if (c->precision == NH_PREC_FP64) {
-    if (c->nb == 20) LZ_HV(2, double, c->blocks64);
-    else LZ_HV(1, double, c->blocks64);
-  } else {
-    if (c->nb == 20) LZ_HV(2, float, c->blocks32);
-    else LZ_HV(1, float, c->blocks32);
-  }
+    if (c->precision == NH_PREC_FP64) {
+      if (c->nb == 20) LZ_HV(2, double, c->blocks64);
+      else LZ_HV(1, double, c->blocks64);
+    } else {
+      if (c->nb == 20) LZ_HV(2, float, c->blocks32);
+      else LZ_HV(1, float, c->blocks32);
+    }
 #undef LZ_HV
-#undef LZ_SK
-#undef LZ_SK0
-#undef LZ_SK1
-#undef LZ_SK2
-#undef LZ_SPL2
-#undef LZ_SKV
-#undef LZ_SKV0
+  }
+  NH_HIP(hipGetLastError());
   if (timed) {
     NH_HIP(hipEventRecord(evp.stop, c->stream));
     ev_.push_back(evp);
   }
-  if (v32_ && red) {
-    // alpha_k, beta_{k+1} from the product's partials; rotate
-    // (r_{k-1}, u_{k-1}) <- (r_k, u_k) (step 0: r_0 stays)
-    hipLaunchKernelGGL(k_lz_scalars3, dim3(1), dim3(kRedThreads), 0, c->stream,
-                       gridA, part_, alpha_ + k, beta_ + k);
-    NH_HIP(hipGetLastError());
-    if (k > 0) std::swap(R32_, Y32_);
-    std::swap(U32_, UN32_);
+  if (red) last_ = k;
+  if (sk && defer_) {
+    // rotate (r_{k-1}, u_{k-1}) <- (r_k, u_k) (step 0: r_0 stays); the
+    // eigenvector pass rotates its slots by index
+    if (red) {
+      if (k > 0) std::swap(r_[0], r_[1]);
+      std::swap(u_[0], u_[1]);
+    }
     return NH_OK;
   }
+  if (sk && !red) return NH_OK;
   if (red)
     hipLaunchKernelGGL(k_lz_scalar, dim3(1), dim3(kRedThreads), 0, c->stream,
-                       gridA, 1, part_, alpha_ + k, 0);
+                       grid_, 1, part_, alpha_ + k, 0);
   const int nb = reduce_blocks(n_);
-  if (!fuse)
-    hipLaunchKernelGGL(k_lz_update, dim3(nb), dim3(kRedThreads), 0, c->stream,
-                       n_, Y_, R_, k > 0 ? Rm1_ : nullptr, alpha_ + k, bprev,
-                       bprev2, part, y32);
+  hipLaunchKernelGGL(k_lz_update, dim3(nb), dim3(kRedThreads), 0, c->stream,
+                     n_, Y_, R_, k > 0 ? Rm1_ : nullptr, alpha_ + k, bprev,
+                     bprev2, red ? part_ : nullptr);
   if (red)
     hipLaunchKernelGGL(k_lz_scalar, dim3(1), dim3(kRedThreads), 0, c->stream,
                        nb, 2, part_, beta_ + k, 1);
   NH_HIP(hipGetLastError());
   // r_{k+1} is in Y: rotate (r_{k-1}, r_k, y) -> (r_k, r_{k+1}, free)
-  if (v32_) {
-    // eigenvector pass: the ring slots rotate by index
-  } else {
-    double2 *free_buf = Rm1_;
-    Rm1_ = R_;
-    R_ = Y_;
-    Y_ = free_buf;
-    std::swap(R32_, Y32_);
-  }
+  double2 *free_buf = Rm1_;
+  Rm1_ = R_;
+  R_ = Y_;
+  Y_ = free_buf;
   return NH_OK;
 }
 
@@ -1246,6 +993,12 @@ bool LanczosRun::window_done(int w, int req, int rule) const {
 // queue the copy of alpha and beta up to step m into the pinned staging
 nh_status LanczosRun::fetch(int m) {
   if (m > fetched_) {
+    // deferred step: the last step's alpha and beta are still partials (the
+    // next step would sum them)
+    if (defer_ && last_ == m - 1)
+      hipLaunchKernelGGL(k_lz_scalars3, dim3(1), dim3(kRedThreads), 0, c_->stream, grid_,
+                         part_ + (size_t)(last_ & 1) * 3 * nparts_, alpha_ + last_,
+                         beta_ + last_);
     NH_HIP(hipMemcpyAsync(pin_ + fetched_, alpha_ + fetched_,
                           (m - fetched_) * sizeof(double), hipMemcpyDeviceToHost,
                           c_->stream));
@@ -1264,6 +1017,15 @@ nh_status LanczosRun::analyse(int m, const nh_lanczos_opts *o) {
   NH_HIP(hipEventSynchronize(fetch_ev_));
   ha_.assign(pin_, pin_ + m);
   hb_.assign(pin_ + pin_cap_, pin_ + pin_cap_ + m);
+  // The deferred FP64 step has beta^2 as a difference of sums, |u|^2 - alpha^2:
+  // below 1e-4 |u|^2 (a start vector in an almost invariant subspace) it loses
+  // more than four of its digits, and the run is repeated with the classic
+  // step, which sums |r|^2 itself.  (FP32 vectors: their rounding is far above
+  // what is lost.)
+  if (defer_ && vbytes_ == sizeof(double2))
+    for (int i = 0; i < m; ++i)
+      if (!(hb_[i] * hb_[i] >= 1e-4 * (ha_[i] * ha_[i] + hb_[i] * hb_[i]))) small_beta_ = true;
+  if (small_beta_) return NH_ERR_STATE;
   const double tol = o->conv_tolerance;
   const double resolution = 100.0 * tol;  // lanczos.c:1970
   const double bias = 1e-80;
@@ -1340,32 +1102,33 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
   NH_CHECK(o->max_iter > 2 && o->conv_tolerance > 0, NH_ERR_ARG,
            "Lanczos: bad max_iter / tolerance");
   n_ = c->n;
-  v32_ = lz_fp32_vectors(c);
-  if (!v32_) {
+  // FP32 products with FP64 vectors (NH_SET_LZ_VECTORS = 0) and stored blocks
+  // take the classic step
+  const bool fp32 = c->precision == NH_PREC_FP32;
+  defer_ = sk_like(c) && !classic_ && (!fp32 || lz_fp32_vectors(c));
+  vbytes_ = defer_ && fp32 ? sizeof(float2) : sizeof(double2);
+  if (!defer_) {
     NH_TRY(alloc((void **)&R_, n_ * sizeof(double2)));
     NH_TRY(alloc((void **)&Rm1_, n_ * sizeof(double2)));
   }
   NH_TRY(alloc((void **)&Y_, n_ * sizeof(double2)));
   NH_TRY(alloc((void **)&alpha_, (size_t)(o->max_iter + 1) * sizeof(double)));
   NH_TRY(alloc((void **)&beta_, (size_t)(o->max_iter + 1) * sizeof(double)));
-  nparts_ = std::max((c->n_atoms + kAtomsPerBlock - 1) / kAtomsPerBlock,
-                     2 * kRedMaxBlocks) + 64;
-  NH_TRY(alloc((void **)&part_, (size_t)nparts_ * 3 * sizeof(double)));
+  // workgroups of the products: as many as run at a time (LDS: 2 a CU with
+  // FP64 entries, 3 with FP32 ones)
+  grid_ = sk_like(c) ? sk_grid(c, vbytes_ == sizeof(float2) ? 3 : 2)
+                     : (c->n_atoms + kAtomsPerBlock - 1) / kAtomsPerBlock;
+  nparts_ = std::max(grid_, 2 * kRedMaxBlocks) + 64;
+  NH_TRY(alloc((void **)&part_, (size_t)nparts_ * 6 * sizeof(double)));
 
   NH_TRY(build_start(o));
-  if (sk_like(c) && c->precision == NH_PREC_FP32) {
-    NH_TRY(alloc((void **)&R32_, n_ * sizeof(float2)));
-    NH_TRY(alloc((void **)&Y32_, n_ * sizeof(float2)));
-    if (v32_) {
-      NH_TRY(alloc((void **)&U32_, n_ * sizeof(float2)));
-      NH_TRY(alloc((void **)&UN32_, n_ * sizeof(float2)));
-      int blocks = 0;
-      sk_grid(c->n_cations, c->n_anions, sk_mixed_roles(c), &blocks,
-              sk_split_lanes(c) ? SkSplit::kLanes : 4);
-      NH_CHECK(blocks <= nparts_, NH_ERR_STATE, "Lanczos: partial sums do not fit");
-    }
+  if (defer_) {
+    for (char **p : {&r_[0], &r_[1], &u_[0], &u_[1]})
+      NH_TRY(alloc((void **)p, n_ * vbytes_));
+    NH_TRY(upload_start(r_[0], vbytes_));
+  } else {
+    NH_TRY(upload_start(R_, vbytes_));
   }
-  NH_TRY(upload_start(R32_));
 
   // pass 1: eigenvalues.  The host analyses the tridiagonal of one check
   // point while the device runs the steps up to the next one: at a check
@@ -1505,28 +1268,23 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
     // free memory (the run's buffers are released before any later stage
     // allocates), else 32, 16 or 8 (each flush reads and writes the
     // eigenvectors once)
-    const bool rring = !R32_ && sk_like(c);
+    const bool rring = sk_like(c);
     {
       size_t fr = 0, tot = 0;
       NH_HIP(hipMemGetInfo(&fr, &tot));
       fr += pool_free_bytes(c);
-      const size_t slot = R32_ ? 2 * n_ * sizeof(float2)
-                               : (rring ? 2 : 1) * n_ * sizeof(double2);
+      const size_t slot = (rring ? 2 : 1) * n_ * vbytes_;
       ring_k_ = kRingMax;
       while (ring_k_ > 8 && (size_t)ring_k_ * slot > fr / 2) ring_k_ /= 2;
       if (c->ring_steps > 0) ring_k_ = std::min(ring_k_, c->ring_steps);
     }
-    if (R32_) {
-      NH_CHECK(n_ % 2 == 0, NH_ERR_STATE, "Lanczos: FP32 ring needs an even N");
-      NH_TRY(alloc((void **)&ring32_, (size_t)2 * ring_k_ * n_ * sizeof(float2)));
-      NH_TRY(upload_start(ring32_));
-    } else if (rring) {
-      NH_TRY(alloc((void **)&ringr_, (size_t)2 * ring_k_ * n_ * sizeof(double2)));
-      NH_HIP(hipMemcpyAsync(ringr_, R0_, n_ * sizeof(double2),
-                            hipMemcpyDeviceToDevice, c->stream));
+    if (rring) {
+      NH_CHECK(n_ % 2 == 0, NH_ERR_STATE, "Lanczos: the ring needs an even N");
+      NH_TRY(alloc((void **)&ringr_, (size_t)2 * ring_k_ * n_ * vbytes_));
+      NH_TRY(upload_start(ringr_, vbytes_));
     } else {
       NH_TRY(alloc((void **)&ring_, (size_t)ring_k_ * n_ * sizeof(double2)));
-      NH_TRY(upload_start(nullptr));
+      NH_TRY(upload_start(R_, sizeof(double2)));
     }
     std::vector<double> hz((size_t)kMaxVec * kRingMax);
     const int rk = ring_k_;
@@ -1540,27 +1298,25 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
         for (int e = 0; e < ne; ++e)
           for (int t = 0; t < K; ++t) {
             const int j = k0 + t;
-            // q_j = r_j / beta_{j-1} for the rings of r (FP32 copies or FP64)
-            const double sc = (ring32_ || ringr_) && j > 0 ? 1.0 / hb_[j - 1] : 1.0;
+            // q_j = r_j / beta_{j-1} for the ring of r
+            const double sc = ringr_ && j > 0 ? 1.0 / hb_[j - 1] : 1.0;
             hz[e * K + t] = j < pick[e].iter ? z[e][j] * sc : 0.0;
           }
         NH_HIP(hipMemcpyAsync(dZ, hz.data(), (size_t)ne * K * sizeof(double),
                               hipMemcpyHostToDevice, c->stream));
         int64_t g = (n_ + 255) / 256;
         if (g > 8192) g = 8192;
-        // ring slots k0..k hold q_k0..q_k in order since k0 % K == 0
-        // (FP32 ring: slots k0 % (2 K) + t hold r_k0+t)
-        if (ring32_)
+        // ring slots k0..k hold q_k0..q_k in order since k0 % K == 0 (ring of
+        // r: slots k0 % (2 K) + t hold r_k0+t)
+        if (ringr_ && vbytes_ == sizeof(float2))
           hipLaunchKernelGGL(k_lz_accum32, dim3((int)g), dim3(256), 0,
                              c->stream, n_, ne, K, dZ,
-                             ring32_ + (int64_t)(k0 % (2 * rk)) * n_, n_, V, n_);
-        else if (ringr_)
-          hipLaunchKernelGGL((k_lz_accum<double2>), dim3((int)g), dim3(256), 0,
-                             c->stream, n_, ne, K, dZ,
-                             ringr_ + (int64_t)(k0 % (2 * rk)) * n_, n_, V, n_);
+                             reinterpret_cast<const float2 *>(slot(k0)), n_, V, n_);
         else
           hipLaunchKernelGGL((k_lz_accum<double2>), dim3((int)g), dim3(256), 0,
-                             c->stream, n_, ne, K, dZ, ring_, n_, V, n_);
+                             c->stream, n_, ne, K, dZ,
+                             ringr_ ? reinterpret_cast<const double2 *>(slot(k0)) : ring_, n_,
+                             V, n_);
         NH_HIP(hipGetLastError());
         // the host array hz is reused next chunk: wait for the copy
         NH_HIP(hipStreamSynchronize(c->stream));
@@ -1611,6 +1367,11 @@ extern "C" nh_status nh_eigensolve_lanczos(nh_context *ctx,
            NH_ERR_ARG, "nh_eigensolve_lanczos: bad arguments");
   (void)hipGetLastError();
   NH_HIP(hipSetDevice(ctx->device));
-  nh::LanczosRun run(ctx);
+  {
+    nh::LanczosRun run(ctx, false);
+    const nh_status st = run.run(opts, res);
+    if (!run.small_beta()) return st;
+  }
+  nh::LanczosRun run(ctx, true);
   return run.run(opts, res);
 }

@@ -1,0 +1,212 @@
+// Product of one bond's sp3d5s* block with one real component vector.
+//
+// The 10x10 block T (rows: anion orbitals, columns: cation orbitals; table
+// in nh_sk.h) is applied without being formed.  With n the bond's direction,
+// sd the five d functions along n, p and d the vector's p and d parts, M(d)
+// the symmetric traceless matrix of the d part and w = M(d) n, its parts are
+//   s, s*      numbers times xs, x_s*, n.p and sd.d;
+//   p-p        ppp p + (pps - ppp) n (n.p);
+//   p-d, d-p   padcp w + A n (sd.d), A = padcs - (2/sqrt 3) padcp, and its
+//              transpose with pcdas, pcdap;
+//   d-d        ddd d + B M^T(n w) + A' sd (sd.d), B = ddp - ddd,
+//              A' = dds - ddd - (4/3) B
+// (M^T(n w): the five components of the symmetric product of n and w).
+// sqrt 3 is the reference's literal, placed so that what its 6.5e-13 error
+// still changes against sk_table is proportional to n^2 - (l^2 + m^2)/2,
+// which vanishes on an unstrained bond.
+// That is 93 multiply-adds per vector and about 40 operations per bond for
+// the scaled vectors, against 100 and about 250 for forming T.
+//
+// Every matrix element is a sum of products of two numbers that are
+// precomputed per bond, added in the same order in both orientations (the
+// anion row applies T, the cation row its transpose: what one projects on,
+// the other expands along), so the two rows of a bond are exact transposes
+// of each other in floating point and H stays exactly Hermitian.  All
+// multiply-adds are explicit: every kernel that applies a bond rounds alike.
+#pragma once
+
+#include "nh_sk.h"
+
+namespace nh {
+
+// The 24 numbers of a bond record.  Pairs whose members swap in the
+// transposed product are neighbours (one 16-byte load in FP64).
+enum : int {
+  K_L = 0, K_M = 1, K_N = 2, K_DDD = 3,
+  K_SSS = 4, K_STSTS = 5, K_STASS = 6, K_SASTS = 7,
+  K_SAPC = 8, K_SCPA = 9, K_STAPC = 10, K_STCPA = 11,
+  K_SADC = 12, K_SCDA = 13, K_STADC = 14, K_STCDA = 15,
+  K_PADP = 16, K_PCDP = 17, K_APD = 18, K_ADP = 19,
+  K_PPP = 20, K_PPC = 21, K_DB = 22, K_DA = 23
+};
+
+// Record of the direction (l, m, n) and the 21 integrals v (parameters
+// 10..30; the signs of the integrals with the lower angular momentum on the
+// cation as in sk_table).
+template <typename R>
+__host__ __device__ __forceinline__ void sk_record(R l, R m, R n, const R *v, R *k) {
+  constexpr R c2 = R(2.0 / kSqrt3Ref), c3 = R(3.0 / (kSqrt3Ref * kSqrt3Ref));
+  k[K_L] = l;
+  k[K_M] = m;
+  k[K_N] = n;
+  k[K_SSS] = v[0];
+  k[K_STSTS] = v[1];
+  k[K_STASS] = v[2];
+  k[K_SASTS] = v[3];
+  k[K_SAPC] = v[4];
+  k[K_SCPA] = -v[5];
+  k[K_STAPC] = v[6];
+  k[K_STCPA] = -v[7];
+  k[K_SADC] = v[8];
+  k[K_SCDA] = v[9];
+  k[K_STADC] = v[10];
+  k[K_STCDA] = v[11];
+  k[K_PPP] = v[13];
+  k[K_PPC] = v[12] - v[13];
+  k[K_PADP] = v[16];
+  k[K_PCDP] = -v[17];
+  k[K_APD] = v[14] - c2 * v[16];
+  k[K_ADP] = c2 * v[17] - v[15];
+  k[K_DDD] = v[20];
+  k[K_DB] = v[19] - v[20];
+  k[K_DA] = c3 * ((v[18] - v[20]) - R(4.0 / 3.0) * (v[19] - v[20]));
+}
+// the 21 integrals of a record
+template <typename R>
+__host__ __device__ __forceinline__ void sk_integrals(const R *k, R *v) {
+  constexpr R c2 = R(2.0 / kSqrt3Ref), c3 = R(3.0 / (kSqrt3Ref * kSqrt3Ref));
+  v[0] = k[K_SSS];
+  v[1] = k[K_STSTS];
+  v[2] = k[K_STASS];
+  v[3] = k[K_SASTS];
+  v[4] = k[K_SAPC];
+  v[5] = -k[K_SCPA];
+  v[6] = k[K_STAPC];
+  v[7] = -k[K_STCPA];
+  v[8] = k[K_SADC];
+  v[9] = k[K_SCDA];
+  v[10] = k[K_STADC];
+  v[11] = k[K_STCDA];
+  v[12] = k[K_PPC] + k[K_PPP];
+  v[13] = k[K_PPP];
+  v[14] = k[K_APD] + c2 * k[K_PADP];
+  v[15] = -k[K_ADP] - c2 * k[K_PCDP];
+  v[16] = k[K_PADP];
+  v[17] = -k[K_PCDP];
+  v[18] = k[K_DA] / c3 + k[K_DDD] + R(4.0 / 3.0) * k[K_DB];
+  v[19] = k[K_DB] + k[K_DDD];
+  v[20] = k[K_DDD];
+}
+
+__host__ __device__ __forceinline__ double sk_fma(double a, double b, double c) {
+  return __builtin_fma(a, b, c);
+}
+__host__ __device__ __forceinline__ float sk_fma(float a, float b, float c) {
+  return __builtin_fmaf(a, b, c);
+}
+
+// y += T x (CATION = false: x on the cation, y on the anion) or y += T^t x
+// (CATION = true: x on the anion, y on the cation); k: the bond's record.
+template <bool CATION, typename R>
+__host__ __device__ __forceinline__ void sk_apply(const R *k, const R (&x)[10], R (&y)[10]) {
+#pragma clang fp contract(off)
+  const R l = k[K_L], m = k[K_M], n = k[K_N];
+  constexpr R s3 = R(kSqrt3Ref), kp = R(kSqrt3Ref / 3.0);
+  // members of the swapping pairs: xy = element from y's role to x's role
+  const R ss_a = CATION ? k[K_SASTS] : k[K_STASS];  // y_s* from x_s
+  const R ss_b = CATION ? k[K_STASS] : k[K_SASTS];  // y_s from x_s*
+  const R sp = CATION ? k[K_SCPA] : k[K_SAPC], ps = CATION ? k[K_SAPC] : k[K_SCPA];
+  const R tp = CATION ? k[K_STCPA] : k[K_STAPC], pt = CATION ? k[K_STAPC] : k[K_STCPA];
+  const R sd_ = CATION ? k[K_SCDA] : k[K_SADC], ds = CATION ? k[K_SADC] : k[K_SCDA];
+  const R td = CATION ? k[K_STCDA] : k[K_STADC], dt = CATION ? k[K_STADC] : k[K_STCDA];
+  const R pdp = CATION ? k[K_PCDP] : k[K_PADP], dpp = CATION ? k[K_PADP] : k[K_PCDP];
+  const R apd = CATION ? k[K_ADP] : k[K_APD], adp = CATION ? k[K_APD] : k[K_ADP];
+  const R ppc = k[K_PPC], ppp = k[K_PPP], ddd = k[K_DDD], db = k[K_DB], da = k[K_DA];
+  const R *p = x + 2, *d = x + 5;
+  const R ml = m * l, mn = m * n, nl = n * l, l2 = l * l, m2 = m * m, n2 = n * n;
+  const R g[5] = {s3 * ml, s3 * mn, s3 * nl, (R(0.5) * s3) * (l2 - m2),
+                  n2 - R(0.5) * (l2 + m2)};
+  // projections
+  const R s = sk_fma(n, p[2], sk_fma(m, p[1], l * p[0]));
+  R t = g[0] * d[0];
+#pragma unroll
+  for (int c = 1; c < 5; ++c) t = sk_fma(g[c], d[c], t);
+  y[0] = sk_fma(td, t, sk_fma(tp, s, sk_fma(ss_a, x[1], sk_fma(k[K_STSTS], x[0], y[0]))));
+  y[1] = sk_fma(sd_, t, sk_fma(sp, s, sk_fma(ss_b, x[0], sk_fma(k[K_SSS], x[1], y[1]))));
+  // w = M(d) n; the z2 part enters as (-1, -1, 2) kp
+  const R kl = kp * l, km = kp * m, kn = (kp * n) * R(2);
+  const R wx = sk_fma(n, d[2], sk_fma(m, d[0], sk_fma(-kl, d[4], l * d[3])));
+  const R wy = sk_fma(n, d[1], sk_fma(l, d[0], sk_fma(-km, d[4], -(m * d[3]))));
+  const R wz = sk_fma(m, d[1], sk_fma(l, d[2], kn * d[4]));
+  // p rows: ppp p + pdp w, then n (...), then the p-p projection
+  R te = (apd * g[0]) * d[0];
+#pragma unroll
+  for (int c = 1; c < 5; ++c) te = sk_fma(apd * g[c], d[c], te);
+  const R cp = sk_fma(ps, x[1], sk_fma(pt, x[0], te));
+  const R cl = ppc * l, cm = ppc * m, cn = ppc * n;
+  R sc;
+  if constexpr (CATION) sc = sk_fma(cn, p[2], sk_fma(cm, p[1], cl * p[0]));
+  y[2] = sk_fma(l, cp, sk_fma(pdp, wx, sk_fma(ppp, p[0], y[2])));
+  y[3] = sk_fma(m, cp, sk_fma(pdp, wy, sk_fma(ppp, p[1], y[3])));
+  y[4] = sk_fma(n, cp, sk_fma(pdp, wz, sk_fma(ppp, p[2], y[4])));
+  if constexpr (CATION) {
+    y[2] = sk_fma(l, sc, y[2]);
+    y[3] = sk_fma(m, sc, y[3]);
+    y[4] = sk_fma(n, sc, y[4]);
+  } else {
+    y[2] = sk_fma(cl, s, y[2]);
+    y[3] = sk_fma(cm, s, y[3]);
+    y[4] = sk_fma(cn, s, y[4]);
+  }
+  // d rows: ddd d, then the symmetric products, then along sd
+  R y5 = sk_fma(ddd, d[0], y[5]), y6 = sk_fma(ddd, d[1], y[6]), y7 = sk_fma(ddd, d[2], y[7]),
+    y8 = sk_fma(ddd, d[3], y[8]);
+  // z2-z2: the table's element has no sqrt(3); the reference's literal one
+  // (1.2e-12 off) enters here through kp^2, which this takes back
+  R ddd4 = ddd;
+  if constexpr (sizeof(R) == 8) {
+    constexpr R e = R(1.0 / 3.0 - (kSqrt3Ref / 3.0) * (kSqrt3Ref / 3.0));
+    ddd4 = sk_fma(sk_fma(R(3) * e, n2, e), db, ddd);
+  }
+  R y9 = sk_fma(ddd4, d[4], y[9]);
+  const R bl = db * l, bm = db * m, bn = db * n;
+  const R kbl = db * kl, kbm = db * km, kbn = db * kn;
+  if constexpr (CATION) {
+    // w along B n, expanded with the p part along n
+    const R vx = sk_fma(bn, d[2], sk_fma(bm, d[0], sk_fma(-kbl, d[4], bl * d[3])));
+    const R vy = sk_fma(bn, d[1], sk_fma(bl, d[0], sk_fma(-kbm, d[4], -(bm * d[3]))));
+    const R vz = sk_fma(bm, d[1], sk_fma(bl, d[2], kbn * d[4]));
+    const R hx = sk_fma(dpp, p[0], vx), hy = sk_fma(dpp, p[1], vy), hz = sk_fma(dpp, p[2], vz);
+    y5 = sk_fma(l, hy, sk_fma(m, hx, y5));
+    y6 = sk_fma(n, hy, sk_fma(m, hz, y6));
+    y7 = sk_fma(n, hx, sk_fma(l, hz, y7));
+    y8 = sk_fma(-m, hy, sk_fma(l, hx, y8));
+    y9 = sk_fma(-km, hy, sk_fma(-kl, hx, sk_fma(kn, hz, y9)));
+  } else {
+    const R hx = dpp * p[0], hy = dpp * p[1], hz = dpp * p[2];
+    y5 = sk_fma(bl, wy, sk_fma(bm, wx, sk_fma(l, hy, sk_fma(m, hx, y5))));
+    y6 = sk_fma(bn, wy, sk_fma(bm, wz, sk_fma(n, hy, sk_fma(m, hz, y6))));
+    y7 = sk_fma(bn, wx, sk_fma(bl, wz, sk_fma(n, hx, sk_fma(l, hz, y7))));
+    y8 = sk_fma(-bm, wy, sk_fma(bl, wx, sk_fma(-m, hy, sk_fma(l, hx, y8))));
+    y9 = sk_fma(-km, hy, sk_fma(-kl, hx, sk_fma(kn, hz, y9)));
+    y9 = sk_fma(-kbm, wy, sk_fma(-kbl, wx, sk_fma(kbn, wz, y9)));
+  }
+  // sd (xs, x_s* parts), A sd (n.p), A' sd (sd.d)
+  const R cs = sk_fma(ds, x[1], dt * x[0]);
+  R ta;
+  if constexpr (CATION) {
+    ta = (da * g[0]) * d[0];
+#pragma unroll
+    for (int c = 1; c < 5; ++c) ta = sk_fma(da * g[c], d[c], ta);
+  } else {
+    ta = t;
+  }
+  R yd[5] = {y5, y6, y7, y8, y9};
+#pragma unroll
+  for (int c = 0; c < 5; ++c) {
+    const R e = adp * g[c], a = CATION ? g[c] : da * g[c];
+    y[5 + c] = sk_fma(a, ta, sk_fma(e, s, sk_fma(g[c], cs, yd[c])));
+  }
+}
+
+}  // namespace nh
