@@ -53,6 +53,62 @@ static nh_status pool_trim(nh_context *c) {
     else NH_HIP(hipFree(b.p));
   }
   c->pool.swap(keep);
+  std::lock_guard<std::mutex> g(c->kept_mu);
+  for (auto &b : c->kept) NH_HIP(hipFree(b.p));
+  c->kept.clear();
+  return NH_OK;
+}
+
+// Blocks of nh_device_alloc freed by the caller stay with the context, at
+// most kKeepBlocks of them and kKeepShare of the device's memory, and serve
+// its next requests of the same size.  A program that asks for its vectors
+// anew on every call otherwise runs at the speed at which the driver clears
+// freed memory: products of 2 GB a call, each freed when the next one is
+// there, took 55 ms a call once the device had been gone through once
+// (37 GB/s), the call itself 3.5 ms.
+constexpr int kKeepBlocks = 8;
+constexpr size_t kKeepShare = 32;
+
+// true: *p is a kept block of exactly `bytes`
+static bool device_take(nh_context *c, void **p, size_t bytes) {
+  std::lock_guard<std::mutex> g(c->kept_mu);
+  for (size_t i = 0; i < c->kept.size(); ++i)
+    if (c->kept[i].bytes == bytes) {
+      *p = c->kept[i].p;
+      c->kept.erase(c->kept.begin() + i);
+      return true;
+    }
+  return false;
+}
+// keep p, or else free it (p that is not the start of a device allocation:
+// hipFree's error)
+static nh_status device_keep(nh_context *c, void *p) {
+  hipDeviceptr_t base = nullptr;
+  size_t bytes = 0, fr = 0, total = 0;
+  hipPointerAttribute_t at{};
+  const bool ours = hipPointerGetAttributes(&at, p) == hipSuccess &&
+                    at.type == hipMemoryTypeDevice && at.device == c->device &&
+                    hipMemGetAddressRange(&base, &bytes, p) == hipSuccess && base == p &&
+                    hipMemGetInfo(&fr, &total) == hipSuccess;
+  (void)hipGetLastError();
+  if (!ours || bytes > total / kKeepShare) {
+    NH_HIP(hipFree(p));
+    return NH_OK;
+  }
+  // as hipFree does: whatever stream used the memory is done with it
+  NH_HIP(hipDeviceSynchronize());
+  std::lock_guard<std::mutex> g(c->kept_mu);
+  for (const auto &b : c->kept)
+    NH_CHECK(b.p != p, NH_ERR_ARG, "nh_device_free: freed twice");
+  c->kept.push_back({p, bytes, false});
+  size_t sum = 0;
+  for (const auto &b : c->kept) sum += b.bytes;
+  while (sum > total / kKeepShare || c->kept.size() > (size_t)kKeepBlocks) {
+    // the oldest one goes
+    sum -= c->kept.front().bytes;
+    NH_HIP(hipFree(c->kept.front().p));
+    c->kept.erase(c->kept.begin());
+  }
   return NH_OK;
 }
 
@@ -111,10 +167,13 @@ void pool_release(nh_context *c, void *p) {
 size_t pool_free_bytes(const nh_context *c) {
   std::lock_guard<std::mutex> g(g_ctx_mu);
   size_t s = 0;
-  for (const nh_context *o : g_ctxs)
-    if (o->device == c->device)
+  for (nh_context *o : g_ctxs)
+    if (o->device == c->device) {
       for (const auto &b : o->pool)
         if (!b.used) s += b.bytes;
+      std::lock_guard<std::mutex> k(o->kept_mu);
+      for (const auto &b : o->kept) s += b.bytes;
+    }
   return s;
 }
 
@@ -150,12 +209,13 @@ static void destroy(nh_context *c) {
                   c->blk_local, c->blk_halo, c->blk_bonds, c->mf_geo, c->mf_q,
                   c->mf_pair, c->mf_ends,
                   c->rev_slot, c->onsite, c->blocks64, c->blocks32,
-                  c->onsite32, c->sk64, c->sk32, c->corr, c->red, c->xbuf,
+                  c->onsite32, c->sk64, c->sk32, c->red, c->xbuf,
                   c->ybuf};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   (void)hipStreamSynchronize(c->stream);
   for (auto &b : c->pool) (void)hipFree(b.p);
+  for (auto &b : c->kept) (void)hipFree(b.p);
   if (c->hred) (void)hipHostFree(c->hred);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -517,7 +577,7 @@ nh_status nh_hV(nh_context *ctx, double shift, const nh_cplx *X, nh_cplx *Y,
 
 nh_status nh_ham_export(nh_context *ctx, double *onsite, double *blocks) {
   NH_TRY(check_ctx(ctx));
-  NH_CHECK(ctx->onsite && ctx->blocks64, NH_ERR_STATE,
+  NH_CHECK(ctx->layout == NH_LAYOUT_BLOCKS && ctx->onsite && ctx->blocks64, NH_ERR_STATE,
            "nh_ham_export: needs a build in NH_LAYOUT_BLOCKS");
   const int A = ctx->n_atoms;
   if (onsite) {
@@ -547,14 +607,14 @@ nh_status nh_context_mem_info(nh_context *ctx, int64_t *free_bytes,
 nh_status nh_device_alloc(nh_context *ctx, int64_t bytes, void **dptr) {
   NH_TRY(check_ctx(ctx));
   NH_CHECK(dptr && bytes >= 0, NH_ERR_ARG, "nh_device_alloc: bad arguments");
+  if (device_take(ctx, dptr, (size_t)bytes)) return NH_OK;
   return device_malloc(ctx, dptr, (size_t)bytes);
 }
 
 nh_status nh_device_free(nh_context *ctx, void *dptr) {
   NH_TRY(check_ctx(ctx));
   NH_HIP(hipStreamSynchronize(ctx->stream));
-  if (dptr) NH_HIP(hipFree(dptr));
-  return NH_OK;
+  return dptr ? device_keep(ctx, dptr) : NH_OK;
 }
 
 nh_status nh_memcpy_h2d(nh_context *ctx, void *dst, const void *src,

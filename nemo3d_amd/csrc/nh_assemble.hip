@@ -264,29 +264,26 @@ inline int grid_for(int64_t n, int block) {
 
 }  // namespace
 
-static void free_ham(nh_context *c) {
-  (void)hipFree(c->onsite);
-  (void)hipFree(c->blocks64);
-  (void)hipFree(c->blocks32);
-  (void)hipFree(c->onsite32);
-  (void)hipFree(c->sk64);
-  (void)hipFree(c->sk32);
-  (void)hipFree(c->corr);
-  (void)hipFree(c->mf_geo);
-  (void)hipFree(c->mf_q);
-  (void)hipFree(c->mf_pair);
-  (void)hipFree(c->mf_ends);
-  c->mf_ends = nullptr;
-  c->mf_geo = nullptr;
-  c->mf_q = nullptr;
-  c->mf_pair = nullptr;
-  c->onsite = nullptr;
-  c->blocks64 = nullptr;
-  c->blocks32 = nullptr;
-  c->onsite32 = nullptr;
-  c->sk64 = nullptr;
-  c->sk32 = nullptr;
-  c->corr = nullptr;
+// What a rebuild does not use of the last build is freed; the rest is written
+// again (its sizes depend on the context alone).  Freeing and allocating all
+// of it took most of a rebuild (786,520 atoms: 2 GB).
+static void free_ham(nh_context *c, int layout) {
+  auto drop = [](auto *&p) {
+    (void)hipFree(p);
+    p = nullptr;
+  };
+  if (layout != NH_LAYOUT_BLOCKS) drop(c->blocks64);
+  // FP32 copies are derived anew (select_precision)
+  drop(c->blocks32);
+  drop(c->onsite32);
+  drop(c->sk32);
+  if (layout != NH_LAYOUT_SK) drop(c->sk64);
+  if (layout != NH_LAYOUT_MATRIX_FREE) {
+    drop(c->mf_geo);
+    drop(c->mf_q);
+    drop(c->mf_pair);
+    drop(c->mf_ends);
+  }
   c->layout = c->precision = -1;
 }
 
@@ -297,32 +294,41 @@ nh_status assemble(nh_context *c, int layout, int precision) {
   NH_CHECK(precision == NH_PREC_FP64 || precision == NH_PREC_FP32, NH_ERR_ARG,
            "precision %d not available", precision);
   NH_HIP(hipStreamSynchronize(c->stream));
-  free_ham(c);
+  free_ham(c, layout);
+  auto need = [c](auto **p, size_t bytes) {
+    return *p ? NH_OK : device_malloc(c, (void **)p, bytes);
+  };
   const int A = c->n_atoms;
   const size_t nblk = (size_t)A * 4 * 100;
-  NH_TRY(device_malloc(c, (void **)&c->onsite, (size_t)A * kOnsiteStride * sizeof(double)));
-  NH_TRY(device_malloc(c, (void **)&c->corr, (size_t)A * 4 * 10 * sizeof(double)));
-  NH_HIP(hipMemsetAsync(c->corr, 0, (size_t)A * 40 * sizeof(double), c->stream));
+  NH_TRY(need(&c->onsite, (size_t)A * kOnsiteStride * sizeof(double)));
+  double *corr = nullptr;
+  NH_TRY(pool_alloc(c, (void **)&corr, (size_t)A * 4 * 10 * sizeof(double)));
+  struct Release {
+    nh_context *c;
+    void *p;
+    ~Release() { pool_release(c, p); }
+  } release{c, corr};  // only the assembly needs the per-bond terms
+  NH_HIP(hipMemsetAsync(corr, 0, (size_t)A * 40 * sizeof(double), c->stream));
   if (layout == NH_LAYOUT_BLOCKS) {
-    NH_TRY(device_malloc(c, (void **)&c->blocks64, nblk * sizeof(double)));
+    NH_TRY(need(&c->blocks64, nblk * sizeof(double)));
     NH_HIP(hipMemsetAsync(c->blocks64, 0, nblk * sizeof(double), c->stream));
   }
   if (layout == NH_LAYOUT_SK) {
-    NH_TRY(device_malloc(c, (void **)&c->sk64, (size_t)c->n_cations * 4 * kSkStride * sizeof(double)));
+    NH_TRY(need(&c->sk64, (size_t)c->n_cations * 4 * kSkStride * sizeof(double)));
     NH_HIP(hipMemsetAsync(c->sk64, 0,
                           (size_t)c->n_cations * 4 * kSkStride * sizeof(double),
                           c->stream));
   }
   const int S = c->n_species;
   if (layout == NH_LAYOUT_MATRIX_FREE) {
-    NH_TRY(device_malloc(c, (void **)&c->mf_geo, (size_t)A * sizeof(double4)));
-    NH_TRY(device_malloc(c, (void **)&c->mf_q, (size_t)A * 4 * sizeof(int32_t)));
-    NH_TRY(device_malloc(c, (void **)&c->mf_pair, (size_t)S * S * kMfPair * sizeof(double)));
+    NH_TRY(need(&c->mf_geo, (size_t)A * sizeof(double4)));
+    NH_TRY(need(&c->mf_q, (size_t)A * 4 * sizeof(int32_t)));
+    NH_TRY(need(&c->mf_pair, (size_t)S * S * kMfPair * sizeof(double)));
     hipLaunchKernelGGL(k_mf_geo, dim3(grid_for(A, 128)), dim3(128), 0, c->stream,
                        A, c->species, c->is_cation, c->bond_q, c->disp,
                        c->mf_geo, c->mf_q);
     const int ne = c->n_blocks * kSkBondPad;
-    NH_TRY(device_malloc(c, (void **)&c->mf_ends, (size_t)ne * sizeof(int2)));
+    NH_TRY(need(&c->mf_ends, (size_t)ne * sizeof(int2)));
     hipLaunchKernelGGL(k_mf_ends, dim3(grid_for(ne, 256)), dim3(256), 0, c->stream, ne,
                        c->blk_bonds, c->cations, c->nbr, c->mf_ends);
     hipLaunchKernelGGL(k_mf_pair, dim3(1), dim3(64 * ((S * S + 63) / 64)), 0,
@@ -335,16 +341,14 @@ nh_status assemble(nh_context *c, int layout, int precision) {
                      dim3(128), 0, c->stream, c->n_cations, S, c->cations,
                      c->species, c->nbr, c->rev_slot, c->bond_q, c->disp,
                      c->lattice[0], c->lattice[1], c->lattice[2], c->parmat,
-                     c->strnmat, c->blocks64, c->corr, c->sk64);
+                     c->strnmat, c->blocks64, corr, c->sk64);
   NH_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_onsite, dim3(grid_for(A, 128)), dim3(128), 0, c->stream,
                      A, S, c->species, c->is_cation, c->nbr, c->bond_q,
                      c->parmat, c->strnmat, c->phi, c->passivate, c->db_shift,
-                     c->corr, c->onsite);
+                     corr, c->onsite);
   NH_HIP(hipGetLastError());
   NH_HIP(hipStreamSynchronize(c->stream));
-  (void)hipFree(c->corr);  // only the assembly needs the per-bond terms
-  c->corr = nullptr;
   c->layout = layout;
   c->precision = NH_PREC_FP64;
   return select_precision(c, precision);

@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <string>
 #include <utility>
+#include <mutex>
 #include <vector>
 
 #include "../../include/nemohip.h"
@@ -101,8 +102,6 @@ struct nh_context {
   float *onsite32 = nullptr;    // [A][kOnsiteStride] (FP32 runs)
   double *sk64 = nullptr;       // [Nc*4][kSkStride] (NH_LAYOUT_SK)
   float *sk32 = nullptr;
-  double *corr = nullptr;       // [A][4][10] Boykin corrections (scratch)
-  // NH_LAYOUT_MATRIX_FREE: bond records recomputed on every product from
   double4 *mf_geo = nullptr;    // [A] displacement (nm) x, y, z; species
   int32_t *mf_q = nullptr;      // [A][4] ideal bond vector of the slot seen
                                 // from its cation, units a/4, 3 x int8
@@ -125,6 +124,10 @@ struct nh_context {
     bool used;
   };
   std::vector<PoolBlock> pool;
+  // blocks of nh_device_alloc that were freed, for its next requests of the
+  // same size (device_keep); several threads may allocate on one context
+  std::vector<PoolBlock> kept;
+  std::mutex kept_mu;
 };
 
 namespace nh {
