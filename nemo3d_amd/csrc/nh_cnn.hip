@@ -5,7 +5,7 @@
 // then a 1x1x1 head W -> c_out.  Activations are FP32, channels last
 // ([point][channel], point = (x*gy + y)*gz + z).  Weights are kept as FP32
 // master copies for Adam and used as BF16 in the forward and backward
-// products (FP32 accumulation).
+// products (FP32 accumulation; kernels in nh_cnn_mfma.h).
 // Parameter vector: for each conv layer W_l[co][ci][27], b_l[co]; then the
 // head W_h[co][ci], b_h[co].
 //
@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "nh_blockla.h"
+#include "nh_cnn_mfma.h"
 #include "nh_vector.h"
 
 struct nh_cnn {
@@ -30,240 +31,34 @@ struct nh_cnn {
   std::vector<int64_t> w_off, b_off;  // per layer (conv layers, then head)
   float *master = nullptr;            // FP32 parameters
   uint16_t *bf = nullptr;             // BF16 copy used by the products
+  uint16_t *packed = nullptr;         // .. in the order of the matrix operands
+  int64_t n_packed = 0;
+  nh::PackList pack{};                // .. its parts
+  std::vector<std::vector<int>> fwd_seg;  // per conv layer: parts of 32 input channels
+  std::vector<int> bwd_seg;               // per conv layer (0: none)
+  int head_seg = 0, headt_seg = 0;
   float *grad = nullptr, *m1 = nullptr, *m2 = nullptr;
   int64_t step = 0;
   // activations for the current grid
   int64_t cap_points = 0;
-  std::vector<float *> pre, act;  // per conv layer, [P][W]
-  float *in = nullptr, *out = nullptr, *dact = nullptr, *dtmp = nullptr;
+  std::vector<float *> act;  // per conv layer, [P][W] (after the relu)
+  float *in = nullptr;
+  // head output or its gradient [P][c_out], gradients before a relu [P][W],
+  // partial sums: allocated by the calls that need them
+  int64_t cap_out = 0, cap_grad = 0;
+  size_t cap_part = 0;
+  float *out = nullptr, *dpre[2] = {nullptr, nullptr};
   double *part = nullptr;
 };
 
 namespace nh {
 namespace {
 
-__device__ __forceinline__ float bf16_to_f(uint16_t h) {
-  return __uint_as_float(((uint32_t)h) << 16);
-}
-// round to nearest even
-__device__ __forceinline__ uint16_t f_to_bf16(float f) {
-  uint32_t u = __float_as_uint(f);
-  const uint32_t lsb = (u >> 16) & 1u;
-  u += 0x7FFFu + lsb;
-  return (uint16_t)(u >> 16);
-}
-
 __global__ void k_to_bf16(int64_t n, const float *__restrict__ a,
                           uint16_t *__restrict__ b) {
   for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < n;
        k += (int64_t)gridDim.x * blockDim.x)
     b[k] = f_to_bf16(a[k]);
-}
-
-// neighbour offset k in 0..26 -> (dx, dy, dz) in {-1,0,1}
-__device__ __forceinline__ void koff(int k, int &dx, int &dy, int &dz) {
-  dx = k / 9 - 1;
-  dy = (k / 3) % 3 - 1;
-  dz = k % 3 - 1;
-}
-
-// forward conv3x3x3 + ReLU: one thread per point, all CO outputs
-template <int CO>
-__global__ __launch_bounds__(128) void k_conv_fwd(
-    int gx, int gy, int gz, int ci_n, const float *__restrict__ in,
-    const uint16_t *__restrict__ W, const uint16_t *__restrict__ b,
-    float *__restrict__ pre, float *__restrict__ act) {
-  extern __shared__ uint16_t wsh[];  // [CO][ci_n][27]
-  const int nw = CO * ci_n * 27;
-  for (int t = threadIdx.x; t < nw; t += blockDim.x) wsh[t] = W[t];
-  __syncthreads();
-  const int64_t P = (int64_t)gx * gy * gz;
-  const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (p >= P) return;
-  const int z = p % gz, y = (p / gz) % gy, x = p / ((int64_t)gy * gz);
-  float acc[CO];
-#pragma unroll
-  for (int co = 0; co < CO; ++co) acc[co] = bf16_to_f(b[co]);
-  for (int k = 0; k < 27; ++k) {
-    int dx, dy, dz;
-    koff(k, dx, dy, dz);
-    const int xx = x + dx, yy = y + dy, zz = z + dz;
-    if (xx < 0 || yy < 0 || zz < 0 || xx >= gx || yy >= gy || zz >= gz) continue;
-    const float *src = in + (((int64_t)xx * gy + yy) * gz + zz) * ci_n;
-    for (int ci = 0; ci < ci_n; ++ci) {
-      const float v = src[ci];
-      if (v == 0.0f) continue;
-#pragma unroll
-      for (int co = 0; co < CO; ++co)
-        acc[co] += bf16_to_f(wsh[(co * ci_n + ci) * 27 + k]) * v;
-    }
-  }
-#pragma unroll
-  for (int co = 0; co < CO; ++co) {
-    pre[p * CO + co] = acc[co];
-    act[p * CO + co] = acc[co] > 0.0f ? acc[co] : 0.0f;
-  }
-}
-
-// head 1x1x1: out[p][co] = b[co] + sum_ci W[co][ci] a[p][ci].  Lane =
-// output channel of a 64-channel chunk (blockIdx.y), so a wavefront writes
-// 64 consecutive outputs of one point and reads that point's inputs as one
-// broadcast; each wavefront walks groups of kHeadPts points.  The chunk's weights sit
-// in LDS as FP32, [ci][64] (lane-consecutive, no bank conflicts).
-constexpr int kHeadPts = 8;
-__global__ __launch_bounds__(256) void k_head_fwd(
-    int64_t P, int ci_n, int co_n, const float *__restrict__ a,
-    const uint16_t *__restrict__ W, const uint16_t *__restrict__ b,
-    float *__restrict__ out) {
-  extern __shared__ float whs[];  // [ci_n][64]
-  const int co0 = blockIdx.y * 64;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  for (int t = threadIdx.x; t < 64 * ci_n; t += blockDim.x) {
-    const int ci = t >> 6, c = t & 63;
-    whs[t] = co0 + c < co_n ? bf16_to_f(W[(size_t)(co0 + c) * ci_n + ci]) : 0.0f;
-  }
-  __syncthreads();
-  const int co = co0 + lane;
-  const bool ok = co < co_n;
-  const float bias = ok ? bf16_to_f(b[co]) : 0.0f;
-  // groups of kHeadPts points, grid-stride (the grid is capped)
-  for (int64_t g = (int64_t)blockIdx.x * 4 + w; g * kHeadPts < P;
-       g += (int64_t)gridDim.x * 4) {
-    for (int k = 0; k < kHeadPts; ++k) {
-      const int64_t p = g * kHeadPts + k;
-      if (p >= P) break;
-      const float *ap = a + p * ci_n;
-      float s = bias;
-      for (int ci = 0; ci < ci_n; ++ci) s += whs[ci * 64 + lane] * ap[ci];
-      if (ok) out[p * co_n + co] = s;
-    }
-  }
-}
-
-// head backward, data: da[p][ci] = sum_co W[co][ci] dout[p][co].  Lane =
-// input channel (ci_n <= 64 lanes of a wavefront per point), so the
-// point's dout is read as broadcasts and da written contiguously; W is
-// read lane-consecutive from the caches; grid-stride over points.
-__global__ __launch_bounds__(256) void k_head_bwd_data(
-    int64_t P, int ci_n, int co_n, const float *__restrict__ dout,
-    const uint16_t *__restrict__ W, float *__restrict__ da) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane >= ci_n) return;
-  for (int64_t p = (int64_t)blockIdx.x * 4 + w; p < P; p += (int64_t)gridDim.x * 4) {
-    const float *dp = dout + p * co_n;
-    float s = 0.0f;
-    for (int co = 0; co < co_n; ++co) s += bf16_to_f(W[(size_t)co * ci_n + lane]) * dp[co];
-    da[p * ci_n + lane] = s;
-  }
-}
-
-// sum over a workgroup of 256 (float accumulate in double for stability)
-__device__ __forceinline__ double wg_sum256(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  __shared__ double s[4];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  __syncthreads();
-  if (lane == 0) s[w] = v;
-  __syncthreads();
-  return s[0] + s[1] + s[2] + s[3];
-}
-
-// head backward, weights: one workgroup per output channel co
-__global__ __launch_bounds__(256) void k_head_bwd_w(
-    int64_t P, int ci_n, int co_n, const float *__restrict__ dout,
-    const float *__restrict__ a, float *__restrict__ gW, float *__restrict__ gb) {
-  const int co = blockIdx.x;
-  double acc[64];
-  for (int ci = 0; ci < ci_n; ++ci) acc[ci] = 0.0;
-  double sb = 0.0;
-  for (int64_t p = threadIdx.x; p < P; p += blockDim.x) {
-    const float g = dout[p * co_n + co];
-    if (g == 0.0f) continue;
-    sb += g;
-    for (int ci = 0; ci < ci_n; ++ci) acc[ci] += (double)g * a[p * ci_n + ci];
-  }
-  for (int ci = 0; ci < ci_n; ++ci) {
-    const double t = wg_sum256(acc[ci]);
-    if (threadIdx.x == 0) gW[(size_t)co * ci_n + ci] = (float)t;
-  }
-  const double t = wg_sum256(sb);
-  if (threadIdx.x == 0) gb[co] = (float)t;
-}
-
-// dpre = dact * relu'(pre)
-__global__ void k_relu_bwd(int64_t n, const float *__restrict__ pre,
-                           const float *__restrict__ dact, float *__restrict__ dpre) {
-  for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < n;
-       k += (int64_t)gridDim.x * blockDim.x)
-    dpre[k] = pre[k] > 0.0f ? dact[k] : 0.0f;
-}
-
-// conv backward, data: din[p][ci] = sum_{co,k} W[co][ci][k] dpre[p - d_k][co]
-template <int CO>
-__global__ __launch_bounds__(128) void k_conv_bwd_data(
-    int gx, int gy, int gz, int ci_n, const float *__restrict__ dpre,
-    const uint16_t *__restrict__ W, float *__restrict__ din) {
-  extern __shared__ uint16_t wsh[];
-  const int nw = CO * ci_n * 27;
-  for (int t = threadIdx.x; t < nw; t += blockDim.x) wsh[t] = W[t];
-  __syncthreads();
-  const int64_t P = (int64_t)gx * gy * gz;
-  const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (p >= P) return;
-  const int z = p % gz, y = (p / gz) % gy, x = p / ((int64_t)gy * gz);
-  for (int ci = 0; ci < ci_n; ++ci) {
-    float s = 0.0f;
-    for (int k = 0; k < 27; ++k) {
-      int dx, dy, dz;
-      koff(k, dx, dy, dz);
-      const int xx = x - dx, yy = y - dy, zz = z - dz;
-      if (xx < 0 || yy < 0 || zz < 0 || xx >= gx || yy >= gy || zz >= gz) continue;
-      const float *g = dpre + (((int64_t)xx * gy + yy) * gz + zz) * CO;
-#pragma unroll
-      for (int co = 0; co < CO; ++co)
-        s += bf16_to_f(wsh[(co * ci_n + ci) * 27 + k]) * g[co];
-    }
-    din[p * ci_n + ci] = s;
-  }
-}
-
-// conv backward, weights: one workgroup per (co, ci); 27 sums over points
-__global__ __launch_bounds__(256) void k_conv_bwd_w(
-    int gx, int gy, int gz, int ci_n, int co_n, const float *__restrict__ dpre,
-    const float *__restrict__ in, float *__restrict__ gW) {
-  const int co = blockIdx.x / ci_n, ci = blockIdx.x % ci_n;
-  const int64_t P = (int64_t)gx * gy * gz;
-  double acc[27];
-#pragma unroll
-  for (int k = 0; k < 27; ++k) acc[k] = 0.0;
-  for (int64_t p = threadIdx.x; p < P; p += blockDim.x) {
-    const float g = dpre[p * co_n + co];
-    if (g == 0.0f) continue;
-    const int z = p % gz, y = (p / gz) % gy, x = p / ((int64_t)gy * gz);
-#pragma unroll
-    for (int k = 0; k < 27; ++k) {
-      const int dx = k / 9 - 1, dy = (k / 3) % 3 - 1, dz = k % 3 - 1;
-      const int xx = x + dx, yy = y + dy, zz = z + dz;
-      if (xx < 0 || yy < 0 || zz < 0 || xx >= gx || yy >= gy || zz >= gz) continue;
-      acc[k] += (double)g * in[(((int64_t)xx * gy + yy) * gz + zz) * ci_n + ci];
-    }
-  }
-  for (int k = 0; k < 27; ++k) {
-    const double t = wg_sum256(acc[k]);
-    if (threadIdx.x == 0) gW[((size_t)co * ci_n + ci) * 27 + k] = (float)t;
-  }
-}
-
-// bias gradient of a conv layer: one workgroup per channel
-__global__ __launch_bounds__(256) void k_bias_bwd(int64_t P, int co_n,
-                                                  const float *__restrict__ dpre,
-                                                  float *__restrict__ gb) {
-  const int co = blockIdx.x;
-  double s = 0.0;
-  for (int64_t p = threadIdx.x; p < P; p += blockDim.x) s += dpre[p * co_n + co];
-  const double t = wg_sum256(s);
-  if (threadIdx.x == 0) gb[co] = (float)t;
 }
 
 __global__ void k_adam(int64_t n, float *__restrict__ w,
@@ -281,42 +76,42 @@ __global__ void k_adam(int64_t n, float *__restrict__ w,
   }
 }
 
-// head output -> start block: y_e[atom*nb + o] from out[point][(e*2nb + slot*nb + o)*2 .. +1]
-__global__ void k_map_out(int64_t A, int nb, int ne, int c_out,
-                          const int32_t *__restrict__ point,
-                          const int32_t *__restrict__ slot,
-                          const float *__restrict__ out, double2 *__restrict__ Y,
-                          int64_t ld) {
+// Gradient w.r.t. the start block, g_e = sum_f v_f M[f][e] + D[e] y_e, to the
+// head output's gradient (points without atoms keep the zeros they were
+// given): one pass over the targets and the prediction, no gradient block in
+// between.
+__global__ __launch_bounds__(256) void k_loss_grad(
+    int64_t A, int nb, int nf, int ne, int c_out, const int32_t *__restrict__ point,
+    const int32_t *__restrict__ slot, const double2 *__restrict__ V,
+    const double2 *__restrict__ Y, int64_t ld, const double2 *__restrict__ MD,
+    float *__restrict__ dout) {
+  __shared__ double2 m[17 * 8];  // M[f][e], then D[e]
+  for (int t = threadIdx.x; t < 17 * 8; t += blockDim.x) m[t] = MD[t];
+  __syncthreads();
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < A * nb;
        t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t a = t / nb;
-    const int o = t % nb;
-    const float *src = out + (int64_t)point[a] * c_out;
-    for (int e = 0; e < ne; ++e) {
-      const int ch = 2 * ((e * 2 + slot[a]) * nb + o);
-      Y[e * ld + t] = make_double2(src[ch], src[ch + 1]);
+    double2 g[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) g[e] = make_double2(0.0, 0.0);
+    for (int f = 0; f < nf; ++f) {
+      const double2 v = V[f * ld + t];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const double2 c = m[f * 8 + e];
+        g[e].x += v.x * c.x - v.y * c.y;
+        g[e].y += v.x * c.y + v.y * c.x;
+      }
     }
-  }
-}
-
-// gradient w.r.t. the start block -> head output gradient (points without
-// atoms get zero: the caller clears dout first)
-__global__ void k_map_grad(int64_t A, int nb, int ne, int c_out,
-                           const int32_t *__restrict__ point,
-                           const int32_t *__restrict__ slot,
-                           const double2 *__restrict__ G, int64_t ld,
-                           float *__restrict__ dout) {
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < A * nb;
-       t += (int64_t)gridDim.x * blockDim.x) {
     const int64_t a = t / nb;
-    const int o = t % nb;
-    float *dst = dout + (int64_t)point[a] * c_out;
-    for (int e = 0; e < ne; ++e) {
-      const int ch = 2 * ((e * 2 + slot[a]) * nb + o);
-      const double2 g = G[e * ld + t];
-      dst[ch] = (float)g.x;
-      dst[ch + 1] = (float)g.y;
-    }
+    float *dst = dout + (int64_t)point[a] * c_out + 2 * (slot[a] * nb + t % nb);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (e < ne) {
+        const double2 y = Y[e * ld + t];
+        const double d = m[16 * 8 + e].x;
+        dst[4 * e * nb] = (float)(g[e].x + d * y.x);
+        dst[4 * e * nb + 1] = (float)(g[e].y + d * y.y);
+      }
   }
 }
 
@@ -325,77 +120,140 @@ int g1(int64_t n, int b = 256) {
   return (int)(g < 1 ? 1 : (g > 65535 ? 65535 : g));
 }
 
+// (re)allocate *p for `bytes`
+template <typename T>
+nh_status regrow(nh_cnn *c, T **p, size_t bytes) {
+  (void)hipFree(*p);
+  *p = nullptr;
+  return device_malloc(c->ctx, (void **)p, bytes);
+}
+
 nh_status ensure_acts(nh_cnn *c, int64_t P) {
   if (P <= c->cap_points) return NH_OK;
-  for (float *q : c->pre) (void)hipFree(q);
-  for (float *q : c->act) (void)hipFree(q);
-  (void)hipFree(c->in);
-  (void)hipFree(c->out);
-  (void)hipFree(c->dact);
-  (void)hipFree(c->dtmp);
-  c->pre.assign(c->layers, nullptr);
-  c->act.assign(c->layers, nullptr);
-  for (int l = 0; l < c->layers; ++l) {
-    NH_TRY(device_malloc(c->ctx, (void **)&c->pre[l], P * c->width * sizeof(float)));
-    NH_TRY(device_malloc(c->ctx, (void **)&c->act[l], P * c->width * sizeof(float)));
-  }
-  const int cmax = std::max(std::max(c->c_in, c->width), c->c_out);
-  NH_TRY(device_malloc(c->ctx, (void **)&c->in, P * c->c_in * sizeof(float)));
-  NH_TRY(device_malloc(c->ctx, (void **)&c->out, P * c->c_out * sizeof(float)));
-  NH_TRY(device_malloc(c->ctx, (void **)&c->dact, P * cmax * sizeof(float)));
-  NH_TRY(device_malloc(c->ctx, (void **)&c->dtmp, P * cmax * sizeof(float)));
+  c->cap_points = 0;
+  c->act.resize(c->layers, nullptr);
+  for (int l = 0; l < c->layers; ++l)
+    NH_TRY(regrow(c, &c->act[l], P * c->width * sizeof(float)));
+  NH_TRY(regrow(c, &c->in, P * c->c_in * sizeof(float)));
   c->cap_points = P;
   return NH_OK;
 }
+nh_status ensure_out(nh_cnn *c, int64_t P) {
+  if (P <= c->cap_out) return NH_OK;
+  c->cap_out = 0;
+  NH_TRY(regrow(c, &c->out, P * c->c_out * sizeof(float)));
+  c->cap_out = P;
+  return NH_OK;
+}
+nh_status ensure_grads(nh_cnn *c, int64_t P) {
+  if (P <= c->cap_grad) return NH_OK;
+  c->cap_grad = 0;
+  for (float *&q : c->dpre) NH_TRY(regrow(c, &q, P * c->width * sizeof(float)));
+  c->cap_grad = P;
+  return NH_OK;
+}
+nh_status ensure_part(nh_cnn *c, size_t count) {
+  if (count <= c->cap_part) return NH_OK;
+  c->cap_part = 0;
+  NH_TRY(regrow(c, &c->part, count * sizeof(double)));
+  c->cap_part = count;
+  return NH_OK;
+}
 
+template <bool BWD>
+void launch_conv(nh_cnn *c, int gx, int gy, int gz, int ld, const PackSeg &g, bool last,
+                 const float *in, const uint16_t *bias, const float *mask, float *out) {
+  const int seg = conv_segment(gx, gy, gz);
+  const dim3 grid((gz + kConvTZ - 1) / kConvTZ, (gy + kConvTY - 1) / kConvTY,
+                  (gx + seg - 1) / seg);
+  const uint4 *W = reinterpret_cast<const uint4 *>(c->packed + g.dst);
+  if (BWD || g.ks == 2)
+    hipLaunchKernelGGL((k_conv<2, BWD>), grid, dim3(256), 0, c->ctx->stream, gx, gy, gz, seg,
+                       ld, g.ci0, in, W, bias, last, mask, out);
+  else
+    hipLaunchKernelGGL((k_conv<1, false>), grid, dim3(256), 0, c->ctx->stream, gx, gy, gz, seg,
+                       ld, g.ci0, in, W, bias, last, mask, out);
+}
+
+// the conv layers: act[l] for every point
 nh_status forward(nh_cnn *c, int gx, int gy, int gz) {
-  const int64_t P = (int64_t)gx * gy * gz;
-  hipStream_t st = c->ctx->stream;
+  NH_CHECK((gy + kConvTY - 1) / kConvTY <= 65535 && gx <= 65535, NH_ERR_ARG,
+           "network: grid %d x %d x %d too large", gx, gy, gz);
   const float *src = c->in;
   int ci = c->c_in;
   for (int l = 0; l < c->layers; ++l) {
-    const size_t shm = (size_t)c->width * ci * 27 * sizeof(uint16_t);
-    NH_CHECK(c->width == 32, NH_ERR_ARG, "network width must be 32");
-    hipLaunchKernelGGL(k_conv_fwd<32>, dim3(g1(P, 128)), dim3(128), shm, st, gx,
-                       gy, gz, ci, src, c->bf + c->w_off[l], c->bf + c->b_off[l],
-                       c->pre[l], c->act[l]);
+    const auto &segs = c->fwd_seg[l];
+    for (size_t k = 0; k < segs.size(); ++k)
+      launch_conv<false>(c, gx, gy, gz, ci, c->pack.s[segs[k]], k + 1 == segs.size(), src,
+                         k == 0 ? c->bf + c->b_off[l] : nullptr, nullptr, c->act[l]);
     src = c->act[l];
     ci = c->width;
   }
+  NH_HIP(hipGetLastError());
+  return NH_OK;
+}
+// the head at every point, to c->out
+nh_status head(nh_cnn *c, int64_t P) {
   const int L = c->layers;
-  hipLaunchKernelGGL(k_head_fwd, dim3(g1(P, 4 * kHeadPts), (c->c_out + 63) / 64),
-                     dim3(256), 64 * ci * sizeof(float), st, P, ci, c->c_out,
-                     src, c->bf + c->w_off[L], c->bf + c->b_off[L], c->out);
+  hipLaunchKernelGGL(k_head_fwd, dim3(g1(P, 128)), dim3(256), 0, c->ctx->stream, P, c->c_out,
+                     c->act[L - 1],
+                     reinterpret_cast<const uint4 *>(c->packed + c->pack.s[c->head_seg].dst),
+                     c->bf + c->b_off[L], c->out);
+  NH_HIP(hipGetLastError());
+  return NH_OK;
+}
+// the head at the atoms, to the start block
+nh_status head_map(nh_cnn *c, int ne, const int32_t *point, const int32_t *slot, double2 *Y) {
+  const nh_context *x = c->ctx;
+  const int L = c->layers;
+  hipLaunchKernelGGL(k_head_map, dim3(g1(x->n_atoms, 128)), dim3(256), 0, x->stream,
+                     (int64_t)x->n_atoms, x->nb, ne, c->c_out, point, slot, c->act[L - 1],
+                     reinterpret_cast<const uint4 *>(c->packed + c->pack.s[c->head_seg].dst),
+                     c->bf + c->b_off[L], Y, x->n);
   NH_HIP(hipGetLastError());
   return NH_OK;
 }
 
-// parameter gradient of sum(out * dout); dout in c->dtmp layout [P][c_out]
+// parameter gradient of sum(out * dout), dout [P][c_out]
 nh_status backward(nh_cnn *c, int gx, int gy, int gz, const float *dout) {
   const int64_t P = (int64_t)gx * gy * gz;
   hipStream_t st = c->ctx->stream;
   const int L = c->layers, W = c->width;
-  const float *alast = L > 0 ? c->act[L - 1] : c->in;
-  hipLaunchKernelGGL(k_head_bwd_w, dim3(c->c_out), dim3(256), 0, st, P, W,
-                     c->c_out, dout, alast, c->grad + c->w_off[L],
-                     c->grad + c->b_off[L]);
-  NH_CHECK(W <= 64, NH_ERR_ARG, "network width above 64");
-  hipLaunchKernelGGL(k_head_bwd_data, dim3(g1(P, 4)), dim3(256), 0, st, P, W,
-                     c->c_out, dout, c->bf + c->w_off[L], c->dact);
+  NH_TRY(ensure_grads(c, P));
+  // chunks of points, none smaller than a few lines: as many workgroups as
+  // run at a time (3 a compute unit for the head, 2 for the conv layers with
+  // their nine offsets)
+  const int co_tiles = (c->c_out + 63) / 64;
+  const int hch = (int)std::max<int64_t>(1, std::min<int64_t>(P / 256, 768 / co_tiles));
+  const int64_t hlen = (int64_t)c->c_out * (W + 1);
+  const int cch = (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)gx * gy / 8, 56));
+  const int cmax = std::max((c->c_in + 15) / 16 * 16, W);
+  NH_TRY(ensure_part(c, std::max(hch * hlen, (int64_t)cch * (27 * W * cmax + W))));
+  auto sum = [&](int chunks, int64_t len, int conv_ci, float *grad) {
+    hipLaunchKernelGGL(k_grad_sum, dim3((len + 255) / 256), dim3(256), 0, st, chunks, len,
+                       conv_ci, c->part, grad);
+  };
+  hipLaunchKernelGGL(k_head_bwd_w, dim3(hch, co_tiles), dim3(256), 0, st, P, c->c_out, dout,
+                     c->act[L - 1], c->part, hlen);
+  sum(hch, hlen, 0, c->grad + c->w_off[L]);
+  hipLaunchKernelGGL(k_head_bwd_data, dim3(g1(P, 128)), dim3(256), 0, st, P, c->c_out, dout,
+                     reinterpret_cast<const uint4 *>(c->packed + c->pack.s[c->headt_seg].dst),
+                     c->act[L - 1], c->dpre[0]);
   for (int l = L - 1; l >= 0; --l) {
     const int ci = l == 0 ? c->c_in : W;
     const float *in = l == 0 ? c->in : c->act[l - 1];
-    // dact (for act[l]) -> dpre in dtmp
-    hipLaunchKernelGGL(k_relu_bwd, dim3(g1(P * W)), dim3(256), 0, st, P * W,
-                       c->pre[l], c->dact, c->dtmp);
-    hipLaunchKernelGGL(k_conv_bwd_w, dim3(W * ci), dim3(256), 0, st, gx, gy, gz,
-                       ci, W, c->dtmp, in, c->grad + c->w_off[l]);
-    hipLaunchKernelGGL(k_bias_bwd, dim3(W), dim3(256), 0, st, P, W, c->dtmp,
-                       c->grad + c->b_off[l]);
+    const int64_t len = 27 * W * (int64_t)((ci + 15) / 16 * 16) + W;
+    if (ci <= 16)
+      hipLaunchKernelGGL(k_conv_bwd_w<1>, dim3(9 * cch), dim3(256), 0, st, gx, gy, gz, ci,
+                         cch, c->dpre[0], in, c->part, len);
+    else
+      hipLaunchKernelGGL(k_conv_bwd_w<2>, dim3(9 * cch, (ci + 31) / 32), dim3(256), 0, st, gx,
+                         gy, gz, ci, cch, c->dpre[0], in, c->part, len);
+    sum(cch, len, ci, c->grad + c->w_off[l]);
     if (l > 0) {
-      const size_t shm = (size_t)W * ci * 27 * sizeof(uint16_t);
-      hipLaunchKernelGGL(k_conv_bwd_data<32>, dim3(g1(P, 128)), dim3(128), shm,
-                         st, gx, gy, gz, ci, c->dtmp, c->bf + c->w_off[l], c->dact);
+      launch_conv<true>(c, gx, gy, gz, W, c->pack.s[c->bwd_seg[l]], true, c->dpre[0], nullptr,
+                        c->act[l - 1], c->dpre[1]);
+      std::swap(c->dpre[0], c->dpre[1]);
     }
   }
   NH_HIP(hipGetLastError());
@@ -419,11 +277,37 @@ void init_layout(nh_cnn *c) {
   c->b_off.push_back(off);
   off += c->c_out;
   c->n_params = off;
+  // packed operands (k_pack_weights)
+  int64_t dst = 0;
+  auto add = [&](int kind, int ci_n, int ci0, int ks, int co_n, int64_t src, int64_t frags) {
+    c->pack.s[c->pack.n] = PackSeg{kind, ci_n, ci0, ks, co_n, src, dst, frags};
+    dst += frags * 512;
+    return c->pack.n++;
+  };
+  c->pack.n = 0;
+  ci = c->c_in;
+  for (int l = 0; l < c->layers; ++l) {
+    c->fwd_seg.emplace_back();
+    for (int ci0 = 0; ci0 < ci; ci0 += 32) {
+      const int ks = std::min(2, (ci - ci0 + 15) / 16);
+      c->fwd_seg[l].push_back(add(kPackConv, ci, ci0, ks, c->width, c->w_off[l], 27 * ks));
+    }
+    c->bwd_seg.push_back(l == 0 ? 0 : add(kPackConvT, ci, 0, 2, c->width, c->w_off[l], 54));
+    ci = c->width;
+  }
+  // the head's rows are padded to whole blocks of k_head_map
+  const int64_t blocks = (c->c_out + kMapRows - 1) / kMapRows;
+  c->head_seg = add(kPackHead, ci, 0, 2, c->c_out, c->w_off[c->layers],
+                    blocks * (kMapRows / 32) * 2);
+  c->headt_seg = add(kPackHeadT, ci, 0, 1, c->c_out, c->w_off[c->layers], (c->c_out + 15) / 16);
+  c->n_packed = dst;
 }
 
 nh_status sync_bf16(nh_cnn *c) {
   hipLaunchKernelGGL(k_to_bf16, dim3(g1(c->n_params)), dim3(256), 0,
                      c->ctx->stream, c->n_params, c->master, c->bf);
+  hipLaunchKernelGGL(k_pack_weights, dim3(54, c->pack.n), dim3(256), 0, c->ctx->stream,
+                     c->pack, c->bf, c->packed);
   NH_HIP(hipGetLastError());
   return NH_OK;
 }
@@ -485,6 +369,7 @@ nh_status nh_cnn_create(nh_context *ctx, int c_in, int width, int layers,
   };
   mk((void **)&c->master, c->n_params * sizeof(float));
   mk((void **)&c->bf, c->n_params * sizeof(uint16_t));
+  mk((void **)&c->packed, c->n_packed * sizeof(uint16_t));
   mk((void **)&c->grad, c->n_params * sizeof(float));
   mk((void **)&c->m1, c->n_params * sizeof(float));
   mk((void **)&c->m2, c->n_params * sizeof(float));
@@ -511,10 +396,9 @@ nh_status nh_cnn_create(nh_context *ctx, int c_in, int width, int layers,
 void nh_cnn_destroy(nh_cnn *c) {
   if (!c) return;
   (void)hipSetDevice(c->device);
-  for (float *q : c->pre) (void)hipFree(q);
   for (float *q : c->act) (void)hipFree(q);
-  void *ps[] = {c->master, c->bf, c->grad, c->m1, c->m2, c->in, c->out,
-                c->dact, c->dtmp, c->part};
+  void *ps[] = {c->master, c->bf, c->packed, c->grad, c->m1, c->m2, c->in, c->out,
+                c->dpre[0], c->dpre[1], c->part};
   for (void *q : ps)
     if (q) (void)hipFree(q);
   delete c;
@@ -543,7 +427,9 @@ nh_status nh_cnn_forward(nh_cnn *c, const float *feat, int gx, int gy, int gz,
   (void)hipGetLastError();
   const int64_t P = (int64_t)gx * gy * gz;
   NH_TRY(upload_feats(c, feat, P));
+  NH_TRY(ensure_out(c, P));
   NH_TRY(forward(c, gx, gy, gz));
+  NH_TRY(head(c, P));
   NH_HIP(hipMemcpyAsync(out, c->out, P * c->c_out * sizeof(float),
                         hipMemcpyDeviceToHost, c->ctx->stream));
   NH_HIP(hipStreamSynchronize(c->ctx->stream));
@@ -556,8 +442,9 @@ nh_status nh_cnn_backward(nh_cnn *c, const float *feat, int gx, int gy, int gz,
   (void)hipGetLastError();
   const int64_t P = (int64_t)gx * gy * gz;
   NH_TRY(upload_feats(c, feat, P));
+  NH_TRY(ensure_out(c, P));
   NH_TRY(forward(c, gx, gy, gz));
-  float *d = c->out;  // reuse the output buffer for dout
+  float *d = c->out;  // holds dout
   NH_HIP(hipMemcpyAsync(d, dout, P * c->c_out * sizeof(float),
                         hipMemcpyHostToDevice, c->ctx->stream));
   NH_TRY(backward(c, gx, gy, gz, d));
@@ -589,38 +476,33 @@ nh_status nh_cnn_start_block(nh_cnn *c, const float *feat, int gx, int gy,
   const int64_t P = (int64_t)gx * gy * gz, A = x->n_atoms;
   NH_TRY(upload_feats(c, feat, P));
   NH_TRY(forward(c, gx, gy, gz));
+  std::vector<void *> mem;  // from the context's pool
+  auto mk = [&](void **p, size_t bytes) -> nh_status {
+    NH_TRY(pool_alloc(x, p, bytes));
+    mem.push_back(*p);
+    return NH_OK;
+  };
   int32_t *dp = nullptr, *ds = nullptr;
-  NH_TRY(device_malloc(x, (void **)&dp, A * sizeof(int32_t)));
-  NH_TRY(device_malloc(x, (void **)&ds, A * sizeof(int32_t)));
-  {
-    hipError_t e = hipMemcpy(dp, atom_point, A * sizeof(int32_t), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(ds, atom_slot, A * sizeof(int32_t), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-      (void)hipFree(dp);
-      (void)hipFree(ds);
-      NH_CHECK(false, NH_ERR_HIP, "nh_cnn_start_block: %s", hipGetErrorString(e));
-    }
-  }
-  double2 *Y = reinterpret_cast<double2 *>(block);
   double2 *tmp = nullptr;
-  if (ptr_kind == NH_PTR_HOST) {
-    if (device_malloc(x, (void **)&tmp, (size_t)n_states * x->n * sizeof(double2)) != NH_OK) {
-      (void)hipFree(dp);
-      (void)hipFree(ds);
-      NH_CHECK(false, NH_ERR_NOMEM, "nh_cnn_start_block: out of memory");
-    }
-    Y = tmp;
+  nh_status st = mk((void **)&dp, A * sizeof(int32_t));
+  if (st == NH_OK) st = mk((void **)&ds, A * sizeof(int32_t));
+  if (st == NH_OK && ptr_kind == NH_PTR_HOST)
+    st = mk((void **)&tmp, (size_t)n_states * x->n * sizeof(double2));
+  hipError_t e = hipSuccess;
+  if (st == NH_OK) {
+    e = hipMemcpyAsync(dp, atom_point, A * sizeof(int32_t), hipMemcpyHostToDevice, x->stream);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(ds, atom_slot, A * sizeof(int32_t), hipMemcpyHostToDevice, x->stream);
+    if (e == hipSuccess)
+      st = head_map(c, n_states, dp, ds, tmp ? tmp : reinterpret_cast<double2 *>(block));
+    if (st == NH_OK && e == hipSuccess && tmp)
+      e = hipMemcpyAsync(block, tmp, (size_t)n_states * x->n * sizeof(double2),
+                         hipMemcpyDeviceToHost, x->stream);
   }
-  hipLaunchKernelGGL(k_map_out, dim3(g1(A * x->nb)), dim3(256), 0, x->stream, A,
-                     x->nb, n_states, c->c_out, dp, ds, c->out, Y, x->n);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess && tmp)
-    e = hipMemcpyAsync(block, tmp, (size_t)n_states * x->n * sizeof(double2),
-                       hipMemcpyDeviceToHost, x->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(x->stream);
-  (void)hipFree(dp);
-  (void)hipFree(ds);
-  if (tmp) (void)hipFree(tmp);
+  const hipError_t es = hipStreamSynchronize(x->stream);
+  if (e == hipSuccess) e = es;
+  for (void *q : mem) pool_release(x, q);
+  NH_TRY(st);
   NH_CHECK(e == hipSuccess, NH_ERR_HIP, "nh_cnn_start_block: %s", hipGetErrorString(e));
   return NH_OK;
 }
@@ -642,29 +524,33 @@ nh_status nh_cnn_train_step(nh_cnn *c, const float *feat, int gx, int gy, int gz
   const int ne = n_states;
   NH_TRY(upload_feats(c, feat, P));
   NH_TRY(forward(c, gx, gy, gz));
-  // device scratch: point/slot maps, Y (prediction, 8 columns), V (targets,
-  // 16 columns), G (gradient, 8 columns)
+  // device scratch from the context's pool: point/slot maps, Y (prediction),
+  // host targets' copy
+  hipPointerAttribute_t pa{};
+  const bool on_device = hipPointerGetAttributes(&pa, targets) == hipSuccess &&
+                         pa.type == hipMemoryTypeDevice && pa.device == x->device &&
+                         reinterpret_cast<uintptr_t>(targets) % sizeof(double2) == 0;
+  (void)hipGetLastError();  // pageable host memory is not a registered pointer
   std::vector<void *> mem;
   auto mk = [&](void **p, size_t bytes) -> nh_status {
-    NH_TRY(device_malloc(x, p, bytes));
+    NH_TRY(pool_alloc(x, p, bytes));
     mem.push_back(*p);
     return NH_OK;
   };
   auto cleanup = [&]() {
-    for (void *q : mem) (void)hipFree(q);
+    for (void *q : mem) pool_release(x, q);
   };
   int32_t *dp, *ds;
-  double2 *Y, *V, *G;
+  double2 *Y, *Vh = nullptr;
   double *part, *sum, *dM;
-  nh_status st = NH_OK;
+  nh_status st = ensure_out(c, P);
   if (st == NH_OK) st = mk((void **)&dp, A * sizeof(int32_t));
   if (st == NH_OK) st = mk((void **)&ds, A * sizeof(int32_t));
-  if (st == NH_OK) st = mk((void **)&Y, (size_t)8 * N * sizeof(double2));
-  if (st == NH_OK) st = mk((void **)&V, (size_t)16 * N * sizeof(double2));
-  if (st == NH_OK) st = mk((void **)&G, (size_t)8 * N * sizeof(double2));
+  if (st == NH_OK) st = mk((void **)&Y, (size_t)ne * N * sizeof(double2));
+  if (st == NH_OK && !on_device) st = mk((void **)&Vh, (size_t)n_targets * N * sizeof(double2));
   if (st == NH_OK) st = mk((void **)&part, (size_t)512 * 2 * 64 * sizeof(double));
-  if (st == NH_OK) st = mk((void **)&sum, 2 * 64 * sizeof(double));
-  if (st == NH_OK) st = mk((void **)&dM, 2 * 64 * sizeof(double));
+  if (st == NH_OK) st = mk((void **)&sum, 3 * 128 * sizeof(double));
+  if (st == NH_OK) st = mk((void **)&dM, 17 * 8 * sizeof(double2));
   if (st != NH_OK) {
     cleanup();
     return st;
@@ -681,27 +567,27 @@ nh_status nh_cnn_train_step(nh_cnn *c, const float *feat, int gx, int gy, int gz
   } while (0)
   TS_HIP(hipMemcpyAsync(dp, atom_point, A * sizeof(int32_t), hipMemcpyHostToDevice, s));
   TS_HIP(hipMemcpyAsync(ds, atom_slot, A * sizeof(int32_t), hipMemcpyHostToDevice, s));
-  TS_HIP(hipMemsetAsync(Y, 0, (size_t)8 * N * sizeof(double2), s));
-  TS_HIP(hipMemsetAsync(V, 0, (size_t)16 * N * sizeof(double2), s));
-  // targets may be host or device memory (unified addressing)
-  TS_HIP(hipMemcpyAsync(V, targets, (size_t)n_targets * N * sizeof(double2),
-                 hipMemcpyDefault, s));
-  hipLaunchKernelGGL(k_map_out, dim3(g1(A * x->nb)), dim3(256), 0, s, A, x->nb,
-                     ne, c->c_out, dp, ds, c->out, Y, N);
-  // C = V^H Y (16 x 8, two 8x8 halves) and the Gram Y^H Y
-  std::vector<double> h(2 * 128), hb(2 * 64);
-  for (int half = 0; half < 2; ++half) {
-    hipLaunchKernelGGL((k_gram<8>), dim3(512), dim3(256), 0, s, N, 8, 8,
-                       V + (int64_t)half * 8 * N, N, Y, N, part);
-    hipLaunchKernelGGL(k_sum_cols, dim3(128), dim3(128), 0, s, 512, 128, part, sum);
-    TS_HIP(hipMemcpyAsync(h.data() + half * 128, sum, 128 * sizeof(double),
-                   hipMemcpyDeviceToHost, s));
-    // the next k_sum_cols overwrites `sum`: wait for the copy
-    TS_HIP(hipStreamSynchronize(s));
+  if (!on_device)
+    TS_HIP(hipMemcpyAsync(Vh, targets, (size_t)n_targets * N * sizeof(double2),
+                          hipMemcpyDefault, s));
+  const double2 *V = on_device ? reinterpret_cast<const double2 *>(targets) : Vh;
+  if (head_map(c, ne, dp, ds, Y) != NH_OK) {
+    cleanup();
+    return NH_ERR_HIP;
   }
-  hipLaunchKernelGGL((k_gram<8>), dim3(512), dim3(256), 0, s, N, 8, 8, Y, N, Y, N, part);
-  hipLaunchKernelGGL(k_sum_cols, dim3(128), dim3(128), 0, s, 512, 128, part, sum);
-  TS_HIP(hipMemcpyAsync(hb.data(), sum, 128 * sizeof(double), hipMemcpyDeviceToHost, s));
+  // C = V^H Y (up to 16 x 8, two halves of 8 rows) and the norms of Y
+  std::vector<double> h(2 * 128, 0.0), hb(16);
+  for (int half = 0; 8 * half < n_targets; ++half) {
+    hipLaunchKernelGGL((k_gram<8>), dim3(512), dim3(256), 0, s, N,
+                       std::min(8, n_targets - 8 * half), ne, V + (int64_t)half * 8 * N, N, Y,
+                       N, part);
+    hipLaunchKernelGGL(k_sum_cols, dim3(128), dim3(128), 0, s, 512, 128, part, sum + 128 * half);
+    TS_HIP(hipMemcpyAsync(h.data() + half * 128, sum + 128 * half, 128 * sizeof(double),
+                   hipMemcpyDeviceToHost, s));
+  }
+  hipLaunchKernelGGL((k_coldot<8>), dim3(512), dim3(256), 0, s, N, ne, Y, N, Y, N, part);
+  hipLaunchKernelGGL(k_sum_cols, dim3(16), dim3(128), 0, s, 512, 16, part, sum + 256);
+  TS_HIP(hipMemcpyAsync(hb.data(), sum + 256, 16 * sizeof(double), hipMemcpyDeviceToHost, s));
   hipError_t e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
     cleanup();
@@ -715,47 +601,28 @@ nh_status nh_cnn_train_step(nh_cnn *c, const float *feat, int gx, int gy, int gz
   // L = mean_e (1 - a_e / b_e), a_e = sum over the targets of e's cluster of
   // |C[f][e]|^2, b_e = ||y_e||^2;  G_e = dL/dRe(y_e) + i dL/dIm(y_e)
   //     = 2 (-sum_f v_f C[f][e] / b_e + a_e y_e / b_e^2) / ne
-  std::vector<cd> M(128, 0.0), D(64, 0.0);
+  std::vector<cd> M(17 * 8, 0.0);  // M[f][e], then D[e]
   double L = 0.0;
   for (int ee = 0; ee < ne; ++ee) {
-    const double b = std::max(hb[2 * (ee * 8 + ee)], 1e-300);
+    const double b = std::max(hb[2 * ee], 1e-300);
     double a = 0.0;
     for (int f = 0; f < n_targets; ++f)
       if (cluster[f] == out_cluster[ee]) a += std::norm(C(f, ee));
     L += (1.0 - a / b) / ne;
     for (int f = 0; f < n_targets; ++f)
       if (cluster[f] == out_cluster[ee]) M[f * 8 + ee] = -2.0 * C(f, ee) / (b * ne);
-    D[ee * 8 + ee] = 2.0 * a / (b * b * ne);
+    M[16 * 8 + ee] = 2.0 * a / (b * b * ne);
   }
   *loss = L;
-  std::vector<double> hm(128);
-  for (int half = 0; half < 2; ++half) {
-    for (int k = 0; k < 64; ++k) {
-      hm[2 * k] = M[half * 64 + k].real();
-      hm[2 * k + 1] = M[half * 64 + k].imag();
-    }
-    TS_HIP(hipMemcpyAsync(dM, hm.data(), 128 * sizeof(double), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL((k_block_gemm<8>), dim3(g1(N)), dim3(256), 0, s, N, 8, 8,
-                       V + (int64_t)half * 8 * N, N, G, N, dM, half ? 1.0 : 0.0);
-    TS_HIP(hipStreamSynchronize(s));  // hm is rewritten next
-  }
-  for (int k = 0; k < 64; ++k) {
-    hm[2 * k] = D[k].real();
-    hm[2 * k + 1] = 0.0;
-  }
-  TS_HIP(hipMemcpyAsync(dM, hm.data(), 128 * sizeof(double), hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL((k_block_gemm<8>), dim3(g1(N)), dim3(256), 0, s, N, 8, 8, Y,
-                     N, G, N, dM, 1.0);
+  TS_HIP(hipMemcpyAsync(dM, M.data(), M.size() * sizeof(cd), hipMemcpyHostToDevice, s));
   // dL/d(out): real and imaginary parts of the complex gradient
-  TS_HIP(hipMemsetAsync(c->dtmp, 0, P * c->c_out * sizeof(float), s));
-  hipLaunchKernelGGL(k_map_grad, dim3(g1(A * x->nb)), dim3(256), 0, s, A, x->nb,
-                     ne, c->c_out, dp, ds, G, N, c->dtmp);
-  // backward needs a dout buffer that survives: move it into c->out
-  TS_HIP(hipMemcpyAsync(c->out, c->dtmp, P * c->c_out * sizeof(float),
-                 hipMemcpyDeviceToDevice, s));
+  TS_HIP(hipMemsetAsync(c->out, 0, P * c->c_out * sizeof(float), s));
+  hipLaunchKernelGGL(k_loss_grad, dim3(g1(A * x->nb)), dim3(256), 0, s, A, x->nb, n_targets,
+                     ne, c->c_out, dp, ds, V, Y, N, reinterpret_cast<const double2 *>(dM),
+                     c->out);
+  TS_HIP(hipGetLastError());
 #undef TS_HIP
-  e = hipStreamSynchronize(s);
-  if (e == hipSuccess) {
+  {
     nh_status bs = backward(c, gx, gy, gz, c->out);
     if (bs != NH_OK) {
       cleanup();
