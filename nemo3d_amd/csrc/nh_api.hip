@@ -217,6 +217,7 @@ static void destroy(nh_context *c) {
   for (auto &b : c->pool) (void)hipFree(b.p);
   for (auto &b : c->kept) (void)hipFree(b.p);
   if (c->hred) (void)hipHostFree(c->hred);
+  if (c->side) (void)hipStreamDestroy(c->side);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }

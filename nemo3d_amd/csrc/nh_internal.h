@@ -66,6 +66,7 @@ struct nh_context {
   int passivate = 0;
   double db_shift = 0;
   hipStream_t stream = nullptr;
+  hipStream_t side = nullptr;  // convergence checks beside the steps (on first use)
 
   // model (device)
   double *parmat = nullptr;     // [S][S][35]

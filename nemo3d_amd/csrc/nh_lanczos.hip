@@ -14,10 +14,10 @@
 // The reference's REDUCE_OPT variant of the iteration (lanczos.c:441-456)
 // defers the vector update into the next iteration in the same spirit, to
 // merge its two reductions into one.
-// alpha and beta stay in device arrays; the host copies the tridiagonal
-// every ConvCheckSkipRate iterations and analyses it (Sturm bisection in
-// the Erange windows, convergence by the trailing components of the
-// tridiagonal eigenvector, find_converged_eigval Method 2,
+// alpha and beta stay in device arrays; every ConvCheckSkipRate iterations
+// the tridiagonal is analysed on a second stream (k_tri_windows, nh_tri.h:
+// eigenvalues in the Erange windows, convergence by the trailing components
+// of the tridiagonal eigenvector, find_converged_eigval Method 2,
 // lanczos.c:764-996).  Eigenvectors come from a second pass over the same
 // recurrence (eigenvectorsLanczos, lanczos.c:1364-1689): the Lanczos
 // vectors land in a ring (K = 128 steps, fewer when memory is short) and
@@ -28,12 +28,12 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
-#include <thread>
 #include <type_traits>
 #include <vector>
 
 #include "nh_hv_row.h"
 #include "nh_hv_sk.h"
+#include "nh_tri.h"
 #include "nh_vector.h"
 
 namespace nh {
@@ -541,31 +541,6 @@ __global__ void k_scale(int64_t n, double2 *__restrict__ x, double s) {
 
 // ---------------- host-side tridiagonal analysis ---------------------------
 
-int sturm(const std::vector<double> &d, const std::vector<double> &e, int m,
-          double x) {
-  int cnt = 0;
-  double q = d[0] - x;
-  if (q < 0) ++cnt;
-  for (int i = 1; i < m; ++i) {
-    if (q == 0.0) q = 1e-300;
-    q = d[i] - x - e[i - 1] * e[i - 1] / q;
-    if (q < 0) ++cnt;
-  }
-  return cnt;
-}
-
-// k-th smallest eigenvalue (0-based) of T_m by bisection on [lo, hi].
-double bisect(const std::vector<double> &d, const std::vector<double> &e,
-              int m, int k, double lo, double hi, double abstol) {
-  for (int it = 0; it < 200 && hi - lo > abstol; ++it) {
-    const double mid = 0.5 * (lo + hi);
-    if (mid <= lo || mid >= hi) break;
-    if (sturm(d, e, m, mid) > k) hi = mid;
-    else lo = mid;
-  }
-  return 0.5 * (lo + hi);
-}
-
 // Eigenvector of T_m at lambda by inverse iteration (tridiagonal Gaussian
 // elimination with partial pivoting), from a fixed pseudo-random start.
 void tri_eigvec(const std::vector<double> &d, const std::vector<double> &e,
@@ -614,23 +589,6 @@ void tri_eigvec(const std::vector<double> &d, const std::vector<double> &e,
   }
 }
 
-// f(j) for j < count on up to 8 host threads (independent j)
-template <typename F>
-void host_parallel_for(int count, F f) {
-  const int hw = (int)std::max(1u, std::thread::hardware_concurrency());
-  const int nt = std::min({count, hw, 8});
-  if (nt <= 1) {
-    for (int j = 0; j < count; ++j) f(j);
-    return;
-  }
-  std::vector<std::thread> pool;
-  for (int t = 0; t < nt; ++t)
-    pool.emplace_back([&f, t, nt, count] {
-      for (int j = t; j < count; j += nt) f(j);
-    });
-  for (auto &th : pool) th.join();
-}
-
 struct Converged {
   double value;
   int iter;
@@ -643,9 +601,13 @@ class LanczosRun {
   LanczosRun(nh_context *c, bool classic) : c_(c), classic_(classic) {}
   ~LanczosRun() {
     release_events();
+    // a check that nobody waited for (error returns) still uses the buffers
+    if (c_->side) (void)hipStreamSynchronize(c_->side);
     for (void *p : allocs_) pool_release(c_, p);
+    if (tri_s_) pool_release(c_, tri_s_);
     if (pin_) (void)hipHostFree(pin_);
-    if (fetch_ev_) (void)hipEventDestroy(fetch_ev_);
+    for (hipEvent_t e : {fetch_ev_, check_ev_})
+      if (e) (void)hipEventDestroy(e);
   }
   nh_status run(const nh_lanczos_opts *o, nh_eig_result *res);
   // run() ended because the deferred step's beta has lost digits
@@ -661,6 +623,7 @@ class LanczosRun {
   nh_status iterate(int k, bool with_reductions);
   nh_status collect_timing();
   nh_status fetch(int m);
+  nh_status check(int m);
   nh_status analyse(int m, const nh_lanczos_opts *o);
   bool window_done(int w, int req, int rule) const;
 
@@ -696,11 +659,16 @@ class LanczosRun {
   double *alpha_ = nullptr, *beta_ = nullptr, *part_ = nullptr;
   int nparts_ = 0;
   std::vector<double> ha_, hb_;
-  // pinned staging of alpha (first half) and beta, filled up to fetched_
-  // by copies behind fetch_ev_
+  // pinned staging of alpha, beta (pin_cap_ each, filled up to fetched_) and
+  // of the last check's results; fetch_ev_: alpha and beta are there on the
+  // context's stream, check_ev_: the check of checked_ steps is done
   double *pin_ = nullptr;
   int pin_cap_ = 0, fetched_ = 0;
-  hipEvent_t fetch_ev_ = nullptr;
+  hipEvent_t fetch_ev_ = nullptr, check_ev_ = nullptr;
+  int checked_ = 0;
+  TriWindows win_{};
+  double *tri_out_ = nullptr, *tri_s_ = nullptr;  // results, scratch of the check
+  int64_t tri_cap_ = 0;                           // doubles in tri_s_
   std::vector<Converged> conv_;
   std::vector<double> lastRitz_[2];
   std::vector<char> lastConv_[2];
@@ -999,22 +967,49 @@ nh_status LanczosRun::fetch(int m) {
       hipLaunchKernelGGL(k_lz_scalars3, dim3(1), dim3(kRedThreads), 0, c_->stream, grid_,
                          part_ + (size_t)(last_ & 1) * 3 * nparts_, alpha_ + last_,
                          beta_ + last_);
-    NH_HIP(hipMemcpyAsync(pin_ + fetched_, alpha_ + fetched_,
-                          (m - fetched_) * sizeof(double), hipMemcpyDeviceToHost,
-                          c_->stream));
+    NH_HIP(hipGetLastError());
+    NH_HIP(hipEventRecord(fetch_ev_, c_->stream));
+    NH_HIP(hipStreamWaitEvent(c_->side, fetch_ev_, 0));
+    NH_HIP(hipMemcpyAsync(pin_ + fetched_, alpha_ + fetched_, (m - fetched_) * sizeof(double),
+                          hipMemcpyDeviceToHost, c_->side));
     NH_HIP(hipMemcpyAsync(pin_ + pin_cap_ + fetched_, beta_ + fetched_,
-                          (m - fetched_) * sizeof(double), hipMemcpyDeviceToHost,
-                          c_->stream));
+                          (m - fetched_) * sizeof(double), hipMemcpyDeviceToHost, c_->side));
     fetched_ = m;
   }
-  NH_HIP(hipEventRecord(fetch_ev_, c_->stream));
+  return check(m);
+}
+
+// queue the check of the first m steps (fetched before) on the side stream;
+// the earlier one has been waited for
+nh_status LanczosRun::check(int m) {
+  const int waves = win_.want[0] + win_.want[1];
+  if (waves > 0) {
+    const int64_t need = (int64_t)waves * 2 * m;
+    if (need > tri_cap_) {
+      if (tri_s_) pool_release(c_, tri_s_);
+      tri_s_ = nullptr;
+      tri_cap_ = 0;
+      const int64_t rows = std::max<int64_t>(2 * m, 2048);
+      NH_TRY(pool_alloc(c_, (void **)&tri_s_, waves * 2 * rows * sizeof(double)));
+      tri_cap_ = waves * 2 * rows;
+    }
+    hipLaunchKernelGGL(k_tri_windows, dim3(waves), dim3(64), 0, c_->side, m, alpha_, beta_, win_,
+                       tri_s_, (int64_t)2 * m, tri_out_);
+    NH_HIP(hipGetLastError());
+    NH_HIP(hipMemcpyAsync(pin_ + 2 * (size_t)pin_cap_, tri_out_,
+                          (kTriHead + (size_t)waves * kTriOut) * sizeof(double),
+                          hipMemcpyDeviceToHost, c_->side));
+  }
+  NH_HIP(hipEventRecord(check_ev_, c_->side));
+  checked_ = m;
   return NH_OK;
 }
 
 // analyse the tridiagonal of the first m steps (fetch(m) queued before)
 nh_status LanczosRun::analyse(int m, const nh_lanczos_opts *o) {
   NH_CHECK(fetched_ >= m, NH_ERR_STATE, "Lanczos: tridiagonal not fetched");
-  NH_HIP(hipEventSynchronize(fetch_ev_));
+  if (checked_ != m) NH_TRY(check(m));
+  NH_HIP(hipEventSynchronize(check_ev_));
   ha_.assign(pin_, pin_ + m);
   hb_.assign(pin_ + pin_cap_, pin_ + pin_cap_ + m);
   // The deferred FP64 step has beta^2 as a difference of sums, |u|^2 - alpha^2:
@@ -1030,7 +1025,7 @@ nh_status LanczosRun::analyse(int m, const nh_lanczos_opts *o) {
   const double resolution = 100.0 * tol;  // lanczos.c:1970
   const double bias = 1e-80;
   const int req[2] = {o->num_eig_vb, o->num_eig_cb};
-  const double *win[2] = {o->erange_vb, o->erange_cb};
+  const double *tri = pin_ + 2 * (size_t)pin_cap_;
   // nearest-the-gap rule: two converged copies of one level differ by up to
   // about 2 tol ||T|| (each Ritz value within beta tol of it), which the
   // reference's relative resolution misses for levels near 0 eV; that rule
@@ -1048,19 +1043,10 @@ nh_status LanczosRun::analyse(int m, const nh_lanczos_opts *o) {
     lastRitz_[w].clear();
     lastConv_[w].clear();
     if (req[w] <= 0) continue;
-    const double lo = win[w][0], hi = win[w][1];
-    const int klo = sturm(ha_, hb_, m, lo), khi = sturm(ha_, hb_, m, hi);
-    // candidates nearest the gap: top of vb, bottom of cb
-    const int want = req[w] + 24;
-    int k0 = klo, k1 = khi;
-    if (w == 0) k0 = std::max(klo, khi - want);
-    else k1 = std::min(khi, klo + want);
-    // bisection of the candidates and the trailing components of their
-    // tridiagonal eigenvectors, each independent: spread over host threads
-    std::vector<double> ev(std::max(0, k1 - k0));
-    host_parallel_for((int)ev.size(), [&](int j) {
-      ev[j] = bisect(ha_, hb_, m, k0 + j, lo, hi, 1e-13);
-    });
+    // the candidates nearest the gap: top of vb, bottom of cb
+    std::vector<double> ev((size_t)tri[w]);
+    const double *o3 = tri + kTriHead + (w ? win_.want[0] : 0) * kTriOut;
+    for (size_t i = 0; i < ev.size(); ++i) ev[i] = o3[kTriOut * i];
     auto duplicate = [&](size_t i) {
       // copies of one eigenvalue (ghosts, degeneracies) count once
       return i > 0 && std::fabs(ev[i - 1] - ev[i]) <
@@ -1071,20 +1057,12 @@ nh_status LanczosRun::analyse(int m, const nh_lanczos_opts *o) {
         if (std::fabs(cv.value - v) < resolution) return true;
       return false;
     };
-    std::vector<double> tail((size_t)2 * ev.size(), 1.0);
-    host_parallel_for((int)ev.size(), [&](int j) {
-      if (duplicate(j) || known_value(ev[j])) return;
-      std::vector<double> xj;
-      tri_eigvec(ha_, hb_, m, ev[j], xj);
-      tail[2 * j] = xj[m - 1];
-      tail[2 * j + 1] = m >= 2 ? xj[m - 2] : 0.0;
-    });
     for (size_t i = 0; i < ev.size(); ++i) {
       if (duplicate(i)) continue;
       const bool known = known_value(ev[i]);
       bool ok = known;
       if (!known) {
-        ok = std::fabs(tail[2 * i]) <= tol && std::fabs(tail[2 * i + 1]) <= tol;
+        ok = std::fabs(o3[kTriOut * i + 1]) <= tol && std::fabs(o3[kTriOut * i + 2]) <= tol;
         if (ok) conv_.push_back({ev[i], m, w});
       }
       lastRitz_[w].push_back(ev[i]);
@@ -1130,16 +1108,23 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
     NH_TRY(upload_start(R_, vbytes_));
   }
 
-  // pass 1: eigenvalues.  The host analyses the tridiagonal of one check
-  // point while the device runs the steps up to the next one: at a check
-  // point the new alpha, beta are copied behind an event, and they are
-  // analysed at the following check point, after that block of steps has
-  // been queued.  Convergence is thus seen one block late; the steps of
+  // pass 1: eigenvalues.  The tridiagonal of one check point is analysed
+  // (k_tri_windows, on a second stream) while the device runs the steps up to
+  // the next one, and its results are looked at there, after that block of
+  // steps has been queued.  Convergence is thus seen one block late; the steps of
   // that block are not used (the run ends at the converged check point).
   pin_cap_ = o->max_iter + 1;
-  NH_HIP(hipHostMalloc((void **)&pin_, 2 * (size_t)pin_cap_ * sizeof(double),
+  win_ = TriWindows{{o->erange_vb[0], o->erange_cb[0]},
+                    {o->erange_vb[1], o->erange_cb[1]},
+                    {o->num_eig_vb > 0 ? o->num_eig_vb + 24 : 0,
+                     o->num_eig_cb > 0 ? o->num_eig_cb + 24 : 0}};
+  const size_t tri = kTriHead + (size_t)(win_.want[0] + win_.want[1]) * kTriOut;
+  NH_TRY(alloc((void **)&tri_out_, tri * sizeof(double)));
+  NH_HIP(hipHostMalloc((void **)&pin_, (2 * (size_t)pin_cap_ + tri) * sizeof(double),
                        hipHostMallocDefault));
+  if (!c->side) NH_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
   NH_HIP(hipEventCreateWithFlags(&fetch_ev_, hipEventDisableTiming));
+  NH_HIP(hipEventCreateWithFlags(&check_ev_, hipEventDisableTiming));
   int m = 0, skip = 0, pending = -1;
   bool done = false;
   int matvecs = 0;
