@@ -1,17 +1,27 @@
 // On-device assembly of the sp3d5s* Hamiltonian.
 //
-// k_bond: one thread per cation-owned bond (every zincblende bond joins one
-// cation-role and one anion-role atom, so each bond is computed exactly
-// once, as the reference stores each bond once in HamZincBlende::Hu).  It
-// evaluates the strain-scaled Slater-Koster block and the Boykin diagonal
-// corrections of both atoms (H_DiagStrainCorr_OffDiag_Wrapper +
-// h3d_offdiag_diag_corr, h_cvectr_mult.c:1007-1126,
-// mb_ham_spds_micro.c:597-1451).
-// k_onsite: one thread per atom builds the onsite record: neighbour-averaged
-// parameters, strain reference shift, dangling-bond passivation, potential
-// and the summed corrections (H_Diag_Wrapper, h_cvectr_mult.c:841-1005;
-// h3d_diag, mb_ham_spds_micro.c:1453-1505;
-// h3d_diag_dangling_bond_shift_zincblende, mb_ham_spds_micro.c:1910-2152).
+// k_assemble: a quad of lanes per atom, a lane per neighbour slot.  A lane
+// evaluates its bond in the cation's frame (so both rows of a bond get the
+// same bits), writes what the layout stores of it (its own row's 10x10 block,
+// or, the cation's lane, the SK record) and the Boykin diagonal corrections
+// of its own atom (H_DiagStrainCorr_OffDiag_Wrapper + h3d_offdiag_diag_corr,
+// h_cvectr_mult.c:1007-1126, mb_ham_spds_micro.c:597-1451); the quad adds
+// them up and builds the onsite record: neighbour-averaged parameters, strain
+// reference shift, dangling-bond passivation, potential and corrections
+// (H_Diag_Wrapper, h_cvectr_mult.c:841-1005; h3d_diag,
+// mb_ham_spds_micro.c:1453-1505; h3d_diag_dangling_bond_shift_zincblende,
+// mb_ham_spds_micro.c:1910-2152).
+// Each bond is evaluated from both ends: that costs 15 exponentials and about
+// 300 operations a bond and saves a pass over 320 B an atom of corrections.
+// The corrections are sums of squares of a row of the block less those of the
+// unstrained block; the squares of a shell pair add up to its integrals'
+// squares weighted by the row's angular functions, so neither block is formed
+// (two tables of 100 numbers in scratch, a division per entry and 21 powers a
+// bond took 0.86 ms for 395,136 atoms, the onsite records 0.07 and the fills
+// 0.04; this 0.19 ms, 0.21 GB written; bound by the FP64 operations and the
+// parameters' loads at two wavefronts a SIMD).
+#include <utility>
+
 #include "nh_internal.h"
 #include "nh_hv_sk.h"
 
@@ -32,122 +42,173 @@ __device__ __forceinline__ void cation_bond_vectors(
   }
 }
 
-__global__ void k_bond(int n_cations, int S, const int32_t *__restrict__ cations,
-                       const int32_t *__restrict__ species,
-                       const int32_t *__restrict__ nbr,
-                       const int32_t *__restrict__ rev_slot,
-                       const int32_t *__restrict__ bond_q,
-                       const double *__restrict__ disp, double lx, double ly,
-                       double lz, const double *__restrict__ parmat,
-                       const double *__restrict__ strnmat,
-                       double *__restrict__ blocks, double *__restrict__ corr,
-                       double *__restrict__ sk) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n_cations * 4) return;
-  const int ci = t >> 2, slot = t & 3;
-  const int i = cations[ci];
-  const int j = nbr[i * 4 + slot];
-  if (j < 0) return;
-  const int jslot = rev_slot[i * 4 + slot];
-  const double *par = parmat + ((size_t)species[i] * S + species[j]) * 35;
-  const double *strn = strnmat + ((size_t)species[i] * S + species[j]) * 33;
-  const double lat[3] = {lx, ly, lz};
-  double nnv[3], nnv0[3];
-  cation_bond_vectors(bond_q, disp, lat, i, slot, j, par[P_A0], nnv, nnv0);
-  const BondGeom g = bond_geom(nnv, nnv0, par[P_A0]);
+// Integrals (index in parameters 10..30) of a shell of the anion with a shell
+// of the cation: sigma, then pi, delta (-1: none)
+__host__ __device__ constexpr int pair_integral(int sa, int sc, int part) {
+  constexpr int s[16] = {1, 2, 6, 10, 3, 0, 4, 8, 7, 5, 12, 14, 11, 9, 15, 18};
+  return part == 0 ? s[sa * 4 + sc]
+         : sa == 2 && sc == 2 ? (part == 1 ? 13 : -1)
+         : sa == 2 && sc == 3 ? (part == 1 ? 16 : -1)
+         : sa == 3 && sc == 2 ? (part == 1 ? 17 : -1)
+         : sa == 3 && sc == 3 ? 18 + part : -1;
+}
+// Weights of the squared sigma, pi and delta integrals in the sum of squares
+// over a row of a shell pair (row: p or d orbital; the same whatever the
+// other shell, which only lacks the later ones)
+struct RowWeights {
+  double p[3], ds[5], dp[5], dd[5];
+  __device__ __forceinline__ RowWeights(double l, double m, double n) {
+    const double l2 = l * l, m2 = m * m, n2 = n * n, dl = l2 - m2, lpm = l2 + m2,
+                 z = n2 - 0.5 * lpm;
+    p[0] = l2, p[1] = m2, p[2] = n2;
+    ds[0] = 3.0 * l2 * m2, ds[1] = 3.0 * m2 * n2, ds[2] = 3.0 * n2 * l2;
+    ds[3] = 0.75 * dl * dl, ds[4] = z * z;
+    dp[0] = lpm - 4.0 * l2 * m2, dp[1] = m2 + n2 - 4.0 * m2 * n2;
+    dp[2] = n2 + l2 - 4.0 * n2 * l2, dp[3] = lpm - dl * dl, dp[4] = 3.0 * n2 * lpm;
+    dd[0] = n2 + l2 * m2, dd[1] = l2 + m2 * n2, dd[2] = m2 + n2 * l2;
+    dd[3] = n2 + 0.25 * dl * dl, dd[4] = 0.75 * lpm * lpm;
+  }
+  // sum over the row of orbital o (0..9) with the squares of a shell pair
+  template <int O>
+  __device__ __forceinline__ double row(double s, double pi, double delta) const {
+    if constexpr (O < 2) return s;
+    else if constexpr (O < 5) return p[O - 2] * s + (1.0 - p[O - 2]) * pi;
+    else return ds[O - 5] * s + dp[O - 5] * pi + dd[O - 5] * delta;
+  }
+};
 
-  double v[21];
-  scale_integrals(par, strn, g.brat, v);
-  double T[100];
-  sk_table(g.l, g.m, g.n, v, T);
-  if (blocks) {  // stored-block layout only
-    double *Ba = blocks + ((size_t)j * 4 + jslot) * 100;  // anion row: T
-    double *Bc = blocks + ((size_t)i * 4 + slot) * 100;   // cation row: T^T
-#pragma unroll
-    for (int a = 0; a < 10; ++a)
-#pragma unroll
-      for (int c = 0; c < 10; ++c) {
-        Ba[a * 10 + c] = T[a * 10 + c];
-        Bc[c * 10 + a] = T[a * 10 + c];
-      }
-  }
-  if (sk) {
-    double *rec = sk + (size_t)t * kSkStride;
-    double k[kSkStride];
-    sk_record(g.l, g.m, g.n, v, k);
-#pragma unroll
-    for (int i = 0; i < kSkStride; ++i) rec[i] = k[i];
-  }
-  // Boykin terms ((V0^2 - V^2) c_strain / (E_a + E_c)) * c_pair
-  // (mb_ham_spds_VoffdEdiag_constructors.h; the pVpE_* macros are not
-  // parenthesised, so the pair coefficient multiplies the quotient).
-  double T0[100];
-  sk_table(g.l0, g.m0, g.n0, par + 10, T0);
-  const double cs = strn[S_CONST];
-  double cc[10];
-#pragma unroll
-  for (int c = 0; c < 10; ++c) cc[c] = 0.0;
-#pragma unroll
-  for (int a = 0; a < 10; ++a) {
-    double ca = 0.0;
-#pragma unroll
-    for (int c = 0; c < 10; ++c) {
-      const int sa = shell_of(a), sc = shell_of(c);
-      const double r1 = T[a * 10 + c], r2 = T0[a * 10 + c];
-      const double r3 = (r2 * r2 - r1 * r1) * cs /
-                        (par[e_anion(sa)] + par[e_cation(sc)]) *
-                        strn[cpair_index(sa, sc)];
-      ca += r3;
-      cc[c] += r3;
-    }
-    corr[((size_t)j * 4 + jslot) * 10 + a] = ca;
-  }
-#pragma unroll
-  for (int c = 0; c < 10; ++c) corr[((size_t)i * 4 + slot) * 10 + c] = cc[c];
+template <int N, typename F, int... I>
+__device__ __forceinline__ void static_for_(F &f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F f) {
+  static_for_<N>(f, std::make_integer_sequence<int, N>{});
 }
 
-__global__ void k_onsite(int A, int S, const int32_t *__restrict__ species,
-                         const int32_t *__restrict__ is_cation,
-                         const int32_t *__restrict__ nbr,
-                         const int32_t *__restrict__ bond_q,
-                         const double *__restrict__ parmat,
-                         const double *__restrict__ strnmat,
-                         const double *__restrict__ phi, int passivate,
-                         double db_shift, const double *__restrict__ corr,
-                         double *__restrict__ onsite) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= A) return;
-  const int ti = species[i];
-  const bool cat = is_cation[i] != 0;
-  // averaged parameters over the present neighbours (only the onsite
-  // energies and the spin-orbit constants are used)
-  double e[10];
+// The quad's sum (lanes 4 q .. 4 q + 3) of x in a fixed order, in every lane
+__device__ __forceinline__ double quad_sum(double x) {
+  x += dpp_f64<0xB1>(x);  // quad_perm 1 0 3 2
+  x += dpp_f64<0x4E>(x);  // quad_perm 2 3 0 1
+  return x;
+}
+
+struct AssembleArgs {
+  int A, S, passivate;
+  const int32_t *species, *is_cation, *nbr, *rev_slot, *bond_q, *bond_of;
+  const double *disp, *parmat, *strnmat, *phi;
+  double lx, ly, lz, db_shift;
+  double *onsite, *blocks, *sk;
+};
+
+enum { kOnsiteOnly = 0, kStoreBlocks = 1, kStoreSk = 2 };
+constexpr int kAsmThreads = 128, kAsmAtoms = kAsmThreads / 4;
+template <int STORE>
+__global__ __launch_bounds__(kAsmThreads) void k_assemble(AssembleArgs g) {
+  // onsite and bond records on their way out (24 doubles a bond, padded
+  // against bank conflicts)
+  constexpr int kRow = kSkStride + 1;
+  __shared__ double lds[kAsmAtoms * kOnsiteStride];
+  __shared__ double recs[STORE == kStoreSk ? kAsmThreads * kRow : 1];
+  __shared__ int32_t rec_of[kAsmAtoms];
+  const int slot = threadIdx.x & 3, la = threadIdx.x >> 2;
+  const int i = blockIdx.x * kAsmAtoms + la;
+  const bool in = i < g.A;
+  const int j = in ? g.nbr[i * 4 + slot] : -1;
+  const bool here = j >= 0;
+  const bool cat = in && g.is_cation[i] != 0;
+  double corr[10], e[10], strain_shift = 0.0;
 #pragma unroll
-  for (int k = 0; k < 10; ++k) e[k] = 0.0;
-  double strain_shift = 0.0;
-  int cnt = 0;
-  for (int n = 0; n < 4; ++n) {
-    const int j = nbr[i * 4 + n];
-    if (j < 0) continue;
-    const int tj = species[j];
-    const int c = cat ? ti : tj, a = cat ? tj : ti;
-    const double *p = parmat + ((size_t)c * S + a) * 35;
+  for (int k = 0; k < 10; ++k) corr[k] = e[k] = 0.0;
+  if (STORE == kStoreSk && !here)
 #pragma unroll
-    for (int k = 0; k < 10; ++k) e[k] += p[k];
-    strain_shift +=
-        strnmat[((size_t)c * S + a) * 33 + (cat ? S_CAT_SHIFT : S_AN_SHIFT)];
-    ++cnt;
+    for (int k = 0; k < kSkStride; ++k) recs[threadIdx.x * kRow + k] = 0.0;
+  if (STORE == kStoreBlocks && in && !here) {
+    double *B = g.blocks + ((size_t)i * 4 + slot) * 100;
+    for (int k = 0; k < 100; ++k) B[k] = 0.0;
   }
-  strain_shift /= cnt;
+  if (here) {
+    const int ti = g.species[i], tj = g.species[j];
+    const int c = cat ? ti : tj, a = cat ? tj : ti;
+    const double *par = g.parmat + ((size_t)c * g.S + a) * 35;
+    const double *strn = g.strnmat + ((size_t)c * g.S + a) * 33;
+    const double lat[3] = {g.lx, g.ly, g.lz};
+    const int back = g.rev_slot[i * 4 + slot];
+    double nnv[3], nnv0[3];
+    if (cat) cation_bond_vectors(g.bond_q, g.disp, lat, i, slot, j, par[P_A0], nnv, nnv0);
+    else cation_bond_vectors(g.bond_q, g.disp, lat, j, back, i, par[P_A0], nnv, nnv0);
+    const BondGeom b = bond_geom(nnv, nnv0, par[P_A0]);
+    double v[21];
+    scale_integrals(par, strn, b.brat, v);
+    if constexpr (STORE == kStoreBlocks) {
+      double T[100];
+      sk_table(b.l, b.m, b.n, v, T);
+      double *B = g.blocks + ((size_t)i * 4 + slot) * 100;
 #pragma unroll
-  for (int k = 0; k < 10; ++k) e[k] /= cnt;
+      for (int r = 0; r < 10; ++r)
+#pragma unroll
+        for (int q = 0; q < 10; ++q) {
+          const double x = T[r * 10 + q], y = T[q * 10 + r];
+          B[r * 10 + q] = cat ? y : x;
+        }
+    }
+    if constexpr (STORE == kStoreSk)
+      if (cat) {
+        double rec[kSkStride];
+        sk_record(b.l, b.m, b.n, v, rec);
+#pragma unroll
+        for (int k = 0; k < kSkStride; ++k) recs[threadIdx.x * kRow + k] = rec[k];
+      }
+    // Boykin terms ((V0^2 - V^2) c_strain / (E_a + E_c)) * c_pair
+    // (mb_ham_spds_VoffdEdiag_constructors.h; the pVpE_* macros are not
+    // parenthesised, so the pair coefficient multiplies the quotient).
+    const RowWeights w(b.l, b.m, b.n), w0(b.l0, b.m0, b.n0);
+    const double cs = strn[S_CONST];
+    auto pair = [&](auto SO, auto SX) {
+      constexpr int so = SO, sx = SX;  // shells of this atom, of the other
+      const double ea = par[cat ? e_anion(sx) : e_anion(so)];
+      const double ec = par[cat ? e_cation(so) : e_cation(sx)];
+      const double f = cs / (ea + ec) * strn[cat ? cpair_index(sx, so) : cpair_index(so, sx)];
+      double q[3], q0[3];
+#pragma unroll
+      for (int part = 0; part < 3; ++part) {
+        q[part] = q0[part] = 0.0;
+        if (pair_integral(so, sx, part) < 0) continue;
+        const int ia = pair_integral(so, sx, part), ic = pair_integral(sx, so, part);
+        const double x = cat ? v[ic] : v[ia], x0 = par[10 + (cat ? ic : ia)];
+        q[part] = x * x;
+        q0[part] = x0 * x0;
+      }
+      auto add = [&](auto O) {
+        constexpr int o = O;
+        if constexpr (shell_of(o) == so)
+          corr[o] += (w0.template row<o>(q0[0], q0[1], q0[2]) -
+                      w.template row<o>(q[0], q[1], q[2])) * f;
+      };
+      static_for<10>(add);
+    };
+    static_for<4>([&](auto SO) { static_for<4>([&](auto SX) { pair(SO, SX); }); });
+    // of the averaged parameters only the onsite energies and the spin-orbit
+    // constants are used
+#pragma unroll
+    for (int k = 0; k < 10; ++k) e[k] = par[k];
+    strain_shift = strn[cat ? S_CAT_SHIFT : S_AN_SHIFT];
+  }
+  const int cnt = (int)quad_sum(here ? 1.0 : 0.0);
+  strain_shift = quad_sum(strain_shift) / cnt;
+#pragma unroll
+  for (int k = 0; k < 10; ++k) {
+    e[k] = quad_sum(e[k]) / cnt;
+    corr[k] = quad_sum(corr[k]);
+  }
   double hd[10];
 #pragma unroll
-  for (int o = 0; o < 10; ++o)
-    hd[o] = e[cat ? e_cation(shell_of(o)) : e_anion(shell_of(o))];
-  const double lambda = cat ? e[P_LC] : e[P_LA];
+  for (int o = 0; o < 10; ++o) {
+    const double ec = e[e_cation(shell_of(o))], ea = e[e_anion(shell_of(o))];
+    hd[o] = cat ? ec : ea;
+  }
   double sp[6] = {0, 0, 0, 0, 0, 0};
-  if (passivate && cnt < 4) {
+  if (g.passivate && in && cnt < 4) {
     // sp3 hybrid directions of the dangling-bond projector
     const double hyb[4][3] = {{0.25, 0.25, 0.25},
                               {-0.25, -0.25, 0.25},
@@ -155,19 +216,19 @@ __global__ void k_onsite(int A, int S, const int32_t *__restrict__ species,
                               {-0.25, 0.25, -0.25}};
     double v[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = 0.25 * db_shift;
+    for (int k = 0; k < 4; ++k) v[k] = 0.25 * g.db_shift;
     double cosv = 0.0;
     for (int n = 0; n < 4; ++n) {
       double d[3];
 #pragma unroll
-      for (int k = 0; k < 3; ++k) d[k] = 0.25 * bond_q[(i * 4 + n) * 3 + k];
+      for (int k = 0; k < 3; ++k) d[k] = 0.25 * g.bond_q[(i * 4 + n) * 3 + k];
       int ib = 0;
       cosv = d[0] * hyb[0][0] + d[1] * hyb[0][1] + d[2] * hyb[0][2];
       while (fabs(cosv) < 0.15 && ib < 3) {
         ++ib;
         cosv = d[0] * hyb[ib][0] + d[1] * hyb[ib][1] + d[2] * hyb[ib][2];
       }
-      if (nbr[i * 4 + n] >= 0) v[ib] = 0.0;
+      if (g.nbr[i * 4 + n] >= 0) v[ib] = 0.0;
     }
     const double s = cosv > 0 ? 1.0 : -1.0;
     const double dsp = v[0] + v[1] + v[2] + v[3];
@@ -180,24 +241,34 @@ __global__ void k_onsite(int A, int S, const int32_t *__restrict__ species,
 #pragma unroll
     for (int k = 1; k < 5; ++k) hd[k] += dsp;
   }
-  const double ph = phi ? phi[i] : 0.0;
+  const double ph = in && g.phi ? g.phi[i] : 0.0;
 #pragma unroll
-  for (int k = 0; k < 10; ++k) {
-    hd[k] += strain_shift;
-    hd[k] -= ph;
+  for (int k = 0; k < 10; ++k) hd[k] = hd[k] + strain_shift - ph + corr[k];
+  // through LDS, so that consecutive lanes write consecutive numbers
+  const int a0 = blockIdx.x * kAsmAtoms, na = min(kAsmAtoms, g.A - a0);
+  if (slot == 0) {
+    double *os = lds + la * kOnsiteStride;
+#pragma unroll
+    for (int k = 0; k < 10; ++k) os[k] = hd[k];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) os[10 + k] = sp[k];
+    os[16] = cat ? e[P_LC] : e[P_LA];
+    os[17] = 0.0;
   }
-  for (int n = 0; n < 4; ++n) {
-    if (nbr[i * 4 + n] < 0) continue;
-#pragma unroll
-    for (int k = 0; k < 10; ++k) hd[k] += corr[((size_t)i * 4 + n) * 10 + k];
+  if constexpr (STORE == kStoreSk) {
+    // a cation's four records follow one another (bond number 4 c + slot)
+    if (here && cat) rec_of[la] = g.bond_of[i * 4 + slot] - slot;
+    else if (slot == 0 && !cat) rec_of[la] = -1;
   }
-  double *os = onsite + (size_t)i * kOnsiteStride;
-#pragma unroll
-  for (int k = 0; k < 10; ++k) os[k] = hd[k];
-#pragma unroll
-  for (int k = 0; k < 6; ++k) os[10 + k] = sp[k];
-  os[16] = lambda;
-  os[17] = 0.0;
+  __syncthreads();
+  for (int t = threadIdx.x; t < na * kOnsiteStride; t += kAsmThreads)
+    g.onsite[(size_t)a0 * kOnsiteStride + t] = lds[t];
+  if constexpr (STORE == kStoreSk) {
+    for (int t = threadIdx.x; t < na * 4 * kSkStride; t += kAsmThreads) {
+      const int r = t / kSkStride, k = t % kSkStride, rr = rec_of[r >> 2];
+      if (rr >= 0) g.sk[((size_t)rr + (r & 3)) * kSkStride + k] = recs[r * kRow + k];
+    }
+  }
 }
 
 // Matrix-free layout tables: per atom its displacement and species, per
@@ -301,24 +372,9 @@ nh_status assemble(nh_context *c, int layout, int precision) {
   const int A = c->n_atoms;
   const size_t nblk = (size_t)A * 4 * 100;
   NH_TRY(need(&c->onsite, (size_t)A * kOnsiteStride * sizeof(double)));
-  double *corr = nullptr;
-  NH_TRY(pool_alloc(c, (void **)&corr, (size_t)A * 4 * 10 * sizeof(double)));
-  struct Release {
-    nh_context *c;
-    void *p;
-    ~Release() { pool_release(c, p); }
-  } release{c, corr};  // only the assembly needs the per-bond terms
-  NH_HIP(hipMemsetAsync(corr, 0, (size_t)A * 40 * sizeof(double), c->stream));
-  if (layout == NH_LAYOUT_BLOCKS) {
-    NH_TRY(need(&c->blocks64, nblk * sizeof(double)));
-    NH_HIP(hipMemsetAsync(c->blocks64, 0, nblk * sizeof(double), c->stream));
-  }
-  if (layout == NH_LAYOUT_SK) {
+  if (layout == NH_LAYOUT_BLOCKS) NH_TRY(need(&c->blocks64, nblk * sizeof(double)));
+  if (layout == NH_LAYOUT_SK)
     NH_TRY(need(&c->sk64, (size_t)c->n_cations * 4 * kSkStride * sizeof(double)));
-    NH_HIP(hipMemsetAsync(c->sk64, 0,
-                          (size_t)c->n_cations * 4 * kSkStride * sizeof(double),
-                          c->stream));
-  }
   const int S = c->n_species;
   if (layout == NH_LAYOUT_MATRIX_FREE) {
     NH_TRY(need(&c->mf_geo, (size_t)A * sizeof(double4)));
@@ -335,18 +391,17 @@ nh_status assemble(nh_context *c, int layout, int precision) {
                        c->stream, S, c->parmat, c->strnmat, c->mf_pair);
     NH_HIP(hipGetLastError());
   }
-  // bonds: the stored blocks or SK records (if kept) and the Boykin terms
-  // of the onsite diagonal, which every layout stores
-  hipLaunchKernelGGL(k_bond, dim3(grid_for((int64_t)c->n_cations * 4, 128)),
-                     dim3(128), 0, c->stream, c->n_cations, S, c->cations,
-                     c->species, c->nbr, c->rev_slot, c->bond_q, c->disp,
-                     c->lattice[0], c->lattice[1], c->lattice[2], c->parmat,
-                     c->strnmat, c->blocks64, corr, c->sk64);
-  NH_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_onsite, dim3(grid_for(A, 128)), dim3(128), 0, c->stream,
-                     A, S, c->species, c->is_cation, c->nbr, c->bond_q,
-                     c->parmat, c->strnmat, c->phi, c->passivate, c->db_shift,
-                     corr, c->onsite);
+  const AssembleArgs g{A, S, c->passivate, c->species, c->is_cation, c->nbr, c->rev_slot,
+                       c->bond_q, c->bond_of, c->disp, c->parmat, c->strnmat, c->phi,
+                       c->lattice[0], c->lattice[1], c->lattice[2], c->db_shift, c->onsite,
+                       c->blocks64, c->sk64};
+  const dim3 grid(grid_for(A, kAsmAtoms)), block(kAsmThreads);
+  if (layout == NH_LAYOUT_BLOCKS)
+    hipLaunchKernelGGL(k_assemble<kStoreBlocks>, grid, block, 0, c->stream, g);
+  else if (layout == NH_LAYOUT_SK)
+    hipLaunchKernelGGL(k_assemble<kStoreSk>, grid, block, 0, c->stream, g);
+  else
+    hipLaunchKernelGGL(k_assemble<kOnsiteOnly>, grid, block, 0, c->stream, g);
   NH_HIP(hipGetLastError());
   NH_HIP(hipStreamSynchronize(c->stream));
   c->layout = layout;

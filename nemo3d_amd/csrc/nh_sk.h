@@ -185,12 +185,17 @@ __device__ __forceinline__ BondGeom bond_geom(const double nnv[3],
   return g;
 }
 
-// Strain-scaled integrals V_k * brat^eta_k (parameters 10..30).
+// Strain-scaled integrals V_k * brat^eta_k (parameters 10..30): one logarithm
+// and 15 exponentials for the 21 of them.
 __device__ __forceinline__ void scale_integrals(const double *par,
                                                 const double *strn,
                                                 double brat, double *v) {
+  const double lb = log(brat);
+  double f[15];
 #pragma unroll
-  for (int k = 0; k < 21; ++k) v[k] = par[10 + k] * pow(brat, strn[eta_index(k)]);
+  for (int e = 0; e < 15; ++e) f[e] = exp(strn[e] * lb);
+#pragma unroll
+  for (int k = 0; k < 21; ++k) v[k] = par[10 + k] * f[eta_index(k)];
 }
 
 }  // namespace nh
