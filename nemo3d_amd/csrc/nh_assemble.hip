@@ -86,11 +86,12 @@ __device__ __forceinline__ void static_for(F f) {
   static_for_<N>(f, std::make_integer_sequence<int, N>{});
 }
 
-// The quad's sum (lanes 4 q .. 4 q + 3) of x in a fixed order, in every lane
-__device__ __forceinline__ double quad_sum(double x) {
-  x += dpp_f64<0xB1>(x);  // quad_perm 1 0 3 2
-  x += dpp_f64<0x4E>(x);  // quad_perm 2 3 0 1
-  return x;
+// s + the quad's four x in slot order, in every lane
+__device__ __forceinline__ double quad_add(double s, double x) {
+  s += dpp_f64<0x00>(x);
+  s += dpp_f64<0x55>(x);
+  s += dpp_f64<0xAA>(x);
+  return s + dpp_f64<0xFF>(x);
 }
 
 struct AssembleArgs {
@@ -194,13 +195,10 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(AssembleArgs g) {
     for (int k = 0; k < 10; ++k) e[k] = par[k];
     strain_shift = strn[cat ? S_CAT_SHIFT : S_AN_SHIFT];
   }
-  const int cnt = (int)quad_sum(here ? 1.0 : 0.0);
-  strain_shift = quad_sum(strain_shift) / cnt;
+  const int cnt = (int)quad_add(0.0, here ? 1.0 : 0.0);
+  strain_shift = quad_add(0.0, strain_shift) / cnt;
 #pragma unroll
-  for (int k = 0; k < 10; ++k) {
-    e[k] = quad_sum(e[k]) / cnt;
-    corr[k] = quad_sum(corr[k]);
-  }
+  for (int k = 0; k < 10; ++k) e[k] = quad_add(0.0, e[k]) / cnt;
   double hd[10];
 #pragma unroll
   for (int o = 0; o < 10; ++o) {
@@ -243,7 +241,7 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(AssembleArgs g) {
   }
   const double ph = in && g.phi ? g.phi[i] : 0.0;
 #pragma unroll
-  for (int k = 0; k < 10; ++k) hd[k] = hd[k] + strain_shift - ph + corr[k];
+  for (int k = 0; k < 10; ++k) hd[k] = quad_add(hd[k] + strain_shift - ph, corr[k]);
   // through LDS, so that consecutive lanes write consecutive numbers
   const int a0 = blockIdx.x * kAsmAtoms, na = min(kAsmAtoms, g.A - a0);
   if (slot == 0) {
@@ -366,6 +364,7 @@ nh_status assemble(nh_context *c, int layout, int precision) {
            "precision %d not available", precision);
   NH_HIP(hipStreamSynchronize(c->stream));
   free_ham(c, layout);
+  if (layout != NH_LAYOUT_BLOCKS) NH_TRY(ensure_blocks(c));
   auto need = [c](auto **p, size_t bytes) {
     return *p ? NH_OK : device_malloc(c, (void **)p, bytes);
   };
