@@ -192,6 +192,8 @@ nh_status ensure_buffers(nh_context *c, int64_t elems) {
 
 template <typename T>
 static nh_status upload(T **dst, const T *src, size_t count) {
+  (void)hipFree(*dst);  // of an attempt that failed later on
+  *dst = nullptr;
   NH_HIP(hipMalloc(dst, count * sizeof(T) + 16));
   NH_HIP(hipMemcpy(*dst, src, count * sizeof(T), hipMemcpyHostToDevice));
   return NH_OK;
@@ -386,6 +388,35 @@ static void build_blocks(const nh_model *m, const std::vector<int32_t> &rev, Blo
   close();
 }
 
+nh_status ensure_blocks(nh_context *c) {
+  if (c->n_blocks > 0) return NH_OK;
+  const size_t A = c->n_atoms;
+  std::vector<int32_t> nbr(A * 4), bond_q(A * 12), is_cation(A), rev(A * 4);
+  auto get = [](std::vector<int32_t> &v, const int32_t *d) {
+    return hipMemcpy(v.data(), d, v.size() * sizeof(int32_t), hipMemcpyDeviceToHost);
+  };
+  NH_HIP(get(nbr, c->nbr));
+  NH_HIP(get(bond_q, c->bond_q));
+  NH_HIP(get(is_cation, c->is_cation));
+  NH_HIP(get(rev, c->rev_slot));
+  nh_model m{};
+  m.n_atoms = c->n_atoms;
+  m.nbr = nbr.data();
+  m.bond_q = bond_q.data();
+  m.is_cation = is_cation.data();
+  BlockTables b;
+  build_blocks(&m, rev, b);
+  NH_TRY(upload(&c->cations, b.cations.data(), b.cations.size()));
+  NH_TRY(upload(&c->bond_of, b.bond_of.data(), b.bond_of.size()));
+  NH_TRY(upload(&c->blk_own, b.own.data(), b.own.size()));
+  NH_TRY(upload(&c->blk_local, reinterpret_cast<const uint2 *>(b.local.data()),
+                b.local.size() / 8));
+  NH_TRY(upload(&c->blk_halo, b.halo.data(), b.halo.size()));
+  NH_TRY(upload(&c->blk_bonds, b.bonds.data(), b.bonds.size()));
+  c->n_blocks = b.n;
+  return NH_OK;
+}
+
 static nh_status create(const nh_model *m, int device, nh_context **out) {
   NH_CHECK(m && out, NH_ERR_ARG, "null model or output pointer");
   NH_CHECK(m->nb == 10 || m->nb == 20, NH_ERR_ARG, "nb must be 10 or 20");
@@ -420,8 +451,6 @@ static nh_status create(const nh_model *m, int device, nh_context **out) {
   }
   for (int i = 0; i < A; ++i) n_cations += m->is_cation[i] != 0;
   NH_CHECK(n_cations > 0, NH_ERR_ARG, "no cation-role atoms");
-  BlockTables blocks;
-  build_blocks(m, rev, blocks);
 
   NH_HIP(hipSetDevice(device));
   NH_TRY(init_noalloc_scratch(device));
@@ -431,7 +460,6 @@ static nh_status create(const nh_model *m, int device, nh_context **out) {
   c->n_atoms = A;
   c->n_species = S;
   c->n_cations = n_cations;
-  c->n_blocks = blocks.n;
   c->n = (int64_t)A * m->nb;
   for (int k = 0; k < 3; ++k) c->lattice[k] = m->lattice[k];
   c->passivate = m->passivate;
@@ -447,12 +475,6 @@ static nh_status create(const nh_model *m, int device, nh_context **out) {
   UP(bond_q, m->bond_q, (size_t)A * 12);
   UP(disp, m->disp, (size_t)A * 3);
   if (m->phi) UP(phi, m->phi, A);
-  UP(cations, blocks.cations.data(), blocks.cations.size());
-  UP(bond_of, blocks.bond_of.data(), (size_t)A * 4);
-  UP(blk_own, blocks.own.data(), blocks.own.size());
-  UP(blk_local, reinterpret_cast<const uint2 *>(blocks.local.data()), blocks.local.size() / 8);
-  UP(blk_halo, blocks.halo.data(), blocks.halo.size());
-  UP(blk_bonds, blocks.bonds.data(), blocks.bonds.size());
   UP(rev_slot, rev.data(), (size_t)A * 4);
 #undef UP
   if (st == NH_OK) {

@@ -231,6 +231,10 @@ nh_status reduce_dot_noalloc(nh_context *c, int64_t n, const nh_cplx *x,
 nh_status launch_axpby(nh_context *c, int64_t n, nh_cplx a, const nh_cplx *x,
                        nh_cplx b, nh_cplx *y);
 nh_status ensure_reduce(nh_context *c, int blocks);
+// the block tables of the SK and matrix-free products (cations, bond_of,
+// blk_*), made by the first build that needs them: the relaxation, the stored
+// blocks and the learned start do without
+nh_status ensure_blocks(nh_context *c);
 // hipMalloc that, when the device is full, frees the idle workspace blocks
 // of every context on the device and tries once more (NH_ERR_NOMEM after
 // that); every device allocation of the library goes through it
