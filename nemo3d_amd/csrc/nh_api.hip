@@ -231,6 +231,11 @@ static void destroy(nh_context *c) {
 // new block unless it fits into the open one whole, so the blocks of a
 // crystal coincide with its cubes (64 atoms, at most 57 halo atoms and 170
 // bonds) and only thin rests of cubes at the surface are put together.
+// Inside a block every atom goes, where it can, to a place that is its color
+// modulo 8, a linear function of its lattice position: eight atoms in
+// consecutive places then have neighbours of eight different colors in any
+// direction, and the quads that read them from LDS together meet eight
+// different groups of banks.  A bond's color is its cation's.
 // Bond numbers are 4 (number of the cation in `cations`) + slot, the cations
 // in block order.
 struct BlockTables {
@@ -241,7 +246,7 @@ struct BlockTables {
 };
 
 static void cube_order(const nh_model *m, std::vector<int32_t> &order,
-                       std::vector<int64_t> &cube) {
+                       std::vector<int64_t> &cube, std::vector<uint8_t> &color) {
   const int A = m->n_atoms;
   std::vector<int32_t> pos((size_t)A * 3, 0);
   std::vector<char> seen(A, 0);
@@ -277,9 +282,36 @@ static void cube_order(const nh_model *m, std::vector<int32_t> &order,
   std::sort(key.begin(), key.end());
   order.resize(A);
   cube.resize(A);
+  color.resize(A);
   for (int i = 0; i < A; ++i) {
     order[i] = key[i].second;
     cube[i] = key[i].first;
+    // cations and anions in units of a/2: 4 x 2 of the 4 x 4 x 2 sites of a
+    // role in a cube are told apart
+    color[i] = (uint8_t)(((pos[(size_t)i * 3] >> 1) + 4 * (pos[(size_t)i * 3 + 1] >> 1)) & 7);
+  }
+}
+// places base .. base + cap of the items, of their color modulo 8 where one is
+// free; taken: places given so far
+template <typename F>
+static void color_places(const std::vector<int32_t> &items, int base, int cap, F color,
+                         std::vector<int32_t> &taken, std::vector<int32_t> &place) {
+  std::vector<int32_t> rest;
+  for (int32_t a : items) {
+    int p = color(a);
+    while (p < cap && taken[base + p] >= 0) p += 8;
+    if (p >= cap) {
+      rest.push_back(a);
+      continue;
+    }
+    taken[base + p] = a;
+    place[a] = base + p;
+  }
+  int p = 0;
+  for (int32_t a : rest) {
+    while (taken[base + p] >= 0) ++p;
+    taken[base + p] = a;
+    place[a] = base + p;
   }
 }
 
@@ -288,7 +320,8 @@ static void build_blocks(const nh_model *m, const std::vector<int32_t> &rev, Blo
   const int A = m->n_atoms;
   std::vector<int32_t> order;
   std::vector<int64_t> cube;
-  cube_order(m, order, cube);
+  std::vector<uint8_t> color;
+  cube_order(m, order, cube, color);
   for (int i : order)
     if (m->is_cation[i]) T.cations.push_back(i);
   T.bond_of.assign((size_t)A * 4, -1);
@@ -309,30 +342,47 @@ static void build_blocks(const nh_model *m, const std::vector<int32_t> &rev, Blo
   std::fill(own, own + kOwn, -1);
   auto close = [&]() {
     if (nc + na == 0) return;
-    int k = 0;
-    for (int32_t a : halo)
-      if (a >= 0) {
-        place[a] = kOwn + k++;
-        T.halo.push_back(a);
+    // final places: cations, anions, halo, bonds
+    const std::vector<int32_t> oc(own, own + nc), oa(own + kHalf, own + kHalf + na);
+    halo.erase(std::remove(halo.begin(), halo.end(), -1), halo.end());
+    std::vector<int32_t> at(kOwn + kHalo, -1), rec(kBondPad, -1);
+    auto col = [&](int32_t i) { return (int)color[i]; };
+    color_places(oc, 0, kHalf, col, at, place);
+    color_places(oa, kHalf, kHalf, col, at, place);
+    color_places(halo, kOwn, kHalo, col, at, place);
+    // bond of slot n of an own cation in place p: 32 n + p; the others after
+    // them and in the gaps
+    std::vector<int32_t> others;
+    for (int32_t q : bonds) {
+      const int p = place[T.cations[q >> 2]];
+      if (p < kHalf) {
+        rec[kHalf * (q & 3) + p] = q;
+        bplace[q] = kHalf * (q & 3) + p;
+      } else {
+        others.push_back(q);
       }
-    T.halo.resize((size_t)(T.n + 1) * kHalo, -1);
-    T.bonds.insert(T.bonds.end(), bonds.begin(), bonds.end());
-    T.bonds.resize((size_t)(T.n + 1) * kBondPad, -1);
-    T.own.insert(T.own.end(), own, own + kOwn);
+    }
+    std::reverse(rec.begin(), rec.begin() + kBonds);  // the free end first
+    for (int32_t q : others) bplace[q] = -1;
+    color_places(others, 0, kBonds,
+                 [&](int32_t q) { return 7 - (int)color[T.cations[q >> 2]]; }, rec, bplace);
+    std::reverse(rec.begin(), rec.begin() + kBonds);
+    for (int32_t q : others) bplace[q] = kBonds - 1 - bplace[q];
+    T.own.insert(T.own.end(), at.begin(), at.begin() + kOwn);
+    T.halo.insert(T.halo.end(), at.begin() + kOwn, at.end());
+    T.bonds.insert(T.bonds.end(), rec.begin(), rec.end());
     const size_t l0 = T.local.size();
     T.local.resize(l0 + kOwn * 8, 255);
     for (int s = 0; s < kOwn; ++s) {
-      if (own[s] < 0) continue;
+      if (at[s] < 0) continue;
       for (int n = 0; n < 4; ++n) {
-        const int j = m->nbr[(size_t)own[s] * 4 + n];
+        const int j = m->nbr[(size_t)at[s] * 4 + n];
         if (j < 0) continue;
         T.local[l0 + s * 8 + n] = (uint8_t)place[j];
-        T.local[l0 + s * 8 + 4 + n] = (uint8_t)bplace[T.bond_of[(size_t)own[s] * 4 + n]];
+        T.local[l0 + s * 8 + 4 + n] = (uint8_t)bplace[T.bond_of[(size_t)at[s] * 4 + n]];
       }
     }
-    for (int s = 0; s < kOwn; ++s)
-      if (own[s] >= 0) place[own[s]] = -1;
-    for (int32_t a : halo)
+    for (int32_t a : at)
       if (a >= 0) place[a] = -1;
     for (int32_t q : bonds) bplace[q] = -1;
     std::fill(own, own + kOwn, -1);

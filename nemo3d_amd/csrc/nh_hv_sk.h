@@ -135,14 +135,22 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Staged items, in 16-byte chunks; odd strides spread the items of a
-// wavefront's atoms over the LDS banks.
+// Staged items, in 16-byte chunks.  20 bands: the chunks of the two spins
+// alternate, so the four components of an orbital that a quad's lanes read
+// together lie in 32 bytes, and the stride is an odd number of 32 bytes: quads
+// reading places that differ modulo 8 (see the places of a block) meet
+// different banks.  10 bands: an odd number of chunks.
 template <int NSP, typename XT>
 struct SkX {  // the entries of an atom
   static constexpr int kChunks = NSP * 10 * (int)sizeof(XT) / 16;  // 20/10, 10/5
   static constexpr int kLoads = (kChunks + 3) / 4;                 // per lane of a quad
   // a place also holds an onsite record (9) or ten FP64 entries
-  static constexpr int kStride = (kChunks < 10 ? 10 : kChunks) | 1;
+  static constexpr int kStride =
+      NSP == 2 ? (kChunks / 2 | 1) * 2 : (kChunks < 10 ? 10 : kChunks) | 1;
+  // where chunk i lies
+  __device__ __forceinline__ static int at(int i) {
+    return NSP == 1 ? i : i < kChunks / 2 ? 2 * i : 2 * i - kChunks + 1;
+  }
 };
 template <typename R>
 struct SkRec {  // a bond record (24 numbers)
@@ -431,7 +439,7 @@ __device__ __forceinline__ void sk_stage_x(uint4 *place, int c,
                                            const uint4 (&X)[SkX<NSP, XT>::kLoads]) {
 #pragma unroll
   for (int i = 0; i < SkX<NSP, XT>::kLoads; ++i)
-    if (4 * i + c < SkX<NSP, XT>::kChunks) place[4 * i + c] = X[i];
+    if (4 * i + c < SkX<NSP, XT>::kChunks) place[SkX<NSP, XT>::at(4 * i + c)] = X[i];
 }
 // r_k from the chunks of u_{k-1} and r_{k-1}
 template <typename XT, int K>
@@ -440,13 +448,14 @@ __device__ __forceinline__ void sk_defer(uint4 (&X)[K], const uint4 (&P)[K], LzC
   for (int i = 0; i < K; ++i) X[i] = lz_defer_chunk<XT>(X[i], P[i], a);
 }
 
-// The thread's component of the item at `place`, from entry `first` on
-template <typename R, typename XT>
-__device__ __forceinline__ void sk_read_x(const uint4 *place, int comp, int first, R (&x)[10]) {
+// The thread's component (of its spin) of the item at `place`
+template <int NSP, typename R, typename XT>
+__device__ __forceinline__ void sk_read_x(const uint4 *place, const SkThread &t, R (&x)[10]) {
   using E = typename std::conditional<sizeof(XT) == 16, double, float>::type;
-  const E *p = reinterpret_cast<const E *>(place) + 2 * first + comp;
+  constexpr int kPer = 16 / (int)sizeof(XT);  // entries of a chunk
+  const E *p = reinterpret_cast<const E *>(place) + (NSP == 2 ? 2 * kPer * t.h : 0) + t.comp;
 #pragma unroll
-  for (int o = 0; o < 10; ++o) x[o] = R(p[2 * o]);
+  for (int o = 0; o < 10; ++o) x[o] = R(p[2 * (NSP * kPer * (o / kPer) + o % kPer)]);
 }
 
 // acc = the thread's component of sum_n T_n x_n from the staged block; R
@@ -467,7 +476,7 @@ __device__ __forceinline__ void sk_bonds(const SkThread &t, uint2 local,
       for (int i = 0; i < SkRec<R>::kChunks; ++i)
         *reinterpret_cast<uint4 *>(&k[i * (16 / (int)sizeof(R))]) =
             L.rec[lb * SkRec<R>::kStride + i];
-      sk_read_x<R, XT>(L.x + lx * SkX<NSP, XT>::kStride, t.comp, NSP == 2 ? 10 * t.h : 0, x);
+      sk_read_x<NSP, R, XT>(L.x + lx * SkX<NSP, XT>::kStride, t, x);
       if constexpr (sizeof(R) == 8) {
         sk_apply<CATION, double>(k, x, acc);
       } else {
@@ -529,7 +538,7 @@ __device__ __forceinline__ void sk_finish(const SkThread &t, SkLds<NSP, R, XT> &
   const uint4 *own = L.x + t.Q * SkX<NSP, XT>::kStride;
   uint4 *halo = L.x + (kSkOwn + t.Q) * SkX<NSP, XT>::kStride;
   double xo[10];
-  sk_read_x<double, XT>(own, t.comp, NSP == 2 ? 10 * t.h : 0, xo);
+  sk_read_x<NSP, double, XT>(own, t, xo);
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < 3; ++i)

@@ -319,7 +319,7 @@ __global__ __launch_bounds__(kSkThreads, sizeof(V) == 8 ? 3 : 2) void k_lz_sk(
         for (int i = 0; i < kPl; ++i) {
           const int q = 4 * i + t.c;
           if (q >= kPer) break;
-          const uint4 rk4 = own[s * kPer + q];
+          const uint4 rk4 = own[S::at(s * kPer + q)];
           uint4 o4;
           if constexpr (sizeof(V) == 16) {
             const double2 y = *reinterpret_cast<const double2 *>(&halo[q]);
