@@ -982,22 +982,22 @@ nh_status LanczosRun::fetch(int m) {
 // queue the check of the first m steps (fetched before) on the side stream;
 // the earlier one has been waited for
 nh_status LanczosRun::check(int m) {
-  const int waves = win_.want[0] + win_.want[1];
-  if (waves > 0) {
-    const int64_t need = (int64_t)waves * 2 * m;
+  const int count = win_.want[0] + win_.want[1];
+  if (count > 0) {
+    const int64_t need = count * tri_scratch(m);
     if (need > tri_cap_) {
       if (tri_s_) pool_release(c_, tri_s_);
       tri_s_ = nullptr;
       tri_cap_ = 0;
-      const int64_t rows = std::max<int64_t>(2 * m, 2048);
-      NH_TRY(pool_alloc(c_, (void **)&tri_s_, waves * 2 * rows * sizeof(double)));
-      tri_cap_ = waves * 2 * rows;
+      const int64_t cap = count * tri_scratch(std::max(2 * m, 2048));
+      NH_TRY(pool_alloc(c_, (void **)&tri_s_, cap * sizeof(double)));
+      tri_cap_ = cap;
     }
-    hipLaunchKernelGGL(k_tri_windows, dim3(waves), dim3(64), 0, c_->side, m, alpha_, beta_, win_,
-                       tri_s_, (int64_t)2 * m, tri_out_);
+    hipLaunchKernelGGL(k_tri_windows, dim3(count), dim3(kTriThreads), 0, c_->side, m, alpha_,
+                       beta_, win_, tri_s_, tri_out_);
     NH_HIP(hipGetLastError());
     NH_HIP(hipMemcpyAsync(pin_ + 2 * (size_t)pin_cap_, tri_out_,
-                          (kTriHead + (size_t)waves * kTriOut) * sizeof(double),
+                          (kTriHead + (size_t)count * kTriOut) * sizeof(double),
                           hipMemcpyDeviceToHost, c_->side));
   }
   NH_HIP(hipEventRecord(check_ev_, c_->side));

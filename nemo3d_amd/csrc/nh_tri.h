@@ -2,18 +2,22 @@
 // two components of their eigenvectors, on the device: the convergence check
 // of the Lanczos runs.
 //
-// One wavefront per eigenvalue.  The 64 lanes count the eigenvalues below 64
-// points of its interval at a time (signs of the leading minors, three-term
-// recurrence with rescaling), which cuts the interval by 65 a pass; then two
-// lanes run the pivots from both ends, and the eigenvector follows from the
-// position where they meet best (twisted factorisation), without inverse
-// iteration.  The kernel uses no LDS and few registers, so that it runs beside
-// a Lanczos step that fills the LDS of every compute unit.
-// Bound by the serial recurrences: about 30 cycles a row and pass (9 passes)
-// and 200 cycles a row for the vector: 0.2 ms at 1,100 rows.  On 8 host
-// threads (bisection with a division a row, threads started for each check) a
-// check took longer than the 25 steps between two of them: a whole solve of
-// 3,888 atoms 57 ms, now 26, a mixed one of 172,032 atoms 355 ms, now 241.
+// A workgroup of four wavefronts per eigenvalue.  Its lanes count the
+// eigenvalues below 256 points of the interval at a time (signs of the leading
+// minors, three-term recurrence with rescaling), which cuts the interval by
+// 257 a pass; then two wavefronts run the pivots from both ends, and the
+// eigenvector follows from the position where they meet best (twisted
+// factorisation), without inverse iteration.  The kernel uses no LDS and few
+// registers, so that it runs beside a Lanczos step that fills the LDS of every
+// compute unit; the wavefronts meet in the scratch memory.
+// Bound by the serial recurrences, 38 cycles a row and pass (6 passes) and
+// about 85 a row for the pivots: 0.30 ms at 1,375 rows.  (One wavefront, 64
+// points, the pivots and the components by two lanes: 547 us; four points a
+// lane: 776 us, the FP64 units are busy with one; rows handed out by readlane
+// instead of scalar loads: 145 cycles a row.)  On 8 host threads (bisection
+// with a division a row, threads started for each check) a check took longer
+// than the 25 steps between two of them: a whole solve of 3,888 atoms 57 ms,
+// now 24, a mixed one of 172,032 atoms 355 ms, now 230.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -26,9 +30,13 @@ struct TriWindows {
   double lo[2], hi[2];
   int want[2];  // at most so many: the highest of window 0, the lowest of 1
 };
-// results: kTriHead doubles (eigenvalues taken of windows 0, 1), then 3 a
-// wavefront: value, last and last but one component
+// results: kTriHead doubles (eigenvalues taken of windows 0, 1), then 3 an
+// eigenvalue: value, last and last but one component
 constexpr int kTriHead = 2, kTriOut = 3;
+constexpr int kTriThreads = 256;
+// scratch of an eigenvalue, in doubles: pivots from both ends, and what the
+// wavefronts tell each other
+inline int64_t tri_scratch(int m) { return 2 * (int64_t)m + 32; }
 
 // eigenvalues of T_m (a diagonal, b off-diagonal) below x
 __device__ inline int tri_count(int m, const double *__restrict__ a,
@@ -78,132 +86,196 @@ __device__ inline int tri_count(int m, const double *__restrict__ a,
   return cnt;
 }
 
-// S: 2 m doubles a wavefront (stride ld)
-__global__ __launch_bounds__(64) void k_tri_windows(int m, const double *__restrict__ a,
-                                                    const double *__restrict__ b,
-                                                    TriWindows win, double *S, int64_t ld,
-                                                    double *__restrict__ out) {
-  const int lane = threadIdx.x;
+// Pivots of T_m - v from the front (BACK: from the back) by one wavefront, the
+// lanes alike; to q[0 .. m)
+template <bool BACK>
+__device__ inline void tri_pivots(int m, const double *__restrict__ a,
+                                  const double *__restrict__ b, double v, double *q) {
+  const int lane = threadIdx.x & 63;
+  double p = 1.0, keep = 0.0;
+  auto row = [&](int t, double d, double e) {
+    // 1 / p to rounding: the hardware's approximation and two Newton steps
+    double r = __builtin_amdgcn_rcp(p);
+    r = __builtin_fma(__builtin_fma(-p, r, 1.0), r, r);
+    r = __builtin_fma(__builtin_fma(-p, r, 1.0), r, r);
+    p = __builtin_fma(-(e * e), r, d - v);
+    if (fabs(p) < 1e-280) p = 1e-280;  // its inverse must be finite
+    if (lane == (t & 63)) keep = p;
+  };
+  auto flush = [&](int t) {  // rows t & ~63 .. t
+    const int s = (t & ~63) + lane;
+    if (s <= t) q[BACK ? m - 1 - s : s] = keep;
+  };
+  constexpr int kU = 8;
+  double d[kU], e[kU];
+  auto load = [&](int t0, double (&dd)[kU], double (&ee)[kU]) {
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int i = BACK ? m - 1 - t0 - u : t0 + u;
+      dd[u] = a[i];
+      ee[u] = BACK ? b[i] : b[i > 0 ? i - 1 : 0];
+    }
+  };
+  const int full = m / kU * kU;
+  if (full > 0) load(0, d, e);
+  for (int t0 = 0; t0 < full; t0 += kU) {
+    double dn[kU], en[kU];
+    load(t0 + kU < full ? t0 + kU : t0, dn, en);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kU; ++u) row(t0 + u, d[u], t0 + u > 0 ? e[u] : 0.0);
+    if ((t0 & 63) == 56) flush(t0 + 7);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      asm volatile("" : "+s"(dn[u]), "+s"(en[u]));  // as in tri_count
+      d[u] = dn[u], e[u] = en[u];
+    }
+  }
+  for (int t = full; t < m; ++t) {
+    const int i = BACK ? m - 1 - t : t;
+    row(t, a[i], t == 0 ? 0.0 : b[BACK ? i : i - 1]);
+  }
+  if ((m & 63) != 0) flush(m - 1);
+}
+
+// Products of the n ratios f[0], f[dir], f[2 dir], .. by one wavefront: the
+// sum of their squares, the first, the last and the last but one
+struct TriProducts {
+  double sum, first, last, before;
+};
+__device__ inline TriProducts tri_products(const double *f, int dir, int n) {
+  const int lane = threadIdx.x & 63;
+  double carry = 1.0, sum = 0.0, first = 1.0, last = 1.0, before = 1.0;
+  for (int c = 0; c < n; c += 64) {
+    const int t = c + lane;
+    double p = t < n ? f[(int64_t)dir * t] : 1.0;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const double o = __shfl_up(p, off, 64);
+      if (lane >= off) p *= o;
+    }
+    p *= carry;
+    if (t < n) sum = __builtin_fma(p, p, sum);
+    if (t == 0) first = p;
+    if (t == n - 1) last = p;
+    if (t == n - 2) before = p;
+    carry = __shfl(p, 63, 64);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  return {sum, __shfl(first, 0, 64), n > 0 ? __shfl(last, (n - 1) & 63, 64) : 1.0,
+          n > 1 ? __shfl(before, (n - 2) & 63, 64) : 1.0};
+}
+
+// S: tri_scratch(m) doubles an eigenvalue
+__global__ __launch_bounds__(kTriThreads) void k_tri_windows(
+    int m, const double *__restrict__ a, const double *__restrict__ b, TriWindows win,
+    double *S, double *__restrict__ out) {
+  constexpr int kPts = kTriThreads, kWaves = kTriThreads / 64;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int w = (int)blockIdx.x >= win.want[0], j = (int)blockIdx.x - (w ? win.want[0] : 0);
-  // numbers of the eigenvalues in the window, and this wavefront's
-  int k, n;
+  double *F = S + (int64_t)blockIdx.x * (2 * (int64_t)m + 32), *B = F + m, *talk = B + m;
+  // the first point with more than k eigenvalues below (kPts: none); slot: of
+  // the talk, in turn
+  auto first_above = [&](int cnt, int k, int slot) {
+    const uint64_t above = __ballot(cnt > k);
+    if (lane == 0)
+      talk[slot * kWaves + wave] = above ? 64 * wave + __builtin_ctzll(above) : kPts;
+    __syncthreads();
+    double l = kPts;
+#pragma unroll
+    for (int q = 0; q < kWaves; ++q) l = fmin(l, talk[slot * kWaves + q]);
+    return (int)l;
+  };
+  // numbers of the eigenvalues in the window, and this workgroup's, from a
+  // first pass with points from end to end of the window
   double lo = win.lo[w], hi = win.hi[w];
+  auto point = [&](double h, int i) { return __builtin_fma(h, (double)i, lo); };
+  int k, n;
   {
-    const int c = tri_count(m, a, b, lane == 0 ? lo : hi);
-    const int klo = __shfl(c, 0, 64), khi = __shfl(c, 1, 64);
+    const double h = (hi - lo) / (kPts - 1);
+    const int cnt = tri_count(m, a, b, tid == kPts - 1 ? hi : point(h, tid));
+    if (tid == 0) talk[4 * kWaves] = cnt;
+    if (tid == kPts - 1) talk[4 * kWaves + 1] = cnt;
+    __syncthreads();
+    const int klo = (int)talk[4 * kWaves], khi = (int)talk[4 * kWaves + 1];
     n = min(khi - klo, win.want[w]);
     k = w == 0 ? khi - n + j : klo + j;
-    if (j == 0 && lane == 0) out[w] = n > 0 ? (double)n : 0.0;
+    if (j == 0 && tid == 0) out[w] = n > 0 ? (double)n : 0.0;
+    if (j >= n) return;
+    const int l = max(first_above(cnt, k, 0), 1);  // klo <= k < khi
+    const double nlo = point(h, l - 1), nhi = l < kPts - 1 ? point(h, l) : hi;
+    lo = nlo;
+    hi = nhi;
   }
-  if (j >= n) return;
-  for (int it = 0; it < 64 && hi - lo > 1e-13; ++it) {
-    const double h = (hi - lo) / 65.0;
-    const double x = __builtin_fma(h, lane + 1.0, lo);
-    const uint64_t above = __ballot(tri_count(m, a, b, x) > k);
-    const int l = above ? __builtin_ctzll(above) : 64;  // first point above it
-    const double nlo = l > 0 ? __builtin_fma(h, (double)l, lo) : lo;
-    const double nhi = l < 64 ? __builtin_fma(h, l + 1.0, lo) : hi;
+  for (int it = 1; it < 64 && hi - lo > 1e-13; ++it) {
+    const double h = (hi - lo) / (kPts + 1);
+    const int l = first_above(tri_count(m, a, b, point(h, tid + 1)), k, it & 1);
+    const double nlo = l > 0 ? point(h, l) : lo;
+    const double nhi = l < kPts ? point(h, l + 1) : hi;
     if (!(nhi - nlo < hi - lo)) break;
     lo = nlo;
     hi = nhi;
   }
   const double v = 0.5 * (lo + hi);
 
-  // pivots from the front (lane 0) and from the back (lane 1)
-  double *F = S + (int64_t)blockIdx.x * ld, *B = F + m;
-  if (lane < 2) {
-    double q = 0.0;
-    double *to = lane ? B : F;
-    constexpr int kU = 8;
-    double d[kU], e[kU];
-    auto load = [&](int t0) {
-#pragma unroll
-      for (int u = 0; u < kU; ++u) {
-        const int t = min(t0 + u, m - 1), i = lane ? m - 1 - t : t;
-        d[u] = a[i];
-        e[u] = t == 0 ? 0.0 : b[lane ? i : i - 1];
-      }
-    };
-    load(0);
-    for (int t0 = 0; t0 < m; t0 += kU) {
-      double dc[kU], ec[kU];
-#pragma unroll
-      for (int u = 0; u < kU; ++u) dc[u] = d[u], ec[u] = e[u];
-      load(t0 + kU);
-#pragma unroll
-      for (int u = 0; u < kU; ++u) {
-        const int t = t0 + u;
-        if (t < m) {
-          q = dc[u] - v - (t == 0 ? 0.0 : ec[u] * ec[u] / q);
-          if (q == 0.0) q = 1e-300;
-          to[lane ? m - 1 - t : t] = q;
-        }
-      }
-    }
-  }
+  if (wave == 0) tri_pivots<false>(m, a, b, v, F);
+  if (wave == 1) tri_pivots<true>(m, a, b, v, B);
   __syncthreads();
   // where they meet best
   double best = INFINITY;
   int r = 0;
-  for (int i = lane; i < m; i += 64) {
+  for (int i = tid; i < m; i += kTriThreads) {
     const double g = fabs(F[i] + B[i] - (a[i] - v));
     if (g < best) {
       best = g;
       r = i;
     }
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const double g = __shfl_xor(best, off, 64);
-    const int o = __shfl_xor(r, off, 64);
+  auto better = [&](double g, int o) {
     if (g < best || (g == best && o < r)) {
       best = g;
       r = o;
     }
+  };
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const double g = __shfl_xor(best, off, 64);
+    better(g, __shfl_xor(r, off, 64));
   }
-  // component ratios away from it
+  if (lane == 0) {
+    talk[2 * kWaves + 2 * wave] = best;
+    talk[2 * kWaves + 2 * wave + 1] = r;
+  }
   __syncthreads();
-  for (int i = lane; i < m; i += 64) {
+#pragma unroll
+  for (int q = 0; q < kWaves; ++q)
+    better(talk[2 * kWaves + 2 * q], (int)talk[2 * kWaves + 2 * q + 1]);
+  // component ratios away from it
+  for (int i = tid; i < m; i += kTriThreads) {
     if (i < r) F[i] = -b[i] / F[i];
     else if (i > r) F[i] = -b[i - 1] / B[i];
   }
   __syncthreads();
-  double x = 1.0, x1 = 1.0, sum = 0.0, first = 0.0;  // lane 0 down, lane 1 up from r
-  if (lane < 2) {
-    const int cnt = lane ? m - 1 - r : r;
-    constexpr int kU = 8;
-    double q[kU];
-    auto load = [&](int t0) {
-#pragma unroll
-      for (int u = 0; u < kU; ++u) {
-        const int t = t0 + u;
-        q[u] = t < cnt ? F[lane ? r + 1 + t : r - 1 - t] : 0.0;
-      }
-    };
-    load(0);
-    for (int t0 = 0; t0 < cnt; t0 += kU) {
-      double c[kU];
-#pragma unroll
-      for (int u = 0; u < kU; ++u) c[u] = q[u];
-      load(t0 + kU);
-#pragma unroll
-      for (int u = 0; u < kU; ++u)
-        if (t0 + u < cnt) {
-          x1 = x;
-          x *= c[u];
-          sum = __builtin_fma(x, x, sum);
-          if (t0 + u == 0) first = x;
-        }
+  if (wave == 0) {
+    const TriProducts down = tri_products(F + (r > 0 ? r - 1 : 0), -1, r);
+    if (lane == 0) {
+      talk[0] = down.sum;
+      talk[1] = down.first;
     }
   }
-  const double norm = sqrt(1.0 + __shfl(sum, 0, 64) + __shfl(sum, 1, 64));
-  const double last = __shfl(x, 1, 64);  // 1 if r is the last row
-  const double before = r == m - 1 ? __shfl(first, 0, 64) : __shfl(x1, 1, 64);
-  if (lane == 0) {
+  TriProducts up{0.0, 1.0, 1.0, 1.0};
+  if (wave == 1) up = tri_products(F + (r < m - 1 ? r + 1 : m - 1), 1, m - 1 - r);
+  __syncthreads();
+  if (wave == 1 && lane == 0) {
+    const double norm = sqrt(1.0 + talk[0] + up.sum);
     double *o = out + kTriHead + (int64_t)blockIdx.x * kTriOut;
     o[0] = v;
-    o[1] = last / norm;
-    o[2] = m >= 2 ? before / norm : 0.0;
+    o[1] = up.last / norm;
+    // the row before the last: the first one down if the last is r
+    o[2] = m >= 2 ? (r == m - 1 ? talk[1] : up.before) / norm : 0.0;
   }
 }
 
