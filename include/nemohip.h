@@ -80,11 +80,10 @@ nh_status nh_context_create(const nh_model *model, int device,
 void nh_context_destroy(nh_context *ctx);
 int64_t nh_context_dim(const nh_context *ctx); /* N = n_atoms * nb */
 
-/* Kernel variants (the same products to rounding).  NH_SET_HV_STAGED, of
- * the stored-block layout: 1 stages the neighbours' vector entries in LDS,
- * 0 reads them from the caches by every lane, -1 (default) direct.  SK and
- * matrix-free products always stage; there 0 only makes FP32 Lanczos runs
- * keep FP64 vectors (as NH_SET_LZ_VECTORS = 0 does). */
+/* NH_SET_HV_STAGED: the products always stage the neighbours' entries in LDS
+ * (one mapping is the fastest in every case measured), whatever the value (-1,
+ * 0 or 1); 0 only makes FP32 Lanczos runs of the SK and matrix-free layouts
+ * keep FP64 vectors, as NH_SET_LZ_VECTORS = 0 does. */
 enum { NH_SET_HV_STAGED = 1 };
 /* NH_SET_RING_STEPS: Lanczos steps between eigenvector accumulations in the
  * eigenvector pass (ring length; 8, 16, 32, 64 or 128), or 0 (default): 128,

@@ -1,19 +1,21 @@
-// Row of the stored-block H·v, shared by the plain operator kernel and
-// the fused Lanczos kernels (the library is built without relocatable
-// device code, so every kernel's translation unit includes this).
+// Rows of the stored-block H·v, shared by the plain operator kernel and the
+// fused Lanczos kernel (the library is built without relocatable device code,
+// so every kernel's translation unit includes this).
 //
-// Row-owner mapping: 10 lanes per atom, lane o owns spatial orbital o of
-// both spins, so the spin-shared 10x10 real neighbour blocks
-// (HamZincBlende::Hu, spin-diagonal and spin-independent) are read once per
-// row and applied to both spin components (Hv_stored_20_Hzb,
-// Hmult_stored.c:176-607, which applies Hu to rows i and i+10).  Each lane
-// reads its block row as 10 contiguous values; the 10 lanes of an atom read
-// one contiguous 800 B (FP64) / 400 B (FP32) block.
+// Row-owner mapping: 10 lanes per atom, six atoms a wavefront; lane o of an
+// atom owns spatial orbital o of both spins, so the spin-shared 10x10 real
+// neighbour blocks (HamZincBlende::Hu, spin-diagonal and spin-independent) are
+// read once per row and applied to both spin components (Hv_stored_20_Hzb,
+// Hmult_stored.c:176-607, which applies Hu to rows i and i+10).
 //
-// Neighbour vector entries: either read by every lane straight from
-// global memory (through L1/L2; hv_row), or first staged in LDS by the 10
-// lanes of the atom, each fetching 8 of the 80 values once (stage_nbr_x +
-// hv_row_staged).
+// The blocks are the traffic (3,200 B an atom in FP64).  Each wavefront loads
+// the six 800-byte blocks of a slot as consecutive 16-byte chunks, all four
+// slots in flight together, and hands them to the rows through its part of
+// LDS, as it does with the neighbours' entries.  A lane that loads its own
+// 80-byte row touches every cache line of the wavefront's 5 KB with each of
+// its five loads; with the lines of all wavefronts larger than the L1 that
+// fetched them several times from L2: 104,976 atoms, FP64, 146 -> 103 us (419
+// MB, 4.1 TB/s; a copy moves 4.7).
 //
 // FP32 storage: each block product is formed in FP32 (values and the FP32
 // image of x) and added to an FP64 row accumulator.
@@ -23,8 +25,9 @@
 
 namespace nh {
 
-constexpr int kAtomsPerBlock = 32;
-constexpr int kThreads = kAtomsPerBlock * 10;  // 320 = 5 wavefronts
+constexpr int kRowAtoms = 6;  // of a wavefront (60 lanes)
+constexpr int kThreads = 256;
+constexpr int kAtomsPerBlock = kThreads / 64 * kRowAtoms;
 
 // Surface s-p coupling partner list for lane o in {1,2,3,4}: partner
 // orbital and index into the 6 stored couplings (1,2),(1,3),(1,4),(2,3),
@@ -98,6 +101,14 @@ __device__ __forceinline__ void hv_onsite(int atom, int o,
   }
 }
 
+// LDS accesses of one wavefront execute in order; this keeps the compiler
+// from moving them across.  No instruction is emitted.
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // One neighbour block row applied to both spins: acc += B[o][:] x_j.
 template <int NSP, typename TB, typename TA>
 __device__ __forceinline__ void hv_block(const TB *__restrict__ B,
@@ -123,62 +134,74 @@ __device__ __forceinline__ void hv_block(const TB *__restrict__ B,
   }
 }
 
-// acc[s] = ((H - shift I) x) at row (atom, spin s, orbital o).
-template <int NSP, typename TB, typename TA>
-__device__ __forceinline__ void hv_row(int atom, int o,
-                                       const double *__restrict__ onsite,
-                                       const TB *__restrict__ blocks,
-                                       const int32_t *__restrict__ nbr,
-                                       double shift,
-                                       const double2 *__restrict__ xc,
-                                       double acc_re[NSP], double acc_im[NSP],
-                                       double2 xi[NSP]) {
-  constexpr int NB = NSP * 10;
-  hv_onsite<NSP>(atom, o, onsite, shift, xc, acc_re, acc_im, xi);
-#pragma unroll
-  for (int n = 0; n < 4; ++n) {
-    const int j = nbr[atom * 4 + n];
-    if (j < 0) continue;
-    hv_block<NSP, TB, TA>(blocks + ((size_t)atom * 4 + n) * 100 + o * 10,
-                          xc + (int64_t)j * NB, acc_re, acc_im);
-  }
-}
+// A wavefront's staging: the blocks of one slot and the neighbours' entries
+template <int NSP, typename TB>
+struct RowLds {
+  static constexpr int kSeg = 100 * (int)sizeof(TB) / 16;  // chunks of a block
+  static constexpr int kNx = NSP * 10;                     // chunks of an atom's entries
+  uint4 b[kRowAtoms * kSeg], x[kRowAtoms * kNx];
+};
 
-// Stages the x entries of the atom's four neighbours (4 x NSP*10 complex
-// values) in shared memory: lane o fetches entries o, o+10, ...; missing
-// neighbours are staged as zeros.  sx: the atom's 40*NSP slots.
-template <int NSP>
-__device__ __forceinline__ void stage_nbr_x(int atom, int o,
-                                            const int32_t *__restrict__ nbr,
-                                            const double2 *__restrict__ xc,
-                                            double2 *sx) {
-  constexpr int NB = NSP * 10;
-#pragma unroll
-  for (int t = 0; t < 4 * NSP; ++t) {
-    const int e = o + 10 * t;  // 0 .. 40*NSP-1
-    const int n = e / NB, k = e % NB;
-    const int j = nbr[atom * 4 + n];
-    sx[e] = j >= 0 ? xc[(int64_t)j * NB + k] : make_double2(0.0, 0.0);
-  }
-}
-
-// hv_row with the neighbour entries read from the staged copy.
+// acc[s] = ((H - shift I) x) at row (atom, spin s, orbital o) of the lane; a0:
+// the wavefront's first atom.  Lanes without a row (atom < 0) take part in the
+// loads.
 template <int NSP, typename TB, typename TA>
-__device__ __forceinline__ void hv_row_staged(int atom, int o,
-                                              const double *__restrict__ onsite,
-                                              const TB *__restrict__ blocks,
-                                              double shift,
-                                              const double2 *__restrict__ xc,
-                                              const double2 *sx,
-                                              double acc_re[NSP],
-                                              double acc_im[NSP],
-                                              double2 xi[NSP]) {
-  constexpr int NB = NSP * 10;
-  hv_onsite<NSP>(atom, o, onsite, shift, xc, acc_re, acc_im, xi);
+__device__ __forceinline__ void hv_rows(int a0, int A, int atom, int o,
+                                        const double *__restrict__ onsite,
+                                        const TB *__restrict__ blocks,
+                                        const int32_t *__restrict__ nbr, double shift,
+                                        const double2 *__restrict__ xc, RowLds<NSP, TB> &L,
+                                        double acc_re[NSP], double acc_im[NSP],
+                                        double2 xi[NSP]) {
+  using S = RowLds<NSP, TB>;
+  constexpr int kB = (kRowAtoms * S::kSeg + 63) / 64, kX = (kRowAtoms * S::kNx + 63) / 64;
+  const int lane = threadIdx.x & 63;
+  const int na = min(kRowAtoms, A - a0);
+  const int4 *nb4 = reinterpret_cast<const int4 *>(nbr);
+  uint4 bl[4][kB], xl[4][kX];
+  int4 nx[kX];
+#pragma unroll
+  for (int i = 0; i < kX; ++i) {
+    const int seg = (lane + 64 * i) / S::kNx;
+    nx[i] = seg < na ? nb4[a0 + seg] : make_int4(-1, -1, -1, -1);
+  }
+  const int4 own = atom >= 0 ? nb4[atom] : make_int4(-1, -1, -1, -1);
 #pragma unroll
   for (int n = 0; n < 4; ++n)
-    hv_block<NSP, TB, TA>(blocks + ((size_t)atom * 4 + n) * 100 + o * 10,
-                          sx + n * NB, acc_re, acc_im);
+#pragma unroll
+    for (int i = 0; i < kB; ++i) {
+      const int c = lane + 64 * i, seg = c / S::kSeg;
+      bl[n][i] = make_uint4(0, 0, 0, 0);
+      if (seg < na)
+        bl[n][i] = reinterpret_cast<const uint4 *>(blocks)[((int64_t)(a0 + seg) * 4 + n) * S::kSeg +
+                                                           c % S::kSeg];
+    }
+#pragma unroll
+  for (int n = 0; n < 4; ++n)
+#pragma unroll
+    for (int i = 0; i < kX; ++i) {
+      const int j = n == 0 ? nx[i].x : n == 1 ? nx[i].y : n == 2 ? nx[i].z : nx[i].w;
+      xl[n][i] = make_uint4(0, 0, 0, 0);
+      if (j >= 0)
+        xl[n][i] = reinterpret_cast<const uint4 *>(xc)[(int64_t)j * S::kNx + (lane + 64 * i) % S::kNx];
+    }
+  if (atom >= 0) hv_onsite<NSP>(atom, o, onsite, shift, xc, acc_re, acc_im, xi);
+  const int la = lane / 10;
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    wave_fence();
+#pragma unroll
+    for (int i = 0; i < kB; ++i)
+      if (lane + 64 * i < kRowAtoms * S::kSeg) L.b[lane + 64 * i] = bl[n][i];
+#pragma unroll
+    for (int i = 0; i < kX; ++i)
+      if (lane + 64 * i < kRowAtoms * S::kNx) L.x[lane + 64 * i] = xl[n][i];
+    wave_fence();
+    const int j = n == 0 ? own.x : n == 1 ? own.y : n == 2 ? own.z : own.w;
+    if (j >= 0)
+      hv_block<NSP, TB, TA>(reinterpret_cast<const TB *>(L.b + la * S::kSeg) + o * 10,
+                            reinterpret_cast<const double2 *>(L.x + la * S::kNx), acc_re, acc_im);
+  }
 }
 
 }  // namespace nh

@@ -89,7 +89,7 @@ struct nh_context {
   // stored-block H·v: neighbour x staged in LDS (measured on the 786,520-
   // atom dot: faster for the plain product, slower inside the fused Lanczos
   // kernel, so off by default)
-  int hv_staged = -1;  // NH_SET_HV_STAGED (-1: by layout, see use_staged)
+  int hv_staged = -1;  // NH_SET_HV_STAGED (0: no FP32 Lanczos vectors)
   int ring_steps = 0;  // NH_SET_RING_STEPS (0: by free memory)
   int block_hv = -1;   // NH_SET_BLOCK_HV (-1: by measurement)
   int lz_vectors = -1; // NH_SET_LZ_VECTORS (-1: default, lz_fp32_vectors)
@@ -132,16 +132,10 @@ struct nh_context {
 };
 
 namespace nh {
-// LDS staging of the neighbours' entries in H·v: measured faster for the SK
-// layout (quad gather), slower for the stored-block layout inside the
-// fused Lanczos step; NH_SET_HV_STAGED overrides.
 // Layouts applied by the 4-lanes-per-atom bond kernels (nh_hv_sk.h): the
 // stored SK records and the matrix-free one.
 inline bool sk_like(const nh_context *c) {
   return c->layout == NH_LAYOUT_SK || c->layout == NH_LAYOUT_MATRIX_FREE;
-}
-inline bool use_staged(const nh_context *c) {
-  return c->hv_staged < 0 ? sk_like(c) : c->hv_staged != 0;
 }
 // Lanczos vectors stored in FP32 (FP32 SK or matrix-free products with the
 // LDS gather only).  Default on (measured on a 786,520-atom dot, FP32 SK
@@ -149,7 +143,7 @@ inline bool use_staged(const nh_context *c) {
 // / 0.228 ms in the two passes against 0.229 / 0.301 ms, FP32 stage 4.73 s
 // against 6.23 s, with a separate update kernel)
 inline bool lz_fp32_vectors(const nh_context *c) {
-  return sk_like(c) && c->precision == NH_PREC_FP32 && use_staged(c) &&
+  return sk_like(c) && c->precision == NH_PREC_FP32 && c->hv_staged != 0 &&
          c->lz_vectors != 0;
 }
 }  // namespace nh

@@ -42,61 +42,41 @@ namespace {
 constexpr int kRingMax = 128;
 constexpr int kMaxVec = 64;
 
-__device__ __forceinline__ double wg_sum320(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  __shared__ double s[kThreads / 64];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (lane == 0) s[w] = v;
-  __syncthreads();
-  double t = 0.0;
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int k = 0; k < kThreads / 64; ++k) t += s[k];
-  }
-  return t;
-}
-
-template <int NSP, typename TB, typename TA, bool STAGED>
-__global__ __launch_bounds__(kThreads) void k_lz_hv(
+template <int NSP, typename TB, typename TA>
+__global__ __launch_bounds__(kThreads, 3) void k_lz_hv(
     int A, const double *__restrict__ onsite, const TB *__restrict__ blocks,
     const int32_t *__restrict__ nbr, const double2 *__restrict__ R,
     double2 *__restrict__ Q, double2 *__restrict__ Y,
     const double *__restrict__ beta_prev, double *__restrict__ part) {
   constexpr int NB = NSP * 10;
-  const int la = threadIdx.x / 10;
-  const int atom = blockIdx.x * kAtomsPerBlock + la;
-  const int o = threadIdx.x % 10;
+  static_assert(kThreads == kRedThreads, "block sums");
+  __shared__ RowLds<NSP, TB> L[kThreads / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int a0 = (blockIdx.x * (kThreads / 64) + wave) * kRowAtoms;
+  const int o = lane % 10;
+  const int atom = lane < 10 * kRowAtoms && a0 + lane / 10 < A ? a0 + lane / 10 : -1;
   const double inv = beta_prev ? 1.0 / beta_prev[0] : 1.0;
-  double local = 0.0;
-  double acc_re[NSP], acc_im[NSP];
-  double2 xi[NSP];
-  if constexpr (STAGED) {
-    __shared__ double2 sx[kAtomsPerBlock * 4 * NB];
-    if (atom < A) stage_nbr_x<NSP>(atom, o, nbr, R, sx + la * 4 * NB);
-    __syncthreads();
-    if (atom < A)
-      hv_row_staged<NSP, TB, TA>(atom, o, onsite, blocks, 0.0, R,
-                                 sx + la * 4 * NB, acc_re, acc_im, xi);
-  } else {
-    if (atom < A)
-      hv_row<NSP, TB, TA>(atom, o, onsite, blocks, nbr, 0.0, R, acc_re, acc_im,
-                          xi);
-  }
-  if (atom < A) {
-    const int64_t base = (int64_t)atom * NB;
+  double local = 0.0, zero = 0.0;
+  if (a0 < A) {
+    double acc_re[NSP], acc_im[NSP];
+    double2 xi[NSP];
+    hv_rows<NSP, TB, TA>(a0, A, atom, o, onsite, blocks, nbr, 0.0, R, L[wave], acc_re, acc_im,
+                         xi);
+    if (atom >= 0) {
+      const int64_t base = (int64_t)atom * NB;
 #pragma unroll
-    for (int s = 0; s < NSP; ++s) {
-      const double2 q = make_double2(xi[s].x * inv, xi[s].y * inv);
-      const double2 y = make_double2(acc_re[s] * inv, acc_im[s] * inv);
-      if (Q) Q[base + s * 10 + o] = q;
-      Y[base + s * 10 + o] = y;
-      local += q.x * y.x + q.y * y.y;
+      for (int s = 0; s < NSP; ++s) {
+        const double2 q = make_double2(xi[s].x * inv, xi[s].y * inv);
+        const double2 y = make_double2(acc_re[s] * inv, acc_im[s] * inv);
+        if (Q) Q[base + s * 10 + o] = q;
+        Y[base + s * 10 + o] = y;
+        local += q.x * y.x + q.y * y.y;
+      }
     }
   }
   if (part) {
-    const double t = wg_sum320(local);
-    if (threadIdx.x == 0) part[blockIdx.x] = t;
+    block_sum2(local, zero);
+    if (threadIdx.x == 0) part[blockIdx.x] = local;
   }
 }
 
@@ -883,16 +863,9 @@ nh_status LanczosRun::iterate(int k, bool red) {
     double2 *Q = red ? nullptr : ring_ + (int64_t)(k % ring_k_) * n_;
     double *part = red ? part_ : nullptr;
 #define LZ_HV(NSP, TB, BLK)                                                    \
-  do {                                                                         \
-    if (use_staged(c))                                                         \
-      hipLaunchKernelGGL((k_lz_hv<NSP, TB, TB, true>), dim3(grid_),            \
-                         dim3(kThreads), 0, c->stream, c->n_atoms, c->onsite,  \
-                         BLK, c->nbr, R_, Q, Y_, bprev, part);                 \
-    else                                                                       \
-      hipLaunchKernelGGL((k_lz_hv<NSP, TB, TB, false>), dim3(grid_),           \
-                         dim3(kThreads), 0, c->stream, c->n_atoms, c->onsite,  \
-                         BLK, c->nbr, R_, Q, Y_, bprev, part);                 \
-  } while (0)
+  hipLaunchKernelGGL((k_lz_hv<NSP, TB, TB>), dim3(grid_), dim3(kThreads), 0,   \
+                     c->stream, c->n_atoms, c->onsite, BLK, c->nbr, R_, Q, Y_, \
+                     bprev, part)
     if (c->precision == NH_PREC_FP64) {
       if (c->nb == 20) LZ_HV(2, double, c->blocks64);
       else LZ_HV(1, double, c->blocks64);
