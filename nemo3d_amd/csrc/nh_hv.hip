@@ -68,29 +68,31 @@ __global__ __launch_bounds__(kSkThreads, 2) void k_hv_sk(
   }
 }
 
-template <int NSP, typename TB, typename TA>
-__global__ __launch_bounds__(kThreads, 3) void k_hv_blocks(
+// A column per grid row, or (COLS) nc columns: the blocks are read once for all
+// of them and stay in registers (104,976 atoms, 8 columns, FP64: XX us, a column
+// per grid row YY).
+template <bool COLS, int NSP, typename TB, typename TA>
+__global__ __launch_bounds__(kThreads, COLS ? 2 : 3) void k_hv_blocks(
     int A, const double *__restrict__ onsite, const TB *__restrict__ blocks,
     const int32_t *__restrict__ nbr, double shift,
-    const double2 *__restrict__ x, double2 *__restrict__ y, int64_t ld) {
+    const double2 *__restrict__ x, double2 *__restrict__ y, int64_t ld, int nc) {
   constexpr int NB = NSP * 10;
   __shared__ RowLds<NSP, TB> L[kThreads / 64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wave = threadIdx.x >> 6;
   const int a0 = (blockIdx.x * (kThreads / 64) + wave) * kRowAtoms;
   if (a0 >= A) return;
-  const int o = lane % 10;
-  const int atom = lane < 10 * kRowAtoms && a0 + lane / 10 < A ? a0 + lane / 10 : -1;
-  const double2 *xc = x + (int64_t)blockIdx.y * ld;
-  double2 *yc = y + (int64_t)blockIdx.y * ld;
-  double acc_re[NSP], acc_im[NSP];
-  double2 xi[NSP];
-  hv_rows<NSP, TB, TA>(a0, A, atom, o, onsite, blocks, nbr, shift, xc, L[wave], acc_re, acc_im,
-                       xi);
-  if (atom < 0) return;
-  const int64_t base = (int64_t)atom * NB;
+  const Rows<NSP, TB> rows(a0, A, blocks, nbr);
+  const int64_t c0 = COLS ? 0 : blockIdx.y;
+  for (int c = 0; c < (COLS ? nc : 1); ++c) {
+    double acc_re[NSP], acc_im[NSP];
+    double2 xi[NSP];
+    rows.template apply<TA>(onsite, shift, x + (c0 + c) * ld, L[wave], acc_re, acc_im, xi);
+    if (rows.atom >= 0) {
+      double2 *yr = y + (c0 + c) * ld + (int64_t)rows.atom * NB + rows.o;
 #pragma unroll
-  for (int s = 0; s < NSP; ++s)
-    yc[base + s * 10 + o] = make_double2(acc_re[s], acc_im[s]);
+      for (int s = 0; s < NSP; ++s) yr[s * 10] = make_double2(acc_re[s], acc_im[s]);
+    }
+  }
 }
 
 }  // namespace
@@ -101,15 +103,13 @@ nh_status launch_hv(nh_context *c, double shift, const nh_cplx *x, nh_cplx *y,
            "H·v: Hamiltonian not built in a supported layout");
   NH_CHECK(ncol >= 1 && ncol <= 65535 && ld >= c->n, NH_ERR_ARG,
            "H·V: bad ncol %d / ld %lld", ncol, (long long)ld);
-  // block products: the matrix-core kernel (FP32, 8 columns) by default for
-  // the row-owner block layout only; in the SK and matrix-free layouts all the
-  // columns in one launch with H read once, measured fastest for 2 columns and
-  // more (395,136 atoms, 8 columns, FP64: 0.65 ms SK and matrix-free against
-  // 0.83 / 1.06 ms with a column per grid row; 4 columns 0.34 / 0.35 ms)
+  // block products: all the columns in one launch with H read once, measured
+  // fastest for 2 columns and more (SK and matrix-free, 395,136 atoms, 8
+  // columns, FP64: 0.65 ms against 0.83 / 1.06 with a column per grid row;
+  // stored blocks, 104,976 atoms, 8 columns: 424 us FP64, 331 FP32 against 720
+  // and 416, and 519 with the matrix-core kernel)
   const int mode = c->block_hv;
-  if ((mode == 2 || (mode == -1 && c->layout == NH_LAYOUT_BLOCKS)) &&
-      hV_mfma_supported(c, ncol))
-    return launch_hV_mfma(c, shift, x, y, ld);
+  if (mode == 2 && hV_mfma_supported(c, ncol)) return launch_hV_mfma(c, shift, x, y, ld);
   if (sk_like(c)) {
     const SkTable tab = sk_table_of(c);
     const double2 *xd = reinterpret_cast<const double2 *>(x);
@@ -149,13 +149,21 @@ nh_status launch_hv(nh_context *c, double shift, const nh_cplx *x, nh_cplx *y,
     NH_HIP(hipGetLastError());
     return NH_OK;
   }
-  const dim3 grid((c->n_atoms + kAtomsPerBlock - 1) / kAtomsPerBlock, ncol);
+  const bool cols = ncol > 1 && mode != 0;
+  const dim3 grid((c->n_atoms + kAtomsPerBlock - 1) / kAtomsPerBlock, cols ? 1 : ncol);
   const double2 *xd = reinterpret_cast<const double2 *>(x);
   double2 *yd = reinterpret_cast<double2 *>(y);
 #define HVB(NSP, TB, TA, BLK)                                                  \
-  hipLaunchKernelGGL((k_hv_blocks<NSP, TB, TA>), grid, dim3(kThreads), 0,    \
-                     c->stream, c->n_atoms, c->onsite, BLK, c->nbr, shift,   \
-                     xd, yd, ld)
+  do {                                                                       \
+    if (cols)                                                                \
+      hipLaunchKernelGGL((k_hv_blocks<true, NSP, TB, TA>), grid,             \
+                         dim3(kThreads), 0, c->stream, c->n_atoms, c->onsite, \
+                         BLK, c->nbr, shift, xd, yd, ld, ncol);              \
+    else                                                                     \
+      hipLaunchKernelGGL((k_hv_blocks<false, NSP, TB, TA>), grid,            \
+                         dim3(kThreads), 0, c->stream, c->n_atoms, c->onsite, \
+                         BLK, c->nbr, shift, xd, yd, ld, 1);                 \
+  } while (0)
   if (c->precision == NH_PREC_FP64) {
     if (c->nb == 20) HVB(2, double, double, c->blocks64);
     else HVB(1, double, double, c->blocks64);

@@ -142,66 +142,77 @@ struct RowLds {
   uint4 b[kRowAtoms * kSeg], x[kRowAtoms * kNx];
 };
 
-// acc[s] = ((H - shift I) x) at row (atom, spin s, orbital o) of the lane; a0:
-// the wavefront's first atom.  Lanes without a row (atom < 0) take part in the
-// loads.
-template <int NSP, typename TB, typename TA>
-__device__ __forceinline__ void hv_rows(int a0, int A, int atom, int o,
-                                        const double *__restrict__ onsite,
-                                        const TB *__restrict__ blocks,
-                                        const int32_t *__restrict__ nbr, double shift,
-                                        const double2 *__restrict__ xc, RowLds<NSP, TB> &L,
-                                        double acc_re[NSP], double acc_im[NSP],
-                                        double2 xi[NSP]) {
+// What a wavefront holds of its six atoms (the first is a0): its share of the
+// 24 blocks' chunks, all requested together, the neighbours of the atoms whose
+// entries it stages and of the lane's own atom (-1: no row, the lane only
+// takes part in the loads).
+template <int NSP, typename TB>
+struct Rows {
   using S = RowLds<NSP, TB>;
-  constexpr int kB = (kRowAtoms * S::kSeg + 63) / 64, kX = (kRowAtoms * S::kNx + 63) / 64;
-  const int lane = threadIdx.x & 63;
-  const int na = min(kRowAtoms, A - a0);
-  const int4 *nb4 = reinterpret_cast<const int4 *>(nbr);
-  uint4 bl[4][kB], xl[4][kX];
-  int4 nx[kX];
-#pragma unroll
-  for (int i = 0; i < kX; ++i) {
-    const int seg = (lane + 64 * i) / S::kNx;
-    nx[i] = seg < na ? nb4[a0 + seg] : make_int4(-1, -1, -1, -1);
-  }
-  const int4 own = atom >= 0 ? nb4[atom] : make_int4(-1, -1, -1, -1);
-#pragma unroll
-  for (int n = 0; n < 4; ++n)
-#pragma unroll
-    for (int i = 0; i < kB; ++i) {
-      const int c = lane + 64 * i, seg = c / S::kSeg;
-      bl[n][i] = make_uint4(0, 0, 0, 0);
-      if (seg < na)
-        bl[n][i] = reinterpret_cast<const uint4 *>(blocks)[((int64_t)(a0 + seg) * 4 + n) * S::kSeg +
-                                                           c % S::kSeg];
-    }
-#pragma unroll
-  for (int n = 0; n < 4; ++n)
+  static constexpr int kB = (kRowAtoms * S::kSeg + 63) / 64, kX = (kRowAtoms * S::kNx + 63) / 64;
+  uint4 bl[4][kB];
+  int4 nx[kX], own;
+  int atom, o;
+
+  __device__ __forceinline__ Rows(int a0, int A, const TB *__restrict__ blocks,
+                                  const int32_t *__restrict__ nbr) {
+    const int lane = threadIdx.x & 63, na = min(kRowAtoms, A - a0);
+    const int4 *nb4 = reinterpret_cast<const int4 *>(nbr);
+    o = lane % 10;
+    atom = lane / 10 < na ? a0 + lane / 10 : -1;
 #pragma unroll
     for (int i = 0; i < kX; ++i) {
-      const int j = n == 0 ? nx[i].x : n == 1 ? nx[i].y : n == 2 ? nx[i].z : nx[i].w;
-      xl[n][i] = make_uint4(0, 0, 0, 0);
-      if (j >= 0)
-        xl[n][i] = reinterpret_cast<const uint4 *>(xc)[(int64_t)j * S::kNx + (lane + 64 * i) % S::kNx];
+      const int seg = (lane + 64 * i) / S::kNx;
+      nx[i] = seg < na ? nb4[a0 + seg] : make_int4(-1, -1, -1, -1);
     }
-  if (atom >= 0) hv_onsite<NSP>(atom, o, onsite, shift, xc, acc_re, acc_im, xi);
-  const int la = lane / 10;
+    own = atom >= 0 ? nb4[atom] : make_int4(-1, -1, -1, -1);
 #pragma unroll
-  for (int n = 0; n < 4; ++n) {
-    wave_fence();
+    for (int n = 0; n < 4; ++n)
 #pragma unroll
-    for (int i = 0; i < kB; ++i)
-      if (lane + 64 * i < kRowAtoms * S::kSeg) L.b[lane + 64 * i] = bl[n][i];
-#pragma unroll
-    for (int i = 0; i < kX; ++i)
-      if (lane + 64 * i < kRowAtoms * S::kNx) L.x[lane + 64 * i] = xl[n][i];
-    wave_fence();
-    const int j = n == 0 ? own.x : n == 1 ? own.y : n == 2 ? own.z : own.w;
-    if (j >= 0)
-      hv_block<NSP, TB, TA>(reinterpret_cast<const TB *>(L.b + la * S::kSeg) + o * 10,
-                            reinterpret_cast<const double2 *>(L.x + la * S::kNx), acc_re, acc_im);
+      for (int i = 0; i < kB; ++i) {
+        const int c = lane + 64 * i, seg = c / S::kSeg;
+        bl[n][i] = make_uint4(0, 0, 0, 0);
+        if (seg < na)
+          bl[n][i] = reinterpret_cast<const uint4 *>(
+              blocks)[((int64_t)(a0 + seg) * 4 + n) * S::kSeg + c % S::kSeg];
+      }
   }
-}
+
+  // acc[s] = ((H - shift I) x) at row (atom, spin s, orbital o)
+  template <typename TA>
+  __device__ __forceinline__ void apply(const double *__restrict__ onsite, double shift,
+                                        const double2 *__restrict__ xc, S &L, double acc_re[NSP],
+                                        double acc_im[NSP], double2 xi[NSP]) const {
+    const int lane = threadIdx.x & 63, la = lane / 10;
+    auto slot = [](const int4 &v, int n) { return n == 0 ? v.x : n == 1 ? v.y : n == 2 ? v.z : v.w; };
+    uint4 xl[4][kX];
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+      for (int i = 0; i < kX; ++i) {
+        const int j = slot(nx[i], n);
+        xl[n][i] = make_uint4(0, 0, 0, 0);
+        if (j >= 0)
+          xl[n][i] =
+              reinterpret_cast<const uint4 *>(xc)[(int64_t)j * S::kNx + (lane + 64 * i) % S::kNx];
+      }
+    if (atom >= 0) hv_onsite<NSP>(atom, o, onsite, shift, xc, acc_re, acc_im, xi);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      wave_fence();
+#pragma unroll
+      for (int i = 0; i < kB; ++i)
+        if (lane + 64 * i < kRowAtoms * S::kSeg) L.b[lane + 64 * i] = bl[n][i];
+#pragma unroll
+      for (int i = 0; i < kX; ++i)
+        if (lane + 64 * i < kRowAtoms * S::kNx) L.x[lane + 64 * i] = xl[n][i];
+      wave_fence();
+      if (slot(own, n) >= 0)
+        hv_block<NSP, TB, TA>(reinterpret_cast<const TB *>(L.b + la * S::kSeg) + o * 10,
+                              reinterpret_cast<const double2 *>(L.x + la * S::kNx), acc_re,
+                              acc_im);
+    }
+  }
+};
 
 }  // namespace nh

@@ -51,25 +51,23 @@ __global__ __launch_bounds__(kThreads, 3) void k_lz_hv(
   constexpr int NB = NSP * 10;
   static_assert(kThreads == kRedThreads, "block sums");
   __shared__ RowLds<NSP, TB> L[kThreads / 64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wave = threadIdx.x >> 6;
   const int a0 = (blockIdx.x * (kThreads / 64) + wave) * kRowAtoms;
-  const int o = lane % 10;
-  const int atom = lane < 10 * kRowAtoms && a0 + lane / 10 < A ? a0 + lane / 10 : -1;
   const double inv = beta_prev ? 1.0 / beta_prev[0] : 1.0;
   double local = 0.0, zero = 0.0;
   if (a0 < A) {
     double acc_re[NSP], acc_im[NSP];
     double2 xi[NSP];
-    hv_rows<NSP, TB, TA>(a0, A, atom, o, onsite, blocks, nbr, 0.0, R, L[wave], acc_re, acc_im,
-                         xi);
-    if (atom >= 0) {
-      const int64_t base = (int64_t)atom * NB;
+    const Rows<NSP, TB> rows(a0, A, blocks, nbr);
+    rows.template apply<TA>(onsite, 0.0, R, L[wave], acc_re, acc_im, xi);
+    if (rows.atom >= 0) {
+      const int64_t base = (int64_t)rows.atom * NB + rows.o;
 #pragma unroll
       for (int s = 0; s < NSP; ++s) {
         const double2 q = make_double2(xi[s].x * inv, xi[s].y * inv);
         const double2 y = make_double2(acc_re[s] * inv, acc_im[s] * inv);
-        if (Q) Q[base + s * 10 + o] = q;
-        Y[base + s * 10 + o] = y;
+        if (Q) Q[base + s * 10] = q;
+        Y[base + s * 10] = y;
         local += q.x * y.x + q.y * y.y;
       }
     }
