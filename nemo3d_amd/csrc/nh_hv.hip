@@ -107,9 +107,8 @@ nh_status launch_hv(nh_context *c, double shift, const nh_cplx *x, nh_cplx *y,
   // fastest for 2 columns and more (SK and matrix-free, 395,136 atoms, 8
   // columns, FP64: 0.65 ms against 0.83 / 1.06 with a column per grid row;
   // stored blocks, 104,976 atoms, 8 columns: 424 us FP64, 331 FP32 against 720
-  // and 416, and 519 with the matrix-core kernel)
+  // and 416; FP32 matrix instructions, a wavefront per atom and 8 columns: 519)
   const int mode = c->block_hv;
-  if (mode == 2 && hV_mfma_supported(c, ncol)) return launch_hV_mfma(c, shift, x, y, ld);
   if (sk_like(c)) {
     const SkTable tab = sk_table_of(c);
     const double2 *xd = reinterpret_cast<const double2 *>(x);

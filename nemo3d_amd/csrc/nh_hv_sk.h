@@ -77,55 +77,6 @@ struct SkWalk {
 __device__ __forceinline__ double2 widen2(double2 v) { return v; }
 __device__ __forceinline__ double2 widen2(float2 v) { return make_double2(v.x, v.y); }
 
-// Onsite contribution (diagonal - shift, surface s-p couplings, spin-orbit)
-// to row (s, o) of atom with vector base pointer xa.
-template <int NSP, typename XA = double2>
-__device__ __forceinline__ void onsite_row(const double *__restrict__ os,
-                                           const XA *__restrict__ xa,
-                                           int s, int o, double shift,
-                                           double &re, double &im) {
-  const double2 xo = widen2(xa[s * 10 + o]);
-  const double d = os[o] - shift;
-  re += d * xo.x;
-  im += d * xo.y;
-  if (o >= 1 && o <= 4) {
-    // partners and stored coupling index: (1,2)0 (1,3)1 (1,4)2 (2,3)3 (2,4)4 (3,4)5
-    const int p0 = o == 1 ? 2 : 1, k0 = o == 1 ? 0 : o == 2 ? 0 : o == 3 ? 1 : 2;
-    const int p1 = o <= 2 ? 3 : 2, k1 = o == 1 ? 1 : o == 2 ? 3 : o == 3 ? 3 : 4;
-    const int p2 = o <= 3 ? 4 : 3, k2 = o == 1 ? 2 : o == 2 ? 4 : 5;
-    const double h0 = os[10 + k0], h1 = os[10 + k1], h2 = os[10 + k2];
-    const double2 a0 = widen2(xa[s * 10 + p0]), a1 = widen2(xa[s * 10 + p1]), a2 = widen2(xa[s * 10 + p2]);
-    re += h0 * a0.x + h1 * a1.x + h2 * a2.x;
-    im += h0 * a0.y + h1 * a1.y + h2 * a2.y;
-  }
-  if (NSP == 2 && o >= 2 && o <= 4) {
-    const double lam = os[16];
-    if (s == 0) {
-      if (o == 2) {
-        re += lam * widen2(xa[3]).y + lam * widen2(xa[14]).x;
-        im += -lam * widen2(xa[3]).x + lam * widen2(xa[14]).y;
-      } else if (o == 3) {
-        re += -lam * widen2(xa[2]).y + lam * widen2(xa[14]).y;
-        im += lam * widen2(xa[2]).x - lam * widen2(xa[14]).x;
-      } else {
-        re += -lam * widen2(xa[12]).x - lam * widen2(xa[13]).y;
-        im += -lam * widen2(xa[12]).y + lam * widen2(xa[13]).x;
-      }
-    } else {
-      if (o == 2) {
-        re += -lam * widen2(xa[13]).y - lam * widen2(xa[4]).x;
-        im += lam * widen2(xa[13]).x - lam * widen2(xa[4]).y;
-      } else if (o == 3) {
-        re += lam * widen2(xa[12]).y + lam * widen2(xa[4]).y;
-        im += -lam * widen2(xa[12]).x - lam * widen2(xa[4]).x;
-      } else {
-        re += lam * widen2(xa[2]).x - lam * widen2(xa[3]).y;
-        im += lam * widen2(xa[2]).y + lam * widen2(xa[3]).x;
-      }
-    }
-  }
-}
-
 // LDS accesses of one wavefront execute in order; this keeps the compiler
 // from moving them across (lanes read what other lanes of the wavefront
 // wrote).  No instruction is emitted.

@@ -71,32 +71,6 @@ __host__ __device__ __forceinline__ void sk_record(R l, R m, R n, const R *v, R 
   k[K_DB] = v[19] - v[20];
   k[K_DA] = c3 * ((v[18] - v[20]) - R(4.0 / 3.0) * (v[19] - v[20]));
 }
-// the 21 integrals of a record
-template <typename R>
-__host__ __device__ __forceinline__ void sk_integrals(const R *k, R *v) {
-  constexpr R c2 = R(2.0 / kSqrt3Ref), c3 = R(3.0 / (kSqrt3Ref * kSqrt3Ref));
-  v[0] = k[K_SSS];
-  v[1] = k[K_STSTS];
-  v[2] = k[K_STASS];
-  v[3] = k[K_SASTS];
-  v[4] = k[K_SAPC];
-  v[5] = -k[K_SCPA];
-  v[6] = k[K_STAPC];
-  v[7] = -k[K_STCPA];
-  v[8] = k[K_SADC];
-  v[9] = k[K_SCDA];
-  v[10] = k[K_STADC];
-  v[11] = k[K_STCDA];
-  v[12] = k[K_PPC] + k[K_PPP];
-  v[13] = k[K_PPP];
-  v[14] = k[K_APD] + c2 * k[K_PADP];
-  v[15] = -k[K_ADP] - c2 * k[K_PCDP];
-  v[16] = k[K_PADP];
-  v[17] = -k[K_PCDP];
-  v[18] = k[K_DA] / c3 + k[K_DDD] + R(4.0 / 3.0) * k[K_DB];
-  v[19] = k[K_DB] + k[K_DDD];
-  v[20] = k[K_DDD];
-}
 
 __host__ __device__ __forceinline__ double sk_fma(double a, double b, double c) {
   return __builtin_fma(a, b, c);
