@@ -368,8 +368,11 @@ __global__ __launch_bounds__(256) void k_head_fwd(
 // point.  A wavefront takes 32 atoms, kMapRows channels at a time (whole
 // states: 4 nb divides them), keeps each atom's slot in LDS and writes them
 // out state by state.  Through the head's output of all points (as large as
-// the start block) it took 5.25 + 0.56 ms for 786,520 atoms, this 0.74 ms
-// (2.0 GB written; half its products are for the slot an atom is not in).
+// the start block) it took 5.25 + 0.56 ms for 786,520 atoms, this 0.50 ms
+// (2.0 GB written, 0.43 ms at the rate of a copy; half its products are for
+// the slot an atom is not in).  The bias goes through LDS and the places are
+// stepped on instead of divided out: with 80 short loads of the bias a block
+// and the divisions the vector units were as busy as the matrix units (0.74).
 constexpr int kMapRows = 160;
 __global__ __launch_bounds__(256) void k_head_map(
     int64_t A, int nb, int ne, int co_n, const int32_t *__restrict__ point,
@@ -379,44 +382,67 @@ __global__ __launch_bounds__(256) void k_head_map(
   // [wave][atom][kMapRows / 2], rows of an odd number of 16-byte chunks
   constexpr int kRow = kMapRows / 2 + 4;
   __shared__ float lds[4][32 * kRow];
+  __shared__ float4 blds[4][kMapRows / 4];  // a block's bias
   const int lane = threadIdx.x & 63, h = lane >> 5, n = lane & 31;
   float *buf = lds[threadIdx.x >> 6];
+  float4 *brow = blds[threadIdx.x >> 6];
   const int per = kMapRows / (4 * nb);  // states of a block
+  const int da = 64 / nb, dq = 64 % nb;  // 64 entries on, in atoms and entries
   for (int64_t g = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); g * 32 < A;
        g += (int64_t)gridDim.x * 4) {
     const int64_t a0 = g * 32, at = a0 + n;
     const bool ok = at < A;
     const int sl = ok ? slot[at] : 0;
     const HeadAct b = load_act(act + (ok ? (int64_t)point[at] : 0) * kCnnW, h, ok);
-    const int64_t rows = (int64_t)min((int64_t)32, A - a0) * nb;  // entries of a state
+    const int rows = (int)min((int64_t)32, A - a0) * nb;  // entries of a state
     for (int e0 = 0; e0 < ne; e0 += per) {
       const int t0 = e0 * 4 * nb / 32;
+      if (lane < kMapRows / 4) {
+        float v[4];
+        head_bias(bias, 32 * t0 + 4 * lane, co_n, v);
+        brow[lane] = make_float4(v[0], v[1], v[2], v[3]);
+      }
+      __builtin_amdgcn_wave_barrier();
+      // rows r .. r + 3 belong to one state and slot (2 nb is a multiple of
+      // 4): o = r % (4 nb) less the slot's rows, dst the state's place
+      int o = 4 * h - (sl ? 2 * nb : 0);
+      float *dst = buf + n * kRow;
 #pragma unroll
       for (int t = 0; t < kMapRows / 32; ++t) {
         f32x16 acc;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          float v[4];
-          head_bias(bias, 32 * (t0 + t) + 8 * q + 4 * h, co_n, v);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[4 * q + j] = v[j];
+          const float4 v = brow[8 * t + 2 * q + h];
+          acc[4 * q] = v.x, acc[4 * q + 1] = v.y, acc[4 * q + 2] = v.z, acc[4 * q + 3] = v.w;
         }
         acc = head_tile(W, t0 + t, lane, b, acc);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          // rows r .. r + 3 belong to one state and slot (2 nb is a multiple of 4)
-          const int r = 32 * t + 8 * q + 4 * h, e = r / (4 * nb), o = r % (4 * nb);
-          if ((o >= 2 * nb) == (sl != 0))
-            *reinterpret_cast<float4 *>(buf + n * kRow + e * 2 * nb + (o - (sl ? 2 * nb : 0))) =
+          if (o >= 0 && o < 2 * nb)
+            *reinterpret_cast<float4 *>(dst + o) =
                 make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+          o += 8;
+          if (o >= (sl ? 2 * nb : 4 * nb)) {  // the next state
+            o -= 4 * nb;
+            dst += 2 * nb;
+          }
         }
       }
       __builtin_amdgcn_wave_barrier();
-      for (int e = 0; e < per && e0 + e < ne; ++e)
+      for (int e = 0; e < per && e0 + e < ne; ++e) {
+        double2 *y = Y + (e0 + e) * ld + a0 * nb;
+        int off = (lane / nb) * kRow + 2 * (lane % nb), q = lane % nb;
         for (int i = lane; i < rows; i += 64) {
-          const float *s = buf + (i / nb) * kRow + e * 2 * nb + 2 * (i % nb);
-          Y[(e0 + e) * ld + a0 * nb + i] = make_double2(s[0], s[1]);
+          const float2 s = *reinterpret_cast<const float2 *>(buf + e * 2 * nb + off);
+          y[i] = make_double2(s.x, s.y);
+          off += da * kRow + 2 * dq;
+          q += dq;
+          if (q >= nb) {
+            q -= nb;
+            off += kRow - 2 * nb;
+          }
         }
+      }
       __builtin_amdgcn_wave_barrier();
     }
   }
