@@ -161,30 +161,30 @@ nh_status ensure_part(nh_cnn *c, size_t count) {
 }
 
 template <bool BWD>
-void launch_conv(nh_cnn *c, int gx, int gy, int gz, int ld, const PackSeg &g, bool last,
-                 const float *in, const uint16_t *bias, const float *mask, float *out) {
-  const int seg = conv_segment(gx, gy, gz);
-  const dim3 grid((gz + kConvTZ - 1) / kConvTZ, (gy + kConvTY - 1) / kConvTY,
-                  (gx + seg - 1) / seg);
+void launch_conv(nh_cnn *c, int gx, int gy, int gz, const ConvTile &tile, int ld,
+                 const PackSeg &g, bool last, const float *in, const uint16_t *bias, const float *mask, float *out) {
+  const dim3 grid((gz + tile.tz - 1) / tile.tz * ((gy + tile.ty - 1) / tile.ty),
+                  (gx + tile.seg - 1) / tile.seg);
   const uint4 *W = reinterpret_cast<const uint4 *>(c->packed + g.dst);
   if (BWD || g.ks == 2)
-    hipLaunchKernelGGL((k_conv<2, BWD>), grid, dim3(256), 0, c->ctx->stream, gx, gy, gz, seg,
-                       ld, g.ci0, in, W, bias, last, mask, out);
+    hipLaunchKernelGGL((k_conv<2, BWD>), grid, dim3(256), 0, c->ctx->stream, gx, gy, gz,
+                       tile, ld, g.ci0, in, W, bias, last, mask, out);
   else
-    hipLaunchKernelGGL((k_conv<1, false>), grid, dim3(256), 0, c->ctx->stream, gx, gy, gz, seg,
-                       ld, g.ci0, in, W, bias, last, mask, out);
+    hipLaunchKernelGGL((k_conv<1, false>), grid, dim3(256), 0, c->ctx->stream, gx, gy, gz,
+                       tile, ld, g.ci0, in, W, bias, last, mask, out);
 }
 
 // the conv layers: act[l] for every point
 nh_status forward(nh_cnn *c, int gx, int gy, int gz) {
-  NH_CHECK((gy + kConvTY - 1) / kConvTY <= 65535 && gx <= 65535, NH_ERR_ARG,
+  NH_CHECK((gy + 7) / 8 <= 65535 && gx <= 65535, NH_ERR_ARG,
            "network: grid %d x %d x %d too large", gx, gy, gz);
+  const ConvTile tile = conv_tile(gx, gy, gz);
   const float *src = c->in;
   int ci = c->c_in;
   for (int l = 0; l < c->layers; ++l) {
     const auto &segs = c->fwd_seg[l];
     for (size_t k = 0; k < segs.size(); ++k)
-      launch_conv<false>(c, gx, gy, gz, ci, c->pack.s[segs[k]], k + 1 == segs.size(), src,
+      launch_conv<false>(c, gx, gy, gz, tile, ci, c->pack.s[segs[k]], k + 1 == segs.size(), src,
                          k == 0 ? c->bf + c->b_off[l] : nullptr, nullptr, c->act[l]);
     src = c->act[l];
     ci = c->width;
@@ -239,6 +239,7 @@ nh_status backward(nh_cnn *c, int gx, int gy, int gz, const float *dout) {
   hipLaunchKernelGGL(k_head_bwd_data, dim3(g1(P, 128)), dim3(256), 0, st, P, c->c_out, dout,
                      reinterpret_cast<const uint4 *>(c->packed + c->pack.s[c->headt_seg].dst),
                      c->act[L - 1], c->dpre[0]);
+  const ConvTile tile = conv_tile(gx, gy, gz);
   for (int l = L - 1; l >= 0; --l) {
     const int ci = l == 0 ? c->c_in : W;
     const float *in = l == 0 ? c->in : c->act[l - 1];
@@ -251,7 +252,7 @@ nh_status backward(nh_cnn *c, int gx, int gy, int gz, const float *dout) {
                          gy, gz, ci, cch, c->dpre[0], in, c->part, len);
     sum(cch, len, ci, c->grad + c->w_off[l]);
     if (l > 0) {
-      launch_conv<true>(c, gx, gy, gz, W, c->pack.s[c->bwd_seg[l]], true, c->dpre[0], nullptr,
+      launch_conv<true>(c, gx, gy, gz, tile, W, c->pack.s[c->bwd_seg[l]], true, c->dpre[0], nullptr,
                         c->act[l - 1], c->dpre[1]);
       std::swap(c->dpre[0], c->dpre[1]);
     }

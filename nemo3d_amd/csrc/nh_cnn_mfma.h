@@ -121,20 +121,23 @@ __global__ __launch_bounds__(256) void k_pack_weights(PackList list,
 //            channels: bias, later ones add to out)
 //  BWD       out = sum where mask > 0, else 0 (gradient before the lower
 //            layer's relu; mask: its output)
-// A workgroup keeps 8 (y) x 16 (z) points and walks along x: it stages one
-// plane of inputs at a time in LDS (10 x 18 points, the next plane's loads in
-// flight meanwhile) and adds each plane to the three output planes it touches,
-// so every operand read from LDS feeds three matrix instructions; planes
-// beyond its segment only to the one it needs.  Bound by the FP32 matrix rate;
-// the weights lie in LDS (54 KB), so that two workgroups share a compute unit.
+// A workgroup keeps up to 128 points of a (y, z) plane, a rectangle that suits
+// the grid, and walks along x: it stages one plane of inputs at a time in LDS
+// (the rectangle and the points around it, the next plane's loads in flight
+// meanwhile) and adds each plane to the three output planes it touches, so
+// every operand read from LDS feeds three matrix instructions; planes beyond
+// its segment only to the one it needs.  Bound by the FP32 matrix rate; the
+// weights lie in LDS (54 KB), so that two workgroups share a compute unit.
 // One thread per point with the weights in LDS took 3.74 ms for a layer of
 // 106 x 106 x 71 points (bound by 864 scalar multiply-adds and LDS reads per
-// point and output block), this 0.52 ms.
-constexpr int kConvTY = 8, kConvTZ = 16;
-constexpr int kConvPos = (kConvTY + 2) * (kConvTZ + 2);
+// point and output block), this 0.46 ms (0.52 with rectangles of 8 x 16 only).
+constexpr int kConvPos = 192;  // points of a staged plane at most
+struct ConvTile {
+  int ty, tz, seg;  // ty tz <= 128, (ty + 2) (tz + 2) <= kConvPos
+};
 template <int KS, bool BWD>
 __global__ __launch_bounds__(256, 2) void k_conv(
-    int gx, int gy, int gz, int seg, int ld, int ci0, const float *__restrict__ in,
+    int gx, int gy, int gz, ConvTile tile, int ld, int ci0, const float *__restrict__ in,
     const uint4 *__restrict__ W, const uint16_t *__restrict__ bias, bool relu,
     const float *__restrict__ mask, float *out) {
   constexpr int kOct = 2 * KS;  // groups of 8 channels
@@ -143,11 +146,14 @@ __global__ __launch_bounds__(256, 2) void k_conv(
   // a plane's even, then its odd channels, four at a time
   __shared__ float4 lds[2 * kOct * kConvPos];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = lane >> 5, n = lane & 31;
-  const int z0 = blockIdx.x * kConvTZ, y0 = blockIdx.y * kConvTY;
-  const int x0 = blockIdx.z * seg, x1 = min(x0 + seg, gx);
-  // this lane's output point (column n: y = 2 w + n / 16, z = n % 16)
-  const int ly = 2 * w + (n >> 4), lz = n & 15;
-  const bool mine = y0 + ly < gy && z0 + lz < gz;
+  const int sz = tile.tz + 2, npos = (tile.ty + 2) * sz;  // the staged plane
+  const int ntz = (gz + tile.tz - 1) / tile.tz;
+  const int z0 = blockIdx.x % ntz * tile.tz, y0 = blockIdx.x / ntz * tile.ty;
+  const int x0 = blockIdx.y * tile.seg, x1 = min(x0 + tile.seg, gx);
+  // this lane's output point (column n of wavefront w); idle ones read point 0
+  const bool in_tile = 32 * w + n < tile.ty * tile.tz;
+  const int lp = in_tile ? 32 * w + n : 0, ly = lp / tile.tz, lz = lp % tile.tz;
+  const bool mine = in_tile && y0 + ly < gy && z0 + lz < gz;
   const int64_t plane = (int64_t)gy * gz, pt = (int64_t)(y0 + ly) * gz + z0 + lz;
 
   for (int f = threadIdx.x; f < 27 * KS * 64; f += 256) wlds[f] = W[f];
@@ -162,10 +168,10 @@ __global__ __launch_bounds__(256, 2) void k_conv(
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     const int t = threadIdx.x + 256 * i, pos = t / kOct, q = t % kOct;
-    const int y = y0 - 1 + pos / (kConvTZ + 2), z = z0 - 1 + pos % (kConvTZ + 2);
+    const int y = y0 - 1 + pos / sz, z = z0 - 1 + pos % sz;
     const int c = ci0 + 8 * q;
     off[i] = ((int64_t)y * gz + z) * ld + c;
-    cnt[i] = t < kItems && y >= 0 && y < gy && z >= 0 && z < gz ? ld - c : 0;
+    cnt[i] = pos < npos && y >= 0 && y < gy && z >= 0 && z < gz ? ld - c : 0;
   }
   const bool vec = ld % 4 == 0;
   float nx[kPer][8];
@@ -185,7 +191,7 @@ __global__ __launch_bounds__(256, 2) void k_conv(
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       const int t = threadIdx.x + 256 * i, pos = t / kOct, q = t % kOct;
-      if (t < kItems)
+      if (pos < npos)
 #pragma unroll
         for (int c = 0; c < 2; ++c)
           lds[(c * kOct + q) * kConvPos + pos] =
@@ -213,7 +219,7 @@ __global__ __launch_bounds__(256, 2) void k_conv(
     for (int i = 0; i < 16; ++i) acc[d][i] = 0.0f;
   acc[2] = init(x0);
   // add the staged plane to the output planes d0 .. d1 (x - 1 + d)
-  const float4 *buf = lds + h * kOct * kConvPos + (ly + 1) * (kConvTZ + 2) + lz + 1;
+  const float4 *buf = lds + h * kOct * kConvPos + (ly + 1) * sz + lz + 1;
   auto apply = [&](auto d0, auto d1) {
 #pragma unroll
     for (int dy = -1; dy <= 1; ++dy)
@@ -221,7 +227,7 @@ __global__ __launch_bounds__(256, 2) void k_conv(
       for (int dz = -1; dz <= 1; ++dz)
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-          const float4 *b = buf + dy * (kConvTZ + 2) + dz + 2 * s * kConvPos;
+          const float4 *b = buf + dy * sz + dz + 2 * s * kConvPos;
           const float4 v0 = b[0], v1 = b[kConvPos];
           // output plane x - 1 + d sees this plane at offset 1 - d
           const int k0 = (dy + 1) * 3 + dz + 1;
@@ -273,19 +279,27 @@ __global__ __launch_bounds__(256, 2) void k_conv(
     acc[2] = init(x + 2);
   }
 }
-// x planes per workgroup: the two planes beyond its ends cost a third each;
-// the split of gx that needs the fewest planes in all rounds of 256
-// workgroups (two on a compute unit take twice as long)
-inline int conv_segment(int gx, int gy, int gz) {
-  const int64_t tiles = (int64_t)((gy + kConvTY - 1) / kConvTY) * ((gz + kConvTZ - 1) / kConvTZ);
-  int best = gx;
+// The tile and the x planes of a workgroup: the split that takes the least
+// time, 3 seg + 2 thirds of a plane (the two planes beyond its ends cost a
+// third each), 12 a round of two workgroups on each compute unit, 7 if every
+// workgroup has one for itself (85 x 85 x 57 points: 484 workgroups of 8
+// planes 274 us, 748 of 5 320, 220 of 17 325; 106 x 106 x 71, tiles of 8 x 16
+// / 16 x 8: 490 of 16 planes 516, 504 of 14 461, 252 of 27 509).  Equal ones:
+// the tile with the fewest points around it.
+inline ConvTile conv_tile(int gx, int gy, int gz) {
+  ConvTile best{8, 16, gx};
   int64_t cost = INT64_MAX;
-  for (int n = 1; n <= gx; ++n) {
-    const int seg = (gx + n - 1) / n;
-    const int64_t c = (tiles * ((gx + seg - 1) / seg) + 255) / 256 * (3 * seg + 2);
-    if (c < cost) {
-      cost = c;
-      best = seg;
+  for (int tz = 4; tz <= 32; ++tz) {
+    const int ty = std::min(128 / tz, kConvPos / (tz + 2) - 2);
+    const int64_t tiles = (int64_t)((gy + ty - 1) / ty) * ((gz + tz - 1) / tz);
+    for (int n = 1; n <= gx; ++n) {
+      const int seg = (gx + n - 1) / n;
+      const int64_t w = tiles * ((gx + seg - 1) / seg);
+      const int64_t c = (w <= 256 ? 7 : (w + 511) / 512 * 12) * (3 * seg + 2);
+      if (c < cost || (c == cost && ty + tz < best.ty + best.tz)) {
+        cost = c;
+        best = {ty, tz, seg};
+      }
     }
   }
   return best;

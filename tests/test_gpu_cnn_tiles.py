@@ -1,4 +1,4 @@
-"""The network's matrix-core kernels at the edges of their tiles (8 x 16
+"""The network's matrix-core kernels at the edges of their tiles (up to 128
 points of a plane, x segments, 16 / 32 input channels, 32 / 160 head rows, 64
 gradient channels) against the FP64 oracle, with the bounds of the device
 network's test: FP32 sums, 1e-5 of the largest output, 1e-4 of the largest
@@ -68,6 +68,30 @@ def test_forward_and_gradient(owner, monkeypatch, dims, c_in, layers, c_out):
     assert any(np.abs(g - r).max() <= 1e-4 * np.abs(r).max()
                for r in gradients(monkeypatch, p, feats, dims, dout, shape))
     assert np.array_equal(g, net.grad(feats, dims, dout))  # sums in a fixed order
+
+
+@pytest.mark.parametrize("dims", [(256, 30, 4), (256, 3, 32), (128, 25, 5), (300, 6, 20)])
+def test_tiles_of_other_shapes(owner, dims):
+    """Grids that take narrow, wide and ragged tiles (30 x 4, 3 x 32, ...):
+    two layers forward and backward.  No gradient is put in where a gate
+    within the rounding of its sum could pass it on or not."""
+    print(dims, flush=True)
+    rng = np.random.default_rng(8)
+    shape = dict(c_in=5, width=32, layers=2, c_out=3)
+    P = int(np.prod(dims))
+    feats = rng.normal(size=(P, 5)).astype(np.float32)
+    net = learned.CNN(owner, 5, 32, 2, 3, seed=9)
+    p = net.get_params().astype(np.float64)
+    ref, cache, _ = cnn_oracle.forward(p, feats, dims, keep=True, **shape)
+    assert np.abs(net.forward(feats, dims) - ref).max() <= 1e-5 * np.abs(ref).max()
+    near = [(np.abs(pre) < 5e-6).any(axis=-1) for _, pre in cache]
+    shut = near[1].copy()
+    for x, y, z in np.argwhere(near[0]):
+        shut[max(x - 1, 0):x + 2, max(y - 1, 0):y + 2, max(z - 1, 0):z + 2] = True
+    dout = rng.normal(size=(P, 3)).astype(np.float32)
+    dout[shut.ravel()] = 0.0
+    r = cnn_oracle.backward(p, feats, dims, dout=dout, **shape)
+    assert np.abs(net.grad(feats, dims, dout) - r).max() <= 1e-4 * np.abs(r).max()
 
 
 @pytest.mark.parametrize("bands,ne,targets,device", [
