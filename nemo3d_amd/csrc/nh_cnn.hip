@@ -221,14 +221,17 @@ nh_status backward(nh_cnn *c, int gx, int gy, int gz, const float *dout) {
   const int L = c->layers, W = c->width;
   NH_TRY(ensure_grads(c, P));
   // chunks of points, none smaller than a few lines: as many workgroups as
-  // run at a time (3 a compute unit for the head, 2 for the conv layers with
-  // their nine offsets)
+  // run at a time (4 a compute unit for the head; the conv layers with their
+  // nine offsets 3, up to 16 channels 4: 85 x 85 x 57 points 415 us, with half
+  // as many 445; 225 and 259)
   const int co_tiles = (c->c_out + 63) / 64;
-  const int hch = (int)std::max<int64_t>(1, std::min<int64_t>(P / 256, 768 / co_tiles));
+  const int hch = (int)std::max<int64_t>(1, std::min<int64_t>(P / 256, 1024 / co_tiles));
   const int64_t hlen = (int64_t)c->c_out * (W + 1);
-  const int cch = (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)gx * gy / 8, 56));
+  auto conv_chunks = [&](int ci) {
+    return (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)gx * gy / 8, ci <= 16 ? 113 : 85));
+  };
   const int cmax = std::max((c->c_in + 15) / 16 * 16, W);
-  NH_TRY(ensure_part(c, std::max(hch * hlen, (int64_t)cch * (27 * W * cmax + W))));
+  NH_TRY(ensure_part(c, std::max(hch * hlen, (int64_t)conv_chunks(1) * (27 * W * cmax + W))));
   auto sum = [&](int chunks, int64_t len, int conv_ci, float *grad) {
     hipLaunchKernelGGL(k_grad_sum, dim3((len + 255) / 256), dim3(256), 0, st, chunks, len,
                        conv_ci, c->part, grad);
@@ -244,6 +247,7 @@ nh_status backward(nh_cnn *c, int gx, int gy, int gz, const float *dout) {
     const int ci = l == 0 ? c->c_in : W;
     const float *in = l == 0 ? c->in : c->act[l - 1];
     const int64_t len = 27 * W * (int64_t)((ci + 15) / 16 * 16) + W;
+    const int cch = conv_chunks(ci);
     if (ci <= 16)
       hipLaunchKernelGGL(k_conv_bwd_w<1>, dim3(9 * cch), dim3(256), 0, st, gx, gy, gz, ci,
                          cch, c->dpre[0], in, c->part, len);

@@ -522,18 +522,22 @@ __device__ __forceinline__ void wave_sums(double (&v)[N], double *lds) {
 }
 
 // conv layer: part[chunk][(k * 32 + co) * cp + ci] = sum_p d[p][co] in[p + d_k][ci]
-// (cp = ci_n rounded up to 16), then 32 sums of d (bias).  blockIdx.x: chunk
-// and (dx, dy); blockIdx.y: 16 NT input channels.  A wavefront takes lines of
-// z.  One
-// workgroup per (co, ci) with 27 sums a thread read both arrays 32 times and
-// took 15.9 ms for 85 x 85 x 57 points, this 0.51 ms (0.31 ms at the FP64
-// matrix rate).
+// (cp = ci_n rounded up to 16; sums of channels from ci_n on are not read),
+// then 32 sums of d (bias).  blockIdx.x: chunk and (dx, dy); blockIdx.y: 16 NT
+// input channels.  A wavefront takes lines of z, each of an instruction's four
+// points a quarter of the line: going along it, a point's inputs serve the
+// next two points as well and are loaded and converted once.  One workgroup
+// per (co, ci) with 27 sums a thread read both arrays 32 times and took 15.9 ms
+// for 85 x 85 x 57 points; four neighbouring points an instruction, each input
+// loaded for all three offsets, 0.51 ms; this 0.42 ms (0.31 ms at the FP64
+// matrix rate; two workgroups a compute unit 0.44).
 template <int NT>
-__global__ __launch_bounds__(256, 2) void k_conv_bwd_w(
+__global__ __launch_bounds__(256, 3) void k_conv_bwd_w(
     int gx, int gy, int gz, int ci_n, int chunks, const float *__restrict__ d,
     const float *__restrict__ in, double *__restrict__ part, int64_t len) {
   __shared__ double lds[3 * 2 * NT * 4 * 64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, kz = lane >> 4;
+  const int lane = threadIdx.x & 63, m = lane & 15, kz = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // the nine (dx, dy) of a chunk follow one another on one XCD (workgroups go
   // round robin over 8)
   const int full = chunks / 8 * 72, g = blockIdx.x;
@@ -552,64 +556,108 @@ __global__ __launch_bounds__(256, 2) void k_conv_bwd_w(
     for (int a = 0; a < 2; ++a)
 #pragma unroll
       for (int b = 0; b < NT; ++b) acc[k][a][b] = f64x4{0.0, 0.0, 0.0, 0.0};
-  // eight points of a line (two instructions' worth) are loaded while the
-  // last eight are multiplied
-  struct Eight {
-    float a[2][2], b[2][3][NT];
+  // lane group kz goes over points kz R .. kz R + R - 1 of a line; four points
+  // are loaded while the last four are multiplied
+  const int R = (gz + 3) / 4;
+  struct Four {
+    float a[4][2], b[4][NT];  // gradients of point j0 + s, inputs of the next
+    float b0[2][NT];          // inputs before and at the line's first point
+    int j0;
   };
+  uint32_t bo[NT];  // the lane's place; channels past the last: the last
+  const uint32_t ao = kz * R * kCnnW + m;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) bo[t] = kz * R * ci_n + min(c0 + 16 * t + m, ci_n - 1);
   int64_t l = chunk * per + w;
-  int z0 = 0;
+  int x = l / gy, y = l % gy, j0 = 0;
   const float *dl = nullptr, *il = nullptr;
   auto line = [&] {  // the next line whose neighbour is in the grid
-    for (; l < l1; l += 4) {
-      const int x = l / gy + dx, y = l % gy + dy;
-      if (x < 0 || y < 0 || x >= gx || y >= gy) continue;
-      dl = d + l * gz * kCnnW + m;
-      il = in + ((int64_t)x * gy + y) * gz * ci_n + c0 + m;
-      return;
-    }
-  };
-  auto load = [&](Eight &e) {
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int z = z0 + 4 * s + kz;
-#pragma unroll
-      for (int t = 0; t < 2; ++t) e.a[s][t] = z < gz ? dl[z * kCnnW + 16 * t] : 0.0f;
-#pragma unroll
-      for (int k = 0; k < 3; ++k)
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-          e.b[s][k][t] = z + k - 1 >= 0 && z + k - 1 < gz && c0 + 16 * t + m < ci_n
-                             ? il[(z + k - 1) * ci_n + 16 * t]
-                             : 0.0f;
-    }
-    z0 += 8;
-    if (z0 >= gz) {
-      z0 = 0;
+    while (l < l1 && (x + dx < 0 || y + dy < 0 || x + dx >= gx || y + dy >= gy)) {
       l += 4;
+      for (y += 4; y >= gy; y -= gy) ++x;
+    }
+    dl = d + l * gz * kCnnW;
+    il = in + (l + dx * (int64_t)gy + dy) * gz * ci_n;
+  };
+  auto load = [&](Four &e) {
+    // inputs of point kz R + j, zero outside the line
+    auto edge = [&](int j, float (&v)[NT]) {
+      const int q = kz * R + j, qc = min(max(q, 0), gz - 1) - kz * R;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const float f = il[(int64_t)bo[t] + qc * ci_n];
+        v[t] = q >= 0 && q < gz ? f : 0.0f;
+      }
+    };
+    e.j0 = j0;
+    if (j0 == 0) {
+      edge(-1, e.b0[0]);
+      edge(0, e.b0[1]);
+    }
+    if (3 * R + j0 + 4 < gz) {  // all points and their neighbours in the line
+      const float *pa = dl + j0 * kCnnW, *pb = il + (int64_t)(j0 + 1) * ci_n;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) e.a[s][t] = (pa + s * kCnnW + 16 * t)[ao];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) e.b[s][t] = (pb + s * ci_n)[bo[t]];
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int p = kz * R + j0 + s, pc = min(p, gz - 1);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const float f = dl[pc * kCnnW + 16 * t + m];
+          e.a[s][t] = p < gz ? f : 0.0f;
+        }
+        edge(j0 + s + 1, e.b[s]);
+      }
+    }
+    j0 += 4;
+    if (j0 >= R) {
+      j0 = 0;
+      l += 4;
+      for (y += 4; y >= gy; y -= gy) ++x;
       line();
     }
   };
   line();
-  Eight next;
+  Four next;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) next.b0[0][t] = next.b0[1][t] = 0.0f;
+  double before[NT], here[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) before[t] = here[t] = 0.0;
   bool more = l < l1;
   if (more) load(next);
   while (more) {
-    const Eight e = next;
+    const Four e = next;
     more = l < l1;
     if (more) load(next);
+    if (e.j0 == 0) {
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
+      for (int t = 0; t < NT; ++t) before[t] = e.b0[0][t], here[t] = e.b0[1][t];
+    }
 #pragma unroll
-      for (int t = 0; t < 2; ++t) sb[t] += e.a[s][t];
+    for (int s = 0; s < 4; ++s) {
+      if (e.j0 + s >= R) break;
+      const double da[2] = {e.a[s][0], e.a[s][1]};
 #pragma unroll
-      for (int k = 0; k < 3; ++k)
+      for (int t = 0; t < 2; ++t) sb[t] += da[t];
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+      for (int u = 0; u < NT; ++u) {
+        const double after = e.b[s][u];
 #pragma unroll
-          for (int u = 0; u < NT; ++u)
-            acc[k][t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                (double)e.a[s][t], (double)e.b[s][k][u], acc[k][t][u], 0, 0, 0);
+        for (int t = 0; t < 2; ++t) {
+          acc[0][t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(da[t], before[u], acc[0][t][u], 0, 0, 0);
+          acc[1][t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(da[t], here[u], acc[1][t][u], 0, 0, 0);
+          acc[2][t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(da[t], after, acc[2][t][u], 0, 0, 0);
+        }
+        before[u] = here[u];
+        here[u] = after;
+      }
     }
   }
   double v[3 * 2 * NT * 4];
@@ -652,12 +700,14 @@ __global__ __launch_bounds__(256, 2) void k_conv_bwd_w(
 }
 // head: part[chunk][co * 32 + ci] = sum_p d[p][co] a[p][ci], then co_n sums of
 // d.  blockIdx.y: 64 output channels.  640 channels of 85 x 85 x 57 points:
-// 33.9 ms with a workgroup per channel, 0.37 ms now (0.23 at the matrix rate).
+// 33.9 ms with a workgroup per channel, 0.34 ms now (0.23 at the matrix rate;
+// 0.37 with every address and bound worked out per lane).
 __global__ __launch_bounds__(256, 3) void k_head_bwd_w(
     int64_t P, int co_n, const float *__restrict__ d, const float *__restrict__ act,
     double *__restrict__ part, int64_t len) {
   __shared__ double lds[4 * 2 * 4 * 64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, kp = lane >> 4;
+  const int lane = threadIdx.x & 63, m = lane & 15, kp = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int co0 = blockIdx.y * 64;
   const int64_t per = (P + gridDim.x - 1) / gridDim.x;
   const int64_t p1 = min((blockIdx.x + 1) * per, P);
@@ -673,15 +723,28 @@ __global__ __launch_bounds__(256, 3) void k_head_bwd_w(
     float a[2][4], b[2][2];
   };
   int64_t p0 = blockIdx.x * per + 8 * w;
+  const uint32_t ao = kp * co_n + m, bo = kp * kCnnW + m;  // the lane's place
   auto load = [&](Eight &e) {
+    if (co0 + 64 <= co_n && p0 + 8 <= p1) {
+      // inside: the wavefront's addresses and the lane's place, no tests
+      const float *pa = d + p0 * co_n + co0, *pb = act + p0 * kCnnW;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int64_t p = p0 + 4 * s + kp;
+      for (int s = 0; s < 2; ++s) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        e.a[s][t] = p < p1 && co0 + 16 * t + m < co_n ? d[p * co_n + co0 + 16 * t + m] : 0.0f;
+        for (int t = 0; t < 4; ++t) e.a[s][t] = (pa + 4 * s * (int64_t)co_n + 16 * t)[ao];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) e.b[s][u] = p < p1 ? act[p * kCnnW + 16 * u + m] : 0.0f;
+        for (int u = 0; u < 2; ++u) e.b[s][u] = (pb + 4 * s * kCnnW + 16 * u)[bo];
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int64_t p = p0 + 4 * s + kp;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          e.a[s][t] = p < p1 && co0 + 16 * t + m < co_n ? d[p * co_n + co0 + 16 * t + m] : 0.0f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) e.b[s][u] = p < p1 ? act[p * kCnnW + 16 * u + m] : 0.0f;
+      }
     }
     p0 += 32;
   };
