@@ -88,12 +88,12 @@ WINDOWS = WORKLOADS["dot786k"]["windows"]
 
 def lanczos_memory(n, free_bytes=288e9, k=8):
     """Device bytes of the Lanczos vectors at N = n (SK layout): the
-    eigenvalue pass keeps r_k, r_(k-1) and y in FP64 (+ two FP32 copies of r
-    with FP32 products; with FP32 Lanczos vectors r and u of two steps in
-    FP32 and one FP64 work vector); the eigenvector pass adds the ring of r
-    vectors (2 K FP64 slots, or 2 K FP32 slots with FP32 products; K = 128
-    steps per flush, halved down to 8 until the ring takes at most half the
-    free memory) and the k FP64 eigenvectors."""
+    eigenvalue pass keeps r and u of two steps in the vectors' precision and
+    the FP64 start vector (FP32 products with FP64 vectors: r_k, r_(k-1), y
+    and the start vector, all FP64); the eigenvector pass adds the ring of r
+    vectors (2 K slots in the vectors' precision; K = 128 steps per flush,
+    halved down to 8 until the ring takes at most half the free memory) and
+    the k FP64 eigenvectors."""
     v64, v32 = n * 16, n * 8
 
     def ring(per_step):  # bytes per step of K: two slots
@@ -104,47 +104,43 @@ def lanczos_memory(n, free_bytes=288e9, k=8):
 
     k64, r64 = ring(2 * v64)
     k32, r32 = ring(2 * v32)
-    return {"eigenvalue_pass_fp64_GB": 3 * v64 / 1e9,
-            "eigenvalue_pass_fp32_products_GB": (3 * v64 + 2 * v32) / 1e9,
-            "eigenvector_pass_fp64_GB": (3 * v64 + r64 + k * v64) / 1e9,
+    return {"eigenvalue_pass_fp64_GB": 5 * v64 / 1e9,
+            "eigenvalue_pass_fp32_products_GB": 4 * v64 / 1e9,
+            "eigenvector_pass_fp64_GB": (5 * v64 + r64 + k * v64) / 1e9,
             "eigenvector_pass_fp64_ring_steps": k64,
-            "eigenvector_pass_fp32_products_GB": (3 * v64 + 2 * v32 + r32 + k * v64) / 1e9,
+            "eigenvector_pass_fp32_products_GB": (4 * v64 + r64 + k * v64) / 1e9,
             "eigenvector_pass_fp32_ring_steps": k32,
             "eigenvalue_pass_fp32_vectors_GB": (4 * v32 + v64) / 1e9,
             "eigenvector_pass_fp32_vectors_GB": (4 * v32 + v64 + r32 + k * v64) / 1e9}
 
 
-def sk_lanczos_bytes(M, rec_bytes=8, fp32_copy=False, fp32_vectors=False):
-    """Algorithmic bytes of one fused Lanczos H·v launch of the eigenvalue
-    pass in the SK layout: onsite record (18 doubles) per atom, one 24-value
-    record per bond (each bond once; rec_bytes per value), neighbour and
-    bond indices (4 + 4 int32 per atom), the atom lists, x read once (FP64)
-    and y written once (q is stored only in the eigenvector pass); with
-    FP32 products the neighbours' entries come from the FP32 copy of x
-    (8 bytes per entry, read once).  fp32_vectors: the Lanczos vectors are
-    FP32 and the step is one launch: u_(k-1) and r_(k-1) read once (own
-    entries and neighbours), r_k and u_k written, all FP32."""
-    A = M.n_atoms
+def sk_matrix_bytes(M, rec_bytes):
+    """Bytes of H and its tables in the SK layout, each once: onsite record
+    (18 doubles), list entry and places in the block (4 + 8) per atom, one
+    24-value record (rec_bytes per value) and one list entry per bond."""
     nb = int((M.structure.nbr >= 0).sum()) // 2
-    mat = A * 18 * 8 + nb * 24 * rec_bytes + A * 4 * 4 * 2 + A * 4
-    if fp32_vectors:
-        return mat + M.n * 4 * 8
-    return mat + 2 * M.n * 16 + (M.n * 8 if fp32_copy else 0)
+    return M.n_atoms * (18 * 8 + 4 + 8) + nb * (24 * rec_bytes + 4)
 
 
-def sk_lanczos_vec_bytes(M, rec_bytes=8, fp32_copy=False, fp32_vectors=False):
-    """Algorithmic bytes of one fused H*v launch of the eigenvector pass
-    (SK layout), which also applies the three-term step: the matrix bytes
-    of sk_lanczos_bytes, r_k read once (FP64), r_(k-1) read and r_(k+1)
-    written (FP64); with FP32 products the neighbours' entries come from
-    the FP32 copy of r_k and the FP32 copy of r_(k+1) is written.
-    fp32_vectors: r_k, r_(k-1) read and r_(k+1) written in FP32 only."""
-    A = M.n_atoms
+def mf_matrix_bytes(M):
+    """The same in the matrix-free layout: per bond its two ends (8) and the
+    packed ideal vector (4), per atom also displacement + species (4 doubles)."""
     nb = int((M.structure.nbr >= 0).sum()) // 2
-    mat = A * 18 * 8 + nb * 24 * rec_bytes + A * 4 * 4 * 2 + A * 4
-    if fp32_vectors:
-        return mat + M.n * 3 * 8
-    return mat + 3 * M.n * 16 + (2 * M.n * 8 if fp32_copy else 0)
+    return M.n_atoms * (18 * 8 + 4 + 8 + 4 * 8) + nb * (8 + 4)
+
+
+def lanczos_bytes(M, mat, vec_bytes=16, deferred=True):
+    """Algorithmic bytes of one launch of the eigenvalue pass: the whole step
+    in one launch (deferred: u_(k-1) and r_(k-1) read, r_k and u_k written),
+    or the product alone (FP32 products with FP64 vectors: r_k read, y
+    written; the update is another launch)."""
+    return mat + M.n * vec_bytes * (4 if deferred else 2)
+
+
+def lanczos_vec_bytes(M, mat, vec_bytes=16):
+    """Algorithmic bytes of one launch of the eigenvector pass, which applies
+    the three-term step: r_k, r_(k-1) read, r_(k+1) written."""
+    return mat + M.n * vec_bytes * 3
 
 
 def layout_probe(M, steps=600):
@@ -228,20 +224,6 @@ def cpu_model():
     except OSError:
         pass
     return "unknown"
-
-
-def mf_lanczos_bytes(M, fp32_copy=False, fp32_vectors=False):
-    """Algorithmic bytes of one fused Lanczos H*v launch in the matrix-free
-    layout: onsite record (18 doubles), displacement + species (4 doubles),
-    the packed ideal bond vectors and the neighbour indices (4 + 4 int32)
-    and the list entry per atom, x read once (FP64), y written once, and
-    with FP32 products the FP32 copy of x (read once); fp32_vectors: u_(k-1)
-    and r_(k-1) read, r_k and u_k written, all FP32."""
-    A = M.n_atoms
-    mat = A * (18 * 8 + 4 * 8 + 4 * 4 * 2 + 4)
-    if fp32_vectors:
-        return mat + M.n * 4 * 8
-    return mat + 2 * M.n * 16 + (M.n * 8 if fp32_copy else 0)
 
 
 def cpu_leg(M, matvecs, checks, sample_iters=2):
@@ -471,11 +453,12 @@ def main():
     mf = args.layout == "mf"
     lname = "matrix-free" if mf else "SK"
 
-    def lz_bytes(fp32):
-        if mf:
-            return mf_lanczos_bytes(M, fp32_copy=fp32, fp32_vectors=fp32 and v32)
-        return (sk_lanczos_bytes(M, rec_bytes=4, fp32_copy=True, fp32_vectors=v32) if fp32
-                else sk_lanczos_bytes(M))
+    def mat_bytes(fp32):
+        return mf_matrix_bytes(M) if mf else sk_matrix_bytes(M, 4 if fp32 else 8)
+
+    def lz_bytes(fp32):  # eigenvalue pass, eigenvector pass
+        m, vb = mat_bytes(fp32), 8 if fp32 and v32 else 16
+        return lanczos_bytes(M, m, vb, not fp32 or v32), lanczos_vec_bytes(M, m, vb)
 
     # the two fused H*v kernels of the headline form (eigenvalue pass and
     # eigenvector pass, which also applies the three-term step); `roofline`
@@ -483,17 +466,18 @@ def main():
     if mixed is not None:
         st = mixed["stage32"]
         prec, p32 = "FP32 products", True
-        passes = [("eigenvalue pass", lz_bytes(True), st["hv_ms"], st["iterations"],
-                   None if mf else "k_lz_hv_sk_fp32" + ("_v32" if v32 else "")),
-                  ("eigenvector pass", None if mf else sk_lanczos_vec_bytes(M, 4, True, v32),
-                   st["hv_ms_vec"], st["matvecs"] - st["iterations"],
-                   None if mf else "k_lz_hv_sk_fp32_vec" + ("_v32" if v32 else ""))]
+        bp = lz_bytes(True)
+        key = "k_lz_sk_fp32" if v32 and not mf else None
+        passes = [("eigenvalue pass", bp[0], st["hv_ms"], st["iterations"], key),
+                  ("eigenvector pass", bp[1], st["hv_ms_vec"],
+                   st["matvecs"] - st["iterations"], key and key + "_vec")]
     else:
         prec, p32 = "FP64", False
-        passes = [("eigenvalue pass", lz_bytes(False), plain["hv_ms"], plain["iterations"],
-                   None if mf else "k_lz_hv_sk"),
-                  ("eigenvector pass", None if mf else sk_lanczos_vec_bytes(M),
-                   plain["hv_ms_vec"], plain["matvecs"] - plain["iterations"], None)]
+        bp = lz_bytes(False)
+        key = None if mf else "k_lz_sk"
+        passes = [("eigenvalue pass", bp[0], plain["hv_ms"], plain["iterations"], key),
+                  ("eigenvector pass", bp[1], plain["hv_ms_vec"],
+                   plain["matvecs"] - plain["iterations"], key and key + "_vec")]
     rooflines = []
     for pname, b, ms, launches, tk in passes:
         if b is None or not ms:
@@ -501,10 +485,12 @@ def main():
         ach = b / (ms * 1e-3) / 1e9
         rooflines.append({
             "bound": "hbm",
-            "kernel": "k_lz_hv_sk<2,%s%s%s> (fused Lanczos H*v, %s, %s %s%s)" % (
-                "float" if p32 else "double", ",FUSE" if pname == "eigenvector pass" else "",
-                ",float2" if (p32 and v32) else "", pname, lname, prec,
-                ", FP32 Lanczos vectors" if (p32 and v32) else ""),
+            "kernel": "k_lz_sk<%s,2,%s,%s> (fused Lanczos H*v, %s, %s %s%s)" % (
+                ("kLzValues" if v32 or not p32 else "kLzProduct")
+                if pname == "eigenvalue pass" else
+                ("kLzVectors" if v32 or not p32 else "kLzFused"),
+                "float" if p32 else "double", "float2" if (p32 and v32) else "double2",
+                pname, lname, prec, ", FP32 Lanczos vectors" if (p32 and v32) else ""),
             "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": ach / HBM_PEAK_GBS,
             # measured (PMC) on the default workload only
@@ -533,13 +519,13 @@ def main():
     if len(rooflines) > 1:
         line["roofline_other_pass"] = rooflines[1]
     if plain is not None:
-        pb = lz_bytes(False)
+        pb = lz_bytes(False)[0]
         line["roofline_plain"] = {
-            "kernel": "k_lz_hv_sk<2,double> (fused Lanczos H*v, %s FP64)" % lname,
+            "kernel": "k_lz_sk<kLzValues,2,double,double2> (fused Lanczos step, %s FP64)" % lname,
             "achieved": pb / (plain["hv_ms"] * 1e-3) / 1e9 if plain["hv_ms"] > 0 else 0.0,
             "peak": HBM_PEAK_GBS, "unit": "GB/s", "bytes_per_launch": pb,
             "launch_ms": plain["hv_ms"],
-            "traffic": traffic_from_profiles("k_lz_hv_sk")
+            "traffic": traffic_from_profiles("k_lz_sk")
             if (args.workload == "dot786k" and not mf) else None}
         line["roofline_plain"]["frac"] = line["roofline_plain"]["achieved"] / HBM_PEAK_GBS
     if args.workload != "dot786k":

@@ -303,7 +303,7 @@ __global__ void k_mf_ends(int n, const int32_t *__restrict__ bonds,
 }
 
 // Per (cation, anion) species pair: integrals 10..30, strain exponents
-// 0..14, lattice constant (the parameters k_bond reads).
+// 0..14, lattice constant (the parameters k_assemble reads).
 __global__ void k_mf_pair(int S, const double *__restrict__ parmat,
                           const double *__restrict__ strnmat,
                           double *__restrict__ pair) {

@@ -364,9 +364,8 @@ def eigensolve_mixed_block(H, block_size=8, num_vb=4, num_cb=4, erange_vb=(-0.6,
                            stage2="block", hnorm=40.0, refine_depth=12,
                            refine_rounds=4, deflation=False):
     """Mixed-precision block Lanczos: the bulk iterations with FP32 H·V
-    (FP32 values, FP32 products inside each block; on the matrix cores for
-    a block of 8) and FP64 recurrences, dots and Ritz solves, to an
-    FP32-level tolerance `tol32`; then, stage2 = "block", FP64 block
+    (FP32 values, FP32 products inside each block) and FP64 recurrences,
+    dots and Ritz solves, to an FP32-level tolerance `tol32`; then, stage2 = "block", FP64 block
     Lanczos started from those Ritz vectors to `tol`, with FP64 Rayleigh
     quotients and residuals, or, stage2 = "refine", the FP64 residual
     refinement of eigensolve_mixed (refine_eigenpairs per side of the gap,
