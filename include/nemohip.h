@@ -90,9 +90,9 @@ enum { NH_SET_HV_STAGED = 1 };
  * halved down to 8 until the ring takes at most half the free memory.
  * The eigenvectors agree to rounding whatever the length. */
 enum { NH_SET_RING_STEPS = 2 };
-/* NH_SET_BLOCK_HV: products of several vectors (block H·V): 0 one column per
- * grid row, else (-1, the default, 1 or 2) all columns in one launch with H
- * read once, the fastest measured in every layout and precision. */
+/* NH_SET_BLOCK_HV: products of several vectors (block H·V): -1 (default) as
+ * many columns to a workgroup, with H read once, as leave the chip full; 0 one
+ * column, 1 or 2 all columns. */
 enum { NH_SET_BLOCK_HV = 3 };
 /* NH_SET_SK_ROLES, NH_SET_SK_LANES: workgroup mappings of earlier SK and
  * matrix-free products; accepted and without effect (one mapping is the

@@ -292,8 +292,8 @@ inline ConvTile conv_tile(int gx, int gy, int gz) {
   for (int tz = 4; tz <= 32; ++tz) {
     const int ty = std::min(128 / tz, kConvPos / (tz + 2) - 2);
     const int64_t tiles = (int64_t)((gy + ty - 1) / ty) * ((gz + tz - 1) / tz);
-    for (int n = 1; n <= gx; ++n) {
-      const int seg = (gx + n - 1) / n;
+    for (int n = 1, seg; n <= gx; n = seg > 1 ? (gx + seg - 2) / (seg - 1) : gx + 1) {
+      seg = (gx + n - 1) / n;
       const int64_t w = tiles * ((gx + seg - 1) / seg);
       const int64_t c = (w <= 256 ? 7 : (w + 511) / 512 * 12) * (3 * seg + 2);
       if (c < cost || (c == cost && ty + tz < best.ty + best.tz)) {

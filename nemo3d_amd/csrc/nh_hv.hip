@@ -1,5 +1,7 @@
 // Sparse H·v and block H·V for the stored-block layout (row computation
 // in nh_hv_row.h).
+#include <algorithm>
+
 #include "nh_hv_row.h"
 #include "nh_hv_sk.h"
 
@@ -68,22 +70,23 @@ __global__ __launch_bounds__(kSkThreads, 2) void k_hv_sk(
   }
 }
 
-// A column per grid row, or (COLS) nc columns: the blocks are read once for all
-// of them and stay in registers (104,976 atoms, 8 columns, FP64: XX us, a column
-// per grid row YY).
+// A column per grid row, or (COLS) `per`: the blocks are read once for all of
+// them and stay in registers (104,976 atoms, 8 columns, FP64: 424 us, a column
+// per grid row 720).
 template <bool COLS, int NSP, typename TB, typename TA>
 __global__ __launch_bounds__(kThreads, COLS ? 2 : 3) void k_hv_blocks(
     int A, const double *__restrict__ onsite, const TB *__restrict__ blocks,
     const int32_t *__restrict__ nbr, double shift,
-    const double2 *__restrict__ x, double2 *__restrict__ y, int64_t ld, int nc) {
+    const double2 *__restrict__ x, double2 *__restrict__ y, int64_t ld, int ncol, int per) {
   constexpr int NB = NSP * 10;
   __shared__ RowLds<NSP, TB> L[kThreads / 64];
   const int wave = threadIdx.x >> 6;
   const int a0 = (blockIdx.x * (kThreads / 64) + wave) * kRowAtoms;
   if (a0 >= A) return;
   const Rows<NSP, TB> rows(a0, A, blocks, nbr);
-  const int64_t c0 = COLS ? 0 : blockIdx.y;
-  for (int c = 0; c < (COLS ? nc : 1); ++c) {
+  const int64_t c0 = COLS ? blockIdx.y * (int64_t)per : blockIdx.y;
+  const int nc = COLS ? min(per, (int)(ncol - c0)) : 1;
+  for (int c = 0; c < nc; ++c) {
     double acc_re[NSP], acc_im[NSP];
     double2 xi[NSP];
     rows.template apply<TA>(onsite, shift, x + (c0 + c) * ld, L[wave], acc_re, acc_im, xi);
@@ -95,6 +98,20 @@ __global__ __launch_bounds__(kThreads, COLS ? 2 : 3) void k_hv_blocks(
   }
 }
 
+// Columns of a workgroup (mode: NH_SET_BLOCK_HV).  All of them, H read once,
+// where the `groups` workgroups of one column fill the chip (`slots` run at a
+// time); fewer where they do not: each further column costs a workgroup about
+// 3 us, one beside it nothing while the chip has room (SK, FP64, 8 columns:
+// 1,000 atoms 39.5 us all / 17.9 one, 11,520 atoms 42.3 / 36.7, 24,576 atoms
+// 56 / 58, 108,160 atoms 180 / 220; stored blocks 39 / 20, 56 / 77, 95 / 152,
+// 417 / 722).
+int hv_columns(int mode, int groups, int slots, int ncol) {
+  if (ncol == 1 || mode == 0) return 1;
+  if (mode > 0) return ncol;
+  const int rows = std::min(ncol, std::max(1, slots / groups));
+  return (ncol + rows - 1) / rows;
+}
+
 }  // namespace
 
 nh_status launch_hv(nh_context *c, double shift, const nh_cplx *x, nh_cplx *y,
@@ -103,28 +120,29 @@ nh_status launch_hv(nh_context *c, double shift, const nh_cplx *x, nh_cplx *y,
            "H·v: Hamiltonian not built in a supported layout");
   NH_CHECK(ncol >= 1 && ncol <= 65535 && ld >= c->n, NH_ERR_ARG,
            "H·V: bad ncol %d / ld %lld", ncol, (long long)ld);
-  // block products: all the columns in one launch with H read once, measured
-  // fastest for 2 columns and more (SK and matrix-free, 395,136 atoms, 8
-  // columns, FP64: 0.65 ms against 0.83 / 1.06 with a column per grid row;
-  // stored blocks, 104,976 atoms, 8 columns: 424 us FP64, 331 FP32 against 720
-  // and 416; FP32 matrix instructions, a wavefront per atom and 8 columns: 519)
+  // block products: several columns of a workgroup with H read once (SK and
+  // matrix-free, 395,136 atoms, 8 columns, FP64: 0.65 ms against 0.83 / 1.06
+  // with a column per grid row; stored blocks, 104,976 atoms, 8 columns: 424 us
+  // FP64, 331 FP32 against 720 and 416; FP32 matrix instructions, a wavefront
+  // per atom and 8 columns: 519)
   const int mode = c->block_hv;
   if (sk_like(c)) {
     const SkTable tab = sk_table_of(c);
     const double2 *xd = reinterpret_cast<const double2 *>(x);
     double2 *yd = reinterpret_cast<double2 *>(y);
-    const bool cols = ncol > 1 && mode != 0;
+    const int per = hv_columns(mode, std::max(1, c->n_blocks), 512, ncol);
+    const bool cols = per > 1;
     // one block per workgroup; the matrix-free product of one vector is
     // faster with as many workgroups as run at a time, their next tables read
     // ahead (786,520 atoms, FP64: 0.273 against 0.292 ms; SK 0.243 / 0.232)
     const bool walk = c->layout == NH_LAYOUT_MATRIX_FREE && !cols;
-    const dim3 g(walk ? sk_grid(c, 2) : sk_grid(c, 1 << 20), cols ? 1 : ncol);
+    const dim3 g(walk ? sk_grid(c, 2) : sk_grid(c, 1 << 20), (ncol + per - 1) / per);
 #define SKL(NSP, R, SRC)                                                       \
   do {                                                                         \
     if (cols)                                                                  \
       hipLaunchKernelGGL((k_hv_sk<true, NSP, R, decltype(SRC)>), g,            \
                          dim3(kSkThreads), 0, c->stream, tab, c->onsite, SRC,  \
-                         shift, xd, yd, ld, ncol, ncol);                       \
+                         shift, xd, yd, ld, ncol, per);                        \
     else                                                                       \
       hipLaunchKernelGGL((k_hv_sk<false, NSP, R, decltype(SRC)>), g,           \
                          dim3(kSkThreads), 0, c->stream, tab, c->onsite, SRC,  \
@@ -148,8 +166,10 @@ nh_status launch_hv(nh_context *c, double shift, const nh_cplx *x, nh_cplx *y,
     NH_HIP(hipGetLastError());
     return NH_OK;
   }
-  const bool cols = ncol > 1 && mode != 0;
-  const dim3 grid((c->n_atoms + kAtomsPerBlock - 1) / kAtomsPerBlock, cols ? 1 : ncol);
+  const int groups = (c->n_atoms + kAtomsPerBlock - 1) / kAtomsPerBlock;
+  const int per = hv_columns(mode, groups, 768, ncol);
+  const bool cols = per > 1;
+  const dim3 grid(groups, (ncol + per - 1) / per);
   const double2 *xd = reinterpret_cast<const double2 *>(x);
   double2 *yd = reinterpret_cast<double2 *>(y);
 #define HVB(NSP, TB, TA, BLK)                                                  \
@@ -157,11 +177,11 @@ nh_status launch_hv(nh_context *c, double shift, const nh_cplx *x, nh_cplx *y,
     if (cols)                                                                \
       hipLaunchKernelGGL((k_hv_blocks<true, NSP, TB, TA>), grid,             \
                          dim3(kThreads), 0, c->stream, c->n_atoms, c->onsite, \
-                         BLK, c->nbr, shift, xd, yd, ld, ncol);              \
+                         BLK, c->nbr, shift, xd, yd, ld, ncol, per);         \
     else                                                                     \
       hipLaunchKernelGGL((k_hv_blocks<false, NSP, TB, TA>), grid,            \
                          dim3(kThreads), 0, c->stream, c->n_atoms, c->onsite, \
-                         BLK, c->nbr, shift, xd, yd, ld, 1);                 \
+                         BLK, c->nbr, shift, xd, yd, ld, ncol, 1);           \
   } while (0)
   if (c->precision == NH_PREC_FP64) {
     if (c->nb == 20) HVB(2, double, double, c->blocks64);

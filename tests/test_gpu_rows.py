@@ -45,3 +45,31 @@ def test_lanczos_on_rows(cells):
     a, b = device_tridiagonal(H, q, 12)
     ar, br = tridiagonal(H, q, 12)
     assert np.abs(a - ar).max() < 1e-9 and np.abs(b - br).max() < 1e-9
+
+
+@pytest.mark.parametrize("precision", [native.PREC_FP64, native.PREC_FP32])
+@pytest.mark.parametrize("layout", [native.LAYOUT_BLOCKS, native.LAYOUT_SK,
+                                    native.LAYOUT_MATRIX_FREE])
+def test_columns_shared_out(layout, precision):
+    """11 columns of a box whose blocks do not fill the chip: the workgroups
+    take two or three columns each, the last ones fewer; the products are
+    those of a column per workgroup (the same operations) and of all columns
+    in one, padding untouched."""
+    M = _models.gaas_box(cells=(9, 8, 6), strain_nm=0.01, seed=3)
+    print("atoms", M.n_atoms, layout, precision, flush=True)
+    H = Hamiltonian(M, layout=layout, precision=precision)
+    n, ld, k = H.n, H.n + 8, 11
+    X = np.zeros((k, ld), dtype=np.complex128)
+    X[:, :n] = _models.random_vectors(n, k, seed=4)
+    dX = native.DeviceArray.from_host(H, X)
+    out = []
+    for mode in (0, 1, -1):
+        H.set(native.SET_BLOCK_HV, mode)
+        dY = native.DeviceArray.from_host(H, np.full((k, ld), 2.0 + 5.0j))
+        native.check(native.load().nh_hV(H.ctx, 0.3, native.ptr(dX), native.ptr(dY),
+                                         k, ld, native.PTR_DEVICE))
+        out.append(dY.download())
+    assert np.all(out[2][:, n:] == 2.0 + 5.0j)
+    for Y in out[1:]:
+        err = np.linalg.norm(Y[:, :n] - out[0][:, :n]) / np.linalg.norm(out[0][:, :n])
+        assert err <= (1e-15 if precision == native.PREC_FP64 else 1e-7)
