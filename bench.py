@@ -230,7 +230,7 @@ def cpu_leg(M, matvecs, checks, sample_iters=2):
     """The oracle (C restatement of the reference's assembly, H*v and
     Lanczos recurrence) on the host: assembly plus `sample_iters` Lanczos
     iterations of the same Hamiltonian, on 1 thread and on every host
-    thread, scaled to the plain solve's H*v count; and, as the checker,
+    thread, scaled to the plain solve's H*v count; and, as a check,
     the FP64 residual and Rayleigh quotient of each GPU eigenpair in
     `checks` ({form: (eigenvalues, vectors)}) under the oracle's operator."""
     from oracle import oracle
