@@ -160,6 +160,26 @@ __device__ __forceinline__ double quad_sum(double v) {
 }
 // Partial sums of a gradient, per workgroup: E, |grad|^2, grad.dir, grad.old
 constexpr int kVffSums = 4;
+// The sums over a workgroup of kRedThreads, in a fixed order, in every thread;
+// s: kVffSums * kRedThreads / 64 doubles.  Each sum has its own part of s, so
+// one barrier does for all of them (sums taken one after another through the
+// same part would need a second one between a sum's read and the next's write)
+__device__ __forceinline__ void vff_block_sums(double (&v)[kVffSums], double *s) {
+  constexpr int kWaves = kRedThreads / 64;
+#pragma unroll
+  for (int k = 0; k < kVffSums; ++k) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
+    if ((threadIdx.x & 63) == 0) s[k * kWaves + (threadIdx.x >> 6)] = v[k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kVffSums; ++k) {
+    v[k] = s[k * kWaves];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) v[k] += s[k * kWaves + w];
+  }
+}
 // Gradient of E at pos (x, y, z, and the species in w) with the sums over it;
 // dir, old: null for 0; st: the descent's state (null: none), nothing is done
 // when it is over.  Bound by the latency of dependent gathers (neighbours,
@@ -291,8 +311,8 @@ __global__ __launch_bounds__(kRedThreads) void k_vff_grad(
       if (old) sum[3] += v * old[o];
     }
   }
-#pragma unroll
-  for (int k = 0; k < kVffSums; k += 2) block_sum2(sum[k], sum[k + 1]);
+  __shared__ double scratch[kVffSums * kRedThreads / 64];
+  vff_block_sums(sum, scratch);
   if (threadIdx.x == 0)
 #pragma unroll
     for (int k = 0; k < kVffSums; ++k) part[kVffSums * blockIdx.x + k] = sum[k];
@@ -301,28 +321,15 @@ __global__ __launch_bounds__(kRedThreads) void k_vff_grad(
 namespace {
 
 // sums of the workgroups' partials, in a fixed order, in every thread of a
-// workgroup of kRedThreads; s: kVffSums * kRedThreads / 64 doubles
+// workgroup of kRedThreads; s as in vff_block_sums
 __device__ __forceinline__ void vff_sums(int nparts, const double *__restrict__ part, double *s,
                                          double (&v)[kVffSums]) {
-  constexpr int kWaves = kRedThreads / 64;
 #pragma unroll
   for (int k = 0; k < kVffSums; ++k) v[k] = 0.0;
   for (int p = threadIdx.x; p < nparts; p += kRedThreads)
 #pragma unroll
     for (int k = 0; k < kVffSums; ++k) v[k] += part[kVffSums * p + k];
-#pragma unroll
-  for (int k = 0; k < kVffSums; ++k) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
-    if ((threadIdx.x & 63) == 0) s[k * kWaves + (threadIdx.x >> 6)] = v[k];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < kVffSums; ++k) {
-    v[k] = s[k * kWaves];
-#pragma unroll
-    for (int w = 1; w < kWaves; ++w) v[k] += s[k * kWaves + w];
-  }
+  vff_block_sums(v, s);
 }
 
 // positions of displacements u (atoms' species in w)
