@@ -53,13 +53,17 @@ __host__ __device__ constexpr int pair_integral(int sa, int sc, int part) {
          : sa == 3 && sc == 3 ? 18 + part : -1;
 }
 // Weights of the squared sigma, pi and delta integrals in the sum of squares
-// over a row of a shell pair (row: p or d orbital; the same whatever the
-// other shell, which only lacks the later ones)
+// over a row of a shell pair, for the true sqrt 3; then what the reference's
+// literal s changes of it (1e-12 relative): its first four d functions in s-d
+// and p-d and its z2 entries of p-d pi and d-d are s / sqrt 3 times as large, so that
+// a sum over the other shell's d functions gains k = s^2 / 3 - 1 times the
+// squares of those entries (the products of sigma and pi still add up to 0).
 struct RowWeights {
-  double p[3], ds[5], dp[5], dd[5];
+  static constexpr double k = kSqrt3Ref * kSqrt3Ref / 3.0 - 1.0;
+  double p[3], ds[5], dp[5], dd[5], z;
   __device__ __forceinline__ RowWeights(double l, double m, double n) {
-    const double l2 = l * l, m2 = m * m, n2 = n * n, dl = l2 - m2, lpm = l2 + m2,
-                 z = n2 - 0.5 * lpm;
+    const double l2 = l * l, m2 = m * m, n2 = n * n, dl = l2 - m2, lpm = l2 + m2;
+    z = n2 - 0.5 * lpm;
     p[0] = l2, p[1] = m2, p[2] = n2;
     ds[0] = 3.0 * l2 * m2, ds[1] = 3.0 * m2 * n2, ds[2] = 3.0 * n2 * l2;
     ds[3] = 0.75 * dl * dl, ds[4] = z * z;
@@ -68,12 +72,33 @@ struct RowWeights {
     dd[0] = n2 + l2 * m2, dd[1] = l2 + m2 * n2, dd[2] = m2 + n2 * l2;
     dd[3] = n2 + 0.25 * dl * dl, dd[4] = 0.75 * lpm * lpm;
   }
-  // sum over the row of orbital o (0..9) with the squares of a shell pair
-  template <int O>
-  __device__ __forceinline__ double row(double s, double pi, double delta) const {
-    if constexpr (O < 2) return s;
-    else if constexpr (O < 5) return p[O - 2] * s + (1.0 - p[O - 2]) * pi;
-    else return ds[O - 5] * s + dp[O - 5] * pi + dd[O - 5] * delta;
+  // sum over the row of orbital O (0..9) with shell X, q the squares of the
+  // pair's integrals
+  template <int O, int X>
+  __device__ __forceinline__ double row(const double (&q)[3]) const {
+    const double s3 = X == 3 ? 1.0 + k * (1.0 - ds[4]) : 1.0;
+    if constexpr (O < 2) {
+      return s3 * q[0];
+    } else if constexpr (O < 5) {
+      const double a = p[O - 2], w = O < 4 ? p[2] : 1.0 - p[2];
+      return (a * s3) * q[0] + (1.0 - a + (X == 3 ? 3.0 * k * a * w * w : 0.0)) * q[1];
+    } else if constexpr (X == 3) {
+      return ds[O - 5] * q[0] + dp[O - 5] * q[1] + dd[O - 5] * q[2];
+    } else {
+      return (O < 9 ? 1.0 + k : 1.0) * ds[O - 5] * q[0] +
+             (O == 9 ? 1.0 + k : 1.0) * dp[O - 5] * q[1];
+    }
+  }
+  // the literal's part of the d-d rows
+  __device__ __forceinline__ void add_dd(double dds, double ddp, double ddd,
+                                         double (&r)[5]) const {
+    const double y = z * dds - 2.0 * p[2] * ddp + 0.5 * (1.0 + p[2]) * ddd;
+    const double w = z * dds + (1.0 - 2.0 * p[2]) * ddp - 0.5 * (1.0 - p[2]) * ddd;
+    const double y2 = k * y * y, w2 = k * w * w;
+    const double e[4] = {ds[0] * y2, ds[1] * w2, ds[2] * w2, ds[3] * y2};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) r[c] += e[c];
+    r[4] += (e[0] + e[1]) + (e[2] + e[3]);
   }
 };
 
@@ -180,11 +205,21 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(AssembleArgs g) {
         q[part] = x * x;
         q0[part] = x0 * x0;
       }
+      double lit[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+      if constexpr (so == 3 && sx == 3) {
+        double less[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        w0.add_dd(par[P_DDS], par[P_DDP], par[P_DDD], lit);
+        w.add_dd(v[18], v[19], v[20], less);
+#pragma unroll
+        for (int c = 0; c < 5; ++c) lit[c] -= less[c];
+      }
       auto add = [&](auto O) {
         constexpr int o = O;
-        if constexpr (shell_of(o) == so)
-          corr[o] += (w0.template row<o>(q0[0], q0[1], q0[2]) -
-                      w.template row<o>(q[0], q[1], q[2])) * f;
+        if constexpr (shell_of(o) == so) {
+          double dif = w0.template row<o, sx>(q0) - w.template row<o, sx>(q);
+          if constexpr (so == 3 && sx == 3) dif += lit[o - 5];
+          corr[o] += dif * f;
+        }
       };
       static_for<10>(add);
     };
