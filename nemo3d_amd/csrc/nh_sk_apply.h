@@ -11,10 +11,15 @@
 //   d-d        ddd d + B M^T(n w) + A' sd (sd.d), B = ddp - ddd,
 //              A' = dds - ddd - (4/3) B
 // (M^T(n w): the five components of the symmetric product of n and w).
-// sqrt 3 is the reference's literal, placed so that what its 6.5e-13 error
-// still changes against sk_table is proportional to n^2 - (l^2 + m^2)/2,
-// which vanishes on an unstrained bond.
-// That is 93 multiply-adds per vector and about 40 operations per bond for
+// The identities behind these forms hold for the true sqrt 3; the table has
+// the reference's literal s (6.5e-13 off), in the first four d functions and
+// in M's z2 part.  What that changes is linear in z = n^2 - (l^2 + m^2)/2, the
+// fifth d function: in FP64 the z2 column of p-d has (2 s / 3) in the place of
+// (2 / s) and the z2 row and column of A' sd sd^T the factor s^2 / 3, added as
+// kz (relative to the table in 80 bits, directions 0.002 / 0.01 / 0.03 off
+// (111): 1.4e-15 / 7.0e-15 / 2.1e-14 without, 2.0e-16 with them; the table in
+// FP64 1.5e-16).
+// That is about 95 multiply-adds per vector and about 40 operations per bond for
 // the scaled vectors, against 100 and about 250 for forming T.
 //
 // Every matrix element is a sum of products of two numbers that are
@@ -112,17 +117,21 @@ __host__ __device__ __forceinline__ void sk_apply(const R *k, const R (&x)[10], 
   const R wx = sk_fma(n, d[2], sk_fma(m, d[0], sk_fma(-kl, d[4], l * d[3])));
   const R wy = sk_fma(n, d[1], sk_fma(l, d[0], sk_fma(-km, d[4], -(m * d[3]))));
   const R wz = sk_fma(m, d[1], sk_fma(l, d[2], kn * d[4]));
-  // p rows: ppp p + pdp w, then n (...), then the p-p projection
-  R te = (apd * g[0]) * d[0];
-#pragma unroll
-  for (int c = 1; c < 5; ++c) te = sk_fma(apd * g[c], d[c], te);
-  const R cp = sk_fma(ps, x[1], sk_fma(pt, x[0], te));
+  // the literal's part (none in FP32): p-d z2 column, d-d z2 row and column
+  constexpr bool kExact = sizeof(R) == 8;
+  constexpr R s2m3 = R(kSqrt3Ref * kSqrt3Ref - 3.0);
+  const R kz = kExact ? (-(R(2) / R(3)) * s2m3 / s3) * g[4] : R(0);
+  const R e4 = kExact ? ((s2m3 / R(3)) * g[4]) * da : R(0);
+  // p rows: ppp p + pdp w, then along n, along A n, then the p-p projection
+  R cp = sk_fma(ps, x[1], pt * x[0]);
+  if constexpr (kExact) cp = sk_fma(kz * pdp, d[4], cp);
+  const R al = apd * l, am = apd * m, an = apd * n;
   const R cl = ppc * l, cm = ppc * m, cn = ppc * n;
   R sc;
   if constexpr (CATION) sc = sk_fma(cn, p[2], sk_fma(cm, p[1], cl * p[0]));
-  y[2] = sk_fma(l, cp, sk_fma(pdp, wx, sk_fma(ppp, p[0], y[2])));
-  y[3] = sk_fma(m, cp, sk_fma(pdp, wy, sk_fma(ppp, p[1], y[3])));
-  y[4] = sk_fma(n, cp, sk_fma(pdp, wz, sk_fma(ppp, p[2], y[4])));
+  y[2] = sk_fma(al, t, sk_fma(l, cp, sk_fma(pdp, wx, sk_fma(ppp, p[0], y[2]))));
+  y[3] = sk_fma(am, t, sk_fma(m, cp, sk_fma(pdp, wy, sk_fma(ppp, p[1], y[3]))));
+  y[4] = sk_fma(an, t, sk_fma(n, cp, sk_fma(pdp, wz, sk_fma(ppp, p[2], y[4]))));
   if constexpr (CATION) {
     y[2] = sk_fma(l, sc, y[2]);
     y[3] = sk_fma(m, sc, y[3]);
@@ -165,8 +174,9 @@ __host__ __device__ __forceinline__ void sk_apply(const R *k, const R (&x)[10], 
     y9 = sk_fma(-km, hy, sk_fma(-kl, hx, sk_fma(kn, hz, y9)));
     y9 = sk_fma(-kbm, wy, sk_fma(-kbl, wx, sk_fma(kbn, wz, y9)));
   }
-  // sd (xs, x_s* parts), A sd (n.p), A' sd (sd.d)
-  const R cs = sk_fma(ds, x[1], dt * x[0]);
+  // sd (xs, x_s* parts, A n.p), A' sd (sd.d)
+  const R sq = sk_fma(adp * n, p[2], sk_fma(adp * m, p[1], (adp * l) * p[0]));
+  const R cs = sk_fma(ds, x[1], sk_fma(dt, x[0], sq));
   R ta;
   if constexpr (CATION) {
     ta = (da * g[0]) * d[0];
@@ -175,12 +185,15 @@ __host__ __device__ __forceinline__ void sk_apply(const R *k, const R (&x)[10], 
   } else {
     ta = t;
   }
-  R yd[5] = {y5, y6, y7, y8, y9};
+  const R cs4 = kExact ? sk_fma(e4, d[4], cs) : cs;
+  if constexpr (kExact) y9 = sk_fma(kz * dpp, s, y9);
+  const R yd[4] = {y5, y6, y7, y8};
 #pragma unroll
-  for (int c = 0; c < 5; ++c) {
-    const R e = adp * g[c], a = CATION ? g[c] : da * g[c];
-    y[5 + c] = sk_fma(a, ta, sk_fma(e, s, sk_fma(g[c], cs, yd[c])));
-  }
+  for (int c = 0; c < 4; ++c)
+    y[5 + c] = sk_fma(CATION ? g[c] : da * g[c], ta, sk_fma(g[c], cs4, yd[c]));
+  y9 = sk_fma(g[4], cs, y9);
+  if constexpr (kExact) y9 = sk_fma(e4, t, y9);
+  y[9] = sk_fma(CATION ? g[4] : da * g[4], ta, y9);
 }
 
 }  // namespace nh
