@@ -361,6 +361,24 @@ __global__ void k_convert(int64_t n, const double *__restrict__ src,
     dst[k] = T(src[k]);
 }
 
+// FP32 SK records (sk_round), a record a thread
+__global__ __launch_bounds__(256) void k_sk32(int64_t n, const double4 *__restrict__ src,
+                                              float4 *__restrict__ dst) {
+  const int64_t b = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (b >= n) return;
+  double d[kSkStride];
+  float k[kSkStride];
+#pragma unroll
+  for (int i = 0; i < kSkStride / 4; ++i) {
+    const double4 v = src[b * (kSkStride / 4) + i];
+    d[4 * i] = v.x, d[4 * i + 1] = v.y, d[4 * i + 2] = v.z, d[4 * i + 3] = v.w;
+  }
+  sk_round(d, k);
+#pragma unroll
+  for (int i = 0; i < kSkStride / 4; ++i)
+    dst[b * (kSkStride / 4) + i] = make_float4(k[4 * i], k[4 * i + 1], k[4 * i + 2], k[4 * i + 3]);
+}
+
 inline int grid_for(int64_t n, int block) {
   int64_t g = (n + block - 1) / block;
   return (int)(g < 1 ? 1 : g);
@@ -464,10 +482,11 @@ nh_status select_precision(nh_context *c, int precision) {
                          (int64_t)nblk, c->blocks64, c->blocks32);
     }
     if (c->layout == NH_LAYOUT_SK && !c->sk32) {
-      const int64_t ns = (int64_t)c->n_cations * 4 * kSkStride;
-      NH_TRY(device_malloc(c, (void **)&c->sk32, ns * sizeof(float)));
-      hipLaunchKernelGGL(k_convert<float>, dim3(1024), dim3(256), 0, c->stream,
-                         ns, c->sk64, c->sk32);
+      const int64_t nr = (int64_t)c->n_cations * 4;
+      NH_TRY(device_malloc(c, (void **)&c->sk32, nr * kSkStride * sizeof(float)));
+      hipLaunchKernelGGL(k_sk32, dim3(grid_for(nr, 256)), dim3(256), 0, c->stream, nr,
+                         reinterpret_cast<const double4 *>(c->sk64),
+                         reinterpret_cast<float4 *>(c->sk32));
     }
     NH_HIP(hipGetLastError());
     NH_HIP(hipStreamSynchronize(c->stream));

@@ -296,7 +296,15 @@ struct MfSrc {
       const double *P = pair + p * kMfPair;
       scale(P, log((0.25 * kSqrt3Ref * P[kMfA0]) / den), v);
     }
-    sk_record(R(nx / den), R(ny / den), R(nz / den), v, rec);
+    if constexpr (sizeof(R) == 8) {
+      sk_record(nx / den, ny / den, nz / den, v, rec);
+    } else {
+      double w[21], k[24];
+#pragma unroll
+      for (int i = 0; i < 21; ++i) w[i] = v[i];
+      sk_record(nx / den, ny / den, nz / den, w, k);
+      sk_round(k, rec);
+    }
   }
 
 

@@ -45,12 +45,13 @@ enum : int {
   K_PPP = 20, K_PPC = 21, K_DB = 22, K_DA = 23
 };
 
+constexpr double kRecC2 = 2.0 / kSqrt3Ref, kRecC3 = 3.0 / (kSqrt3Ref * kSqrt3Ref);
 // Record of the direction (l, m, n) and the 21 integrals v (parameters
 // 10..30; the signs of the integrals with the lower angular momentum on the
 // cation as in sk_table).
 template <typename R>
 __host__ __device__ __forceinline__ void sk_record(R l, R m, R n, const R *v, R *k) {
-  constexpr R c2 = R(2.0 / kSqrt3Ref), c3 = R(3.0 / (kSqrt3Ref * kSqrt3Ref));
+  constexpr R c2 = R(kRecC2), c3 = R(kRecC3);
   k[K_L] = l;
   k[K_M] = m;
   k[K_N] = n;
@@ -75,6 +76,20 @@ __host__ __device__ __forceinline__ void sk_record(R l, R m, R n, const R *v, R 
   k[K_DDD] = v[20];
   k[K_DB] = v[19] - v[20];
   k[K_DA] = c3 * ((v[18] - v[20]) - R(4.0 / 3.0) * (v[19] - v[20]));
+}
+
+// The FP32 record of an FP64 one: the combinations take up the rounding of the
+// integrals in them, so that what T has of the others (dds = K_DDD + 4/3 K_DB +
+// K_DA / c3, pps = K_PPP + K_PPC, ..) is rounded once
+__host__ __device__ __forceinline__ void sk_round(const double (&d)[24], float (&k)[24]) {
+#pragma unroll
+  for (int i = 0; i < 24; ++i) k[i] = (float)d[i];
+  auto lost = [&](int i) { return d[i] - (double)k[i]; };
+  k[K_PPC] = (float)(d[K_PPC] + lost(K_PPP));
+  k[K_APD] = (float)(d[K_APD] + kRecC2 * lost(K_PADP));
+  k[K_ADP] = (float)(d[K_ADP] + kRecC2 * lost(K_PCDP));
+  k[K_DB] = (float)(d[K_DB] + lost(K_DDD));
+  k[K_DA] = (float)(d[K_DA] + kRecC3 * (lost(K_DDD) + (4.0 / 3.0) * lost(K_DB)));
 }
 
 __host__ __device__ __forceinline__ double sk_fma(double a, double b, double c) {
@@ -102,14 +117,32 @@ __host__ __device__ __forceinline__ void sk_apply(const R *k, const R (&x)[10], 
   const R apd = CATION ? k[K_ADP] : k[K_APD], adp = CATION ? k[K_APD] : k[K_ADP];
   const R ppc = k[K_PPC], ppp = k[K_PPP], ddd = k[K_DDD], db = k[K_DB], da = k[K_DA];
   const R *p = x + 2, *d = x + 5;
-  const R ml = m * l, mn = m * n, nl = n * l, l2 = l * l, m2 = m * m, n2 = n * n;
-  const R g[5] = {s3 * ml, s3 * mn, s3 * nl, (R(0.5) * s3) * (l2 - m2),
-                  n2 - R(0.5) * (l2 + m2)};
-  // projections
-  const R s = sk_fma(n, p[2], sk_fma(m, p[1], l * p[0]));
-  R t = g[0] * d[0];
+  // sd and the projections on it and on n.  FP32: sd's five functions are
+  // formed and projected on in FP64 and rounded once (as products of rounded
+  // products their errors, alike in all three of (111), made up most of the
+  // product's error)
+  R g[5], t;
+  if constexpr (sizeof(R) == 8) {
+    const R l2 = l * l, m2 = m * m;
+    g[0] = s3 * (m * l), g[1] = s3 * (m * n), g[2] = s3 * (n * l);
+    g[3] = (R(0.5) * s3) * (l2 - m2), g[4] = n * n - R(0.5) * (l2 + m2);
+    t = g[0] * d[0];
 #pragma unroll
-  for (int c = 1; c < 5; ++c) t = sk_fma(g[c], d[c], t);
+    for (int c = 1; c < 5; ++c) t = sk_fma(g[c], d[c], t);
+  } else {
+    const double dl = l, dm = m, dn = n, m2 = dm * dm;
+    const double sl = kSqrt3Ref * dl, sn = kSqrt3Ref * dn;
+    const double e[5] = {sl * dm, sn * dm, sl * dn,
+                         (0.5 * kSqrt3Ref) * sk_fma(dl, dl, -m2),
+                         sk_fma(dn, dn, -0.5 * sk_fma(dl, dl, m2))};
+    double td_ = e[0] * (double)d[0];
+#pragma unroll
+    for (int c = 1; c < 5; ++c) td_ = sk_fma(e[c], (double)d[c], td_);
+    t = R(td_);
+#pragma unroll
+    for (int c = 0; c < 5; ++c) g[c] = R(e[c]);
+  }
+  const R s = sk_fma(n, p[2], sk_fma(m, p[1], l * p[0]));
   y[0] = sk_fma(td, t, sk_fma(tp, s, sk_fma(ss_a, x[1], sk_fma(k[K_STSTS], x[0], y[0]))));
   y[1] = sk_fma(sd_, t, sk_fma(sp, s, sk_fma(ss_b, x[0], sk_fma(k[K_SSS], x[1], y[1]))));
   // w = M(d) n; the z2 part enters as (-1, -1, 2) kp
@@ -149,7 +182,7 @@ __host__ __device__ __forceinline__ void sk_apply(const R *k, const R (&x)[10], 
   R ddd4 = ddd;
   if constexpr (sizeof(R) == 8) {
     constexpr R e = R(1.0 / 3.0 - (kSqrt3Ref / 3.0) * (kSqrt3Ref / 3.0));
-    ddd4 = sk_fma(sk_fma(R(3) * e, n2, e), db, ddd);
+    ddd4 = sk_fma(sk_fma(R(3) * e, n * n, e), db, ddd);
   }
   R y9 = sk_fma(ddd4, d[4], y[9]);
   const R bl = db * l, bm = db * m, bn = db * n;
