@@ -112,8 +112,8 @@ enum { NH_SET_SK_LANES = 5 };
  * way the eigenvector pass retraces the eigenvalue pass; other layouts
  * and FP64 products always keep FP64 vectors.  FP64 SK and matrix-free
  * products run the one-launch step too, with FP64 u and r; there
- * beta_{k+1}^2 = |u_k|^2 - 2 alpha_k^2 + alpha_k^2 |q_k|^2, and a run in
- * which it falls below 1e-4 |u_k|^2 (a start in an almost invariant
+ * beta_{k+1}^2 is a difference of sums over w = u_k - alpha_{k-1} q_k, and a
+ * run in which it falls below |w|^2 / 8 (a start in an almost invariant
  * subspace) is repeated with |r_{k+1}|^2 summed directly. */
 enum { NH_SET_LZ_VECTORS = 6 };
 nh_status nh_context_set(nh_context *ctx, int what, int value);

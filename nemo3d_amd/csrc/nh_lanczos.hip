@@ -10,7 +10,7 @@
 // FP32 products keep FP32 vectors): the product sums the previous step's
 // partials to alpha_{k-1} and beta_k, forms r_k from u_{k-1} and r_{k-1} as it
 // reads them, computes u_k = H q_k - beta_k q_{k-1} and the partials of
-// alpha_k, |u_k|^2 and |q_k|^2.
+// alpha_k and beta_{k+1} (LzPart3).
 // The reference's REDUCE_OPT variant of the iteration (lanczos.c:441-456)
 // defers the vector update into the next iteration in the same spirit, to
 // merge its two reductions into one.
@@ -115,16 +115,28 @@ __device__ __forceinline__ double2 lz_three_term(double2 y, double2 q,
 __device__ __forceinline__ double lz_u(double y, double rp, double be, double invp) {
   return __builtin_fma(-be, rp * invp, y);
 }
-// partials of an eigenvalue-pass step: alpha_k, |u_k|^2, |q_k|^2
-// (beta_{k+1}^2 = |u|^2 - 2 alpha^2 + alpha^2 |q|^2)
+// partials of an eigenvalue-pass step: with w = u_k - sigma_k q_k, <q_k, w>,
+// |w|^2 and |q_k|^2 (lz_alpha_beta).  sigma_k = alpha_{k-1}: u's part along q_k
+// is gone but for alpha_k - alpha_{k-1}, and beta as exact as from |r_{k+1}|^2
+// (600 steps, N = 20,000: 7.5e-17 root mean square against 8.5e-17; without
+// sigma 1.9e-16, and 8e-14 with H shifted by 300 eV)
 struct LzPart3 {
-  double a = 0.0, u = 0.0, q = 0.0;
-  __device__ __forceinline__ void add(double qv, double uv) {
-    a = __builtin_fma(qv, uv, a);
-    u = __builtin_fma(uv, uv, u);
-    q = __builtin_fma(qv, qv, q);
+  double a = 0.0, w2 = 0.0, q2 = 0.0;
+  __device__ __forceinline__ void add(double sigma, double qv, double uv) {
+    const double w = __builtin_fma(-sigma, qv, uv);
+    a = __builtin_fma(qv, w, a);
+    w2 = __builtin_fma(w, w, w2);
+    q2 = __builtin_fma(qv, qv, q2);
   }
 };
+// alpha_k = <q, u> and beta_{k+1}^2 = |u - alpha_k q|^2 from the partials' sums;
+// d: <q, u> - sigma
+__device__ __forceinline__ void lz_alpha_beta(const double (&s)[3], double sigma, double &alpha,
+                                              double &beta) {
+  const double d = __builtin_fma(sigma, s[2] - 1.0, s[0]);
+  alpha = sigma + d;
+  beta = sqrt(fmax(__builtin_fma(d, __builtin_fma(d, s[2], -2.0 * s[0]), s[1]), 0.0));
+}
 // sums of three values over a workgroup of kRedThreads in a fixed order, in
 // every thread; scratch: 3 * kRedThreads / 64 doubles
 __device__ __forceinline__ void lz_block_sum3(double (&s)[3], double *scratch) {
@@ -146,21 +158,21 @@ __device__ __forceinline__ void lz_block_sum3(double (&s)[3], double *scratch) {
 // alpha_k and beta_{k+1} from the partials of nparts workgroups (fixed order:
 // every workgroup that evaluates it gets the same bits)
 __device__ __forceinline__ void lz_scalars3(int nparts, const double *__restrict__ part,
-                                            double *scratch, double &alpha, double &beta) {
+                                            double sigma, double *scratch, double &alpha,
+                                            double &beta) {
   double s[3] = {0.0, 0.0, 0.0};
   for (int k = threadIdx.x; k < nparts; k += kRedThreads)
 #pragma unroll
     for (int c = 0; c < 3; ++c) s[c] += part[3 * k + c];
   lz_block_sum3(s, scratch);
-  alpha = s[0];
-  beta = sqrt(fmax(s[1] - 2.0 * s[0] * s[0] + s[0] * s[0] * s[2], 0.0));
+  lz_alpha_beta(s, sigma, alpha, beta);
 }
 __global__ __launch_bounds__(kRedThreads) void k_lz_scalars3(
     int nparts, const double *__restrict__ part, double *__restrict__ alpha,
     double *__restrict__ beta) {
   __shared__ double scratch[3 * kRedThreads / 64];
   double a, b;
-  lz_scalars3(nparts, part, scratch, a, b);
+  lz_scalars3(nparts, part, alpha[-1], scratch, a, b);
   if (threadIdx.x == 0) {
     alpha[0] = a;
     beta[0] = b;
@@ -194,9 +206,11 @@ struct LzArgs {
   const V *x, *rp;
   V *out, *rout;
   const double *alpha, *beta_prev, *beta_prev2;  // beta null: 1 (start vector)
-  const double *part_prev;  // kLzValues: partials of the previous step
+  const double *part_prev;  // kLzValues: partials of the previous step (null: none)
   int nparts;
-  double *alpha_out, *beta_out;  // .. whose alpha and beta go here
+  // .. whose alpha and beta go here; alpha_out[-1]: its sigma, or (no previous
+  // step) this one's is alpha_out[0]
+  double *alpha_out, *beta_out;
   double *part;
 };
 template <int MODE, int NSP, typename R, typename V, typename SRC>
@@ -220,10 +234,14 @@ __global__ __launch_bounds__(kSkThreads, sizeof(V) == 8 ? 3 : 2) void k_lz_sk(
   SkIndex<SRC> ix;
   if (w.b < w.end) ix.read(tab, src, w.b, t.Q);
   LzCoef<V> ap{};
+  double sigma = 0.0;
   if constexpr (VALUES) {
     double alp = 0.0;
-    if (g.part_prev) {
-      lz_scalars3(g.nparts, g.part_prev, scratch, alp, be);
+    if (!g.part_prev) {
+      sigma = g.alpha_out[0];
+    } else {
+      lz_scalars3(g.nparts, g.part_prev, g.alpha_out[-1], scratch, alp, be);
+      sigma = alp;
       inv = 1.0 / be;
       if (blockIdx.x == 0 && threadIdx.x == 0) {
         g.alpha_out[0] = alp;
@@ -312,8 +330,8 @@ __global__ __launch_bounds__(kSkThreads, sizeof(V) == 8 ? 3 : 2) void k_lz_sk(
               if constexpr (MODE == kLzVectors) {
                 o = make_double2(lz_defer1(o.x, rk.x, af), lz_defer1(o.y, rk.y, af));
               } else {
-                p3.add(qk.x, o.x);
-                p3.add(qk.y, o.y);
+                p3.add(sigma, qk.x, o.x);
+                p3.add(sigma, qk.y, o.y);
               }
             } else {
               local += qk.x * o.x + qk.y * o.y;
@@ -331,7 +349,7 @@ __global__ __launch_bounds__(kSkThreads, sizeof(V) == 8 ? 3 : 2) void k_lz_sk(
                 o[e] = lz_defer1(u, rk[e], af);
               } else {
                 o[e] = u;
-                p3.add((double)rk[e] * inv, (double)u);
+                p3.add(sigma, (double)rk[e] * inv, (double)u);
               }
             }
           }
@@ -342,7 +360,7 @@ __global__ __launch_bounds__(kSkThreads, sizeof(V) == 8 ? 3 : 2) void k_lz_sk(
     }
   }
   if constexpr (VALUES || MODE == kLzProduct) {
-    double s[3] = {VALUES ? p3.a : local, p3.u, p3.q};
+    double s[3] = {VALUES ? p3.a : local, p3.w2, p3.q2};
     __syncthreads();  // the last block's records have been read
     lz_block_sum3(s, scratch);
     if (threadIdx.x == 0) {
@@ -584,12 +602,13 @@ class LanczosRun {
     for (void *p : allocs_) pool_release(c_, p);
     if (tri_s_) pool_release(c_, tri_s_);
     if (pin_) (void)hipHostFree(pin_);
-    for (hipEvent_t e : {fetch_ev_, check_ev_})
+    for (hipEvent_t e : {fetch_ev_, check_ev_, look_ev_})
       if (e) (void)hipEventDestroy(e);
   }
   nh_status run(const nh_lanczos_opts *o, nh_eig_result *res);
   // run() ended because the deferred step's beta has lost digits
   bool small_beta() const { return small_beta_; }
+  int matvecs() const { return matvecs_; }
 
  private:
   // from the context's workspace pool, handed back when the run ends
@@ -602,6 +621,12 @@ class LanczosRun {
   nh_status collect_timing();
   nh_status fetch(int m);
   nh_status check(int m);
+  nh_status look(bool wait);
+  // whether the deferred step's beta_i has lost digits (LzPart3)
+  static bool lost(double sigma, double alpha, double beta) {
+    const double d = alpha - sigma;
+    return !(beta * beta >= 0.125 * (d * d + beta * beta));
+  }
   hipStream_t check_stream() const { return alone_ ? c_->stream : c_->side; }
   bool alone_ = false;
   nh_status analyse(int m, const nh_lanczos_opts *o);
@@ -636,15 +661,16 @@ class LanczosRun {
   nh_status build_start(const nh_lanczos_opts *o);
   nh_status upload_start(void *r, size_t bytes);
   double2 *R0_ = nullptr;  // the normalised start vector (device)
-  double *alpha_ = nullptr, *beta_ = nullptr, *part_ = nullptr;
+  double *alpha_ = nullptr, *beta_ = nullptr, *part_ = nullptr;  // (alpha_[-1]: sigma_0)
   int nparts_ = 0;
   std::vector<double> ha_, hb_;
-  // pinned staging of alpha, beta (pin_cap_ each, filled up to fetched_) and
-  // of the last check's results; fetch_ev_: alpha and beta are there on the
+  // pinned staging of sigma_0 and alpha, of beta (pin_cap_ each, filled up to
+  // fetched_) and of the last check's results; fetch_ev_: alpha and beta are there on the
   // context's stream, check_ev_: the check of checked_ steps is done
   double *pin_ = nullptr;
   int pin_cap_ = 0, fetched_ = 0;
-  hipEvent_t fetch_ev_ = nullptr, check_ev_ = nullptr;
+  hipEvent_t fetch_ev_ = nullptr, check_ev_ = nullptr, look_ev_ = nullptr;
+  int matvecs_ = 0;
   int checked_ = 0;
   TriWindows win_{};
   double *tri_out_ = nullptr, *tri_s_ = nullptr;  // results, scratch of the check
@@ -710,11 +736,21 @@ __global__ __launch_bounds__(256) void k_start_fill(int64_t n, int kind, int L,
     r[j] = kind == 0 ? make_double2(cyc[(2 * j) % L], cyc[(2 * j + 1) % L])
                      : make_double2(1.0, 1.0);
 }
+// (and sigma_0, see LzPart3: the mean diagonal entry of 256 atoms)
 __global__ __launch_bounds__(256) void k_div(int64_t n, double2 *__restrict__ r,
-                                             double s) {
+                                             double s, int A, const double *__restrict__ onsite,
+                                             double *__restrict__ sigma) {
   for (int64_t j = blockIdx.x * (int64_t)256 + threadIdx.x; j < n;
        j += (int64_t)gridDim.x * 256)
     r[j] = make_double2(r[j].x / s, r[j].y / s);
+  if (blockIdx.x == 0) {
+    const double *os = onsite + (int64_t)threadIdx.x * A / 256 * kOnsiteStride;
+    double d = 0.0, z = 0.0;
+#pragma unroll
+    for (int k = 0; k < 10; ++k) d += os[k];
+    block_sum2(d, z);
+    if (threadIdx.x == 0) sigma[0] = d / 2560.0;
+  }
 }
 
 nh_status LanczosRun::build_start(const nh_lanczos_opts *o) {
@@ -754,7 +790,8 @@ nh_status LanczosRun::build_start(const nh_lanczos_opts *o) {
   double s = 0.0;
   NH_TRY(reduce_nrm2sq(c_, n_, reinterpret_cast<const nh_cplx *>(R0_), &s));
   NH_CHECK(s > 0, NH_ERR_ARG, "zero start vector");
-  hipLaunchKernelGGL(k_div, dim3(g), dim3(256), 0, c_->stream, n_, R0_, std::sqrt(s));
+  hipLaunchKernelGGL(k_div, dim3(g), dim3(256), 0, c_->stream, n_, R0_, std::sqrt(s),
+                     c_->n_atoms, c_->onsite, alpha_ - 1);
   NH_HIP(hipGetLastError());
   return NH_OK;
 }
@@ -792,11 +829,11 @@ void LanczosRun::launch_sk(int k, bool red, const SRC &src) {
     g.out = vec(u_[1]);
     g.rout = k == 0 ? nullptr : vec(r_[1]);
     g.beta_prev = nullptr;  // summed by this launch
+    g.alpha_out = alpha_ + (k - 1);
+    g.beta_out = beta_ + (k - 1);
     if (k > 0) {
       g.part_prev = part_ + (size_t)((k - 1) & 1) * 3 * nparts_;
       g.nparts = grid_;
-      g.alpha_out = alpha_ + (k - 1);
-      g.beta_out = beta_ + (k - 1);
     }
   } else if (red) {
     g.x = reinterpret_cast<V *>(R_);
@@ -945,7 +982,8 @@ nh_status LanczosRun::fetch(int m) {
       NH_HIP(hipEventRecord(fetch_ev_, c_->stream));
       NH_HIP(hipStreamWaitEvent(c_->side, fetch_ev_, 0));
     }
-    NH_HIP(hipMemcpyAsync(pin_ + fetched_, alpha_ + fetched_, (m - fetched_) * sizeof(double),
+    const int from = fetched_ > 0 ? fetched_ : -1;
+    NH_HIP(hipMemcpyAsync(pin_ + 1 + from, alpha_ + from, (m - from) * sizeof(double),
                           hipMemcpyDeviceToHost, check_stream()));
     NH_HIP(hipMemcpyAsync(pin_ + pin_cap_ + fetched_, beta_ + fetched_,
                           (m - fetched_) * sizeof(double), hipMemcpyDeviceToHost, check_stream()));
@@ -981,21 +1019,39 @@ nh_status LanczosRun::check(int m) {
   return NH_OK;
 }
 
+// A caller's start vector may lie in an almost invariant subspace (an
+// eigenvector): a look at the first step beside the ones that follow, so that
+// such a run is not first taken to its first check
+nh_status LanczosRun::look(bool wait) {
+  double *first = pin_ + 2 * (size_t)pin_cap_ - 3;  // the places of the last beta
+  if (!wait) {
+    NH_HIP(hipEventRecord(fetch_ev_, c_->stream));
+    NH_HIP(hipStreamWaitEvent(c_->side, fetch_ev_, 0));
+    NH_HIP(hipMemcpyAsync(first, alpha_ - 1, 2 * sizeof(double), hipMemcpyDeviceToHost, c_->side));
+    NH_HIP(hipMemcpyAsync(first + 2, beta_, sizeof(double), hipMemcpyDeviceToHost, c_->side));
+    NH_HIP(hipEventRecord(look_ev_, c_->side));
+    return NH_OK;
+  }
+  NH_HIP(hipEventSynchronize(look_ev_));
+  small_beta_ = lost(first[0], first[1], first[2]);
+  return small_beta_ ? NH_ERR_STATE : NH_OK;
+}
+
 // analyse the tridiagonal of the first m steps (fetch(m) queued before)
 nh_status LanczosRun::analyse(int m, const nh_lanczos_opts *o) {
   NH_CHECK(fetched_ >= m, NH_ERR_STATE, "Lanczos: tridiagonal not fetched");
   if (checked_ != m) NH_TRY(check(m));
   NH_HIP(hipEventSynchronize(check_ev_));
-  ha_.assign(pin_, pin_ + m);
+  ha_.assign(pin_ + 1, pin_ + 1 + m);
   hb_.assign(pin_ + pin_cap_, pin_ + pin_cap_ + m);
-  // The deferred FP64 step has beta^2 as a difference of sums, |u|^2 - alpha^2:
-  // below 1e-4 |u|^2 (a start vector in an almost invariant subspace) it loses
-  // more than four of its digits, and the run is repeated with the classic
-  // step, which sums |r|^2 itself.  (FP32 vectors: their rounding is far above
-  // what is lost.)
+  // The deferred FP64 step has beta^2 as a difference of sums, |w|^2 - (alpha -
+  // sigma)^2 (LzPart3): below |w|^2 / 8 (a start vector in an almost invariant
+  // subspace; 0.83 |w|^2 was the least in 1,400 steps from ordinary ones) three
+  // of its bits are lost, and the run is repeated with the classic step, which
+  // sums |r|^2 itself.  (FP32 vectors: their rounding is far above what is lost.)
   if (defer_ && vbytes_ == sizeof(double2))
     for (int i = 0; i < m; ++i)
-      if (!(hb_[i] * hb_[i] >= 1e-4 * (ha_[i] * ha_[i] + hb_[i] * hb_[i]))) small_beta_ = true;
+      if (lost(pin_[i], ha_[i], hb_[i])) small_beta_ = true;
   if (small_beta_) return NH_ERR_STATE;
   const double tol = o->conv_tolerance;
   const double resolution = 100.0 * tol;  // lanczos.c:1970
@@ -1066,7 +1122,8 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
     NH_TRY(alloc((void **)&Rm1_, n_ * sizeof(double2)));
   }
   NH_TRY(alloc((void **)&Y_, n_ * sizeof(double2)));
-  NH_TRY(alloc((void **)&alpha_, (size_t)(o->max_iter + 1) * sizeof(double)));
+  NH_TRY(alloc((void **)&alpha_, (size_t)(o->max_iter + 2) * sizeof(double)));
+  ++alpha_;  // alpha_[-1]: sigma_0
   NH_TRY(alloc((void **)&beta_, (size_t)(o->max_iter + 1) * sizeof(double)));
   // workgroups of the products: as many as run at a time (LDS: 2 a CU with
   // FP64 entries, 3 with FP32 ones)
@@ -1089,7 +1146,7 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
   // the next one, and its results are looked at there, after that block of
   // steps has been queued.  Convergence is thus seen one block late; the steps of
   // that block are not used (the run ends at the converged check point).
-  pin_cap_ = o->max_iter + 1;
+  pin_cap_ = o->max_iter + 2;
   win_ = TriWindows{{o->erange_vb[0], o->erange_cb[0]},
                     {o->erange_vb[1], o->erange_cb[1]},
                     {o->num_eig_vb > 0 ? o->num_eig_vb + 24 : 0,
@@ -1101,9 +1158,12 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
   if (!c->side) NH_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
   NH_HIP(hipEventCreateWithFlags(&fetch_ev_, hipEventDisableTiming));
   NH_HIP(hipEventCreateWithFlags(&check_ev_, hipEventDisableTiming));
+  constexpr int kLook = 2, kLookAt = 8;  // steps queued before look() and its wait
+  const bool looks = defer_ && vbytes_ == sizeof(double2) && (o->start == 2 || o->start == 3) &&
+                     o->restore_len <= 0 && o->max_iter > kLookAt + 3;
+  if (looks) NH_HIP(hipEventCreateWithFlags(&look_ev_, hipEventDisableTiming));
   int m = 0, skip = 0, pending = -1;
   bool done = false;
-  int matvecs = 0;
   Progress prog;
   if (o->restore_len > 0) {
     // restart from the tridiagonal of an earlier run (restoreState,
@@ -1143,8 +1203,9 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
     NH_TRY(iterate(m, true));
     ++m;
     prog.tick("lanczos", m, (int)conv_.size());
-    ++matvecs;
+    ++matvecs_;
     ++skip;
+    if (looks && (m == kLook || m == kLookAt)) NH_TRY(look(m == kLookAt));
     if (o->conv_check_start < m && o->conv_check_skip <= skip) {
       skip = 0;
       if (pending > 0) {
@@ -1253,7 +1314,7 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
     const int rk = ring_k_;
     for (int k = 0; k < mmax; ++k) {
       NH_TRY(iterate(k, false));
-      ++matvecs;
+      ++matvecs_;
       prog.tick("lanczos eigenvectors", k + 1, mmax);
       if ((k + 1) % rk == 0 || k + 1 == mmax) {
         const int k0 = k + 1 - ((k % rk) + 1);
@@ -1295,7 +1356,7 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
       hipLaunchKernelGGL(k_scale, dim3((int)g), dim3(256), 0, c->stream, n_,
                          V + (int64_t)e * n_, 1.0 / std::sqrt(nrm2));
       NH_TRY(launch_hv(c, 0.0, v, reinterpret_cast<nh_cplx *>(Y_), 1, n_));
-      ++matvecs;
+      ++matvecs_;
       double rq[2];
       NH_TRY(reduce_dot(c, n_, v, reinterpret_cast<nh_cplx *>(Y_), rq));
       const nh_cplx a = {-rq[0], 0.0}, b = {1.0, 0.0};
@@ -1310,7 +1371,7 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
     }
   }
   NH_HIP(hipStreamSynchronize(c->stream));
-  res->matvecs = matvecs;
+  res->matvecs = matvecs_;
   NH_TRY(collect_timing());
   res->hv_ms = hv_ms(0);
   res->hv_timed = hv_timed(0);
@@ -1330,11 +1391,18 @@ extern "C" nh_status nh_eigensolve_lanczos(nh_context *ctx,
            NH_ERR_ARG, "nh_eigensolve_lanczos: bad arguments");
   (void)hipGetLastError();
   NH_HIP(hipSetDevice(ctx->device));
+  const auto t0 = std::chrono::steady_clock::now();
+  int before = 0;
   {
     nh::LanczosRun run(ctx, false);
     const nh_status st = run.run(opts, res);
     if (!run.small_beta()) return st;
+    before = run.matvecs();
   }
   nh::LanczosRun run(ctx, true);
-  return run.run(opts, res);
+  const nh_status st = run.run(opts, res);
+  if (st != NH_OK && st != NH_ERR_NOCONV) return st;
+  res->matvecs += before;
+  res->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+  return st;
 }
