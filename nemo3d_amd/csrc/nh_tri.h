@@ -192,6 +192,36 @@ __global__ __launch_bounds__(kTriThreads) void k_tri_windows(
   // numbers of the eigenvalues in the window, and this workgroup's, from a
   // first pass with points from end to end of the window
   double lo = win.lo[w], hi = win.hi[w];
+  // window ends beyond T's Gershgorin bounds (an open window: +-1e99, infinity)
+  // are moved to them: eight minors at such a point leave the range of a double
+  {
+    double mn = INFINITY, mx = -INFINITY;
+    for (int i = tid; i < m; i += kTriThreads) {
+      const double r = (i > 0 ? fabs(b[i - 1]) : 0.0) + (i + 1 < m ? fabs(b[i]) : 0.0);
+      mn = fmin(mn, a[i] - r);
+      mx = fmax(mx, a[i] + r);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      mn = fmin(mn, __shfl_xor(mn, off, 64));
+      mx = fmax(mx, __shfl_xor(mx, off, 64));
+    }
+    double *ends = talk + 5 * kWaves;
+    if (lane == 0) {
+      ends[2 * wave] = mn;
+      ends[2 * wave + 1] = mx;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kWaves; ++q) {
+      mn = fmin(mn, ends[2 * q]);
+      mx = fmax(mx, ends[2 * q + 1]);
+    }
+    const double eps = 1e-12 * (fabs(mn) + fabs(mx)) + 1e-30;
+    auto inside = [&](double x) { return x < mn - eps ? mn - eps : x > mx + eps ? mx + eps : x; };
+    lo = inside(lo);
+    hi = inside(hi);
+  }
   auto point = [&](double h, int i) { return __builtin_fma(h, (double)i, lo); };
   int k, n;
   {
