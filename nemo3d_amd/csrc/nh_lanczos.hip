@@ -673,6 +673,12 @@ class LanczosRun {
   int matvecs_ = 0;
   int checked_ = 0;
   TriWindows win_{};
+  // no more eigenvalues are asked for than T_m has
+  TriWindows win_at(int m) const {
+    TriWindows w = win_;
+    for (int &n : w.want) n = std::min(n, m);
+    return w;
+  }
   double *tri_out_ = nullptr, *tri_s_ = nullptr;  // results, scratch of the check
   int64_t tri_cap_ = 0;                           // doubles in tri_s_
   std::vector<Converged> conv_;
@@ -996,19 +1002,21 @@ nh_status LanczosRun::fetch(int m) {
 // (alone_: the run's only check, with no steps beside it, on the run's own);
 // the earlier one has been waited for
 nh_status LanczosRun::check(int m) {
-  const int count = win_.want[0] + win_.want[1];
+  const TriWindows win = win_at(m);
+  const int count = win.want[0] + win.want[1];
   if (count > 0) {
-    const int64_t need = count * tri_scratch(m);
+    const int groups = std::min(count, kTriGroups);
+    const int64_t need = groups * tri_scratch(m);
     if (need > tri_cap_) {
       if (tri_s_) pool_release(c_, tri_s_);
       tri_s_ = nullptr;
       tri_cap_ = 0;
-      const int64_t cap = count * tri_scratch(std::max(2 * m, 2048));
+      const int64_t cap = groups * tri_scratch(std::max(2 * m, 2048));
       NH_TRY(pool_alloc(c_, (void **)&tri_s_, cap * sizeof(double)));
       tri_cap_ = cap;
     }
-    hipLaunchKernelGGL(k_tri_windows, dim3(count), dim3(kTriThreads), 0, check_stream(), m, alpha_,
-                       beta_, win_, tri_s_, tri_out_);
+    hipLaunchKernelGGL(k_tri_windows, dim3(groups), dim3(kTriThreads), 0, check_stream(), m,
+                       alpha_, beta_, win, tri_s_, tri_out_);
     NH_HIP(hipGetLastError());
     NH_HIP(hipMemcpyAsync(pin_ + 2 * (size_t)pin_cap_, tri_out_,
                           (kTriHead + (size_t)count * kTriOut) * sizeof(double),
@@ -1077,7 +1085,7 @@ nh_status LanczosRun::analyse(int m, const nh_lanczos_opts *o) {
     if (req[w] <= 0) continue;
     // the candidates nearest the gap: top of vb, bottom of cb
     std::vector<double> ev((size_t)tri[w]);
-    const double *o3 = tri + kTriHead + (w ? win_.want[0] : 0) * kTriOut;
+    const double *o3 = tri + kTriHead + (w ? win_at(m).want[0] : 0) * kTriOut;
     for (size_t i = 0; i < ev.size(); ++i) ev[i] = o3[kTriOut * i];
     auto duplicate = [&](size_t i) {
       // copies of one eigenvalue (ghosts, degeneracies) count once
@@ -1149,8 +1157,8 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
   pin_cap_ = o->max_iter + 2;
   win_ = TriWindows{{o->erange_vb[0], o->erange_cb[0]},
                     {o->erange_vb[1], o->erange_cb[1]},
-                    {o->num_eig_vb > 0 ? o->num_eig_vb + 24 : 0,
-                     o->num_eig_cb > 0 ? o->num_eig_cb + 24 : 0}};
+                    {o->num_eig_vb > 0 ? std::min(o->num_eig_vb, o->max_iter) + 24 : 0,
+                     o->num_eig_cb > 0 ? std::min(o->num_eig_cb, o->max_iter) + 24 : 0}};
   const size_t tri = kTriHead + (size_t)(win_.want[0] + win_.want[1]) * kTriOut;
   NH_TRY(alloc((void **)&tri_out_, tri * sizeof(double)));
   NH_HIP(hipHostMalloc((void **)&pin_, (2 * (size_t)pin_cap_ + tri) * sizeof(double),

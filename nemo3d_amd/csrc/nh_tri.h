@@ -34,7 +34,8 @@ struct TriWindows {
 // eigenvalue: value, last and last but one component
 constexpr int kTriHead = 2, kTriOut = 3;
 constexpr int kTriThreads = 256;
-// scratch of an eigenvalue, in doubles: pivots from both ends, and what the
+constexpr int kTriGroups = 512;  // workgroups at most (their scratch)
+// scratch of a workgroup, in doubles: pivots from both ends, and what the
 // wavefronts tell each other
 inline int64_t tri_scratch(int m) { return 2 * (int64_t)m + 32; }
 
@@ -168,15 +169,17 @@ __device__ inline TriProducts tri_products(const double *f, int dir, int n) {
           n > 1 ? __shfl(before, (n - 2) & 63, 64) : 1.0};
 }
 
-// S: tri_scratch(m) doubles an eigenvalue
-__global__ __launch_bounds__(kTriThreads) void k_tri_windows(
-    int m, const double *__restrict__ a, const double *__restrict__ b, TriWindows win,
-    double *S, double *__restrict__ out) {
+// eigenvalue idx of the windows' want[0] + want[1] by a workgroup; F: its
+// scratch
+__device__ __forceinline__ void tri_eigenvalue(int m, const double *__restrict__ a,
+                                               const double *__restrict__ b,
+                                               const TriWindows &win, int idx, double *F,
+                                               double *__restrict__ out) {
   constexpr int kPts = kTriThreads, kWaves = kTriThreads / 64;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int w = (int)blockIdx.x >= win.want[0], j = (int)blockIdx.x - (w ? win.want[0] : 0);
-  double *F = S + (int64_t)blockIdx.x * (2 * (int64_t)m + 32), *B = F + m, *talk = B + m;
+  const int w = idx >= win.want[0], j = idx - (w ? win.want[0] : 0);
+  double *B = F + m, *talk = B + m;
   // the first point with more than k eigenvalues below (kPts: none); slot: of
   // the talk, in turn
   auto first_above = [&](int cnt, int k, int slot) {
@@ -301,11 +304,21 @@ __global__ __launch_bounds__(kTriThreads) void k_tri_windows(
   __syncthreads();
   if (wave == 1 && lane == 0) {
     const double norm = sqrt(1.0 + talk[0] + up.sum);
-    double *o = out + kTriHead + (int64_t)blockIdx.x * kTriOut;
+    double *o = out + kTriHead + (int64_t)idx * kTriOut;
     o[0] = v;
     o[1] = up.last / norm;
     // the row before the last: the first one down if the last is r
     o[2] = m >= 2 ? (r == m - 1 ? talk[1] : up.before) / norm : 0.0;
+  }
+}
+// S: tri_scratch(m) doubles a workgroup
+__global__ __launch_bounds__(kTriThreads) void k_tri_windows(
+    int m, const double *__restrict__ a, const double *__restrict__ b, TriWindows win,
+    double *S, double *__restrict__ out) {
+  double *F = S + (int64_t)blockIdx.x * (2 * (int64_t)m + 32);
+  for (int idx = blockIdx.x; idx < win.want[0] + win.want[1]; idx += gridDim.x) {
+    tri_eigenvalue(m, a, b, win, idx, F, out);
+    __syncthreads();  // the scratch is free
   }
 }
 

@@ -2,6 +2,7 @@
 spectrum's own bound finds."""
 import numpy as np
 import pytest
+from scipy.linalg import eigh_tridiagonal
 
 import _models
 from nemo3d_amd import native
@@ -28,3 +29,30 @@ def test_open_ends(end):
     assert want["converged"] and got["converged"]
     assert got["eigenvalues"].size == want["eigenvalues"].size == 24
     assert np.abs(got["eigenvalues"] - want["eigenvalues"]).max() < 1e-12
+
+
+@pytest.mark.parametrize("num", [40, 700, 10 ** 7, 2 ** 31 - 30])
+def test_every_eigenvalue_asked_for(num):
+    """As many eigenvalues as the check has workgroups for, more than the windows
+    hold (168 and 309) or than the tridiagonal has: the 64 lowest of those asked
+    for, LAPACK's to 1e-12 (|T| < 40; bisection to 1e-13), copies within 100 tol
+    counted once."""
+    H = Hamiltonian(_models.gaas_box(cells=(1, 1, 1)), layout=native.LAYOUT_SK)
+    rng = np.random.default_rng(4)
+    m = 601
+    a, b = rng.uniform(-5.0, 15.0, m), rng.uniform(3.0, 10.0, m)
+    b[-9:] = 1e-9  # cuts the last rows off: all but two eigenvalues count as converged
+    b[-1] = 1e-3
+    w = eigh_tridiagonal(a, b[:-1], eigvals_only=True)
+    r = eigensolve_lanczos(H, num_vb=num, num_cb=num, erange_vb=(-60.0, -3.0),
+                           erange_cb=(4.9, 60.0), tol=1e-6, max_iter=m + 1, start_iter=10 * m,
+                           want_vectors=False, restore=(a, b))
+    got = r["eigenvalues"]
+    print(num, "found", got.size, "from", got[0], flush=True)
+    assert r["converged"] == (num == 40) and got.size == 64
+    assert max(np.abs(w - e).min() for e in got) < 1e-12
+    if num > 300:
+        assert abs(got[0] - w[0]) < 1e-12
+        # none is missing between the lowest and the highest one but copies
+        inner = w[(w > got[0]) & (w < got[-1])]
+        assert max(np.abs(got - e).min() for e in inner) < 1e-4 * 20
