@@ -191,10 +191,10 @@ nh_status ensure_buffers(nh_context *c, int64_t elems) {
 }
 
 template <typename T>
-static nh_status upload(T **dst, const T *src, size_t count) {
+static nh_status upload(nh_context *c, T **dst, const T *src, size_t count) {
   (void)hipFree(*dst);  // of an attempt that failed later on
   *dst = nullptr;
-  NH_HIP(hipMalloc(dst, count * sizeof(T) + 16));
+  NH_TRY(device_malloc(c, (void **)dst, count * sizeof(T) + 16));
   NH_HIP(hipMemcpy(*dst, src, count * sizeof(T), hipMemcpyHostToDevice));
   return NH_OK;
 }
@@ -456,13 +456,13 @@ nh_status ensure_blocks(nh_context *c) {
   m.is_cation = is_cation.data();
   BlockTables b;
   build_blocks(&m, rev, b);
-  NH_TRY(upload(&c->cations, b.cations.data(), b.cations.size()));
-  NH_TRY(upload(&c->bond_of, b.bond_of.data(), b.bond_of.size()));
-  NH_TRY(upload(&c->blk_own, b.own.data(), b.own.size()));
-  NH_TRY(upload(&c->blk_local, reinterpret_cast<const uint2 *>(b.local.data()),
+  NH_TRY(upload(c, &c->cations, b.cations.data(), b.cations.size()));
+  NH_TRY(upload(c, &c->bond_of, b.bond_of.data(), b.bond_of.size()));
+  NH_TRY(upload(c, &c->blk_own, b.own.data(), b.own.size()));
+  NH_TRY(upload(c, &c->blk_local, reinterpret_cast<const uint2 *>(b.local.data()),
                 b.local.size() / 8));
-  NH_TRY(upload(&c->blk_halo, b.halo.data(), b.halo.size()));
-  NH_TRY(upload(&c->blk_bonds, b.bonds.data(), b.bonds.size()));
+  NH_TRY(upload(c, &c->blk_halo, b.halo.data(), b.halo.size()));
+  NH_TRY(upload(c, &c->blk_bonds, b.bonds.data(), b.bonds.size()));
   c->n_blocks = b.n;
   return NH_OK;
 }
@@ -516,7 +516,7 @@ static nh_status create(const nh_model *m, int device, nh_context **out) {
   c->db_shift = m->db_shift;
   nh_status st = NH_OK;
 #define UP(dst, src, cnt)                              \
-  if (st == NH_OK) st = upload(&c->dst, src, (size_t)(cnt));
+  if (st == NH_OK) st = upload(c, &c->dst, src, (size_t)(cnt));
   UP(parmat, m->parmat, (size_t)S * S * 35);
   UP(strnmat, m->strnmat, (size_t)S * S * 33);
   UP(species, m->species, A);

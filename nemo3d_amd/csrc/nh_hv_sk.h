@@ -36,8 +36,9 @@ namespace nh {
 
 // ---- blocks of atoms ---------------------------------------------------------
 
-// Blocks (built at context creation): capacity 32 cations and 32 anions of
-// its own, 64 more neighbours (the halo), 176 bonds; -1 pads the tables.
+// Blocks (built by the first SK or matrix-free build, ensure_blocks): capacity
+// 32 cations and 32 anions of its own, 64 more neighbours (the halo), 176
+// bonds; -1 pads the tables.
 constexpr int kSkOwn = 64, kSkHalo = 64, kSkBonds = 176, kSkBondPad = 192;
 constexpr int kSkThreads = 256;
 
