@@ -90,10 +90,11 @@ def lanczos_memory(n, free_bytes=288e9, k=8):
     """Device bytes of the Lanczos vectors at N = n (SK layout): the
     eigenvalue pass keeps r and u of two steps in the vectors' precision and
     the FP64 start vector (FP32 products with FP64 vectors: r_k, r_(k-1), y
-    and the start vector, all FP64); the eigenvector pass adds the ring of r
-    vectors (2 K slots in the vectors' precision; K = 128 steps per flush,
-    halved down to 8 until the ring takes at most half the free memory) and
-    the k FP64 eigenvectors."""
+    and the start vector, all FP64), which the eigenvector pass gives back but
+    for the start vector (with FP64 vectors and FP32 products keeps); it has
+    the ring of r vectors (2 K slots in the vectors' precision; K = 128 steps
+    per flush, halved down to 8 until the ring takes at most half the free
+    memory) and the k FP64 eigenvectors."""
     v64, v32 = n * 16, n * 8
 
     def ring(per_step):  # bytes per step of K: two slots
@@ -106,12 +107,12 @@ def lanczos_memory(n, free_bytes=288e9, k=8):
     k32, r32 = ring(2 * v32)
     return {"eigenvalue_pass_fp64_GB": 5 * v64 / 1e9,
             "eigenvalue_pass_fp32_products_GB": 4 * v64 / 1e9,
-            "eigenvector_pass_fp64_GB": (5 * v64 + r64 + k * v64) / 1e9,
+            "eigenvector_pass_fp64_GB": (v64 + r64 + k * v64) / 1e9,
             "eigenvector_pass_fp64_ring_steps": k64,
             "eigenvector_pass_fp32_products_GB": (4 * v64 + r64 + k * v64) / 1e9,
             "eigenvector_pass_fp32_ring_steps": k32,
             "eigenvalue_pass_fp32_vectors_GB": (4 * v32 + v64) / 1e9,
-            "eigenvector_pass_fp32_vectors_GB": (4 * v32 + v64 + r32 + k * v64) / 1e9}
+            "eigenvector_pass_fp32_vectors_GB": (v64 + r32 + k * v64) / 1e9}
 
 
 def sk_matrix_bytes(M, rec_bytes):

@@ -617,6 +617,10 @@ class LanczosRun {
     allocs_.push_back(*p);
     return NH_OK;
   }
+  void release(void *p) {
+    pool_release(c_, p);
+    allocs_.erase(std::remove(allocs_.begin(), allocs_.end(), p), allocs_.end());
+  }
   nh_status iterate(int k, bool with_reductions);
   nh_status collect_timing();
   nh_status fetch(int m);
@@ -1128,8 +1132,8 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
   if (!defer_) {
     NH_TRY(alloc((void **)&R_, n_ * sizeof(double2)));
     NH_TRY(alloc((void **)&Rm1_, n_ * sizeof(double2)));
+    NH_TRY(alloc((void **)&Y_, n_ * sizeof(double2)));
   }
-  NH_TRY(alloc((void **)&Y_, n_ * sizeof(double2)));
   NH_TRY(alloc((void **)&alpha_, (size_t)(o->max_iter + 2) * sizeof(double)));
   ++alpha_;  // alpha_[-1]: sigma_0
   NH_TRY(alloc((void **)&beta_, (size_t)(o->max_iter + 1) * sizeof(double)));
@@ -1291,6 +1295,9 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
     std::vector<std::vector<double>> z(ne);
     for (int e = 0; e < ne; ++e)
       tri_eigvec(ha_, hb_, pick[e].iter, pick[e].value, z[e]);
+    // the deferred step's vectors of the eigenvalue pass are done with
+    if (defer_)
+      for (char *p : {r_[0], r_[1], u_[0], u_[1]}) release(p);
     double2 *V = nullptr;
     double *dZ = nullptr;
     NH_TRY(alloc((void **)&V, (size_t)ne * n_ * sizeof(double2)));
@@ -1314,6 +1321,7 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
       NH_CHECK(n_ % 2 == 0, NH_ERR_STATE, "Lanczos: the ring needs an even N");
       NH_TRY(alloc((void **)&ringr_, (size_t)2 * ring_k_ * n_ * vbytes_));
       NH_TRY(upload_start(ringr_, vbytes_));
+      if (defer_) Y_ = R0_;  // the start vector is in the ring: free for H v
     } else {
       NH_TRY(alloc((void **)&ring_, (size_t)ring_k_ * n_ * sizeof(double2)));
       NH_TRY(upload_start(R_, sizeof(double2)));
