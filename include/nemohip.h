@@ -237,7 +237,10 @@ typedef struct nh_lanczos_opts {
    * eigenvalue pass is skipped and the tridiagonal alpha[0..len),
    * beta[0..len) of an earlier run (nh_eig_result.tridiag_*, host arrays)
    * is analysed instead; the eigenvector pass then starts from the start
-   * vector these options describe, which must be that run's */
+   * vector these options describe, which should be that run's.  Where the
+   * eigenvectors' residuals show that it does not retrace the run (another
+   * start, an older version's order of the step, other vectors or products),
+   * the whole solve is done without the restart */
   const double *restore_alpha;
   const double *restore_beta;
   int32_t restore_len;

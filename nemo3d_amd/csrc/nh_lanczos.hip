@@ -608,6 +608,8 @@ class LanczosRun {
   nh_status run(const nh_lanczos_opts *o, nh_eig_result *res);
   // run() ended because the deferred step's beta has lost digits
   bool small_beta() const { return small_beta_; }
+  // a restart's vectors are not those of its tridiagonal
+  bool stale() const { return stale_; }
   int matvecs() const { return matvecs_; }
 
  private:
@@ -645,7 +647,7 @@ class LanczosRun {
   // the products' type (vbytes_ an entry).  The eigenvalue pass keeps r_{k-1},
   // u_{k-1} in r_[0], u_[0] and writes r_k, u_k to r_[1], u_[1]; part_ holds
   // the partials of two steps in turn, grid_ of each.
-  bool defer_ = false, small_beta_ = false;
+  bool defer_ = false, small_beta_ = false, stale_ = false;
   size_t vbytes_ = sizeof(double2);
   char *r_[2] = {nullptr, nullptr}, *u_[2] = {nullptr, nullptr};
   int grid_ = 0, last_ = -1;  // the last step of the eigenvalue pass queued
@@ -1381,6 +1383,22 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
       NH_TRY(reduce_nrm2sq(c, n_, reinterpret_cast<nh_cplx *>(Y_), &r2));
       res->eigenvalues[e] = rq[0];
       if (res->residuals) res->residuals[e] = std::sqrt(r2);
+      // A tridiagonal of another recurrence (an older version's order of the
+      // step, another precision or setting of the vectors) is not retraced:
+      // its vectors drift from this recurrence's as far as rounding grows, and
+      // what they add up to is no eigenvector.  A retraced one's residual is
+      // beta times the last component, or the rounding of the vectors.
+      if (o->restore_len > 0) {
+        const int it = pick[e].iter;
+        double tn = 0.0;
+        for (int i = 0; i < it; ++i) tn = std::max(tn, std::fabs(ha_[i]) + 2.0 * std::fabs(hb_[i]));
+        const double eps = c->precision == NH_PREC_FP64 ? 1e-16 : 1e-8;
+        const double tail = std::fabs(hb_[it - 1] * z[e][it - 1]);
+        if (!(std::sqrt(r2) <= 100.0 * tail + std::sqrt(eps) * tn)) {
+          stale_ = true;
+          return NH_ERR_STATE;
+        }
+      }
       if (res->eigenvectors)
         NH_HIP(hipMemcpy(res->eigenvectors + (int64_t)e * n_, v,
                          n_ * sizeof(nh_cplx), hipMemcpyDefault));  // host or device
@@ -1408,17 +1426,25 @@ extern "C" nh_status nh_eigensolve_lanczos(nh_context *ctx,
   (void)hipGetLastError();
   NH_HIP(hipSetDevice(ctx->device));
   const auto t0 = std::chrono::steady_clock::now();
+  nh_lanczos_opts o = *opts;
   int before = 0;
-  {
-    nh::LanczosRun run(ctx, false);
-    const nh_status st = run.run(opts, res);
-    if (!run.small_beta()) return st;
-    before = run.matvecs();
+  for (bool classic = false;;) {
+    nh::LanczosRun run(ctx, classic);
+    const nh_status st = run.run(&o, res);
+    if (run.small_beta()) {
+      classic = true;
+    } else if (run.stale()) {
+      // the eigenvalue pass after all
+      o.restore_len = 0;
+      classic = false;
+    } else {
+      if (st != NH_OK && st != NH_ERR_NOCONV) return st;
+      res->matvecs += before;
+      if (before > 0)
+        res->seconds =
+            std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+      return st;
+    }
+    before += run.matvecs();
   }
-  nh::LanczosRun run(ctx, true);
-  const nh_status st = run.run(opts, res);
-  if (st != NH_OK && st != NH_ERR_NOCONV) return st;
-  res->matvecs += before;
-  res->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-  return st;
 }
