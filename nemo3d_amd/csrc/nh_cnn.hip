@@ -232,13 +232,15 @@ nh_status backward(nh_cnn *c, int gx, int gy, int gz, const float *dout) {
   };
   const int cmax = std::max((c->c_in + 15) / 16 * 16, W);
   NH_TRY(ensure_part(c, std::max(hch * hlen, (int64_t)conv_chunks(1) * (27 * W * cmax + W))));
-  auto sum = [&](int chunks, int64_t len, int conv_ci, float *grad) {
+  auto sum = [&](int chunks, int64_t len, int conv_ci, const float *d, const float *x,
+                 float *grad) {
+    const GradIn g{gx, gy, gz, conv_ci ? W : c->c_out, conv_ci ? conv_ci : W, d, x};
     hipLaunchKernelGGL(k_grad_sum, dim3((len + 255) / 256), dim3(256), 0, st, chunks, len,
-                       conv_ci, c->part, grad);
+                       conv_ci, c->part, g, grad);
   };
   hipLaunchKernelGGL(k_head_bwd_w, dim3(hch, co_tiles), dim3(256), 0, st, P, c->c_out, dout,
                      c->act[L - 1], c->part, hlen);
-  sum(hch, hlen, 0, c->grad + c->w_off[L]);
+  sum(hch, hlen, 0, dout, c->act[L - 1], c->grad + c->w_off[L]);
   hipLaunchKernelGGL(k_head_bwd_data, dim3(g1(P, 128)), dim3(256), 0, st, P, c->c_out, dout,
                      reinterpret_cast<const uint4 *>(c->packed + c->pack.s[c->headt_seg].dst),
                      c->act[L - 1], c->dpre[0]);
@@ -254,7 +256,7 @@ nh_status backward(nh_cnn *c, int gx, int gy, int gz, const float *dout) {
     else
       hipLaunchKernelGGL(k_conv_bwd_w<2>, dim3(9 * cch, (ci + 31) / 32), dim3(256), 0, st, gx,
                          gy, gz, ci, cch, c->dpre[0], in, c->part, len);
-    sum(cch, len, ci, c->grad + c->w_off[l]);
+    sum(cch, len, ci, c->dpre[0], in, c->grad + c->w_off[l]);
     if (l > 0) {
       launch_conv<true>(c, gx, gy, gz, tile, W, c->pack.s[c->bwd_seg[l]], true, c->dpre[0], nullptr,
                         c->act[l - 1], c->dpre[1]);

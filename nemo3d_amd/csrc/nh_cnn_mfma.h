@@ -797,26 +797,61 @@ __global__ __launch_bounds__(256, 3) void k_head_bwd_w(
 }
 
 // grad[..] = sum of the chunks' partials, in order; conv: partials
-// [k][co][cp] and 32 of the bias to W[co][ci][k], b; else as they stand
+// [k][co][cp] and 32 of the bias to W[co][ci][k], b; else as they stand.
+// A sum that is not finite is taken again by the workgroup, point by point,
+// without the points whose gradient is zero: the matrix units multiply those
+// too, and a zero times an infinite activation (a point that the loss does not
+// reach) is NaN.
+struct GradIn {  // gradients d [P][co_n], inputs x [P][ci_n] of the layer
+  int gx, gy, gz, co_n, ci_n;
+  const float *d, *x;
+};
 __global__ __launch_bounds__(256) void k_grad_sum(int chunks, int64_t len, int conv_ci,
-                                                  const double *__restrict__ part,
+                                                  const double *__restrict__ part, GradIn g,
                                                   float *__restrict__ grad) {
-  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (t >= len) return;
+  __shared__ int32_t bad[256];
+  __shared__ double lds[4];
+  const int64_t t0 = blockIdx.x * (int64_t)blockDim.x, t = t0 + threadIdx.x;
+  const int cp = conv_ci ? (conv_ci + 15) / 16 * 16 : kCnnW;
+  const int64_t nw = (int64_t)(conv_ci ? 27 : 1) * g.co_n * cp;  // products, then the bias
+  auto place = [&](int64_t e) {  // -1: padding
+    if (!conv_ci) return e;
+    if (e >= nw) return (int64_t)kCnnW * conv_ci * 27 + (e - nw);
+    const int ci = e % cp;
+    const int64_t r = e / cp;
+    return ci >= conv_ci ? (int64_t)-1 : ((r % kCnnW) * conv_ci + ci) * 27 + r / kCnnW;
+  };
+  const int64_t o = t < len ? place(t) : -1;
   double s = 0.0;
+  if (o >= 0)
 #pragma unroll 8
-  for (int c = 0; c < chunks; ++c) s += part[c * len + t];
-  int64_t o = t;
-  if (conv_ci) {
-    const int cp = (conv_ci + 15) / 16 * 16;
-    const int64_t nw = (int64_t)27 * kCnnW * cp;
-    const int ci = t % cp;
-    const int64_t r = t / cp;
-    if (t >= nw) o = (int64_t)kCnnW * conv_ci * 27 + (t - nw);
-    else if (ci >= conv_ci) return;
-    else o = ((r % kCnnW) * conv_ci + ci) * 27 + r / kCnnW;
+    for (int c = 0; c < chunks; ++c) s += part[c * len + t];
+  if (o >= 0) grad[o] = (float)s;
+  const bool again = o >= 0 && t < nw && !isfinite(s);
+  bad[threadIdx.x] = again;
+  if (!__syncthreads_or(again)) return;
+  for (int e = 0; e < 256; ++e) {
+    if (!bad[e]) continue;
+    const int64_t r = (t0 + e) / cp;
+    const int ci = (t0 + e) % cp, co = r % g.co_n, k = conv_ci ? (int)(r / g.co_n) : 13;
+    const int dx = k / 9 - 1, dy = k / 3 % 3 - 1, dz = k % 3 - 1;
+    const int64_t P = (int64_t)g.gx * g.gy * g.gz;
+    double v = 0.0;
+    for (int64_t p = threadIdx.x; p < P; p += 256) {
+      const float d = g.d[p * g.co_n + co];
+      if (d == 0.0f) continue;
+      const int z = p % g.gz + dz, y = p / g.gz % g.gy + dy;
+      const int x = (int)(p / ((int64_t)g.gy * g.gz)) + dx;
+      if (x < 0 || y < 0 || z < 0 || x >= g.gx || y >= g.gy || z >= g.gz) continue;
+      v += (double)d * g.x[(((int64_t)x * g.gy + y) * g.gz + z) * g.ci_n + ci];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) grad[place(t0 + e)] = (float)(lds[0] + lds[1] + lds[2] + lds[3]);
   }
-  grad[o] = (float)s;
 }
 
 }  // namespace nh
