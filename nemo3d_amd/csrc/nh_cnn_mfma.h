@@ -21,6 +21,8 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "nh_internal.h"
+
 namespace nh {
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
@@ -416,7 +418,7 @@ __global__ __launch_bounds__(256) void k_head_map(
         head_bias(bias, 32 * t0 + 4 * lane, co_n, v);
         brow[lane] = make_float4(v[0], v[1], v[2], v[3]);
       }
-      __builtin_amdgcn_wave_barrier();
+      wave_sync();
       // rows r .. r + 3 belong to one state and slot (2 nb is a multiple of
       // 4): o = r % (4 nb) less the slot's rows, dst the state's place
       int o = 4 * h - (sl ? 2 * nb : 0);
@@ -442,7 +444,7 @@ __global__ __launch_bounds__(256) void k_head_map(
           }
         }
       }
-      __builtin_amdgcn_wave_barrier();
+      wave_sync();
       for (int e = 0; e < per && e0 + e < ne; ++e) {
         double2 *y = Y + (e0 + e) * ld + a0 * nb;
         int off = (lane / nb) * kRow + 2 * (lane % nb), q = lane % nb;
@@ -457,7 +459,7 @@ __global__ __launch_bounds__(256) void k_head_map(
           }
         }
       }
-      __builtin_amdgcn_wave_barrier();
+      wave_sync();
     }
   }
 }

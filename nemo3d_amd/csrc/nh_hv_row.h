@@ -101,14 +101,6 @@ __device__ __forceinline__ void hv_onsite(int atom, int o,
   }
 }
 
-// LDS accesses of one wavefront execute in order; this keeps the compiler
-// from moving them across.  No instruction is emitted.
-__device__ __forceinline__ void wave_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // One neighbour block row applied to both spins: acc += B[o][:] x_j.
 template <int NSP, typename TB, typename TA>
 __device__ __forceinline__ void hv_block(const TB *__restrict__ B,
@@ -199,14 +191,14 @@ struct Rows {
     if (atom >= 0) hv_onsite<NSP>(atom, o, onsite, shift, xc, acc_re, acc_im, xi);
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
-      wave_fence();
+      wave_sync();
 #pragma unroll
       for (int i = 0; i < kB; ++i)
         if (lane + 64 * i < kRowAtoms * S::kSeg) L.b[lane + 64 * i] = bl[n][i];
 #pragma unroll
       for (int i = 0; i < kX; ++i)
         if (lane + 64 * i < kRowAtoms * S::kNx) L.x[lane + 64 * i] = xl[n][i];
-      wave_fence();
+      wave_sync();
       if (slot(own, n) >= 0)
         hv_block<NSP, TB, TA>(reinterpret_cast<const TB *>(L.b + la * S::kSeg) + o * 10,
                               reinterpret_cast<const double2 *>(L.x + la * S::kNx), acc_re,

@@ -78,15 +78,6 @@ struct SkWalk {
 __device__ __forceinline__ double2 widen2(double2 v) { return v; }
 __device__ __forceinline__ double2 widen2(float2 v) { return make_double2(v.x, v.y); }
 
-// LDS accesses of one wavefront execute in order; this keeps the compiler
-// from moving them across (lanes read what other lanes of the wavefront
-// wrote).  No instruction is emitted.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Staged items, in 16-byte chunks.  20 bands: the chunks of the two spins
 // alternate, so the four components of an orbital that a quad's lanes read
 // together lie in 32 bytes, and the stride is an odd number of 32 bytes: quads

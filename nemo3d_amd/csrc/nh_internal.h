@@ -53,6 +53,15 @@ constexpr int kSkStride = 24;
 constexpr int kMfPair = 40;
 constexpr int kMfEta = 21, kMfA0 = 36;
 
+// LDS accesses of one wavefront execute in order; this keeps the compiler
+// from moving them across (lanes read what other lanes of the wavefront
+// wrote).  No instruction is emitted.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 }  // namespace nh
 
 struct nh_context {
