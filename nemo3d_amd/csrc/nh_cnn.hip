@@ -176,8 +176,6 @@ void launch_conv(nh_cnn *c, int gx, int gy, int gz, const ConvTile &tile, int ld
 
 // the conv layers: act[l] for every point
 nh_status forward(nh_cnn *c, int gx, int gy, int gz) {
-  NH_CHECK((gy + 7) / 8 <= 65535 && gx <= 65535, NH_ERR_ARG,
-           "network: grid %d x %d x %d too large", gx, gy, gz);
   const ConvTile tile = conv_tile(gx, gy, gz);
   const float *src = c->in;
   int ci = c->c_in;

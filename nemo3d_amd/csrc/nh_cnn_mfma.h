@@ -287,7 +287,8 @@ __global__ __launch_bounds__(256, 2) void k_conv(
 // workgroup has one for itself (85 x 85 x 57 points: 484 workgroups of 8
 // planes 274 us, 748 of 5 320, 220 of 17 325; 106 x 106 x 71, tiles of 8 x 16
 // / 16 x 8: 490 of 16 planes 516, 504 of 14 461, 252 of 27 509).  Equal ones:
-// the tile with the fewest points around it.
+// the tile with the fewest points around it.  No more than 65,535 parts of x
+// (a grid's rows).
 inline ConvTile conv_tile(int gx, int gy, int gz) {
   ConvTile best{8, 16, gx};
   int64_t cost = INT64_MAX;
@@ -296,6 +297,7 @@ inline ConvTile conv_tile(int gx, int gy, int gz) {
     const int64_t tiles = (int64_t)((gy + ty - 1) / ty) * ((gz + tz - 1) / tz);
     for (int n = 1, seg; n <= gx; n = seg > 1 ? (gx + seg - 2) / (seg - 1) : gx + 1) {
       seg = (gx + n - 1) / n;
+      if ((gx + seg - 1) / seg > 65535) break;
       const int64_t w = tiles * ((gx + seg - 1) / seg);
       const int64_t c = (w <= 256 ? 7 : (w + 511) / 512 * 12) * (3 * seg + 2);
       if (c < cost || (c == cost && ty + tz < best.ty + best.tz)) {
