@@ -159,8 +159,9 @@ nh_status nh_ham_export(nh_context *ctx, double *onsite, double *blocks);
  * every allocation of the library, nh_device_alloc included, first hands
  * the idle pool blocks of all contexts on the device back when the device
  * is full.  Blocks given to nh_device_free (which waits for the device, as
- * hipFree does) are kept for requests of the same size, at most 8 of them and
- * 1/32 of the device's memory in a context; they count as idle pool blocks.
+ * hipFree does) are kept for requests of the same size, at most 8 of them in a
+ * context and 1/32 of the device's memory in all; they count as idle pool
+ * blocks.
  * nh_context_mem_info reports the device's free bytes and the
  * idle pool bytes of all contexts on it (either pointer may be NULL). */
 nh_status nh_context_mem_info(nh_context *ctx, int64_t *free_bytes,

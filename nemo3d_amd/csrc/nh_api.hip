@@ -60,8 +60,8 @@ static nh_status pool_trim(nh_context *c) {
 }
 
 // Blocks of nh_device_alloc freed by the caller stay with the context, at
-// most kKeepBlocks of them and kKeepShare of the device's memory, and serve
-// its next requests of the same size.  A program that asks for its vectors
+// most kKeepBlocks of them and, over all contexts, one part in kKeepShare of
+// the device's memory, and serve its next requests of the same size.  A program that asks for its vectors
 // anew on every call otherwise runs at the speed at which the driver clears
 // freed memory: products of 2 GB a call, each freed when the next one is
 // there, took 55 ms a call once the device had been gone through once
@@ -97,13 +97,20 @@ static nh_status device_keep(nh_context *c, void *p) {
   }
   // as hipFree does: whatever stream used the memory is done with it
   NH_HIP(hipDeviceSynchronize());
+  std::lock_guard<std::mutex> all(g_ctx_mu);
+  size_t sum = bytes;  // with the other contexts' blocks
+  for (nh_context *o : g_ctxs) {
+    if (o->device != c->device) continue;
+    std::lock_guard<std::mutex> k(o->kept_mu);
+    for (const auto &b : o->kept) {
+      NH_CHECK(b.p != p, NH_ERR_ARG, "nh_device_free: freed twice");
+      sum += b.bytes;
+    }
+  }
   std::lock_guard<std::mutex> g(c->kept_mu);
-  for (const auto &b : c->kept)
-    NH_CHECK(b.p != p, NH_ERR_ARG, "nh_device_free: freed twice");
   c->kept.push_back({p, bytes, false});
-  size_t sum = 0;
-  for (const auto &b : c->kept) sum += b.bytes;
-  while (sum > total / kKeepShare || c->kept.size() > (size_t)kKeepBlocks) {
+  while (!c->kept.empty() &&
+         (sum > total / kKeepShare || c->kept.size() > (size_t)kKeepBlocks)) {
     // the oldest one goes
     sum -= c->kept.front().bytes;
     NH_HIP(hipFree(c->kept.front().p));
