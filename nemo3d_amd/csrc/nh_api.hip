@@ -218,8 +218,7 @@ static void destroy(nh_context *c) {
                   c->blk_local, c->blk_halo, c->blk_bonds, c->mf_geo, c->mf_q,
                   c->mf_pair, c->mf_ends,
                   c->rev_slot, c->onsite, c->blocks64, c->blocks32,
-                  c->onsite32, c->sk64, c->sk32, c->red, c->xbuf,
-                  c->ybuf};
+                  c->sk64, c->sk32, c->red, c->xbuf, c->ybuf};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   (void)hipStreamSynchronize(c->stream);

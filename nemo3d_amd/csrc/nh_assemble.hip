@@ -397,7 +397,6 @@ static void free_ham(nh_context *c, int layout) {
   if (layout != NH_LAYOUT_BLOCKS) drop(c->blocks64);
   // FP32 copies are derived anew (select_precision)
   drop(c->blocks32);
-  drop(c->onsite32);
   drop(c->sk32);
   if (layout != NH_LAYOUT_SK) drop(c->sk64);
   if (layout != NH_LAYOUT_MATRIX_FREE) {
@@ -468,13 +467,8 @@ nh_status select_precision(nh_context *c, int precision) {
            "precision %d not available", precision);
   const int A = c->n_atoms;
   if (precision == NH_PREC_FP32) {
-    // the FP64 values are always kept: derive the FP32 copies once (the
-    // matrix-free layout needs none)
-    if (c->layout == NH_LAYOUT_BLOCKS && !c->onsite32) {
-      NH_TRY(device_malloc(c, (void **)&c->onsite32, (size_t)A * kOnsiteStride * sizeof(float)));
-      hipLaunchKernelGGL(k_convert<float>, dim3(1024), dim3(256), 0, c->stream,
-                         (int64_t)A * kOnsiteStride, c->onsite, c->onsite32);
-    }
+    // the FP64 values are always kept: derive the FP32 blocks or records once
+    // (the matrix-free layout needs none; onsite terms are FP64 always)
     if (c->layout == NH_LAYOUT_BLOCKS && !c->blocks32) {
       const size_t nblk = (size_t)A * 4 * 100;
       NH_TRY(device_malloc(c, (void **)&c->blocks32, nblk * sizeof(float)));

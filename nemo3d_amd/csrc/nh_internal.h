@@ -109,7 +109,6 @@ struct nh_context {
   double *onsite = nullptr;     // [A][kOnsiteStride]
   double *blocks64 = nullptr;   // [A][4][100] (NH_LAYOUT_BLOCKS, FP64)
   float *blocks32 = nullptr;    // [A][4][100] (NH_LAYOUT_BLOCKS, FP32)
-  float *onsite32 = nullptr;    // [A][kOnsiteStride] (FP32 runs)
   double *sk64 = nullptr;       // [Nc*4][kSkStride] (NH_LAYOUT_SK)
   float *sk32 = nullptr;
   double4 *mf_geo = nullptr;    // [A] displacement (nm) x, y, z; species
