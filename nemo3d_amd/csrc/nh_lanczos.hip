@@ -42,19 +42,19 @@ namespace {
 constexpr int kRingMax = 128;
 constexpr int kMaxVec = 64;
 
-template <int NSP, typename TB, typename TA>
-__global__ __launch_bounds__(kThreads, 3) void k_lz_hv(
+template <int WAVES, int NSP, typename TB, typename TA>
+__global__ __launch_bounds__(64 * WAVES, 3) void k_lz_hv(
     int A, const double *__restrict__ onsite, const TB *__restrict__ blocks,
     const int32_t *__restrict__ nbr, const double2 *__restrict__ R,
     double2 *__restrict__ Q, double2 *__restrict__ Y,
     const double *__restrict__ beta_prev, double *__restrict__ part) {
   constexpr int NB = NSP * 10;
-  static_assert(kThreads == kRedThreads, "block sums");
-  __shared__ RowLds<NSP, TB> L[kThreads / 64];
+  __shared__ RowLds<NSP, TB> L[WAVES];
+  __shared__ double sums[WAVES];
   const int wave = threadIdx.x >> 6;
-  const int a0 = (blockIdx.x * (kThreads / 64) + wave) * kRowAtoms;
+  const int a0 = (blockIdx.x * WAVES + wave) * kRowAtoms;
   const double inv = beta_prev ? 1.0 / beta_prev[0] : 1.0;
-  double local = 0.0, zero = 0.0;
+  double local = 0.0;
   if (a0 < A) {
     double acc_re[NSP], acc_im[NSP];
     double2 xi[NSP];
@@ -73,9 +73,26 @@ __global__ __launch_bounds__(kThreads, 3) void k_lz_hv(
     }
   }
   if (part) {
-    block_sum2(local, zero);
-    if (threadIdx.x == 0) part[blockIdx.x] = local;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) local += __shfl_down(local, off, 64);
+    if ((threadIdx.x & 63) == 0) sums[wave] = local;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      local = 0.0;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) local += sums[w];
+      part[blockIdx.x] = local;
+    }
   }
+}
+// Wavefronts of a workgroup of k_lz_hv: four, and up to eight where with more
+// the compute units take the atoms in one round (one workgroup on each; a
+// second one on some of them holds up the whole step: 60 steps, FP64, 6,720
+// atoms 1475 us with four, 1379 with six; 9,984 atoms 1666, with eight 1594).
+inline int hv_waves(int A) {
+  for (int w : {4, 6, 8})
+    if ((A + w * kRowAtoms - 1) / (w * kRowAtoms) <= 256) return w;
+  return 4;
 }
 
 // One element of the three-term step y - alpha q - beta_prev q_prev with
@@ -650,6 +667,7 @@ class LanczosRun {
   bool defer_ = false, small_beta_ = false, stale_ = false;
   size_t vbytes_ = sizeof(double2);
   char *r_[2] = {nullptr, nullptr}, *u_[2] = {nullptr, nullptr};
+  int waves_ = 4;  // of a workgroup of k_lz_hv
   int grid_ = 0, last_ = -1;  // the last step of the eigenvalue pass queued
   // ring length of the eigenvector pass (<= kRingMax)
   int ring_k_ = kRingMax;
@@ -911,10 +929,16 @@ nh_status LanczosRun::iterate(int k, bool red) {
     // accumulates from it; the update forms q_k, q_{k-1} from r_k, r_{k-1}
     double2 *Q = red ? nullptr : ring_ + (int64_t)(k % ring_k_) * n_;
     double *part = red ? part_ : nullptr;
-#define LZ_HV(NSP, TB, BLK)                                                    \
-  hipLaunchKernelGGL((k_lz_hv<NSP, TB, TB>), dim3(grid_), dim3(kThreads), 0,   \
+#define LZ_HVW(W, NSP, TB, BLK)                                                \
+  hipLaunchKernelGGL((k_lz_hv<W, NSP, TB, TB>), dim3(grid_), dim3(64 * W), 0,  \
                      c->stream, c->n_atoms, c->onsite, BLK, c->nbr, R_, Q, Y_, \
                      bprev, part)
+#define LZ_HV(NSP, TB, BLK)                                                    \
+  do {                                                                         \
+    if (waves_ == 8) LZ_HVW(8, NSP, TB, BLK);                                  \
+    else if (waves_ == 6) LZ_HVW(6, NSP, TB, BLK);                             \
+    else LZ_HVW(4, NSP, TB, BLK);                                              \
+  } while (0)
     if (c->precision == NH_PREC_FP64) {
       if (c->nb == 20) LZ_HV(2, double, c->blocks64);
       else LZ_HV(1, double, c->blocks64);
@@ -923,6 +947,7 @@ nh_status LanczosRun::iterate(int k, bool red) {
       else LZ_HV(1, float, c->blocks32);
     }
 #undef LZ_HV
+#undef LZ_HVW
   }
   NH_HIP(hipGetLastError());
   if (timed) {
@@ -1141,8 +1166,9 @@ nh_status LanczosRun::run(const nh_lanczos_opts *o, nh_eig_result *res) {
   NH_TRY(alloc((void **)&beta_, (size_t)(o->max_iter + 1) * sizeof(double)));
   // workgroups of the products: as many as run at a time (LDS: 2 a CU with
   // FP64 entries, 3 with FP32 ones)
+  waves_ = hv_waves(c->n_atoms);
   grid_ = sk_like(c) ? sk_grid(c, vbytes_ == sizeof(float2) ? 3 : 2)
-                     : (c->n_atoms + kAtomsPerBlock - 1) / kAtomsPerBlock;
+                     : (c->n_atoms + waves_ * kRowAtoms - 1) / (waves_ * kRowAtoms);
   nparts_ = std::max(grid_, 2 * kRedMaxBlocks) + 64;
   NH_TRY(alloc((void **)&part_, (size_t)nparts_ * 6 * sizeof(double)));
 
