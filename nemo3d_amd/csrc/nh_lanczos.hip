@@ -1046,8 +1046,9 @@ nh_status LanczosRun::check(int m) {
       NH_TRY(pool_alloc(c_, (void **)&tri_s_, cap * sizeof(double)));
       tri_cap_ = cap;
     }
-    hipLaunchKernelGGL(k_tri_windows, dim3(groups), dim3(kTriThreads), 0, check_stream(), m,
-                       alpha_, beta_, win, tri_s_, tri_out_);
+    for (int first = 0; first < count; first += groups)
+      hipLaunchKernelGGL(k_tri_windows, dim3(std::min(groups, count - first)), dim3(kTriThreads),
+                         0, check_stream(), m, alpha_, beta_, win, first, tri_s_, tri_out_);
     NH_HIP(hipGetLastError());
     NH_HIP(hipMemcpyAsync(pin_ + 2 * (size_t)pin_cap_, tri_out_,
                           (kTriHead + (size_t)count * kTriOut) * sizeof(double),

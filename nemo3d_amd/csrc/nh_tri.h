@@ -9,7 +9,9 @@
 // eigenvector follows from the position where they meet best (twisted
 // factorisation), without inverse iteration.  The kernel uses no LDS and few
 // registers, so that it runs beside a Lanczos step that fills the LDS of every
-// compute unit; the wavefronts meet in the scratch memory.
+// compute unit; the wavefronts meet in the scratch memory.  (Three workgroups of
+// an FP32 step leave 56 registers of a SIMD; with 80 of them for the check, for
+// a loop over eigenvalues, the step went from 239 to 255 us, 786,520 atoms.)
 // Bound by the serial recurrences, 38 cycles a row and pass (6 passes) and
 // about 85 a row for the pivots: 0.30 ms at 1,375 rows.  (One wavefront, 64
 // points, the pivots and the components by two lanes: 547 us; four points a
@@ -34,7 +36,7 @@ struct TriWindows {
 // eigenvalue: value, last and last but one component
 constexpr int kTriHead = 2, kTriOut = 3;
 constexpr int kTriThreads = 256;
-constexpr int kTriGroups = 512;  // workgroups at most (their scratch)
+constexpr int kTriGroups = 512;  // workgroups of a launch at most (their scratch)
 // scratch of a workgroup, in doubles: pivots from both ends, and what the
 // wavefronts tell each other
 inline int64_t tri_scratch(int m) { return 2 * (int64_t)m + 32; }
@@ -169,17 +171,17 @@ __device__ inline TriProducts tri_products(const double *f, int dir, int n) {
           n > 1 ? __shfl(before, (n - 2) & 63, 64) : 1.0};
 }
 
-// eigenvalue idx of the windows' want[0] + want[1] by a workgroup; F: its
-// scratch
-__device__ __forceinline__ void tri_eigenvalue(int m, const double *__restrict__ a,
-                                               const double *__restrict__ b,
-                                               const TriWindows &win, int idx, double *F,
-                                               double *__restrict__ out) {
+// Eigenvalues first, first + 1, .. of the windows' want[0] + want[1], one a
+// workgroup.  S: tri_scratch(m) doubles a workgroup
+__global__ __launch_bounds__(kTriThreads) void k_tri_windows(
+    int m, const double *__restrict__ a, const double *__restrict__ b, TriWindows win,
+    int first, double *S, double *__restrict__ out) {
   constexpr int kPts = kTriThreads, kWaves = kTriThreads / 64;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int idx = first + (int)blockIdx.x;
   const int w = idx >= win.want[0], j = idx - (w ? win.want[0] : 0);
-  double *B = F + m, *talk = B + m;
+  double *F = S + (int64_t)blockIdx.x * (2 * (int64_t)m + 32), *B = F + m, *talk = B + m;
   // the first point with more than k eigenvalues below (kPts: none); slot: of
   // the talk, in turn
   auto first_above = [&](int cnt, int k, int slot) {
@@ -309,16 +311,6 @@ __device__ __forceinline__ void tri_eigenvalue(int m, const double *__restrict__
     o[1] = up.last / norm;
     // the row before the last: the first one down if the last is r
     o[2] = m >= 2 ? (r == m - 1 ? talk[1] : up.before) / norm : 0.0;
-  }
-}
-// S: tri_scratch(m) doubles a workgroup
-__global__ __launch_bounds__(kTriThreads) void k_tri_windows(
-    int m, const double *__restrict__ a, const double *__restrict__ b, TriWindows win,
-    double *S, double *__restrict__ out) {
-  double *F = S + (int64_t)blockIdx.x * (2 * (int64_t)m + 32);
-  for (int idx = blockIdx.x; idx < win.want[0] + win.want[1]; idx += gridDim.x) {
-    tri_eigenvalue(m, a, b, win, idx, F, out);
-    __syncthreads();  // the scratch is free
   }
 }
 
