@@ -107,8 +107,8 @@ enum { NH_SET_SK_LANES = 5 };
  * into two FP32 parts, and the product of step k
  * forms r_k from u_{k-1} and r_{k-1} as it reads them, so a step is one
  * launch (no FP64 vector in either pass; alpha, beta and the sums stay
- * FP64); -1 the default (1 where the products use the
- * LDS gather: measured faster, with the same number of steps).  Either
+ * FP64); -1 the default (1: faster, with about the same number of steps).
+ * Either
  * way the eigenvector pass retraces the eigenvalue pass; other layouts
  * and FP64 products always keep FP64 vectors.  FP64 SK and matrix-free
  * products run the one-launch step too, with FP64 u and r; there

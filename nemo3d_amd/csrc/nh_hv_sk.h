@@ -21,8 +21,8 @@
 // twice) and kept the texture addresser busy 76% of 255 us whatever the order
 // of the atoms; the block moves the entries 1.7 times and the records 1.2
 // times: 786,520 atoms FP64 0.312 -> 0.238 ms (SK), 8 columns of 395,136
-// atoms 1.25 -> 0.65 ms (matrix-free); what is left is FP64 VALU (93 FMAs a
-// bond, component and row) and LDS reads about evenly, behind 0.94 GB of HBM.
+// atoms 1.25 -> 0.65 ms (matrix-free); what is left is FP64 VALU (93 operations
+// a bond, component and row) and LDS reads about evenly, behind 0.94 GB of HBM.
 // The role (cation or anion) is uniform in a wavefront, so whether T or its
 // transpose is applied is a scalar branch.
 #pragma once

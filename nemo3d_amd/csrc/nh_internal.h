@@ -45,7 +45,8 @@ void set_error(const char *fmt, ...);
 // Onsite record per atom: 10 diagonal energies, 6 surface s-p couplings,
 // spin-orbit lambda (17 doubles, padded to 18 for 16-byte alignment).
 constexpr int kOnsiteStride = 18;
-// Per-bond SK record: l, m, n and the 21 scaled integrals (24 values).
+// Per-bond SK record: l, m, n and 21 combinations of the scaled integrals
+// (sk_record, nh_sk_apply.h).
 constexpr int kSkStride = 24;
 // Matrix-free layout, per (cation species, anion species) pair: the 21
 // unscaled two-centre integrals (parameters 10..30), the 15 strain
@@ -94,13 +95,10 @@ struct nh_context {
   int32_t *blk_own = nullptr, *blk_halo = nullptr, *blk_bonds = nullptr;
   uint2 *blk_local = nullptr;
 
-  // kernel variants (nh_context_set)
-  // stored-block H·v: neighbour x staged in LDS (measured on the 786,520-
-  // atom dot: faster for the plain product, slower inside the fused Lanczos
-  // kernel, so off by default)
+  // settings (nh_context_set)
   int hv_staged = -1;  // NH_SET_HV_STAGED (0: no FP32 Lanczos vectors)
   int ring_steps = 0;  // NH_SET_RING_STEPS (0: by free memory)
-  int block_hv = -1;   // NH_SET_BLOCK_HV (-1: by measurement)
+  int block_hv = -1;   // NH_SET_BLOCK_HV (-1: by size, hv_columns)
   int lz_vectors = -1; // NH_SET_LZ_VECTORS (-1: default, lz_fp32_vectors)
 
   // assembled Hamiltonian
@@ -140,16 +138,14 @@ struct nh_context {
 };
 
 namespace nh {
-// Layouts applied by the 4-lanes-per-atom bond kernels (nh_hv_sk.h): the
-// stored SK records and the matrix-free one.
+// Layouts applied bond by bond from records (nh_hv_sk.h): the stored SK records
+// and the matrix-free one.
 inline bool sk_like(const nh_context *c) {
   return c->layout == NH_LAYOUT_SK || c->layout == NH_LAYOUT_MATRIX_FREE;
 }
-// Lanczos vectors stored in FP32 (FP32 SK or matrix-free products with the
-// LDS gather only).  Default on (measured on a 786,520-atom dot, FP32 SK
-// products: the same 7,901 steps to the same eigenvalues, fused H*v 0.208
-// / 0.228 ms in the two passes against 0.229 / 0.301 ms, FP32 stage 4.73 s
-// against 6.23 s, with a separate update kernel)
+// Lanczos vectors stored in FP32 (FP32 SK or matrix-free products).  Default on
+// (786,520-atom dot, mixed solve: 3.87 s and 7,976 FP32 steps, 5.88 s and 8,001
+// with FP64 vectors, to the same eigenvalues)
 inline bool lz_fp32_vectors(const nh_context *c) {
   return sk_like(c) && c->precision == NH_PREC_FP32 && c->hv_staged != 0 &&
          c->lz_vectors != 0;

@@ -19,7 +19,7 @@
 // kz (relative to the table in 80 bits, directions 0.002 / 0.01 / 0.03 off
 // (111): 1.4e-15 / 7.0e-15 / 2.1e-14 without, 2.0e-16 with them; the table in
 // FP64 1.5e-16).
-// That is about 95 multiply-adds per vector and about 40 operations per bond for
+// That is 93 operations per vector and about 45 per bond for
 // the scaled vectors, against 100 and about 250 for forming T.
 //
 // Every matrix element is a sum of products of two numbers that are
