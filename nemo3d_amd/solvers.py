@@ -34,7 +34,8 @@ def eigensolve_lanczos(H, num_vb=4, num_cb=4, erange_vb=(-0.6, 0.2),
     with the same start (the result's "alpha"/"beta" with
     return_tridiag=True, or ndio.read_tridiagonal of a saved one): no
     eigenvalue pass, only the analysis and the eigenvector pass
-    (restoreState, lanczos.c:1905-1960)."""
+    (restoreState, lanczos.c:1905-1960); where the eigenvectors' residuals
+    show that it does not retrace that run, the solve without it."""
     lib = native.load()
     o = native.NHLanczosOpts()
     o.max_iter = int(max_iter)
